@@ -53,9 +53,14 @@ constexpr int kShortRow = 32;    // bottom-up: lane-sequential scan up to this l
 constexpr uint32_t kNoNbr = 0xFFFFFFFFu;
 
 // counters: vertices found; the root (new id); head words (k_td_head_size);
-// frontier edges of the next level, summed by a small top-down level
+// frontier edges of the next level, summed by a small top-down level.  The
+// found and next-edge sums of whole grids go to the stripes behind them
+// (words S_FOUND and S_NEXT_E of each); k_publish adds the stripes up.
+// C_FOUND itself only hands out queue positions in a small top-down level.
 enum { C_FOUND = 0, C_AUX = 1, C_HEAD = 2, C_NEXT_E = 3, C_NUM = 4 };
-
+enum { S_FOUND = 0, S_NEXT_E = 1 };
+constexpr int kStripeBase = 8;  // words: the stripes start on a 64-byte line of their own
+constexpr int kBfsCounters = kStripeBase + kStripes * kStripeWords;
 
 __global__ void __launch_bounds__(kBlock) k_bfs_init(uint8_t* __restrict__ level, uint64_t* __restrict__ vis,
                                                      int64_t rows, int64_t words) {
@@ -74,10 +79,11 @@ __global__ void k_bfs_root(const uint32_t* __restrict__ old2new, int64_t root_or
                            uint8_t* __restrict__ level, uint32_t* __restrict__ parent,
                            uint64_t* __restrict__ vis, uint32_t* __restrict__ queue,
                            unsigned long long* __restrict__ counters) {
-  const uint32_t r = old2new[root_orig];
   // the first level's counters start at zero; k_publish clears them after
   // every later level
-  for (int i = 0; i < C_NUM; ++i) counters[i] = 0;
+  for (int i = threadIdx.x; i < kBfsCounters; i += blockDim.x) counters[i] = 0;
+  if (threadIdx.x != 0) return;
+  const uint32_t r = old2new[root_orig];
   if ((int64_t)r < rows) {
     level[r] = 0;
     parent[r] = r;
@@ -185,7 +191,7 @@ __global__ void __launch_bounds__(kBlock) k_td_expand(
   }
   // the next level's frontier edges, so that the host can skip the launches
   // of the other form there
-  if (!kBulk) block_add(next_e, counters + C_NEXT_E);
+  if (!kBulk) block_add(next_e, stripe_of(counters + kStripeBase, S_NEXT_E));
 }
 
 // --- piece-ordered hub levels ---------------------------------------------
@@ -673,7 +679,7 @@ __global__ void __launch_bounds__(kBlock) k_td_finish(const uint8_t* __restrict_
       total += __popcll(m);
     }
   }
-  block_add(total, counters + C_FOUND);
+  block_add(total, stripe_of(counters + kStripeBase, S_FOUND));
 }
 
 // Bottom-up level.  A wave reads `span` bitmap words at a time (one
@@ -736,7 +742,7 @@ __global__ void __launch_bounds__(kBlock) k_bu(
       found_total += __popcll(fm0) + __popcll(fm1);  // identical in every lane
     }
   }
-  block_add(lane == 0 ? found_total : 0, counters + C_FOUND);
+  block_add(lane == 0 ? found_total : 0, stripe_of(counters + kStripeBase, S_FOUND));
 }
 
 // Frontier bitmap -> frontier queue in ascending vertex order: an exclusive
@@ -989,12 +995,24 @@ __global__ void __launch_bounds__(kFuseThreads) k_td_fused(
 // level's frontier edge count after a top-down level) are published straight
 // into coherent host memory, each tagged with the level's sequence number, so
 // the host need not wait for a copy and a stream synchronisation.
-__global__ void k_publish(unsigned long long* __restrict__ counters, const uint64_t* __restrict__ prefix,
-                          int64_t nf, int forward, Published* pub, uint64_t seq) {
-  for (int i = 0; i < C_NUM; ++i) {
-    const uint64_t v = (forward && i == 1) ? prefix[nf] : (uint64_t)counters[i];
-    counters[i] = 0;  // ready for the next level, with no fill launched before it
-    publish(pub + i, v, seq);
+// One wave: lane i takes stripe i.
+static_assert(kStripes == 64, "k_publish sums one stripe per lane of a wave");
+__global__ void __launch_bounds__(64) k_publish(unsigned long long* __restrict__ counters,
+                                                const uint64_t* __restrict__ prefix, int64_t nf, int forward,
+                                                Published* pub, uint64_t seq) {
+  const int t = threadIdx.x;
+  unsigned long long* mine = counters + kStripeBase + t * kStripeWords;
+  const uint64_t found = wave_sum(mine[S_FOUND]);
+  const uint64_t next_e = wave_sum(mine[S_NEXT_E]);
+  // ready for the next level, with no fill launched before it
+  mine[S_FOUND] = 0;
+  mine[S_NEXT_E] = 0;
+  if (t < C_NUM) {
+    uint64_t v = (forward && t == C_AUX) ? prefix[nf] : (uint64_t)counters[t];
+    if (t == C_FOUND) v += found;
+    if (t == C_NEXT_E) v += next_e;
+    counters[t] = 0;
+    publish(pub + t, v, seq);
   }
 }
 
@@ -1048,7 +1066,7 @@ void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   b.chunk_rows.alloc(2 * ((uint64_t)g.nnz / kEpb + 2));
   const size_t scan_n = (size_t)rows + 1;
   b.scan_tmp.alloc(scan_tmp_elems(scan_n));
-  b.counters.alloc(C_NUM);
+  b.counters.alloc(kBfsCounters);
   bfs_tuning_buffers(ctx, b, s);
   G5_HIP(hipHostMalloc((void**)&b.h_counters, C_NUM * sizeof(uint64_t), hipHostMallocDefault));
   b.pub.alloc(C_NUM);
@@ -1102,7 +1120,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   hipLaunchKernelGGL(k_bfs_init, dim3(grid_of(rows, kBlock, 4096)), dim3(kBlock), 0, s, b.level.p,
                      b.vis[0].p, rows, b.words);
   G5_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_bfs_root, dim3(1), dim3(1), 0, s, g.old2new.p, root, rows, b.level.p,
+  hipLaunchKernelGGL(k_bfs_root, dim3(1), dim3(kBlock), 0, s, g.old2new.p, root, rows, b.level.p,
                      b.parent.p, b.vis[0].p, b.queue[0].p, cnt);
   G5_HIP(hipGetLastError());
 
@@ -1323,7 +1341,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     G5_HIP(hipGetLastError());
     G5_HIP(hipEventRecord(b.lev_end[lvl], s));
     ++b.pub_seq;
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, cnt, b.prefix.p, nf, td ? 1 : 0, b.pub.d,
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, td ? 1 : 0, b.pub.d,
                        b.pub_seq);
     G5_HIP(hipGetLastError());
     wait_published(b, s);
