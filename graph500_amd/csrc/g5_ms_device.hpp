@@ -13,6 +13,30 @@ constexpr int kMsShortRow = 32;
 
 enum { M_LIVE = 0, M_PAIRS = 1, M_NZ = 2, M_FDEG = 3, M_NUM = 8 };
 
+// A level's counters: M_NUM level counters, a list count, 64 per-lane counts
+// and 64 per-lane degree sums, one more list count (serving).  Per-level
+// launches keep kMsStripes copies of them, kMsStride words apart, and a
+// workgroup adds to the copy its id picks (see kStripes in g5_frontier.hpp
+// for what one contended word costs: 8,192 workgroups adding per-lane sums
+// to one copy queued 1 M atomics on 16 lines); the publishing kernel sums
+// the copies.  The list counts hand out positions and live in copy 0 alone.
+constexpr int kMsStripes = 32;
+constexpr int kMsStride = 144;
+constexpr int kMsLanes = M_NUM + 1;  // first of the 128 per-lane words
+__device__ __forceinline__ unsigned long long* ms_stripe(unsigned long long* c) {
+  return c + (blockIdx.x % kMsStripes) * kMsStride;
+}
+// Counter t summed (M_LIVE: ORed) over the copies.
+__device__ __forceinline__ uint64_t ms_stripe_total(const unsigned long long* c, int t) {
+  uint64_t v = 0;
+#pragma unroll 8
+  for (int i = 0; i < kMsStripes; ++i) {
+    const uint64_t x = c[i * kMsStride + t];
+    v = t == M_LIVE ? v | x : v + x;
+  }
+  return v;
+}
+
 __device__ __forceinline__ uint64_t wave_or(uint64_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);

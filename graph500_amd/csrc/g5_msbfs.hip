@@ -29,7 +29,9 @@
 
 namespace g5 {
 
-constexpr int kMsCounters = M_NUM + 1 + 128;  // level counters, a list count, per-lane counts and degree sums
+constexpr int kMsCounters = kMsLanes + 128;  // level counters, a list count, per-lane counts and degree sums
+constexpr size_t kMsCounterWords = (size_t)kMsStripes * kMsStride;
+static_assert(kMsCounters <= kMsStride, "a counter copy holds every counter");
 
 __global__ void __launch_bounds__(kBlock) k_ms_clear(uint64_t* __restrict__ a, uint64_t* __restrict__ b,
                                                      int64_t n) {
@@ -150,10 +152,11 @@ __global__ void __launch_bounds__(kBlock) k_ms_finish_list(uint64_t* __restrict_
                                                            int lane_stats) {
   const uint64_t n = *list_count;
   if (lane_stats) {
-    const LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
-    ms_finish_list_body(seen, next, nz_next, offsets, list, n, c, blockIdx.x, gridDim.x, epi);
+    LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
+    epi.lane_nq = ms_stripe(epi.lane_nq);
+    ms_finish_list_body(seen, next, nz_next, offsets, list, n, ms_stripe(c), blockIdx.x, gridDim.x, epi);
   } else {
-    ms_finish_list_body(seen, next, nz_next, offsets, list, n, c, blockIdx.x, gridDim.x);
+    ms_finish_list_body(seen, next, nz_next, offsets, list, n, ms_stripe(c), blockIdx.x, gridDim.x);
   }
 }
 
@@ -161,7 +164,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_finish(uint64_t* __restrict__ see
                                                       uint64_t* __restrict__ nz_next,
                                                       const uint64_t* __restrict__ offsets, int64_t rows,
                                                       unsigned long long* __restrict__ c) {
-  ms_finish_body(seen, next, nz_next, offsets, rows, c, blockIdx.x, gridDim.x);
+  ms_finish_body(seen, next, nz_next, offsets, rows, ms_stripe(c), blockIdx.x, gridDim.x);
 }
 
 template <int kU, int kW>
@@ -175,8 +178,8 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull(uint64_t* __restrict__ seen,
                                                     const uint64_t* __restrict__ compact, uint32_t filter_from,
                                                     unsigned long long* __restrict__ c, uint64_t* __restrict__ miss) {
   const FrontView fv{front, nz_front, pack, compact, mode, filter_from};
-  ms_pull_body<NoEpilogue, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, c, blockIdx.x,
-                                   gridDim.x, ~UINT64_C(0), NoEpilogue(), false, miss);
+  ms_pull_body<NoEpilogue, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+                                   blockIdx.x, gridDim.x, ~UINT64_C(0), NoEpilogue(), false, miss);
 }
 
 // The pull of a tail level over the listed vertices (see ms_pull_list_body).
@@ -190,8 +193,8 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull_list(uint64_t* __restrict__ 
                                                          uint64_t* __restrict__ miss,
                                                          unsigned long long* __restrict__ c) {
   const FrontView fv{front, nullptr, nullptr, nullptr, kFrontPlain, 0};
-  ms_pull_list_body(seen, fv, next, nz_next, first_nbr, offsets, cols, list, *list_count, live_in, miss, c,
-                    blockIdx.x, gridDim.x);
+  ms_pull_list_body(seen, fv, next, nz_next, first_nbr, offsets, cols, list, *list_count, live_in, miss,
+                    ms_stripe(c), blockIdx.x, gridDim.x);
 }
 
 // --- per-root directions (lane_rule 1) ---
@@ -199,8 +202,9 @@ __global__ void __launch_bounds__(kBlock) k_ms_finish_lanes(uint64_t* __restrict
                                                             uint64_t* __restrict__ nz_next,
                                                             const uint64_t* __restrict__ offsets, int64_t rows,
                                                             unsigned long long* __restrict__ c, LaneEpi epi_in) {
-  const LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
-  ms_finish_body(seen, next, nz_next, offsets, rows, c, blockIdx.x, gridDim.x, ~UINT64_C(0), epi);
+  LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
+  epi.lane_nq = ms_stripe(epi.lane_nq);
+  ms_finish_body(seen, next, nz_next, offsets, rows, ms_stripe(c), blockIdx.x, gridDim.x, ~UINT64_C(0), epi);
 }
 
 // Pull for the lanes in live_in; with merge, next already holds this level's
@@ -214,10 +218,11 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull_lanes(uint64_t* __restrict__
                                                           const uint32_t* __restrict__ cols, int64_t rows,
                                                           uint64_t live_in, int filter, int merge,
                                                           unsigned long long* __restrict__ c, LaneEpi epi_in) {
-  const LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
+  LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
+  epi.lane_nq = ms_stripe(epi.lane_nq);
   const FrontView fv{front, nz_front, nullptr, nullptr, filter ? kFrontFilter : kFrontPlain, 0};
-  ms_pull_body<LaneEpi, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, c, blockIdx.x,
-                                gridDim.x, ~UINT64_C(0), epi, merge != 0);
+  ms_pull_body<LaneEpi, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+                                blockIdx.x, gridDim.x, ~UINT64_C(0), epi, merge != 0);
 }
 
 // One bit per vertex whose frontier word has one of `lanes`.
@@ -276,18 +281,14 @@ __global__ void __launch_bounds__(kBlock) k_ms_sweep(const uint32_t* __restrict_
 // vertex) pairs are unreached.
 constexpr double kListBelow = 16.0;
 
+// The listed pulls run on at most this many workgroups: their list is far
+// shorter than its bound, and workgroups that find nothing to do still cost
+// (SCALE 28, per listed level: 0.070 ms on up to 4,096, 0.093 on 16,384).
+constexpr int64_t kListGrid = 2048;
+
 // A push level lists the vertices it touches when its frontier edges times
 // this are fewer than the rows (the touched vertices are at most the edges).
 constexpr double kTouchBelow = 8.0;
-
-// Pull levels with fewer than 1/kLightBelow of the (root, vertex) pairs
-// unreached run on at most kLightGrid workgroups: their pass over every
-// vertex finds little to probe, and at SCALE 28 it took 0.48 ms on 2,048
-// workgroups against 0.86 ms on 16,384 and 1.59 ms on 32,768, while the
-// mixed level gains from the larger grids (26.2 ms on 2,048, 24.6 ms on
-// 32,768).
-constexpr double kLightBelow = 8.0;
-constexpr int64_t kLightGrid = 2048;
 
 constexpr unsigned kBarGroup = 16;
 constexpr unsigned kBarMaxGroups = 1024;
@@ -535,7 +536,7 @@ void ms_prepare(g5_ctx* ctx) {
   m.prefix.alloc(rows + 1);
   m.chunk_rows.alloc(2 * ((uint64_t)g.nnz / kEpb + 2));
   m.scan_tmp.alloc(scan_tmp_elems(rows + 1));
-  m.counters.alloc(kMsCounters);
+  m.counters.alloc(kMsCounterWords);
   m.roots.alloc(64);
   m.frp.alloc(G5_MAX_LEVELS);
   if (g.reorder_mode != 0 && g.nnz > 0) {
@@ -590,9 +591,13 @@ void ms_prepare(g5_ctx* ctx) {
 // fill starts a level).
 __global__ void k_ms_publish(unsigned long long* __restrict__ c, int n_pub, Published* __restrict__ p,
                              uint64_t seq) {
-  for (int t = threadIdx.x; t < kMsCounters; t += blockDim.x) {
-    const uint64_t v = c[t];
-    c[t] = 0;
+  // one thread per counter; counters past the published ones (the per-lane
+  // sums of a level that kept none) were not written, but for the list count
+  const int n = n_pub > M_NUM ? n_pub : M_NUM + 1;
+  for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    const uint64_t v = ms_stripe_total(c, t);
+#pragma unroll 8
+    for (int i = 0; i < kMsStripes; ++i) c[i * kMsStride + t] = 0;
     if (t < n_pub) publish(p + t, v, seq);
   }
 }
@@ -677,7 +682,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
   m.level_masks = lanes_mode;
   double lane_fd[64] = {}, lane_vd[64] = {};
   uint64_t pulled = 0;  // roots that have pulled: they pull from then on
-  const uint64_t* h_lane = m.h_counters + M_NUM + 1;
+  const uint64_t* h_lane = m.h_counters + kMsLanes;
   unsigned* d_list_count = (unsigned*)(cnt + M_NUM);
   bool have_miss = false;  // m.miss holds the vertices still missing a live root
   int l = l0 - 1;
@@ -721,7 +726,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     m.level_pull[l] = push ? 0 : (lanes_mode ? bu : live);
     G5_HIP(hipEventRecord(m.lev_begin[l], s));
     // statistics for the roots still choosing (a root that pulled keeps pulling)
-    const LaneEpi lepi{cnt + M_NUM + 1, g.offsets.p, lanes_mode ? td : live};
+    const LaneEpi lepi{cnt + kMsLanes, g.offsets.p, lanes_mode ? td : live};
     if (lanes_mode && td && bu) {
       // the pushing roots first, then the pull of the others, merging the
       // pushed lanes
@@ -854,8 +859,6 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       // next pull takes only those, listed by a scan of the bits (after
       // clearing its frontier array, which must hold zeros elsewhere).
       const double unreached = std::max(0.0, total_pairs - reached);
-      const int64_t grid_cap =
-          unreached * kLightBelow < total_pairs ? std::min<int64_t>(m.pull_grid, kLightGrid) : m.pull_grid;
       if (have_miss && mode == kFrontPlain) {
         const uint64_t ub = (uint64_t)std::min<double>((double)rows, unreached);  // list length bound
         m.ulist.alloc(std::max<uint64_t>(ub, 1));
@@ -865,7 +868,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         ms_clear_frontier(m, l, rows, s, marked);
         G5_HIP(hipMemsetAsync(nz_next, 0, words * 8, s));
         G5_HIP(hipMemsetAsync(m.miss.p, 0, words * 8, s));
-        hipLaunchKernelGGL(k_ms_pull_list, dim3(grid_of((int64_t)ub, kBlock, grid_cap)), dim3(kBlock), 0, s,
+        hipLaunchKernelGGL(k_ms_pull_list, dim3(grid_of((int64_t)ub, kBlock, std::min(m.pull_grid, kListGrid))), dim3(kBlock), 0, s,
                            m.seen.p, front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, m.ulist.p,
                            m.ulist_count.p, live, m.miss.p, cnt);
         list_level = true;
@@ -875,7 +878,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         // the pull writes every word of the level's frontier array (clearing
         // its old words first, one store per marked vertex, so that the pull
         // could skip its zero words, measured no faster)
-        hipLaunchKernelGGL(kp, dim3(grid_of(words, kBlock / 64, grid_cap)), dim3(kBlock), 0, s, m.seen.p, front,
+        hipLaunchKernelGGL(kp, dim3(grid_of(words, kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
                            nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, rows, live, mode,
                            m.pack.p, m.compact.p, filter_from, cnt, mark ? m.miss.p : nullptr);
         list_level = mark;
@@ -1098,7 +1101,7 @@ static void ms_run_persistent(g5_ctx* ctx, const int64_t* roots, int nroots) {
     // which reads the last level's nonzero bitmap from its per-level slot
     const int64_t words = (g.n_rows + 63) / 64;
     G5_HIP(hipMemcpyAsync(ms_marks(m, done, words), m.nz[done & 1].p, words * 8, hipMemcpyDeviceToDevice, s));
-    G5_HIP(hipMemsetAsync(m.counters.p, 0, kMsCounters * 8, s));  // the host levels expect them clear
+    G5_HIP(hipMemsetAsync(m.counters.p, 0, kMsCounterWords * 8, s));  // the host levels expect them clear
     ms_host_levels(ctx, done + 1, last[M_LIVE], last[M_NZ], last[M_FDEG], reached, roots_live);
   }
   (void)g;
@@ -1131,7 +1134,7 @@ void ms_run(g5_ctx* ctx, const int64_t* roots, int nroots) {
     uint64_t* nz0 = ms_marks(m, 0, words);
     G5_HIP(hipMemcpyAsync(m.roots.p, roots, nroots * sizeof(int64_t), hipMemcpyHostToDevice, s));
     G5_HIP(hipEventRecord(m.ev0, s));
-    G5_HIP(hipMemsetAsync(m.counters.p, 0, kMsCounters * 8, s));  // then cleared by every publish
+    G5_HIP(hipMemsetAsync(m.counters.p, 0, kMsCounterWords * 8, s));  // then cleared by every publish
     G5_HIP(hipMemsetAsync(m.seen.p, 0, rows * 8, s));
     const bool marked = m.fr_exact[0] != 0;
     m.fr_exact[0] = 0;

@@ -112,7 +112,7 @@ struct ServeLocal {
       atomicAdd(&lds()[64 + me], (unsigned long long)d_acc);
     }
     __syncthreads();
-    if (threadIdx.x < 128 && lds()[threadIdx.x]) atomicAdd(p.lane_nq + threadIdx.x, lds()[threadIdx.x]);
+    if (threadIdx.x < 128 && lds()[threadIdx.x]) atomicAdd(ms_stripe(p.lane_nq) + threadIdx.x, lds()[threadIdx.x]);
   }
 };
 
@@ -124,14 +124,15 @@ struct ServeLocal {
 // commands on the stream.
 constexpr int kSvTeps = M_NUM + 128;
 constexpr int kSvPub = kSvTeps + 64;
-constexpr int kSvTouch = M_NUM + 1 + 128;  // device counter slot of a listed push's touched vertices
-constexpr int kSvCounters = kSvTouch + 1;
+constexpr int kSvTouch = kMsLanes + 128;  // device counter slot of a listed push's touched vertices
+constexpr size_t kSvCounterWords = (size_t)kMsStripes * kMsStride;
+static_assert(kSvTouch < kMsStride, "a counter copy holds every counter");
 __global__ void k_sv_publish(const unsigned long long* __restrict__ c, const unsigned long long* __restrict__ tacc,
                              Published* __restrict__ p, uint64_t seq) {
   const int t = threadIdx.x;
-  if (t < M_NUM) publish(p + t, c[t], seq);
-  if (t < 128) publish(p + M_NUM + t, c[M_NUM + 1 + t], seq);
-  if (t < 64) publish(p + kSvTeps + t, tacc[t], seq);
+  // [0, M_NUM) level counters, [M_NUM, kSvTeps) per-lane sums, then the weight sums
+  if (t < kSvTeps) publish(p + t, ms_stripe_total(c, t < M_NUM ? t : kMsLanes + t - M_NUM), seq);
+  else if (t < kSvPub) publish(p + t, tacc[t - kSvTeps], seq);
 }
 
 struct ServeRoots {
@@ -152,8 +153,8 @@ __global__ void __launch_bounds__(kBlock) k_sv_pull(uint64_t* __restrict__ seen,
   // two probes per step on a short row, one per lane and step on a long row:
   // the batch's fastest pull unrolling at SCALE 28 (fewer probes past the
   // point where a vertex's searches are all found)
-  ms_pull_body<ServeLocal, 2, 1>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, c, blockIdx.x,
-                                 gridDim.x, keep, el, merge != 0);
+  ms_pull_body<ServeLocal, 2, 1>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+                                 blockIdx.x, gridDim.x, keep, el, merge != 0);
 }
 
 __global__ void __launch_bounds__(kBlock) k_sv_finish(uint64_t* __restrict__ seen, uint64_t* __restrict__ next,
@@ -162,7 +163,7 @@ __global__ void __launch_bounds__(kBlock) k_sv_finish(uint64_t* __restrict__ see
                                                       unsigned long long* __restrict__ c, uint64_t keep,
                                                       ServeEpi epi) {
   const ServeLocal el{epi};
-  ms_finish_body(seen, next, nz_next, offsets, rows, c, blockIdx.x, gridDim.x, keep, el);
+  ms_finish_body(seen, next, nz_next, offsets, rows, ms_stripe(c), blockIdx.x, gridDim.x, keep, el);
 }
 
 __global__ void __launch_bounds__(kBlock) k_sv_collect(const uint32_t* __restrict__ chunk_rows, uint64_t nchunks,
@@ -206,7 +207,8 @@ __global__ void __launch_bounds__(kBlock) k_sv_finish_list(uint64_t* __restrict_
                                                            const unsigned long long* __restrict__ touch_count,
                                                            unsigned long long* __restrict__ c, ServeEpi epi) {
   const ServeLocal el{epi};
-  ms_finish_list_body(seen, next, nz_next, offsets, touch, (uint64_t)*touch_count, c, blockIdx.x, gridDim.x, el);
+  ms_finish_list_body(seen, next, nz_next, offsets, touch, (uint64_t)*touch_count, ms_stripe(c), blockIdx.x,
+                      gridDim.x, el);
 }
 
 // Zeroes the frontier words marked in a nonzero bitmap (one bitmap word per
@@ -385,7 +387,6 @@ struct Engine {
   uint64_t pulled = 0;  // lane rule 3: searches that have pulled keep pulling
   bool lane_growing[64];
   int64_t lane_prev_nq[64];
-  int lane_pulls[64];    // pull levels each search has taken
   int64_t lane_visited[64];
   double lane_vdeg[64];  // row lengths of the vertices each search has reached
   uint64_t active = 0, cooling = 0;
@@ -474,7 +475,7 @@ static void sv_setup_engine(g5_server* srv, Engine& e, g5_ctx* ctx) {
   e.nchunks = ((uint64_t)e.nnz + kSweepEpb - 1) / kSweepEpb;
   e.chunk_rows.alloc(2 * e.nchunks + 2);
   e.chunk_list.alloc(e.nchunks + 1);
-  e.cnt.alloc(kSvCounters);
+  e.cnt.alloc(kSvCounterWords);
   e.touch.alloc(e.rows ? e.rows : 1);
   e.tacc.alloc(64);
   G5_HIP(hipMemsetAsync(e.tacc.p, 0, 64 * 8, e.s));
@@ -500,7 +501,6 @@ static void sv_setup_engine(g5_server* srv, Engine& e, g5_ctx* ctx) {
   for (int r = 0; r < 64; ++r) {
     e.lane_req[r] = -1;
     e.lane_l0[r] = 0;
-    e.lane_pulls[r] = 0;
     e.teps_req[r] = -1;
   }
   G5_HIP(hipStreamSynchronize(s));
@@ -644,7 +644,6 @@ static uint64_t sv_admit(g5_server* srv, Engine& e, double t) {
     e.lane_fwd[r] = true;
     e.pulled &= ~(UINT64_C(1) << r);
     e.lane_growing[r] = true;
-    e.lane_pulls[r] = 0;
     e.lane_prev_nq[r] = 0;
     e.lane_visited[r] = 1;
     e.lane_vdeg[r] = 0;
@@ -701,7 +700,7 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
     if (e.lane_fwd[r]) fwd |= UINT64_C(1) << r;
   const uint64_t td = e.active & fwd, bu = e.active & ~fwd;
   unsigned long long* c = e.cnt.p;
-  epi.lane_nq = c + M_NUM + 1;
+  epi.lane_nq = c + kMsLanes;
   epi.offsets = g.offsets.p;
   epi.nz_sel = e.nzs[cur ^ 1].p;
   epi.sel = td;
@@ -716,7 +715,7 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
   if (reselect)
     hipLaunchKernelGGL(k_sv_select, dim3(grid_of(e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, front, e.rows, td,
                        e.nzs[cur].p);
-  G5_HIP(hipMemsetAsync(c, 0, kSvCounters * 8, s));
+  G5_HIP(hipMemsetAsync(c, 0, kSvCounterWords * 8, s));
   ++e.st.levels;
   if (td && bu) ++e.st.mixed_levels; else if (td) ++e.st.push_levels; else ++e.st.pull_levels;
   e.st.lane_levels += __builtin_popcountll(e.active);
@@ -751,17 +750,7 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
     hipLaunchKernelGGL(k_sv_finish_list, dim3(grid_of(e.rows / 8 + 1, kBlock, 2048)), dim3(kBlock), 0, s, e.seen.p,
                        next, nz_next, g.offsets.p, e.touch.p, (const unsigned long long*)(c + kSvTouch), c, epi);
   } else if (bu) {
-    // a pull of searches that have each pulled twice before finds little to
-    // probe (their frontiers have passed the hubs): its pass over every
-    // vertex runs on a smaller grid, as the batch's light levels do
-    bool light = true;
-    for (uint64_t x = bu; x; x &= x - 1) {
-      const int r = __builtin_ctzll(x);
-      light = light && e.lane_pulls[r] >= 2;
-      ++e.lane_pulls[r];
-    }
-    hipLaunchKernelGGL(k_sv_pull, dim3(grid_of(e.words, kBlock / 64, light ? 2048 : 8192)), dim3(kBlock), 0, s,
-                       e.seen.p, front,
+    hipLaunchKernelGGL(k_sv_pull, dim3(grid_of(e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, e.seen.p, front,
                        nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, e.rows, bu,
                        srv->cfg.pull_filter, c, keep, td ? 1 : 0, epi);
   } else {
