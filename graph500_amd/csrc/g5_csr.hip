@@ -11,14 +11,16 @@
 //   isolateFirstEdge     first (smallest new id) neighbour kept apart  (:845-879)
 //   computeNumVertices   n_active = vertices with an edge              (:1444-1464)
 //
-// Device pipeline: OR-reduce -> atomic degree count -> stable radix sort of
-// (degree key, id) -> one uint64 key (new_src << S | new_tgt) per directed
-// entry -> LSD radix sort over 2S bits -> one scan that drops duplicates,
-// writes columns and row offsets.  The tuples themselves are never re-sorted.
+// Device pipeline: OR-reduce -> directed entries grouped by vertex range ->
+// degrees counted in LDS per range -> stable radix sort of (degree key, id) ->
+// entries relabelled range by range, grouped by row ranges, then by estimated
+// position, sorted and deduplicated in LDS (g5_entries.hpp).  The tuples
+// themselves are never re-sorted.
 #include "g5_ctx.hpp"
+#include "g5_entries.hpp"
 #include "g5_prims.hpp"
 
-#include <chrono>
+#include <algorithm>
 
 namespace g5 {
 
@@ -29,32 +31,26 @@ __device__ __forceinline__ uint64_t tuple_v1(const g5_packed_edge& e) {
   return (uint64_t)e.v1_low | ((uint64_t)(e.high >> 16) << 32);
 }
 
+// One atomic per workgroup, and none once the bits are there: a wave's OR per
+// wave of a 65,536-workgroup grid spent 3 ms on that one word (12 ns each).
 __global__ void __launch_bounds__(kBlock) k_or_ids(const g5_packed_edge* __restrict__ e, int64_t m,
                                                    unsigned long long* out) {
+  __shared__ uint64_t s_or[kBlock / 64];
   uint64_t acc = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * kBlock) {
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+#pragma unroll 4
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < m; i += stride) {
     const g5_packed_edge t = e[i];
     acc |= tuple_v0(t) | tuple_v1(t);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) acc |= __shfl_xor(acc, o, 64);
-  if ((threadIdx.x & 63) == 0 && acc) atomicOr(out, (unsigned long long)acc);
-}
-
-__global__ void __launch_bounds__(kBlock) k_degree(const g5_packed_edge* __restrict__ e, int64_t m,
-                                                   uint32_t* __restrict__ deg,
-                                                   uint32_t* __restrict__ loops) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * kBlock) {
-    const g5_packed_edge t = e[i];
-    const uint64_t a = tuple_v0(t), b = tuple_v1(t);
-    if (a == b) {
-      atomicAdd(&loops[a], 1u);
-    } else {
-      atomicAdd(&deg[a], 1u);
-      atomicAdd(&deg[b], 1u);
-    }
+  if ((threadIdx.x & 63) == 0) s_or[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; ++w) acc |= s_or[w];
+    if (acc & ~__hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicOr(out, (unsigned long long)acc);
   }
 }
 
@@ -69,52 +65,29 @@ __global__ void k_order_keys(const uint32_t* __restrict__ deg, int64_t n, uint32
   }
 }
 
-struct NonZeroU32 {
-  const uint32_t* p;
-  __device__ uint64_t operator()(size_t i) const { return p[i] ? 1 : 0; }
-};
-
 __global__ void k_iota(int64_t n, uint32_t* __restrict__ out) {
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
        v += (int64_t)gridDim.x * blockDim.x)
     out[v] = (uint32_t)v;
 }
 
-__global__ void k_invert(const uint32_t* __restrict__ new2old, int64_t n, uint32_t* __restrict__ old2new) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-       v += (int64_t)gridDim.x * blockDim.x)
-    old2new[new2old[v]] = (uint32_t)v;
-}
-
-__global__ void k_weights(const uint32_t* __restrict__ new2old, const uint32_t* __restrict__ deg,
-                          const uint32_t* __restrict__ loops, int64_t rows, uint32_t* __restrict__ w) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < rows;
+// Degree (duplicates counted) and tuple weight (degree + 2 * loops) per row.
+__global__ void k_row_info(const uint32_t* __restrict__ new2old, const uint32_t* __restrict__ deg,
+                           const uint32_t* __restrict__ loops, int64_t rows, uint32_t* __restrict__ row_deg,
+                           uint32_t* __restrict__ w) {
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= rows;
        v += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t o = new2old[v];
-    w[v] = deg[o] + 2u * loops[o];
-  }
-}
-
-// One key per directed entry: (new src << S) | new tgt; loops get an all-ones
-// key that sorts after every real key and is cut off by the count.
-__global__ void __launch_bounds__(kBlock) k_pair_keys(const g5_packed_edge* __restrict__ e, int64_t m,
-                                                      const uint32_t* __restrict__ old2new, int scale,
-                                                      uint64_t* __restrict__ keys) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * kBlock) {
-    const g5_packed_edge t = e[i];
-    const uint64_t a = tuple_v0(t), b = tuple_v1(t);
-    uint64_t k0 = ~UINT64_C(0), k1 = ~UINT64_C(0);
-    if (a != b) {
-      const uint64_t na = old2new[a], nb = old2new[b];
-      k0 = (na << scale) | nb;
-      k1 = (nb << scale) | na;
+    if (v == rows) {
+      row_deg[v] = 0;  // the prefix's last element, the total
+      continue;
     }
-    keys[2 * i] = k0;
-    keys[2 * i + 1] = k1;
+    const uint32_t o = new2old[v], d = deg[o];
+    row_deg[v] = d;
+    w[v] = loops ? d + 2u * loops[o] : d;
   }
 }
 
+// --- sorted entries to rows, for graphs whose entries were sorted by radix ---
 struct UniqueFlag {
   const uint64_t* keys;
   size_t nvalid;
@@ -178,6 +151,47 @@ static unsigned grid_for(int64_t n, int64_t per_block = kBlock) {
   return (unsigned)(b > 0 ? b : 1);
 }
 
+// Ranges of vertex ids for the degree counts and the relabelling: up to
+// kPartMax of at least 64 vertices; at least 256 where the ids allow, so that
+// small graphs fill the chip, and beyond that as many as keep a range within
+// one workgroup's LDS counters (kDegVerts).
+static int range_bits(int scale) { return std::min(10, std::max(std::min(8, std::max(scale - 6, 0)), scale - 15)); }
+
+// From here on both endpoints of an entry are relabelled in one pass by
+// lookups of old2new wherever they fall; a larger table is looked up one side
+// at a time with the entries grouped by that side, one more pass over the
+// entries but no lookup past the L2 (4 MB per XCD).  Random lookups of a
+// 128 MB table run at 55 G/s, 20 ms per 10^9, the pass takes 5 ms; in a table
+// that fits the L2 they run at the pass's own rate.
+constexpr int kRelabelBothScale = 20;
+
+// Workgroups of a pass over the tuples that ends with atomics on shared words
+// (12 ns each, one after another).
+constexpr unsigned kTupleGrid = 1024;
+
+// Positions per sub-bucket, as a shift: 2^11 as long as two partitions by
+// about 512 reach it, 2^12 beyond (2^31 entries on).
+static int sub_shift_for(uint64_t entries) { return entries >> 31 ? 12 : 11; }
+
+// L1 buckets: stretches of 2^wshift positions, at most 512 of them, or
+// kPartMax once a sub-bucket has 2^12 positions.
+static int l1_shift(uint64_t entries, int sub) {
+  const uint64_t most = sub == 11 ? 512 : kPartMax;
+  int w = sub;
+  while ((entries - 1) >> w >= most) ++w;
+  return w;
+}
+
+// Persistent grid of the partition passes: one workgroup per CU.
+static unsigned part_grid(int64_t tiles) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 256)); }
+
+template <class Src>
+static void partition(const Src& src, unsigned long long* cursor, uint64_t* out, hipStream_t s) {
+  const int64_t tiles = src.tiles();
+  hipLaunchKernelGGL(k_partition<Src>, dim3(part_grid(tiles)), dim3(kPartThreads), 0, s, src, tiles, cursor, out);
+  G5_HIP(hipGetLastError());
+}
+
 void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   G5_CHECK(mode >= 0 && mode <= 2, "g5_construct: reorder_mode must be 0, 1 or 2");
   G5_CHECK(ctx->num_edges > 0, "g5_construct: the edge list is empty");
@@ -195,7 +209,7 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
 
   // 1. estimated SCALE
   G5_HIP(hipMemsetAsync(ctx->acc.p, 0, 8, s));
-  hipLaunchKernelGGL(k_or_ids, dim3(grid_for(m, kBlock * 8)), dim3(kBlock), 0, s, e, m,
+  hipLaunchKernelGGL(k_or_ids, dim3(std::min(grid_for(m, kBlock * 8), kTupleGrid)), dim3(kBlock), 0, s, e, m,
                      (unsigned long long*)ctx->acc.p);
   G5_HIP(hipGetLastError());
   uint64_t orv = 0;
@@ -212,19 +226,46 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   g.num_tuples = m;
   g.reorder_mode = mode;
 
-  // 2. degrees (duplicates counted, loops apart)
+  // 2. directed entries grouped by ranges of 2^shift ids, and the degrees
+  // (duplicates counted, loops apart)
+  const int shift = scale - range_bits(scale), nb = 1 << range_bits(scale);
+  const int sub_shift = std::min(shift, 15);
+  static_assert(kDegVerts == 1 << 15, "one workgroup counts 2^15 vertices");
   DevBuf<uint32_t> deg, loops;
   deg.alloc(n);
   loops.alloc(n);
-  G5_HIP(hipMemsetAsync(deg.p, 0, n * 4, s));
+  // counts | cursors of the two range partitions | of the row partition, then bucket bounds and the info words
+  DevBuf<unsigned long long> ctl;
+  const size_t pad = (size_t)kPartMax * kCursorPad;
+  ctl.alloc(4 * pad + 2 * (kPartMax + 1) + I_NUM);
+  unsigned long long *counts = ctl.p, *cur0 = ctl.p + pad, *cur1 = cur0 + pad, *cur2 = cur1 + pad;
+  uint64_t* range_off = (uint64_t*)(cur2 + pad);
+  uint64_t* l1_base = range_off + kPartMax + 1;
+  unsigned long long* info = cur2 + pad + 2 * (kPartMax + 1);
+  G5_HIP(hipMemsetAsync(ctl.p, 0, ctl.bytes(), s));
   G5_HIP(hipMemsetAsync(loops.p, 0, n * 4, s));
-  hipLaunchKernelGGL(k_degree, dim3(grid_for(m, kBlock * 4)), dim3(kBlock), 0, s, e, m, deg.p, loops.p);
+  hipLaunchKernelGGL(k_part_count, dim3(std::min(grid_for(m, kBlock * 8), kTupleGrid)), dim3(kBlock), 0, s, e, m, shift, nb,
+                     counts, info);
+  hipLaunchKernelGGL(k_part_offsets, dim3(1), dim3(kPartMax), 0, s, counts, nb, range_off, cur0, cur1);
+  const size_t nkeys = 2 * (size_t)m;
+  DevBuf<uint64_t> xa, xb;
+  xa.alloc(nkeys);
+  partition(SrcTuples{e, m, loops.p, shift}, cur0, xa.p, s);
+  hipLaunchKernelGGL(k_bucket_degrees, dim3((unsigned)nb << (shift - sub_shift)), dim3(1024), 0, s, xa.p, range_off,
+                     shift, sub_shift, n, deg.p, info);
   G5_HIP(hipGetLastError());
-  g.max_degree = (int64_t)device_reduce_max(LoadU32{deg.p}, (size_t)n, ctx->acc.p, s);
-  g.self_loops = (int64_t)device_reduce_sum(LoadU32{loops.p}, (size_t)n, ctx->acc.p, s);
-  g.n_active = (int64_t)device_reduce_sum(NonZeroU32{deg.p}, (size_t)n, ctx->acc.p, s);
+  uint64_t h_info[I_NUM];
+  G5_HIP(hipMemcpyAsync(h_info, info, sizeof(h_info), hipMemcpyDeviceToHost, s));
+  G5_HIP(hipStreamSynchronize(s));
+  g.max_degree = (int64_t)h_info[I_MAXDEG];
+  g.self_loops = (int64_t)h_info[I_LOOPS];
+  g.n_active = (int64_t)h_info[I_ACTIVE];
   g.directed_before = 2 * (m - g.self_loops);
   g.n_rows = (mode == 0) ? n : g.n_active;
+  if (release_edges) {
+    ctx->edges.release();
+    ctx->num_edges = 0;
+  }
 
   // has_edge bitmap by original id, kept on the host for root selection
   {
@@ -251,7 +292,6 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   if (mode == 0) {
     hipLaunchKernelGGL(k_iota, dim3(grid_for(n)), dim3(kBlock), 0, s, n, g.new2old.p);
     G5_HIP(hipGetLastError());
-    G5_HIP(hipMemcpyAsync(g.old2new.p, g.new2old.p, n * 4, hipMemcpyDeviceToDevice, s));
   } else {
     DevBuf<uint32_t> k0, k1, v1;
     k0.alloc(n);
@@ -267,58 +307,114 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     radix_sort_pairs_u32(&kp, &ka, &vp, &va, (size_t)n, 0, bits, rs, s);
     if (vp != g.new2old.p)
       G5_HIP(hipMemcpyAsync(g.new2old.p, vp, n * 4, hipMemcpyDeviceToDevice, s));
-    hipLaunchKernelGGL(k_invert, dim3(grid_for(n)), dim3(kBlock), 0, s, g.new2old.p, n, g.old2new.p);
-    G5_HIP(hipGetLastError());
     G5_HIP(hipStreamSynchronize(s));
   }
   const int64_t rows = g.n_rows;
   g.weight.alloc(rows);
-  hipLaunchKernelGGL(k_weights, dim3(grid_for(rows)), dim3(kBlock), 0, s, g.new2old.p, deg.p, loops.p,
-                     rows, g.weight.p);
-  G5_HIP(hipGetLastError());
-  G5_HIP(hipStreamSynchronize(s));
-  deg.release();
-  loops.release();
-
-  // 4. directed entry keys and their sort
-  const size_t nkeys = 2 * (size_t)m;
-  const size_t nvalid = (size_t)g.directed_before;
-  DevBuf<uint64_t> keys, alt;
-  keys.alloc(nkeys);
-  hipLaunchKernelGGL(k_pair_keys, dim3(grid_for(m, kBlock * 4)), dim3(kBlock), 0, s, e, m,
-                     g.old2new.p, scale, keys.p);
-  G5_HIP(hipGetLastError());
-  if (release_edges) {
-    G5_HIP(hipStreamSynchronize(s));
-    ctx->edges.release();
-    ctx->num_edges = 0;
-  }
-  alt.alloc(nkeys);
-  uint64_t *kp = keys.p, *ka = alt.p;
-  radix_sort_u64(&kp, &ka, nkeys, 0, 2 * scale, rs, s);
-  G5_HIP(hipStreamSynchronize(s));
-  rs.counts.release();
-  rs.offsets.release();
-  // keep the sorted buffer, free the other
-  if (kp == keys.p) alt.release(); else keys.release();
-  const uint64_t* sorted = kp;
-
-  // 5. duplicate removal, columns, offsets
-  const uint64_t nnz = device_reduce_sum(UniqueFlag{sorted, nvalid}, nkeys, ctx->acc.p, s);
-  g.nnz = (int64_t)nnz;
-  g.cols.alloc(nnz);
   g.offsets.alloc(rows + 1);
-  DevBuf<uint64_t> tmp;
-  tmp.alloc(scan_tmp_elems(nvalid));
-  device_scan(UniqueFlag{sorted, nvalid}, UniqueStore{sorted, nvalid, scale, g.cols.p, g.offsets.p},
-              nvalid, tmp.p, s);
-  hipLaunchKernelGGL(k_offsets_tail, dim3(grid_for(rows)), dim3(kBlock), 0, s, sorted, nvalid, scale,
-                     rows, nnz, g.offsets.p);
+  DevBuf<uint32_t> row_cnt;  // degrees with duplicates, then unique entries per row
+  DevBuf<uint64_t> P, tmp;   // degree prefix: P[r] = entries of the rows before r
+  row_cnt.alloc(rows + 1);
+  P.alloc(rows + 1);
+  tmp.alloc(scan_tmp_elems(rows + 1));
+  hipLaunchKernelGGL(k_row_info, dim3(grid_for(rows + 1)), dim3(kBlock), 0, s, g.new2old.p, deg.p,
+                     g.self_loops ? loops.p : nullptr, rows, row_cnt.p, g.weight.p);
   G5_HIP(hipGetLastError());
-  G5_HIP(hipStreamSynchronize(s));
-  keys.release();
-  alt.release();
-  tmp.release();
+  device_scan(LoadU32{row_cnt.p}, StoreU64{P.p}, (size_t)rows + 1, tmp.p, s);
+  DevBuf<uint64_t> row_word;
+  row_word.alloc(n);
+  hipLaunchKernelGGL(k_row_words, dim3(grid_for(n)), dim3(kBlock), 0, s, g.new2old.p, n, P.p, rows, g.old2new.p,
+                     row_word.p);
+  G5_HIP(hipGetLastError());
+
+  // 4. entries to sorted, deduplicated rows
+  const uint64_t E = (uint64_t)g.directed_before;
+  xb.alloc(nkeys);
+  uint64_t nnz = 0;
+  if (E == 0) {
+    g.cols.alloc(0);
+    G5_HIP(hipMemsetAsync(g.offsets.p, 0, (rows + 1) * 8, s));
+  } else {
+    const int sub = sub_shift_for(E), wshift = l1_shift(E, sub);
+    const int nb1 = (int)(((E - 1) >> wshift) + 1);
+    const size_t max_subs = (size_t)(E >> sub) + nb1 + 1;
+    DevBuf<uint64_t> sub64;  // first position | first entry | first unique column
+    DevBuf<uint32_t> sub32;  // entries | first row | unique columns | L1 first sub-buckets | column shares
+    sub64.alloc(3 * (max_subs + 1));
+    sub32.alloc(3 * max_subs + kPartMax + 1 + kFracMax);
+    uint64_t *sub_pos = sub64.p, *sub_off = sub_pos + max_subs + 1, *out_off = sub_off + max_subs + 1;
+    uint32_t *sub_cnt = sub32.p, *sub_row = sub_cnt + max_subs, *sub_unique = sub_row + max_subs;
+    uint32_t *l1_sub0 = sub_unique + max_subs, *frac = l1_sub0 + kPartMax + 1;
+    int flat = -1;  // degree order: share samples by octave
+    if (mode != 2) {
+      flat = 0;
+      while (((rows - 1) >> flat) >= 4096) ++flat;
+    }
+    int sh = 0;
+    const int frac_count = (int)FracMap::index((uint32_t)(rows - 1), flat, sh) + 2;
+    G5_CHECK(frac_count <= kFracMax && nb1 <= kPartMax, "g5_construct: share table or bucket count too small");
+    hipLaunchKernelGGL(k_frac_table, dim3(grid_for(frac_count)), dim3(kBlock), 0, s, P.p, rows, flat, frac_count, frac);
+    hipLaunchKernelGGL(k_l1_setup, dim3(1), dim3(kPartMax), 0, s, P.p, rows, wshift, sub, nb1, l1_base, l1_sub0, cur2,
+                       sub_pos, info);
+    hipLaunchKernelGGL(k_sub_rows, dim3(std::min(grid_for(rows), 4096u)), dim3(kBlock), 0, s, P.p, rows, wshift, sub,
+                       l1_base, l1_sub0, info, sub_row);
+    G5_HIP(hipGetLastError());
+    uint64_t *grouped, *refined;  // entries by L1 bucket (kept until the sort is known to have fit), by sub-bucket
+    if (scale <= kRelabelBothScale) {
+      grouped = xb.p;
+      refined = xa.p;
+      partition(SrcPosition<true>{xa.p, (int64_t)E, g.old2new.p, row_word.p, l1_base, nb1, wshift, frac, frac_count,
+                                  flat}, cur2, grouped, s);
+    } else {
+      grouped = xa.p;
+      refined = xb.p;
+      partition(SrcRelabel{xa.p, (int64_t)E, g.old2new.p, shift}, cur1, xb.p, s);
+      partition(SrcPosition<false>{xb.p, (int64_t)E, g.old2new.p, row_word.p, l1_base, nb1, wshift, frac, frac_count,
+                                   flat}, cur2, grouped, s);
+    }
+    hipLaunchKernelGGL(k_refine, dim3((unsigned)nb1), dim3(1024), 0, s, grouped, refined, sub, l1_base, l1_sub0,
+                       sub_pos, sub_off, sub_cnt, info);
+    G5_HIP(hipMemsetAsync(row_cnt.p, 0, (rows + 1) * 4, s));
+    if (sub == 11)
+      hipLaunchKernelGGL(k_sort_sub<11>, dim3((unsigned)max_subs), dim3(SubSort<11>::kThreads), 0, s, refined, sub_off,
+                         sub_cnt, sub_pos, sub_row, P.p, rows, row_cnt.p, sub_unique, info);
+    else
+      hipLaunchKernelGGL(k_sort_sub<12>, dim3((unsigned)max_subs), dim3(SubSort<12>::kThreads), 0, s, refined, sub_off,
+                         sub_cnt, sub_pos, sub_row, P.p, rows, row_cnt.p, sub_unique, info);
+    G5_HIP(hipGetLastError());
+    DevBuf<uint64_t> stmp;
+    stmp.alloc(scan_tmp_elems(max_subs));
+    device_scan(LoadU32{row_cnt.p}, StoreU64{g.offsets.p}, (size_t)rows + 1, tmp.p, s);
+    device_scan(LoadU32{sub_unique}, StoreU64{out_off}, max_subs, stmp.p, s);
+    G5_HIP(hipMemcpyAsync(h_info, info, sizeof(h_info), hipMemcpyDeviceToHost, s));
+    G5_HIP(hipMemcpyAsync(&nnz, g.offsets.p + rows, 8, hipMemcpyDeviceToHost, s));
+    G5_HIP(hipStreamSynchronize(s));
+    if (!h_info[I_WIDE] && !h_info[I_OVERFLOW]) {
+      g.cols.alloc(nnz);
+      hipLaunchKernelGGL(k_compact, dim3((unsigned)max_subs), dim3(kBlock), 0, s, refined, sub_off, sub_unique, out_off,
+                         info, g.cols.p);
+      G5_HIP(hipGetLastError());
+    } else {
+      // Rows whose columns crowd into few positions (very long rows, many
+      // copies of one tuple): the entries, still whole in `grouped`, are
+      // sorted by radix instead.
+      hipLaunchKernelGGL(k_entry_keys, dim3(grid_for((int64_t)E)), dim3(kBlock), 0, s, grouped, E, P.p, rows, l1_base,
+                         nb1, refined);
+      uint64_t *kp = refined, *ka = grouped;
+      radix_sort_u64(&kp, &ka, E, 0, scale, rs, s);
+      radix_sort_u64(&kp, &ka, E, 32, 32 + scale, rs, s);
+      const UniqueFlag flag{kp, (size_t)E};
+      nnz = device_reduce_sum(flag, E, ctx->acc.p, s);
+      g.cols.alloc(nnz);
+      stmp.alloc(scan_tmp_elems(E));
+      device_scan(flag, UniqueStore{kp, (size_t)E, 32, g.cols.p, g.offsets.p}, E, stmp.p, s);
+      hipLaunchKernelGGL(k_offsets_tail, dim3(grid_for(rows)), dim3(kBlock), 0, s, kp, (size_t)E, 32, rows, nnz,
+                         g.offsets.p);
+      G5_HIP(hipGetLastError());
+    }
+    G5_HIP(hipStreamSynchronize(s));
+  }
+  g.nnz = (int64_t)nnz;
 
   g.first_nbr.alloc(rows);
   hipLaunchKernelGGL(k_first_nbr, dim3(grid_for(rows)), dim3(kBlock), 0, s, g.offsets.p, g.cols.p,
