@@ -58,6 +58,7 @@ int g5_create(int device, g5_ctx** out) {
     delete ctx;
     return G5_ERR_HIP;
   }
+  pool_context(device, 1);
   *out = ctx;
   return G5_OK;
 }
@@ -77,7 +78,9 @@ int g5_destroy(g5_ctx* ctx) {
   ctx->wstage.release();
   ctx->acc.release();
   (void)hipStreamDestroy(ctx->stream);
+  const int device = ctx->device;
   delete ctx;
+  pool_context(device, -1);
   return G5_OK;
 }
 

@@ -1068,19 +1068,14 @@ void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   b.scan_tmp.alloc(scan_tmp_elems(scan_n));
   b.counters.alloc(kBfsCounters);
   bfs_tuning_buffers(ctx, b, s);
-  G5_HIP(hipHostMalloc((void**)&b.h_counters, C_NUM * sizeof(uint64_t), hipHostMallocDefault));
+  static_assert(C_NUM <= sizeof(b.h_counters) / 8, "host counters");
+  G5_HIP(hipStreamSynchronize(s));  // the published blocks are reset below
   b.pub.alloc(C_NUM);
   b.pub_seq = 0;
   b.fuse.alloc(F_NUM);
   b.fuse_seq = 0;
-  G5_HIP(hipEventCreate(&b.ev0));
-  G5_HIP(hipEventCreate(&b.ev1));
-  b.lev_begin.assign(G5_MAX_LEVELS, nullptr);
-  b.lev_end.assign(G5_MAX_LEVELS, nullptr);
-  for (int i = 0; i < G5_MAX_LEVELS; ++i) {
-    G5_HIP(hipEventCreate(&b.lev_begin[i]));
-    G5_HIP(hipEventCreate(&b.lev_end[i]));
-  }
+  if (!b.ev0) G5_HIP(hipEventCreate(&b.ev0));
+  if (!b.ev1) G5_HIP(hipEventCreate(&b.ev1));
   b.prepared = true;
 }
 
@@ -1159,7 +1154,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     ++lvl;
     G5_CHECK(lvl < 255, "g5_run_bfs: more than 254 levels (uint8 level array)");
     const bool forward = next_forward;
-    G5_HIP(hipEventRecord(b.lev_begin[lvl], s));
+    G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
     if (forward && fuse_next && b.small_edges > 0 && nf <= kFuseNf &&
         (e_next < 0 || e_next <= b.small_edges)) {
       // small top-down levels, as many as fit, in one single-workgroup launch
@@ -1169,7 +1164,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
                          g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p, (uint32_t)lvl, max_levels,
                          b.small_edges, na, prev_nq, growing ? 1 : 0, b.fuse.d, b.fuse_seq);
       G5_HIP(hipGetLastError());
-      G5_HIP(hipEventRecord(b.lev_end[lvl], s));
+      G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
       const char* unpublished = "g5_run_bfs: fused levels were not published";
       b.fuse.wait(F_LEVELS, F_NUM, b.fuse_seq, s, unpublished);
       const int k = (int)b.fuse.value(F_LEVELS);
@@ -1190,11 +1185,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
         st.nq[l] = nq;
         st.num_levels = l + 1;
         visited += nq;
-        if (j > 0) {
-          // the launch's time is the first fused level's; the others show 0
-          G5_HIP(hipEventRecord(b.lev_begin[l], s));
-          G5_HIP(hipEventRecord(b.lev_end[l], s));
-        }
+        st.level_ms[l] = j ? 0 : -1;  // the launch's time is the first fused level's; the others show 0
       }
       prev_nq = (int64_t)b.fuse.value(k - 1);
       qi = (int)b.fuse.value(F_QI);
@@ -1339,7 +1330,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
                          b.level.p, b.parent.p, b.words, span, (uint32_t)lvl, cnt);
     }
     G5_HIP(hipGetLastError());
-    G5_HIP(hipEventRecord(b.lev_end[lvl], s));
+    G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
     ++b.pub_seq;
     hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, td ? 1 : 0, b.pub.d,
                        b.pub_seq);
@@ -1353,6 +1344,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     st.bu_kernel[lvl] = td ? 0 : 1;
     st.nq[lvl] = nq;
     st.num_levels = lvl + 1;
+    st.level_ms[lvl] = -1;  // read from the events at the end
     visited += nq;
     if (nq == 0) break;
     // direction switch, mpi/bfs.hpp:2799-2829
@@ -1386,6 +1378,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   G5_HIP(hipEventElapsedTime(&ms, b.ev0, b.ev1));
   st.device_ms = ms;
   for (int l = 1; l <= lvl && root_active; ++l) {
+    if (st.level_ms[l] == 0) continue;
     float lms = 0;
     G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[l], b.lev_end[l]));
     st.level_ms[l] = lms;

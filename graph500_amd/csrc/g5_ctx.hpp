@@ -42,6 +42,18 @@ struct Graph {
   }
 };
 
+// Events of a run's levels, created as levels are first reached.
+inline hipEvent_t level_event(std::vector<hipEvent_t>& v, int l) {
+  if ((int)v.size() <= l) v.resize(l + 1, nullptr);
+  if (!v[l]) G5_HIP(hipEventCreate(&v[l]));
+  return v[l];
+}
+inline void destroy_events(std::vector<hipEvent_t>& v) {
+  for (auto e : v)
+    if (e) (void)hipEventDestroy(e);
+  v.clear();
+}
+
 // Single-root BFS state.
 struct BfsState {
   bool prepared = false;
@@ -57,7 +69,7 @@ struct BfsState {
   DevBuf<uint32_t> chunk_rows;    // 2 per top-down edge chunk: first/last frontier index
   DevBuf<uint64_t> scan_tmp;
   DevBuf<uint64_t> counters;      // device counters (see g5_bfs.hip)
-  uint64_t* h_counters = nullptr; // pinned host mirror
+  uint64_t h_counters[8] = {};    // the last level's counters on the host
   PublishBlock pub;               // the level counters, published by k_publish
   uint64_t pub_seq = 0;
   PublishBlock fuse;              // the fused small levels' state (g5_bfs.hip)
@@ -117,19 +129,15 @@ struct BfsState {
     seg_start.release();
     hub_bnd.release();
     hub_built_shift = 0;
-    if (h_counters) (void)hipHostFree(h_counters);
-    h_counters = nullptr;
-    pub.release();
-    fuse.release();
-    if (ev0) (void)hipEventDestroy(ev0);
-    if (ev1) (void)hipEventDestroy(ev1);
-    ev0 = ev1 = nullptr;
-    for (auto e : lev_begin) (void)hipEventDestroy(e);
-    for (auto e : lev_end) (void)hipEventDestroy(e);
-    lev_begin.clear();
-    lev_end.clear();
     prepared = false;
     have_result = false;
+  }
+  // events and published blocks stay with the state from one graph to the next
+  ~BfsState() {
+    destroy_events(lev_begin);
+    destroy_events(lev_end);
+    if (ev0) (void)hipEventDestroy(ev0);
+    if (ev1) (void)hipEventDestroy(ev1);
   }
 };
 
@@ -199,7 +207,7 @@ struct MsState {
   DevBuf<uint64_t> scan_tmp;
   DevBuf<uint64_t> counters;
   DevBuf<int64_t> roots;
-  uint64_t* h_counters = nullptr;
+  std::vector<uint64_t> h_counters;  // the last level's counters on the host
   PublishBlock pub;             // the counters as each level publishes them (g5_msbfs.hip)
   uint64_t pub_seq = 0;
   g5_batch_stats stats{};
@@ -240,18 +248,15 @@ struct MsState {
     p_dir.release();
     if (h_persist) (void)hipHostFree(h_persist);
     h_persist = nullptr;
-    if (h_counters) (void)hipHostFree(h_counters);
-    h_counters = nullptr;
-    pub.release();
-    if (ev0) (void)hipEventDestroy(ev0);
-    if (ev1) (void)hipEventDestroy(ev1);
-    ev0 = ev1 = nullptr;
-    for (auto e : lev_begin) (void)hipEventDestroy(e);
-    for (auto e : lev_end) (void)hipEventDestroy(e);
-    lev_begin.clear();
-    lev_end.clear();
     prepared = false;
     have_result = false;
+  }
+  // events and published blocks stay with the state from one graph to the next
+  ~MsState() {
+    destroy_events(lev_begin);
+    destroy_events(lev_end);
+    if (ev0) (void)hipEventDestroy(ev0);
+    if (ev1) (void)hipEventDestroy(ev1);
   }
 };
 

@@ -571,17 +571,12 @@ void ms_prepare(g5_ctx* ctx) {
   m.fr_exact.assign(m.fr.size(), 0);
   m.fr_count.assign(m.fr.size(), 0);
   if (m.compact_below > 0) ms_alloc_compact(ctx);
-  G5_HIP(hipHostMalloc((void**)&m.h_counters, kMsCounters * sizeof(uint64_t), hipHostMallocDefault));
+  m.h_counters.assign(kMsCounters, 0);
+  G5_HIP(hipStreamSynchronize(ctx->stream));  // the published block is reset below
   m.pub.alloc(kMsCounters);
   m.pub_seq = 0;
-  G5_HIP(hipEventCreate(&m.ev0));
-  G5_HIP(hipEventCreate(&m.ev1));
-  m.lev_begin.assign(G5_MAX_LEVELS, nullptr);
-  m.lev_end.assign(G5_MAX_LEVELS, nullptr);
-  for (int i = 0; i < G5_MAX_LEVELS; ++i) {
-    G5_HIP(hipEventCreate(&m.lev_begin[i]));
-    G5_HIP(hipEventCreate(&m.lev_end[i]));
-  }
+  if (!m.ev0) G5_HIP(hipEventCreate(&m.ev0));
+  if (!m.ev1) G5_HIP(hipEventCreate(&m.ev1));
   m.prepared = true;
 }
 
@@ -682,7 +677,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
   m.level_masks = lanes_mode;
   double lane_fd[64] = {}, lane_vd[64] = {};
   uint64_t pulled = 0;  // roots that have pulled: they pull from then on
-  const uint64_t* h_lane = m.h_counters + kMsLanes;
+  const uint64_t* h_lane = m.h_counters.data() + kMsLanes;
   unsigned* d_list_count = (unsigned*)(cnt + M_NUM);
   bool have_miss = false;  // m.miss holds the vertices still missing a live root
   int l = l0 - 1;
@@ -724,7 +719,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     }
     m.level_push[l] = push ? live : td;
     m.level_pull[l] = push ? 0 : (lanes_mode ? bu : live);
-    G5_HIP(hipEventRecord(m.lev_begin[l], s));
+    G5_HIP(hipEventRecord(level_event(m.lev_begin, l), s));
     // statistics for the roots still choosing (a root that pulled keeps pulling)
     const LaneEpi lepi{cnt + kMsLanes, g.offsets.p, lanes_mode ? td : live};
     if (lanes_mode && td && bu) {
@@ -886,7 +881,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     }
     G5_HIP(hipGetLastError());
     m.fr_exact[l] = 1;  // every level form leaves next non-zero exactly at the bits of nz_next
-    G5_HIP(hipEventRecord(m.lev_end[l], s));
+    G5_HIP(hipEventRecord(level_event(m.lev_end, l), s));
     ms_publish_wait(m, lane_stats ? kMsCounters : M_NUM, s);
     st.direction[l] = (lanes_mode && td && bu) ? 3 : (push ? 1 : (sweep ? 2 : 0));
     if (lane_stats)

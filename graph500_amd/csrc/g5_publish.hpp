@@ -38,7 +38,12 @@ struct PublishBlock {
   PublishBlock& operator=(const PublishBlock&) = delete;
   ~PublishBlock() { release(); }
 
+  // every tag 0 again; an equal block is kept (no kernel that publishes into it may be in flight)
   void alloc(int count) {
+    if (h && n == count) {
+      for (int i = 0; i < count; ++i) h[i] = Published{0, 0};
+      return;
+    }
     release();
     G5_HIP(hipHostMalloc((void**)&h, (size_t)count * sizeof(Published),
                          hipHostMallocCoherent | hipHostMallocMapped));
