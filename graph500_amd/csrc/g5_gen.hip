@@ -7,11 +7,12 @@
 //   scramble constants / scramble   generator/graph_generator.hpp:375-384,405-469
 //   generateRange/make_one_edge     generator/graph_generator.hpp:612-704
 //
-// Device design: one lane per tuple.  The lane skips the seed state by
-// edge_index * 2^64 (the "middle" exponent word) with one 5x5 transition per
-// non-zero byte of edge_index (at most 4 for 2^32 tuples), then draws SCALE
-// quadrant choices.  Arithmetic mod 2^31-1 uses 64-bit multiply-accumulate
-// (v_mad_u64_u32) and a two-fold Mersenne reduction instead of division.
+// Device design: one lane per tuple.  The tuple's state is the seed state
+// skipped by edge_index * 2^64 (the "middle" exponent word): one 5x5
+// transition per byte of edge_index, the upper bytes' once per 256 tuples and
+// the low byte's per lane, then SCALE quadrant draws.  Arithmetic mod 2^31-1
+// uses 64-bit multiply-accumulate (v_mad_u64_u32) and Mersenne folds instead
+// of division.
 #include "g5_internal.hpp"
 
 #include <mutex>
@@ -157,19 +158,21 @@ struct DevEntry {
   uint32_t pad[3];
 };
 
+// x < 2^64 mod 2^31 - 1: two folds leave at most 2^31 + 4, one conditional
+// subtraction (the smaller of r and r - M as unsigned numbers) the residue.
 __device__ __forceinline__ uint32_t mred(uint64_t x) {
   x = (x & kM) + (x >> 31);
-  x = (x & kM) + (x >> 31);
-  uint32_t r = (uint32_t)x;
-  return r >= kM ? r - kM : r;
+  const uint32_t r = (uint32_t)(x & kM) + (uint32_t)(x >> 31);
+  return min(r, r - kM);
 }
 
-// Five-term dot product mod 2^31-1; each product < 2^62, four of them < 2^64.
+// Five-term dot product mod 2^31-1; each product < 2^62, four of them < 2^64;
+// folded once they are < 2^34 and the fifth fits beside them.
 __device__ __forceinline__ uint32_t dot5(uint32_t a1, uint32_t b1, uint32_t a2, uint32_t b2,
                                          uint32_t a3, uint32_t b3, uint32_t a4, uint32_t b4,
                                          uint32_t a5, uint32_t b5) {
   uint64_t acc = (uint64_t)a1 * b1 + (uint64_t)a2 * b2 + (uint64_t)a3 * b3 + (uint64_t)a4 * b4;
-  acc = (uint64_t)mred(acc) + (uint64_t)a5 * b5;
+  acc = (acc & kM) + (acc >> 31) + (uint64_t)a5 * b5;
   return mred(acc);
 }
 
@@ -191,7 +194,10 @@ __device__ __forceinline__ void dapply(const DevEntry& e, DState& s) {
 }
 
 __device__ __forceinline__ uint32_t dstep(DState& s) {
-  const uint32_t nz = mred((uint64_t)kX * s.z1 + (uint64_t)kY * s.z5);
+  // below 2^27 * 2^31 + 2^17 * 2^31 < 2^59: one fold leaves less than 2 M
+  const uint64_t x = (uint64_t)kX * s.z1 + (uint64_t)kY * s.z5;
+  const uint32_t r = (uint32_t)(x & kM) + (uint32_t)(x >> 31);
+  const uint32_t nz = min(r, r - kM);
   s.z5 = s.z4;
   s.z4 = s.z3;
   s.z3 = s.z2;
@@ -209,52 +215,99 @@ __device__ __forceinline__ uint64_t dscramble(uint64_t v, int scale, uint64_t va
   return v;
 }
 
+// The same for scale <= 32: only the low 32 bits of a product reach the
+// reversed result.
+__device__ __forceinline__ uint32_t dscramble32(uint32_t v, int scale, uint64_t val0, uint64_t val1) {
+  v += (uint32_t)val0 + (uint32_t)val1;
+  v *= (uint32_t)(val0 | UINT64_C(0x4519840211493211));
+  v = __builtin_bitreverse32(v) >> (32 - scale);
+  v *= (uint32_t)(val1 | UINT64_C(0x3050852102C843A5));
+  return __builtin_bitreverse32(v) >> (32 - scale);
+}
+
 struct GenParams {
   DState seed;
   uint64_t val0, val1;
   int64_t start, count;
   int scale;
   uint32_t a_num, bc_num;
+  int groups;  // 256-tuple groups per workgroup
 };
 
+// One draw's quadrant number below 10000 (draws under the rejection bound
+// 2^32 mod 10000 are taken again, as the generator defines it).
+__device__ __forceinline__ uint32_t ddraw(DState& st) {
+  constexpr uint32_t kLimit = UINT32_C(0xFFFFFFFF) % 10000u;  // 7295
+  uint32_t v = dstep(st);
+  while (v < kLimit) v = dstep(st);
+  return v - __umul24(v / 10000u, 10000u);  // the quotient has 18 bits: one full-rate multiply
+}
+
 // tab: the 8 byte-tables of the middle exponent word (entries [8*256, 16*256)).
+// A workgroup takes p.groups runs of 256 tuple indices, aligned to 256, so
+// that a run shares every byte of its indices but the lowest: thread k makes
+// run k's state once (LDS), and lane t applies the low byte's transition,
+// which it keeps in registers over all runs.  The kernel is bound by the
+// integer multiplies of the draws (two 64-bit multiply-adds and a high
+// multiply per level, quarter rate); with four transitions per tuple, read
+// from the table, SCALE 25 (2^29 tuples) took 17.3 ms.
+template <bool k32>
 __global__ void __launch_bounds__(256) k_kronecker(g5_packed_edge* __restrict__ out,
                                                    const DevEntry* __restrict__ tab,
                                                    GenParams p) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const uint32_t limit = UINT32_C(0xFFFFFFFF) % 10000u;  // 7295: rejection bound
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p.count; i += stride) {
-    const uint64_t idx = (uint64_t)(p.start + i);
+  __shared__ DState s_run[256];
+  const int t = threadIdx.x;
+  const int64_t g0 = (p.start >> 8) + (int64_t)blockIdx.x * p.groups;
+  if (t < p.groups) {
     DState st = p.seed;
-    uint64_t e = idx;
-    for (int b = 0; e; ++b, e >>= 8) {
+    uint64_t e = (uint64_t)(g0 + t);
+    for (int b = 1; e; ++b, e >>= 8) {
       const uint32_t v = (uint32_t)(e & 0xFF);
       if (v) dapply(tab[b * 256 + v], st);
     }
+    s_run[t] = st;
+  }
+  const DevEntry low = tab[t];
+  __syncthreads();
+  const uint32_t bc = p.bc_num, bc2 = 2 * p.bc_num, abc = bc2 + p.a_num;
+  for (int k = 0; k < p.groups; ++k) {
+    const int64_t i = ((g0 + k) << 8) + t - p.start;
+    if (i < 0 || i >= p.count) continue;
+    DState st = s_run[k];
+    dapply(low, st);
     uint64_t bs = 0, bt = 0;
+    uint32_t bs32 = 0, bt32 = 0;
+    bool same = true;  // bs == bt so far
     for (int lvl = p.scale - 1; lvl >= 0; --lvl) {
-      uint32_t val = dstep(st);
-      while (val < limit) val = dstep(st);
-      val %= 10000u;
-      int sq;
-      if (val < p.bc_num) sq = 1;
-      else if (val - p.bc_num < p.bc_num) sq = 2;
-      else if (val - 2 * p.bc_num < p.a_num) sq = 0;
-      else sq = 3;
-      uint32_t so = (uint32_t)sq >> 1, to = (uint32_t)sq & 1;
-      if (bs == bt && so > to) {  // clip-and-flip
-        so = 0;
-        to = 1;
+      const uint32_t val = ddraw(st);
+      // below bc: quadrant 1, below 2 bc: 2, below 2 bc + a: 0, else 3
+      const bool both = val >= abc;
+      bool so = both || (val >= bc && val < bc2), to = both || val < bc;
+      if (same && so && !to) {  // clip-and-flip
+        so = false;
+        to = true;
       }
-      bs += (uint64_t)so << lvl;
-      bt += (uint64_t)to << lvl;
+      same = same && so == to;
+      if (k32) {
+        bs32 = 2 * bs32 + so;
+        bt32 = 2 * bt32 + to;
+      } else {
+        bs = 2 * bs + so;
+        bt = 2 * bt + to;
+      }
     }
-    const uint64_t v0 = dscramble(bs, p.scale, p.val0, p.val1);
-    const uint64_t v1 = dscramble(bt, p.scale, p.val0, p.val1);
     g5_packed_edge r;
-    r.v0_low = (uint32_t)v0;
-    r.v1_low = (uint32_t)v1;
-    r.high = (uint32_t)(((v0 >> 32) & 0xFFFF) | ((v1 >> 16) & 0xFFFF0000u));
+    if (k32) {
+      r.v0_low = dscramble32(bs32, p.scale, p.val0, p.val1);
+      r.v1_low = dscramble32(bt32, p.scale, p.val0, p.val1);
+      r.high = 0;
+    } else {
+      const uint64_t v0 = dscramble(bs, p.scale, p.val0, p.val1);
+      const uint64_t v1 = dscramble(bt, p.scale, p.val0, p.val1);
+      r.v0_low = (uint32_t)v0;
+      r.v1_low = (uint32_t)v1;
+      r.high = (uint32_t)(((v0 >> 32) & 0xFFFF) | ((v1 >> 16) & 0xFFFF0000u));
+    }
     out[i] = r;
   }
 }
@@ -374,9 +427,16 @@ void launch_kronecker(int device, g5_packed_edge* out, int64_t start, int64_t co
   p.bc_num = (uint32_t)bc_num;
   if (count <= 0) return;
   // Edge indices up to 2^64 use at most the 8 middle-word tables.
-  int64_t blocks = (count + 255) / 256;
-  if (blocks > 256 * 256) blocks = 256 * 256;
-  hipLaunchKernelGGL(k_kronecker, dim3((unsigned)blocks), dim3(256), 0, stream, out, t.tab.p, p);
+  const int64_t runs = ((start + count + 255) >> 8) - (start >> 8);
+  int64_t groups = runs / 4096;  // at least 4,096 workgroups where there are as many runs
+  groups = groups < 1 ? 1 : (groups > 256 ? 256 : groups);
+  p.groups = (int)groups;
+  const int64_t blocks = (runs + groups - 1) / groups;
+  G5_CHECK(blocks <= INT32_MAX, "g5_generate_kronecker: too many tuples for one launch");
+  if (scale <= 32)
+    hipLaunchKernelGGL(k_kronecker<true>, dim3((unsigned)blocks), dim3(256), 0, stream, out, t.tab.p, p);
+  else
+    hipLaunchKernelGGL(k_kronecker<false>, dim3((unsigned)blocks), dim3(256), 0, stream, out, t.tab.p, p);
   G5_HIP(hipGetLastError());
 }
 

@@ -103,3 +103,17 @@ def test_star(ctx, leaves):
     assert np.array_equal(g["cols"][:leaves], leaf)
     assert not g["cols"][leaves:].any() and len(g["cols"]) == 2 * leaves
     assert np.array_equal(g["offsets"], np.concatenate([[0], np.arange(leaves, 2 * leaves + 1)]))
+
+
+@pytest.mark.parametrize("scale,edgefactor", [(19, 13), (20, 17), (33, 1)])
+def test_generator_slices(oracle_mod, scale, edgefactor):
+    """Runs that do not fill the last workgroup, and ids beyond 32 bits."""
+    import graph500_amd
+    print("slices", scale, edgefactor, flush=True)
+    m = edgefactor << scale
+    with graph500_amd.G5Context(0) as c:
+        c.generate_kronecker(scale, edgefactor, 5, 9)
+        for start in (0, 255, m // 3, (1 << min(scale, 32)) - 300, m - 1001):
+            got = c.edges_download(start, 1001 if start + 1001 <= m else m - start)
+            exp = oracle_mod.generate_edges(scale, edgefactor, 5, 9, start=start, end=start + len(got))
+            assert np.array_equal(got, exp), start
