@@ -62,36 +62,6 @@ enum { S_FOUND = 0, S_NEXT_E = 1 };
 constexpr int kStripeBase = 8;  // words: the stripes start on a 64-byte line of their own
 constexpr int kBfsCounters = kStripeBase + kStripes * kStripeWords;
 
-__global__ void __launch_bounds__(kBlock) k_bfs_init(uint8_t* __restrict__ level, uint64_t* __restrict__ vis,
-                                                     int64_t rows, int64_t words) {
-  const int64_t stride = (int64_t)gridDim.x * kBlock;
-  for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < rows; v += stride) level[v] = 0xFF;
-  for (int64_t w = (int64_t)blockIdx.x * kBlock + threadIdx.x; w < words; w += stride) {
-    // bits past the last row read as visited so no sweep ever picks them
-    const int64_t first = w * 64;
-    uint64_t x = 0;
-    if (first + 64 > rows) x = (rows <= first) ? ~UINT64_C(0) : (~UINT64_C(0) << (rows - first));
-    vis[w] = x;
-  }
-}
-
-__global__ void k_bfs_root(const uint32_t* __restrict__ old2new, int64_t root_orig, int64_t rows,
-                           uint8_t* __restrict__ level, uint32_t* __restrict__ parent,
-                           uint64_t* __restrict__ vis, uint32_t* __restrict__ queue,
-                           unsigned long long* __restrict__ counters) {
-  // the first level's counters start at zero; k_publish clears them after
-  // every later level
-  for (int i = threadIdx.x; i < kBfsCounters; i += blockDim.x) counters[i] = 0;
-  if (threadIdx.x != 0) return;
-  const uint32_t r = old2new[root_orig];
-  if ((int64_t)r < rows) {
-    level[r] = 0;
-    parent[r] = r;
-    vis[r >> 6] |= UINT64_C(1) << (r & 63);
-    queue[0] = r;
-  }
-}
-
 // Top-down expansion of one level.  The frontier's rows form one virtual edge
 // list (prefix = exclusive scan of frontier degrees, E = prefix[nf]); every
 // workgroup takes kEpb-edge chunks and each lane walks kEpt consecutive edges.
@@ -413,12 +383,16 @@ __global__ void __launch_bounds__(kBlock) k_td_expand_segs(
   }
 }
 
-// Row part of the bottom-up probe: the first entry of [offsets[v] + 1,
-// offsets[v + 1]) (the first neighbour is probed apart, from the coalesced
-// first_nbr array) whose bit is set in bm.  Every lane of the wave calls it;
-// lanes with active=false only help.  Rows up to kShortRow are scanned by
-// their lane, longer rows by the whole wave 64 entries at a time with a ballot
-// for the first hit.
+// Row part of the bottom-up probe: an entry of [offsets[v] + 1, offsets[v + 1])
+// (the first neighbour is probed apart, from the coalesced first_nbr array)
+// whose bit is set in bm.  Every lane of the wave calls it; lanes with
+// active=false only help.  Rows up to kShortRow are scanned by their lane, kU
+// entries a turn; longer rows by the whole wave, kR rows a turn, 64 entries of
+// each (the last one left takes all kR x 64), a ballot giving a row's first
+// hit.  A turn is a chain of two dependent loads, so on small graphs, whose
+// bottom-up levels are a few such chains, the turns are what counts (kU 8, kR
+// 4); on large ones the probes past a hit are (kU 4, kR 1 with two per lane).
+template <int kU, int kR>
 __device__ __forceinline__ bool row_marked_nbr(bool active, uint32_t v, const uint64_t* __restrict__ bm,
                                                const uint64_t* __restrict__ offsets,
                                                const uint32_t* __restrict__ cols, uint32_t& p) {
@@ -431,44 +405,99 @@ __device__ __forceinline__ bool row_marked_nbr(bool active, uint32_t v, const ui
     need = rb < re;
   }
   if (need && re - rb <= (uint64_t)kShortRow) {
-    // four independent probes per step (entries past the row repeat the
-    // first); any marked neighbour is a valid parent, the first is taken
-    for (uint64_t k = rb; k < re && !found; k += 4) {
-      const uint32_t c0 = cols[k];
-      const uint32_t c1 = k + 1 < re ? cols[k + 1] : c0;
-      const uint32_t c2 = k + 2 < re ? cols[k + 2] : c0;
-      const uint32_t c3 = k + 3 < re ? cols[k + 3] : c0;
-      const bool h0 = bit_set(bm, c0), h1 = bit_set(bm, c1), h2 = bit_set(bm, c2), h3 = bit_set(bm, c3);
-      if (h0 | h1 | h2 | h3) {
-        found = true;
-        p = h0 ? c0 : (h1 ? c1 : (h2 ? c2 : c3));
-      }
+    // independent probes (entries past the row repeat the first); any marked
+    // neighbour is a valid parent, the first is taken
+    for (uint64_t k = rb; k < re && !found; k += kU) {
+      uint32_t c[kU];
+      c[0] = cols[k];
+#pragma unroll
+      for (int j = 1; j < kU; ++j) c[j] = k + j < re ? cols[k + j] : c[0];
+      bool h[kU];
+#pragma unroll
+      for (int j = 0; j < kU; ++j) h[j] = bit_set(bm, c[j]);
+#pragma unroll
+      for (int j = kU - 1; j >= 0; --j)
+        if (h[j]) {
+          found = true;
+          p = c[j];
+        }
     }
     need = false;
   }
   uint64_t lm = __ballot(need);
   while (lm) {
-    const int src = __ffsll((unsigned long long)lm) - 1;
-    lm &= lm - 1;
-    const uint64_t b = __shfl(rb, src, 64), e = __shfl(re, src, 64);
-    // 128 entries per step, two independent probes per lane
-    for (uint64_t base = b; base < e; base += 128) {
-      const uint64_t k = base + lane;
-      uint32_t c0 = 0, c1 = 0;
-      bool h0 = false, h1 = false;
-      if (k < e) c0 = cols[k];
-      if (k + 64 < e) c1 = cols[k + 64];
-      if (k < e) h0 = bit_set(bm, c0);
-      if (k + 64 < e) h1 = bit_set(bm, c1);
-      const uint64_t m0 = __ballot(h0), m1 = __ballot(h1);
-      if (m0 | m1) {
-        const uint32_t hp = m0 ? __shfl(c0, __ffsll((unsigned long long)m0) - 1, 64)
-                               : __shfl(c1, __ffsll((unsigned long long)m1) - 1, 64);
-        if (lane == src) {
-          found = true;
-          p = hp;
+    constexpr int kSlots = kR > 1 ? kR : 2;
+    int src[kSlots];
+    uint64_t b[kSlots], e[kSlots];
+    int n = 0;  // rows of this turn
+#pragma unroll
+    for (int j = 0; j < kR; ++j) {
+      src[j] = -1;
+      b[j] = e[j] = 0;
+      if (lm) {
+        src[j] = __builtin_ctzll(lm);
+        lm &= lm - 1;
+        b[j] = __shfl(rb, src[j], 64);
+        e[j] = __shfl(re, src[j], 64);
+        ++n;
+      }
+    }
+    while (n > 1) {  // 64 entries of every row
+      uint32_t c[kR];
+      bool h[kR];
+#pragma unroll
+      for (int j = 0; j < kR; ++j) c[j] = b[j] + lane < e[j] ? cols[b[j] + lane] : 0;
+#pragma unroll
+      for (int j = 0; j < kR; ++j) h[j] = b[j] + lane < e[j] && bit_set(bm, c[j]);
+#pragma unroll
+      for (int j = 0; j < kR; ++j) {
+        if (b[j] >= e[j]) continue;
+        const uint64_t m = __ballot(h[j]);
+        if (m) {
+          const uint32_t hp = __shfl(c[j], __builtin_ctzll(m), 64);
+          if (lane == src[j]) {
+            found = true;
+            p = hp;
+          }
         }
-        break;
+        b[j] = m ? e[j] : b[j] + 64;
+        if (b[j] >= e[j]) --n;
+      }
+    }
+    if (n == 1) {  // one row: all slots
+      int s1 = -1;
+      uint64_t b1 = 0, e1 = 0;
+#pragma unroll
+      for (int j = 0; j < kR; ++j)
+        if (b[j] < e[j]) {
+          s1 = src[j];
+          b1 = b[j];
+          e1 = e[j];
+        }
+      for (; b1 < e1; b1 += 64 * kSlots) {
+        uint32_t c[kSlots];
+        bool h[kSlots];
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) c[j] = b1 + 64 * j + lane < e1 ? cols[b1 + 64 * j + lane] : 0;
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) h[j] = b1 + 64 * j + lane < e1 && bit_set(bm, c[j]);
+        uint32_t hp = 0;
+        bool any = false;
+#pragma unroll
+        for (int j = kSlots - 1; j >= 0; --j) {
+          const uint64_t m = __ballot(h[j]);
+          if (m) {
+            any = true;
+            hp = __shfl(c[j], __builtin_ctzll(m), 64);
+          }
+        }
+        if (any) {
+          if (lane == s1) {
+            found = true;
+            p = hp;
+          }
+          break;
+        }
       }
     }
   }
@@ -485,7 +514,7 @@ __device__ __forceinline__ bool first_marked_nbr(bool active, uint32_t v, const 
   const uint32_t f = active ? first_nbr[v] : kNoNbr;
   const bool hit = f != kNoNbr && bit_set(bm, f);
   if (hit) p = f;
-  const bool more = row_marked_nbr(f != kNoNbr && !hit, v, bm, offsets, cols, p);
+  const bool more = row_marked_nbr<4, 1>(f != kNoNbr && !hit, v, bm, offsets, cols, p);
   return hit || more;
 }
 
@@ -682,69 +711,6 @@ __global__ void __launch_bounds__(kBlock) k_td_finish(const uint8_t* __restrict_
   block_add(total, stripe_of(counters + kStripeBase, S_FOUND));
 }
 
-// Bottom-up level.  A wave reads `span` bitmap words at a time (one
-// coalesced load, one word per lane, span a power of two from 2 to 64),
-// copies the words whose vertices are all visited to the next bitmap (one
-// coalesced store) and walks the others two at a time, one lane per vertex
-// of each, so both words' first-neighbour probes are in flight together.
-// The host sizes span so that the grid still has a step per wave or more;
-// late levels, where almost every word is full, then cost little more than
-// a pass over the bitmap.
-__global__ void __launch_bounds__(kBlock) k_bu(
-    const uint64_t* __restrict__ vis, uint64_t* __restrict__ vis_next,
-    const uint32_t* __restrict__ first_nbr, const uint64_t* __restrict__ offsets,
-    const uint32_t* __restrict__ cols, uint8_t* __restrict__ level, uint32_t* __restrict__ parent,
-    int64_t words, int span, uint32_t lvl, unsigned long long* __restrict__ counters) {
-  const int lane = threadIdx.x & 63;
-  const int64_t nwaves = (int64_t)gridDim.x * (kBlock / 64);
-  uint64_t found_total = 0;
-  for (int64_t base = ((int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * span; base < words;
-       base += nwaves * span) {
-    const int64_t wl = base + lane;
-    const bool mine = lane < span && wl < words;
-    const uint64_t cl = mine ? vis[wl] : ~UINT64_C(0);  // lanes beyond the span or the end read as visited
-    uint64_t open = __ballot(cl != ~UINT64_C(0));        // words with an unvisited vertex
-    if (mine && cl == ~UINT64_C(0)) vis_next[wl] = cl;
-    while (open) {
-      // the next two open words (identical in every lane)
-      const int j0 = __builtin_ctzll(open);
-      open &= open - 1;
-      const bool has1 = open != 0;
-      const int j1 = has1 ? __builtin_ctzll(open) : j0;
-      if (has1) open &= open - 1;
-      const uint64_t c0 = __shfl(cl, j0, 64);
-      const uint64_t c1 = has1 ? __shfl(cl, j1, 64) : ~UINT64_C(0);
-      const int64_t w0 = base + j0, w1 = base + j1;
-      const uint32_t v0 = (uint32_t)(w0 * 64 + lane), v1 = (uint32_t)(w1 * 64 + lane);
-      const bool a0 = !((c0 >> lane) & 1), a1 = !((c1 >> lane) & 1);
-      const uint32_t f0 = a0 ? first_nbr[v0] : kNoNbr;
-      const uint32_t f1 = a1 ? first_nbr[v1] : kNoNbr;
-      const bool h0 = f0 != kNoNbr && bit_set(vis, f0);
-      const bool h1 = f1 != kNoNbr && bit_set(vis, f1);
-      uint32_t p0 = f0, p1 = f1;
-      // every lane makes both calls (the long-row scan needs the whole wave)
-      const bool r0 = row_marked_nbr(f0 != kNoNbr && !h0, v0, vis, offsets, cols, p0);
-      const bool r1 = row_marked_nbr(f1 != kNoNbr && !h1, v1, vis, offsets, cols, p1);
-      const bool g0 = h0 || r0, g1 = h1 || r1;
-      const uint64_t fm0 = __ballot(g0), fm1 = __ballot(g1);
-      if (lane == 0) {
-        vis_next[w0] = c0 | fm0;
-        if (has1) vis_next[w1] = c1 | fm1;
-      }
-      if (g0) {
-        level[v0] = (uint8_t)lvl;
-        parent[v0] = p0;
-      }
-      if (g1) {
-        level[v1] = (uint8_t)lvl;
-        parent[v1] = p1;
-      }
-      found_total += __popcll(fm0) + __popcll(fm1);  // identical in every lane
-    }
-  }
-  block_add(lane == 0 ? found_total : 0, stripe_of(counters + kStripeBase, S_FOUND));
-}
-
 // Frontier bitmap -> frontier queue in ascending vertex order: an exclusive
 // scan of per-word popcounts gives every word its output position, so no
 // atomics are involved.  The bits are 'now & ~before' (before may be null).
@@ -866,128 +832,580 @@ __global__ void k_make_levels(const uint32_t* __restrict__ old2new, const uint8_
   }
 }
 
-// --- fused small top-down levels ---------------------------------------------
-// Consecutive top-down levels whose frontiers are small (at most kFuseNf
-// vertices with at most max_edges edges) run inside one launch of one
-// workgroup: per level, the frontier's degree prefix in LDS, its edges taken
-// kFuseThreads at a time (a lane finds its row by binary search in LDS), the
-// visited bitmap test-and-set (plain-load filter, then atomicOr) and the next
-// queue; between levels the workgroup applies the reference's switch rule
-// (mpi/bfs.hpp:2799-2829: a growing top-down level that finds more vertices
-// than the previous one and more than n_active/2000 hands over to bottom-up),
-// so these levels cost no host round trip and no further launches.  The
-// launch stops when a level finds nothing, before a level that pulls, before
-// a frontier too large for it, or at max_levels.  Each level's vertex count
-// and, at the end, the launch's state are published to coherent host memory,
-// every value tagged with the launch's sequence number.
-constexpr int kFuseThreads = 1024;
-constexpr int kFuseNf = 4096;
-constexpr int kFuseMaxLevels = 64;
-enum { F_LEVELS = kFuseMaxLevels, F_STOP, F_QI, F_NF, F_E, F_NUM };
-enum { FUSE_EMPTY = 0, FUSE_PULL = 1, FUSE_LARGE = 2, FUSE_LIMIT = 3 };
+// --- steps: the levels a search decides for itself -----------------------------
+// A search is an init launch and a row of step launches, each of which starts
+// by folding the previous step's vertex count into the search's state and
+// applying the reference's switch rule (mpi/bfs.hpp:2799-2829), so that a
+// level costs one launch and no host round trip (18 us a level before, of 4 to
+// 12 us of kernel on graphs up to SCALE 21).  Every workgroup folds the same
+// values and so takes the same decision; workgroup 0 passes the state on.
+// The host keeps one step queued behind the running one until a step
+// publishes the end; steps launched past it find it and leave.  A step runs
+//   * consecutive small top-down levels (at most kStepNf vertices with at
+//     most small_edges edges each) in workgroup 0 alone;
+//   * a top-down level of at most kTdSmall edges: every workgroup makes the
+//     frontier's degree prefix in LDS, the waves take 256 edges at a time (row
+//     by binary search in LDS), test-and-set the visited bitmap and append
+//     the winners through an LDS list;
+//   * a bottom-up level: a wave reads `span` bitmap words at a time (one
+//     coalesced load, one word per lane, span a power of two from 2 to 64),
+//     copies the words whose vertices are all visited to the next bitmap (one
+//     coalesced store) and walks the others two at a time, one lane per vertex
+//     of each, so both words' first-neighbour probes are in flight together.
+//     The host sizes span so that the grid still has a step per wave or more;
+//     late levels, where almost every word is full, then cost little more than
+//     a pass over the bitmap.  The new vertices are listed as well, as far as
+//     each workgroup's LDS list holds them, for a top-down level that follows;
+// and hands any other level back to the host (larger top-down levels, a
+// frontier whose queue has to be rebuilt from the bitmaps).  Graphs of one
+// workgroup's size run all their levels in one step.
+constexpr int kStepThreads = 1024;
+constexpr int kStepNf = 4096;
+constexpr int kStepList = 2048;    // LDS list of a workgroup's new vertices
+constexpr int kStepTdGrid = 256;   // workgroups of a top-down level: kTdSmall edges are 4,096 waves of 256
+constexpr int kStepMaxLevel = 254; // levels are bytes, 0xFF = unreached
+enum { STEP_GO = 0, STEP_DONE = 1, STEP_LARGE = 2, STEP_QUEUE = 3, STEP_LIMIT = 4, STEP_BOTTOM_UP = 5 };
 
-__global__ void __launch_bounds__(kFuseThreads) k_td_fused(
-    uint32_t* __restrict__ q0, uint32_t* __restrict__ q1, int qi0, int64_t nf0,
-    const uint64_t* __restrict__ offsets, const uint32_t* __restrict__ cols, uint64_t* vis,
-    uint8_t* __restrict__ level, uint32_t* __restrict__ parent, uint32_t lvl0, int max_levels, int64_t max_edges,
-    double na, int64_t prev_nq0, int growing, Published* out, uint64_t seq) {
-  __shared__ uint64_t s_pre[kFuseNf + 1];
-  __shared__ uint32_t s_src[kFuseNf];
-  __shared__ uint64_t s_wave[kFuseThreads / 64];
-  __shared__ uint32_t s_cnt;
-  constexpr int kPer = kFuseNf / kFuseThreads;  // frontier entries per thread in the scan
+struct StepState {
+  int32_t lvl;       // levels completed
+  int32_t stop;
+  int32_t forward, growing;
+  int32_t cur, qi;   // current visited bitmap, queue holding the frontier
+  int32_t queued;    // queue[qi] holds the frontier whole
+  int32_t pending;   // 1: a level has run whose count is still in the counters, 2: by the bottom-up body
+  int64_t nf;        // frontier of the coming level
+  int64_t prev_nq, visited;
+  uint64_t edges;    // its edges, where a step that hands the level back has summed them (0: not known)
+  uint64_t start;    // clock at the start of the pending level
+};
+
+// Control words: three sets of {queue count, list overflow, found stripes} in
+// turn by step (a step adds to its own, reads the previous one's and clears
+// the next one's), the passed state (two slots in turn), the clock of the start.
+constexpr int kSetWords = 2 * kStripeWords + kStripes * kStripeWords;
+enum { SET_QUEUE = 0, SET_OVER = kStripeWords, SET_FOUND = 2 * kStripeWords };
+constexpr int kStateWords = 16;
+static_assert(sizeof(StepState) <= kStateWords * 8, "state slot");
+constexpr int kStepState = 3 * kSetWords;
+constexpr int kStepClock = kStepState + 2 * kStateWords;
+constexpr int kStepArgs = kStepClock + 8;  // the arguments every step reads (StepArgs)
+constexpr int kStepWords = kStepArgs + 32;
+
+// Published: two entries per level (count, kind and clock ticks), then
+enum { P_STEP = 2 * (kStepMaxLevel + 1), P_STOP, P_LVL, P_BITS, P_NF, P_PREV, P_VISITED, P_EDGES, P_TICKS, P_NUM };
+
+struct StepArgs {
+  const uint64_t* offsets;
+  const uint32_t* cols;
+  const uint32_t* first_nbr;
+  uint64_t* vis[2];
+  uint32_t* queue[3];
+  uint8_t* level;
+  uint32_t* parent;
+  Published* pub;
+  int64_t words, n_active, small_edges, tail_pull;
+  int span;
+  int host_bu;  // bottom-up levels go back to the host
+};
+
+__device__ __forceinline__ void step_publish_level(const StepArgs& a, uint64_t seq, int lvl, int64_t nq, int kind,
+                                                   uint64_t ticks) {
+  publish(a.pub + 2 * lvl, ((uint64_t)nq << 2) | (uint64_t)kind, seq);
+  publish(a.pub + 2 * lvl + 1, ticks, seq);
+}
+
+// Least workgroups of a step, the bitmap words and edges up to which one
+// workgroup takes the whole search in one launch, the bitmap words beyond
+// which bottom-up levels go back to the host, and the steps launched ahead.
+constexpr unsigned kStepMinGrid = 64;
+constexpr int64_t kStepAloneWords = 64;
+constexpr int64_t kStepAloneEdges = 1 << 18;
+constexpr int64_t kStepMaxWords = 100000;
+constexpr int kStepAhead = 3;
+
+// Counts a finished level in (kind: bit 0 forward, bit 1 bottom-up body) and
+// applies the switch rule.
+__host__ __device__ __forceinline__ void step_fold(int64_t n_active, StepState& st, int64_t nq) {
+  ++st.lvl;
+  st.visited += nq;
+  st.nf = nq;
+  if (nq == 0) {
+    st.stop = STEP_DONE;
+    return;
+  }
+  const double na = (double)n_active;
+  if (st.growing && nq > st.prev_nq) {
+    if (st.forward && (double)nq > na / 2000.0) st.forward = 0;
+  } else if (!st.forward && n_active - st.visited < (int64_t)(na / 8.0)) {
+    st.forward = 1;
+    st.growing = 0;
+  }
+  st.prev_nq = nq;
+}
+
+// A top-down level after the bottom-up phase whose frontier holds more than
+// 1/tail_pull as many vertices as remain unvisited (and more than kStepNf) is
+// found by the bottom-up body: an unvisited vertex with a visited neighbour is
+// on this level (an older neighbour would have reached it before), so both
+// find the same vertices, and this one probes from the few unvisited ones
+// instead of expanding the frontier.  The level keeps its top-down place in
+// the schedule.
+__host__ __device__ __forceinline__ bool tail_pulls(int forward, int growing, int64_t tail_pull, int64_t nf,
+                                                    int64_t unvisited) {
+  return forward && !growing && tail_pull > 0 && nf > kStepNf && tail_pull * nf > unvisited;
+}
+
+static_assert(sizeof(StepArgs) <= 32 * 8, "argument block");
+
+struct StepLds {
+  uint64_t base[kStepNf];     // cols index of frontier row i's first entry - pre[i]
+  uint32_t pre[kStepNf + 1];  // first virtual edge of the row
+  uint32_t src[kStepNf];
+  uint32_t list[kStepList];
+  uint64_t wave[kStepThreads / 64];
+  uint32_t n;
+  uint64_t lap;  // clock at the start of a level of workgroup 0's own
+  union {
+    StepState st;
+    uint64_t st_words[kStateWords];
+  };
+};
+
+// Degree prefix of the frontier in LDS (cur[0, nf), nf <= kStepNf); returns
+// its edge count.  The 32-bit prefix is whole when that is at most 2^32 - 1.
+__device__ __forceinline__ uint64_t step_prefix(StepLds& L, const uint32_t* __restrict__ cur, int nf,
+                                                const uint64_t* __restrict__ offsets) {
+  constexpr int kPer = kStepNf / kStepThreads;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  int qi = qi0;
-  int64_t nf = nf0, prev_nq = prev_nq0;
-  uint64_t stop = FUSE_LIMIT, E = 0;
-  int k = 0;
-  while (k < max_levels) {
-    const uint32_t* cur = qi ? q1 : q0;
-    uint32_t* nxt = qi ? q0 : q1;
-    if (nf > kFuseNf) {
-      stop = FUSE_LARGE;
-      E = 0;  // not known here
-      break;
-    }
-    // degrees of the frontier, exclusive prefix in LDS (kPer per thread)
-    uint64_t d[kPer], sum = 0;
+  const int per = (nf + kStepThreads - 1) / kStepThreads;  // entries per thread
+  uint64_t o[kPer], d[kPer], sum = 0;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int64_t i = (int64_t)t * kPer + j;
-      d[j] = 0;
-      if (i < nf) {
-        const uint32_t u = cur[i];
-        s_src[i] = u;
-        d[j] = offsets[u + 1] - offsets[u];
-      }
-      sum += d[j];
+  for (int j = 0; j < kPer; ++j) {
+    const int i = t * per + j;
+    o[j] = d[j] = 0;
+    if (j < per && i < nf) {
+      const uint32_t u = cur[i];
+      L.src[i] = u;
+      o[j] = offsets[u];
+      d[j] = offsets[u + 1] - o[j];
     }
-    uint64_t inc = sum;  // inclusive scan of the per-thread sums within the wave
+    sum += d[j];
+  }
+  const uint64_t inc = wave_incl_scan(sum);
+  if (lane == 63) L.wave[wave] = inc;
+  if (t == 0) L.n = 0;
+  __syncthreads();
+  uint64_t run = inc - sum, total = 0;
+  for (int w = 0; w < kStepThreads / 64; ++w) {
+    if (w < wave) run += L.wave[w];
+    total += L.wave[w];
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = t * per + j;
+    if (j < per && i < nf) {
+      L.pre[i] = (uint32_t)run;
+      L.base[i] = o[j] - run;
+    }
+    run += d[j];
+  }
+  __syncthreads();
+  return total;
+}
+
+// Row of virtual edge e: the last one that starts at or before it.
+__device__ __forceinline__ int step_row(const StepLds& L, int nf, uint32_t e) {
+  int lo = 0, hi = nf - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (L.pre[mid] <= e) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+// Sets bit w of the bitmap for every lane with ok; true for the one lane whose
+// claim finds it unset.  Every lane of the wave calls it.  Neighbouring lanes
+// whose targets share a word (a row is sorted, and every row holds the hubs)
+// claim with one atomic: the frontier's rows all meet in the first words, and
+// atomics on one word are performed one after another (160 rows, 10,000 claims
+// of the hubs' words: 0.18 ms of a level of 0.05 at SCALE 23).
+__device__ __forceinline__ bool claim_bits(uint64_t* vis, uint32_t w, bool ok) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t key = ok ? w >> 6 : 0x80000000u | (uint32_t)lane;  // words are below 2^26
+  const uint64_t bit = ok ? UINT64_C(1) << (w & 63) : 0;
+  const uint32_t left = __shfl_up(key, 1, 64);
+  const uint64_t heads = __ballot(lane == 0 || key != left);  // first lanes of the runs
+  const uint64_t upto = ~UINT64_C(0) >> (63 - lane);
+  const int start = 63 - __builtin_clzll(heads & upto);
+  const uint64_t later = heads & ~upto;
+  const int end = later ? __builtin_ctzll(later) - 1 : 63;
+  uint64_t run = bit;  // OR over the run up to this lane
+  if (heads != ~UINT64_C(0)) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const uint64_t x = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += x;
-    }
-    if (lane == 63) s_wave[wave] = inc;
-    if (t == 0) s_cnt = 0;
-    __syncthreads();
-    uint64_t base = 0;
-    for (int w = 0; w < wave; ++w) base += s_wave[w];
-    uint64_t run = base + inc - sum;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int64_t i = (int64_t)t * kPer + j;
-      if (i < nf) s_pre[i] = run;
-      run += d[j];
-    }
-    if (t == kFuseThreads - 1) s_pre[nf] = run;
-    __syncthreads();
-    E = s_pre[nf];
-    if ((int64_t)E > max_edges) {
-      stop = FUSE_LARGE;
-      break;
-    }
-    const uint32_t lvl = lvl0 + (uint32_t)k;
-    for (uint64_t e = t; e < E; e += kFuseThreads) {
-      int lo = 0, hi = (int)nf - 1;  // last row starting at or before e
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (s_pre[mid] <= e) lo = mid; else hi = mid - 1;
-      }
-      const uint32_t u = s_src[lo];
-      const uint32_t w = cols[offsets[u] + (e - s_pre[lo])];
-      const uint64_t bit = UINT64_C(1) << (w & 63);
-      if (vis[w >> 6] & bit) continue;
-      const uint64_t old = atomicOr((unsigned long long*)(vis + (w >> 6)), (unsigned long long)bit);
-      if (old & bit) continue;
-      level[w] = (uint8_t)lvl;
-      parent[w] = u;
-      nxt[atomicAdd(&s_cnt, 1u)] = w;
-    }
-    __syncthreads();
-    const int64_t nq = s_cnt;
-    if (t == 0) publish(out + k, (uint64_t)nq, seq);
-    const bool pull = growing && nq > prev_nq && (double)nq > na / 2000.0;
-    prev_nq = nq;
-    nf = nq;
-    qi ^= 1;
-    ++k;
-    __syncthreads();  // every lane has read s_cnt and s_pre before the next level writes them
-    if (nq == 0) {
-      stop = FUSE_EMPTY;
-      break;
-    }
-    if (pull) {
-      stop = FUSE_PULL;
-      break;
+      const uint64_t x = __shfl_up(run, o, 64);
+      if (lane - o >= start) run |= x;
     }
   }
-  if (t == 0) {
-    publish(out + F_LEVELS, (uint64_t)k, seq);
-    publish(out + F_STOP, stop, seq);
-    publish(out + F_QI, (uint64_t)qi, seq);
-    publish(out + F_NF, (uint64_t)nf, seq);
-    publish(out + F_E, E, seq);
+  uint64_t before = __shfl_up(run, 1, 64);
+  if (lane == start) before = 0;
+  uint64_t old = 0;
+  if (ok && lane == end) old = atomicOr((unsigned long long*)(vis + key), (unsigned long long)run);
+  old = __shfl(old, end, 64);
+  return ok && !((old | before) & bit);
+}
+
+// A lane's claims of the edges e, e + stride, ... below end, four in flight:
+// rows, columns and the bitmap filter of all four before the first claim.
+// Every lane of the wave calls it.
+template <class F>
+__device__ __forceinline__ void step_expand(const StepArgs& a, const StepLds& L, int nf, uint64_t* vis, uint32_t e,
+                                            uint32_t end, uint32_t stride, int lvl, F&& append) {
+  uint32_t w[4], u[4];
+  bool ok[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t x = e + j * stride;
+    ok[j] = x < end;
+    w[j] = u[j] = 0;
+    if (ok[j]) {
+      const int i = step_row(L, nf, x);
+      u[j] = L.src[i];
+      w[j] = a.cols[L.base[i] + x];
+    }
+  }
+  uint64_t b[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) b[j] = ok[j] ? vis[w[j] >> 6] : 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ok[j] = claim_bits(vis, w[j], ok[j] && !((b[j] >> (w[j] & 63)) & 1));
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (ok[j]) {
+      a.level[w[j]] = (uint8_t)lvl;
+      a.parent[w[j]] = u[j];
+      append(w[j]);
+    }
+}
+
+// The bottom-up body over waves wave0, wave0 + nwaves, ...; with a list (LDS,
+// kStepList entries and their count) found vertices are appended to it.
+// Returns the wave's count (in every lane).
+template <int kU, int kR>
+__device__ __forceinline__ uint64_t step_bottom_up(const StepArgs& a, uint32_t* list, uint32_t* list_n,
+                                                   const uint64_t* __restrict__ vis, uint64_t* __restrict__ vis_next,
+                                                   int lvl, int64_t wave0, int64_t nwaves) {
+  const int lane = threadIdx.x & 63, span = a.span;
+  const uint64_t below = lane ? ~UINT64_C(0) >> (64 - lane) : 0;
+  uint64_t total = 0;
+  for (int64_t base = wave0 * span; base < a.words; base += nwaves * span) {
+    const int64_t wl = base + lane;
+    const bool mine = lane < span && wl < a.words;
+    const uint64_t cl = mine ? vis[wl] : ~UINT64_C(0);  // lanes beyond the span or the end read as visited
+    uint64_t open = __ballot(cl != ~UINT64_C(0));        // words with an unvisited vertex
+    if (mine && cl == ~UINT64_C(0)) vis_next[wl] = cl;
+    while (open) {
+      // the next two open words (identical in every lane)
+      const int j0 = __builtin_ctzll(open);
+      open &= open - 1;
+      const bool has1 = open != 0;
+      const int j1 = has1 ? __builtin_ctzll(open) : j0;
+      if (has1) open &= open - 1;
+      const uint64_t c0 = __shfl(cl, j0, 64);
+      const uint64_t c1 = has1 ? __shfl(cl, j1, 64) : ~UINT64_C(0);
+      const int64_t w0 = base + j0, w1 = base + j1;
+      const uint32_t v0 = (uint32_t)(w0 * 64 + lane), v1 = (uint32_t)(w1 * 64 + lane);
+      const bool a0 = !((c0 >> lane) & 1), a1 = !((c1 >> lane) & 1);
+      const uint32_t f0 = a0 ? a.first_nbr[v0] : kNoNbr;
+      const uint32_t f1 = a1 ? a.first_nbr[v1] : kNoNbr;
+      const bool h0 = f0 != kNoNbr && bit_set(vis, f0);
+      const bool h1 = f1 != kNoNbr && bit_set(vis, f1);
+      uint32_t p0 = f0, p1 = f1;
+      // every lane makes both calls (the long-row scan needs the whole wave)
+      const bool r0 = row_marked_nbr<kU, kR>(f0 != kNoNbr && !h0, v0, vis, a.offsets, a.cols, p0);
+      const bool r1 = row_marked_nbr<kU, kR>(f1 != kNoNbr && !h1, v1, vis, a.offsets, a.cols, p1);
+      const bool g0 = h0 || r0, g1 = h1 || r1;
+      const uint64_t m0 = __ballot(g0), m1 = __ballot(g1);
+      const uint32_t n0 = (uint32_t)__popcll(m0), n1 = (uint32_t)__popcll(m1);
+      uint32_t pos = 0;
+      if (lane == 0) {
+        vis_next[w0] = c0 | m0;
+        if (has1) vis_next[w1] = c1 | m1;
+        // a full list stays full: further counts are not needed
+        pos = kStepList;
+        if (list && n0 + n1 && *list_n <= (uint32_t)kStepList) pos = atomicAdd(list_n, n0 + n1);
+      }
+      if (list) pos = __builtin_amdgcn_readfirstlane(pos);
+      if (g0) {
+        a.level[v0] = (uint8_t)lvl;
+        a.parent[v0] = p0;
+        const uint32_t i = pos + (uint32_t)__popcll(m0 & below);
+        if (list && i < (uint32_t)kStepList) list[i] = v0;
+      }
+      if (g1) {
+        a.level[v1] = (uint8_t)lvl;
+        a.parent[v1] = p1;
+        const uint32_t i = pos + n0 + (uint32_t)__popcll(m1 & below);
+        if (list && i < (uint32_t)kStepList) list[i] = v1;
+      }
+      total += n0 + n1;
+    }
+  }
+  return total;
+}
+
+// The address of the argument block, opaque from here on: fields are loaded
+// where they are used instead of being held in registers across the bodies.
+__device__ __forceinline__ const StepArgs& step_args(const unsigned long long* ctl) {
+  const StepArgs* p = reinterpret_cast<const StepArgs*>(ctl + kStepArgs);
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
+__global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* __restrict__ ctl, int k, uint64_t seq) {
+  __shared__ StepLds L;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const bool lead = blockIdx.x == 0;
+  const uint64_t now = wall_clock64();
+  // the state, with the previous step's level folded in (the same in every workgroup)
+  if (wave == 0) {
+    const unsigned long long* const set_prev = ctl + ((k + 2) % 3) * kSetWords;
+    const uint64_t f = set_prev[SET_FOUND + lane * kStripeWords], over = set_prev[SET_OVER];
+    if (lane < kStateWords) L.st_words[lane] = ctl[kStepState + ((k + 1) & 1) * kStateWords + lane];
+    const int64_t nq = (int64_t)wave_sum(f);
+    if (lane == 0) {
+      const StepArgs& a = step_args(ctl);
+      StepState& st = L.st;
+      if (!st.stop && st.pending) {
+        const bool bu = st.pending == 2;
+        if (lead) step_publish_level(a, seq, st.lvl + 1, nq, st.forward | (st.pending & 2), now - st.start);
+        st.queued = !bu || (nq <= kStepNf && !over);
+        st.qi = st.qi == 2 ? 0 : st.qi + 1;
+        if (bu) st.cur ^= 1;
+        st.pending = 0;
+        step_fold(a.n_active, st, nq);
+      }
+      if (!st.stop && st.nf == 0) st.stop = STEP_DONE;
+      L.lap = now;
+    }
+  }
+  if (lead) {
+    unsigned long long* const set_next = ctl + ((k + 1) % 3) * kSetWords;
+    for (int i = t; i < kSetWords; i += kStepThreads) set_next[i] = 0;
+    if (t == 64) publish(step_args(ctl).pub + P_STEP, (uint64_t)k + 1, seq);
+  }
+  __syncthreads();
+  const bool alone = gridDim.x == 1;
+  // The queue the step starts from stays as it is while the step runs: every
+  // workgroup makes its prefix, some after workgroup 0 has gone on to the next
+  // small level.  Small levels use the other two in turn.
+  const int entry = L.st.qi, lvl0 = L.st.lvl + 1;
+  while (!L.st.stop) {
+    const int lvl = __builtin_amdgcn_readfirstlane(L.st.lvl) + 1;
+    int stop = STEP_GO;
+    uint64_t E = 0;
+    bool td = false;
+    {
+      const StepArgs& a = step_args(ctl);
+      td = L.st.forward &&
+           !tail_pulls(L.st.forward, L.st.growing, a.tail_pull, L.st.nf, a.n_active - L.st.visited);
+      if (lvl > kStepMaxLevel) stop = STEP_LIMIT;
+      else if (td && !L.st.queued) stop = STEP_QUEUE;
+      else if (td && L.st.nf > kStepNf) stop = STEP_LARGE;
+      else if (!td && a.host_bu) stop = STEP_BOTTOM_UP;
+      if (!stop && td) {
+        if (blockIdx.x >= kStepTdGrid) return;
+        E = step_prefix(L, a.queue[L.st.qi], (int)L.st.nf, a.offsets);
+        if (E > kTdSmall) stop = STEP_LARGE;
+      }
+    }
+    if (stop) {
+      __syncthreads();  // every thread has read L.st
+      if (t == 0) {
+        L.st.stop = stop;
+        L.st.edges = E;
+      }
+      __syncthreads();
+      break;
+    }
+    const int qi = __builtin_amdgcn_readfirstlane(L.st.qi);
+    const int nqi = qi == entry ? (entry == 2 ? 0 : entry + 1) : 3 - entry - qi;
+    unsigned long long* const set = ctl + (k % 3) * kSetWords;
+    if (td) {
+      const StepArgs& a = step_args(ctl);
+      const bool small = alone || (int64_t)E <= a.small_edges;
+      if (small && !lead) return;
+      if (!small && lvl != lvl0) break;  // the other workgroups left at the first small level: the next step's
+      const int nf = __builtin_amdgcn_readfirstlane((int)L.st.nf);
+      uint64_t* const vis = a.vis[L.st.cur];
+      uint32_t* const next = a.queue[nqi];
+      if (small) {
+        // the winners straight into the next queue
+        for (uint32_t e = t; (e & ~63u) < (uint32_t)E; e += 4 * kStepThreads)  // whole waves
+          step_expand(a, L, nf, vis, e, (uint32_t)E, kStepThreads, lvl,
+                      [&](uint32_t w) { next[atomicAdd(&L.n, 1u)] = w; });
+        __syncthreads();
+        // the bitmap words the atomics changed are read past this CU's cache by a bottom-up level
+        if (alone) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (t == 0) {
+          const uint32_t n = L.n;
+          const uint64_t end = wall_clock64();
+          step_publish_level(a, seq, lvl, (int64_t)n, L.st.forward, end - L.lap);
+          L.lap = end;
+          L.st.qi = nqi;
+          L.st.queued = 1;
+          step_fold(a.n_active, L.st, (int64_t)n);
+        }
+        __syncthreads();
+        if (!alone && (!L.st.forward || tail_pulls(L.st.forward, L.st.growing, a.tail_pull, L.st.nf,
+                                                   a.n_active - L.st.visited)))
+          break;  // a bottom-up level takes the grid
+        continue;
+      }
+      // consecutive stretches go to different workgroups, so that the winners
+      // spread over their lists (past a full list each costs a global atomic)
+      const uint32_t nblk = gridDim.x < kStepTdGrid ? gridDim.x : kStepTdGrid;
+      for (uint32_t c = wave * nblk + blockIdx.x; (uint64_t)c * 256 < E; c += nblk * (kStepThreads / 64)) {
+        const uint64_t end = (uint64_t)(c + 1) * 256 < E ? (uint64_t)(c + 1) * 256 : E;
+        step_expand(a, L, nf, vis, c * 256 + lane, (uint32_t)end, 64, lvl, [&](uint32_t w) {
+          const uint32_t pos = atomicAdd(&L.n, 1u);
+          if (pos < (uint32_t)kStepList) L.list[pos] = w;
+          else next[atomicAdd(set + SET_QUEUE, 1ull)] = w;
+        });
+      }
+    } else {
+      if (t == 0) L.n = 0;
+      __syncthreads();
+      const StepArgs& a = step_args(ctl);
+      const int cur = __builtin_amdgcn_readfirstlane(L.st.cur);
+      const uint64_t f = step_bottom_up<8, 4>(a, L.list, &L.n, a.vis[cur], a.vis[cur ^ 1], lvl,
+                                              (int64_t)blockIdx.x * (kStepThreads / 64) + wave,
+                                              (int64_t)gridDim.x * (kStepThreads / 64));
+      if (lane == 0) L.wave[wave] = f;
+    }
+    __syncthreads();
+    // the level's vertices so far (a top-down level: all were listed or queued)
+    const StepArgs& a = step_args(ctl);
+    uint32_t* const next = a.queue[nqi];
+    const uint32_t n = L.n;
+    uint64_t found = 0;
+    if (td) {
+      found = n;
+    } else {
+      for (int w = 0; w < kStepThreads / 64; ++w) found += L.wave[w];
+    }
+    const bool whole = td || n <= (uint32_t)kStepList;  // a full list says nothing about the rest
+    const uint32_t listed = !whole ? 0 : (n < (uint32_t)kStepList ? n : (uint32_t)kStepList);
+    if (alone) {
+      // a bottom-up level of the only workgroup
+      for (uint32_t i = t; i < listed; i += kStepThreads) next[i] = L.list[i];
+      __syncthreads();
+      if (t == 0) {
+        const uint64_t end = wall_clock64();
+        step_publish_level(a, seq, lvl, (int64_t)found, L.st.forward | 2, end - L.lap);
+        L.lap = end;
+        L.st.qi = nqi;
+        L.st.cur ^= 1;
+        L.st.queued = whole;
+        step_fold(a.n_active, L.st, (int64_t)found);
+      }
+      __syncthreads();
+      continue;
+    }
+    // a level of the whole grid: the next step folds it
+    __syncthreads();  // L.wave has been read
+    if (t == 0) {
+      if (found) atomicAdd(set + SET_FOUND + (blockIdx.x % kStripes) * kStripeWords, (unsigned long long)found);
+      if (!whole) set[SET_OVER] = 1;
+      L.wave[0] = listed ? atomicAdd(set + SET_QUEUE, (unsigned long long)listed) : 0;
+      if (lead) {
+        L.st.pending = td ? 1 : 2;
+        L.st.start = L.lap;
+      }
+    }
+    __syncthreads();
+    const uint64_t at = L.wave[0];
+    for (uint32_t i = t; i < listed; i += kStepThreads) next[at + i] = L.list[i];
+    if (lead && t < kStateWords) ctl[kStepState + (k & 1) * kStateWords + t] = L.st_words[t];
+    return;
+  }
+  // the end, a level for the host, or a level of the whole grid after small ones
+  if (!lead) return;
+  if (t < kStateWords) ctl[kStepState + (k & 1) * kStateWords + t] = L.st_words[t];
+  if (L.st.stop && t >= 64 && t < 64 + 8) {
+    const StepState& st = L.st;
+    uint64_t v = 0;
+    switch (t - 64 + P_STOP) {
+      case P_STOP: v = (uint64_t)st.stop; break;
+      case P_LVL: v = (uint64_t)st.lvl; break;
+      case P_BITS:
+        v = (uint64_t)(st.forward | (st.growing << 1) | (st.cur << 2) | (st.queued << 3) | (st.qi << 4));
+        break;
+      case P_NF: v = (uint64_t)st.nf; break;
+      case P_PREV: v = (uint64_t)st.prev_nq; break;
+      case P_VISITED: v = (uint64_t)st.visited; break;
+      case P_EDGES: v = st.edges; break;
+      default: v = wall_clock64() - ctl[kStepClock]; break;
+    }
+    publish(step_args(ctl).pub + P_STOP + (t - 64), v, seq);
+  }
+}
+
+// A bottom-up level of a large graph, launched by the host: the body above in
+// 256-thread workgroups without a list, at twice the waves per CU a step
+// leaves room for (its registers and LDS hold 16).
+__global__ void __launch_bounds__(kBlock) k_bu(StepArgs a, int cur, int lvl, unsigned long long* __restrict__ counters) {
+  const uint64_t f = step_bottom_up<4, 1>(a, nullptr, nullptr, a.vis[cur], a.vis[cur ^ 1], lvl,
+                                          (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
+                                          (int64_t)gridDim.x * (kBlock / 64));
+  block_add((threadIdx.x & 63) == 0 ? f : 0, stripe_of(counters + kStripeBase, S_FOUND));
+}
+
+// The state a row of steps goes on from after a level run by the host (slot:
+// the one the next step reads).
+__global__ void k_step_resume(unsigned long long* __restrict__ ctl, StepState st, int k) {
+  *reinterpret_cast<StepState*>(ctl + kStepState + ((k + 1) & 1) * kStateWords) = st;
+}
+
+// Everything a search starts from: levels unreached, the visited bitmap (bits
+// past the last row read as visited so no sweep ever picks them), the root on
+// level 0 and in the queue, the control words and level counters zero.
+__global__ void __launch_bounds__(kBlock) k_bfs_init(const uint32_t* __restrict__ old2new, int64_t root_orig,
+                                                     int64_t rows, int64_t words, uint8_t* __restrict__ level,
+                                                     uint32_t* __restrict__ parent, uint64_t* __restrict__ vis,
+                                                     uint32_t* __restrict__ queue, unsigned long long* __restrict__ ctl,
+                                                     unsigned long long* __restrict__ counters, StepArgs args) {
+  const int64_t stride = (int64_t)gridDim.x * kBlock, me = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t r = old2new[root_orig];  // >= rows for a root without edges (modes 1 and 2)
+  for (int64_t q = me; q * 16 < rows; q += stride) {
+    if (q * 16 + 16 <= rows && (r < q * 16 || r >= q * 16 + 16)) {
+      reinterpret_cast<uint4*>(level)[q] = uint4{~0u, ~0u, ~0u, ~0u};
+    } else {
+      for (int64_t v = q * 16; v < q * 16 + 16 && v < rows; ++v) level[v] = v == r ? 0 : 0xFF;
+    }
+  }
+  for (int64_t w = me; w < words; w += stride) {
+    const int64_t first = w * 64;
+    uint64_t x = 0;
+    if (first + 64 > rows) x = ~UINT64_C(0) << (rows - first);
+    if (r < rows && (r >> 6) == w) x |= UINT64_C(1) << (r & 63);
+    vis[w] = x;
+  }
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < 3 * kSetWords; i += kBlock) ctl[i] = 0;
+    for (int i = threadIdx.x; i < kBfsCounters; i += kBlock) counters[i] = 0;
+    if (threadIdx.x == 0) {
+      ctl[kStepClock] = wall_clock64();
+      *reinterpret_cast<StepArgs*>(ctl + kStepArgs) = args;
+      StepState st{};
+      st.forward = st.growing = st.queued = 1;
+      st.nf = st.visited = 1;
+      *reinterpret_cast<StepState*>(ctl + kStepState + kStateWords) = st;  // the slot step 0 reads
+      if (r < rows) {
+        parent[r] = (uint32_t)r;
+        queue[0] = (uint32_t)r;
+      }
+    }
   }
 }
 
@@ -1072,10 +1490,14 @@ void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   G5_HIP(hipStreamSynchronize(s));  // the published blocks are reset below
   b.pub.alloc(C_NUM);
   b.pub_seq = 0;
-  b.fuse.alloc(F_NUM);
-  b.fuse_seq = 0;
-  if (!b.ev0) G5_HIP(hipEventCreate(&b.ev0));
-  if (!b.ev1) G5_HIP(hipEventCreate(&b.ev1));
+  b.step_ctl.alloc(kStepWords);
+  b.step_pub.alloc(P_NUM);
+  b.step_seq = 0;
+  if (!b.tick_khz) {
+    int khz = 0;
+    G5_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+    b.tick_khz = khz > 0 ? khz : 100000;
+  }
   b.prepared = true;
 }
 
@@ -1098,6 +1520,277 @@ static void build_hub_index(g5_ctx* ctx, BfsState& b, hipStream_t s) {
 
 void bfs_run(g5_ctx* ctx, int64_t root) { bfs_run(ctx, ctx->bfs, ctx->stream, root); }
 
+// A top-down level too large for a step: the frontier's rows as one virtual
+// edge list over the whole grid (see k_td_expand), then the switch rule.
+static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& state) {
+  Graph& g = ctx->graph;
+  const int64_t rows = g.n_rows, nf = state.nf, visited = state.visited;
+  const int lvl = state.lvl + 1, cur = state.cur, qi = state.qi, qn = (qi + 1) % 3;
+  const double na = (double)g.n_active;
+  unsigned long long* cnt = (unsigned long long*)b.counters.p;
+  g5_bfs_stats& st = b.stats;
+  // the frontier's edges when the step summed them (-1: not known, both forms
+  // are launched and the device picks)
+  const int64_t e_next = state.edges ? (int64_t)state.edges : -1;
+  G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
+  device_scan(FrontierDegree{b.queue[qi].p, g.offsets.p, nf}, StoreU64{b.prefix.p},
+              (size_t)nf + 1, b.scan_tmp.p, s);
+  if (b.bin_edges > 0) {
+    // the binned form sizes its pair buffer from E: wait for it
+    G5_HIP(hipMemcpyAsync(b.h_counters + 1, b.prefix.p + nf, 8, hipMemcpyDeviceToHost, s));
+    G5_HIP(hipStreamSynchronize(s));
+  }
+  const uint64_t E_known = b.bin_edges > 0 ? b.h_counters[1] : 0;
+  // past the bottom-up phase most targets are visited: a bulk level then
+  // tests the visited bitmap before the level array
+  const int probe_vis = (double)visited > na / 4 ? 1 : 0;
+  // the level's frontier edge count when the previous level summed it
+  const bool known_small = e_next >= 0 && (uint64_t)e_next <= kTdSmall;
+  const bool known_bulk = e_next >= 0 && (uint64_t)e_next > kTdSmall;
+  // while the search grows, a bulk level can take its rows block by
+  // block (exact target blocks) or piece by piece (positional pieces)
+  const int64_t seg_max = b.seg_max > 0 ? std::min<int64_t>(b.seg_max, kSegMax) : kSegMax;
+  const bool blocked = b.hub_shift > 0 && !probe_vis && nf * b.hub_pieces <= seg_max;
+  // a growing bulk level settles its highest-degree targets bottom-up
+  // first (degree order only)
+  bool head = b.td_head > 0 && !probe_vis && g.reorder_mode == 2;
+  if (head && e_next > (int64_t)kTdSmall) {
+    // E known on the host: no head when no row reaches the threshold
+    // (the same test k_td_head_size makes)
+    const double r = (double)g.nnz / (double)e_next;
+    if ((double)b.td_head / 16.0 * r * r > (double)g.max_degree) head = false;
+  }
+  unsigned long long* head_words = head ? cnt + C_HEAD : nullptr;
+  const bool pieces = blocked || (b.td_pieces > 0 && !probe_vis && nf * b.td_pieces <= seg_max);
+  // with a head and row order, the expansion walks row suffixes (one
+  // segment per frontier row: the segment count field bounds nf)
+  if (head && !pieces && nf > seg_max) head = false;
+  head_words = head ? cnt + C_HEAD : nullptr;
+  const bool suffix = head && !pieces;
+  const bool binned = b.bin_edges > 0 && E_known > kTdSmall && E_known >= (uint64_t)b.bin_edges;
+  // Without binning no launch waits for E on the host: chunk rows and the
+  // expansion take upper-bound grids and read E (prefix[nf]) on the
+  // device; the small and the bulk expansion are both launched and the
+  // one that does not fit E exits at once, as does k_td_finish after a
+  // small level.  The host learns E with the level's counters.
+  const uint64_t max_chunks = b.chunk_rows.n / 2;  // sized for every edge of the graph
+  const uint64_t nchunks = b.bin_edges > 0 ? (E_known + kEpb - 1) / kEpb : max_chunks;
+  const unsigned grid = b.bin_edges > 0 ? grid_of((int64_t)E_known, kEpb, 2048) : 2048u;
+  if (nchunks)
+    hipLaunchKernelGGL(k_chunk_rows<kEpb>,
+                       dim3(b.bin_edges > 0 ? grid_of((int64_t)(2 * nchunks), kBlock, 65536) : 4096u),
+                       dim3(kBlock), 0, s, b.prefix.p, nf, nchunks, b.chunk_rows.p);
+  if (!known_bulk)
+    hipLaunchKernelGGL(k_td_expand<false>, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
+                       b.chunk_rows.p, g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p,
+                       b.queue[qn].p, cnt, (uint32_t)lvl, 0, nullptr);
+  if (head && !binned && !known_small) {
+    hipLaunchKernelGGL(k_td_head_size, dim3(1), dim3(1), 0, s, b.prefix.p, nf, g.offsets.p, rows, b.words,
+                       (double)g.nnz, (double)b.td_head / 16.0, head_words);
+    hipLaunchKernelGGL(k_td_head, dim3(grid_of(b.words, kBlock / 64, 8192)), dim3(kBlock), 0, s,
+                       b.vis[cur].p, g.first_nbr.p, g.offsets.p, g.cols.p, b.level.p, b.parent.p, head_words,
+                       (uint32_t)lvl);
+    G5_HIP(hipGetLastError());
+  }
+  if (known_small) {
+    // nothing else to launch: the small expansion keeps the queue exact
+  } else if (binned) {
+    // binned by target range (see k_td_bin_count)
+    const uint64_t E = E_known;
+    int shift = kBinShift;
+    while ((rows >> shift) >= kBinMaxBuckets) ++shift;
+    const int nb = (int)(((rows - 1) >> shift) + 1);
+    b.bin_pairs.alloc(E);
+    b.bin_cnt.alloc(2 * kBinMaxBuckets);
+    unsigned long long* bc = (unsigned long long*)b.bin_cnt.p;
+    G5_HIP(hipMemsetAsync(bc, 0, nb * 8, s));
+    hipLaunchKernelGGL(k_td_bin_count, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
+                       b.chunk_rows.p, g.offsets.p, g.cols.p, shift, nb, bc);
+    hipLaunchKernelGGL(k_td_bin_offsets, dim3(1), dim3(kBlock), 0, s, bc, nb, bc + kBinMaxBuckets);
+    hipLaunchKernelGGL(k_td_bin_scatter, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
+                       b.chunk_rows.p, g.offsets.p, g.cols.p, shift, nb, bc + kBinMaxBuckets, b.bin_pairs.p);
+    hipLaunchKernelGGL(k_td_bin_apply, dim3(grid_of((int64_t)E, kBlock, 2048)), dim3(kBlock), 0, s,
+                       b.bin_pairs.p, E, b.level.p, b.parent.p, (uint32_t)lvl);
+  } else if (pieces || suffix) {
+    // segment-list bulk level; a small level makes an empty segment list
+    // and the expansion exits (both read E on the device)
+    const size_t np = (size_t)(suffix ? nf : nf * (blocked ? b.hub_pieces : b.td_pieces)) + 1;
+    b.seg_pre.alloc(np);
+    b.seg_base.alloc(np);
+    b.seg_src.alloc(np);
+    b.seg_count.alloc(1);
+    b.seg_scan_tmp.alloc(scan_tmp_elems(np));
+    if (suffix) {
+      b.seg_start.alloc(np);
+      hipLaunchKernelGGL(k_suffix_start, dim3(grid_of(nf, kBlock, 4096)), dim3(kBlock), 0, s, b.queue[qi].p, nf,
+                         b.prefix.p, g.offsets.p, g.cols.p, head_words, b.seg_start.p);
+      const SuffixLen sl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, 1, b.seg_start.p};
+      device_scan(sl, PieceEmit<SuffixLen>{sl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
+                  b.seg_scan_tmp.p, s);
+    } else if (blocked) {
+      const BlockLen bl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, b.hub_pieces, b.hub_bnd.p, b.hub_rows};
+      device_scan(bl, PieceEmit<BlockLen>{bl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
+                  b.seg_scan_tmp.p, s);
+    } else {
+      const PieceLen pl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, b.td_pieces};
+      device_scan(pl, PieceEmit<PieceLen>{pl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
+                  b.seg_scan_tmp.p, s);
+    }
+    hipLaunchKernelGGL(k_chunk_segs, dim3(4096), dim3(kBlock), 0, s, b.seg_pre.p, b.seg_count.p, max_chunks,
+                       b.chunk_rows.p);
+    hipLaunchKernelGGL(k_td_expand_segs, dim3(grid), dim3(kBlock), 0, s, b.prefix.p, nf, b.seg_pre.p,
+                       b.seg_base.p, b.seg_src.p, b.seg_count.p, b.chunk_rows.p, g.cols.p, b.vis[cur].p,
+                       b.level.p, b.parent.p, (uint32_t)lvl, head_words);
+  } else {
+    hipLaunchKernelGGL(k_td_expand<true>, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
+                       b.chunk_rows.p, g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p,
+                       (uint32_t*)nullptr, cnt, (uint32_t)lvl, probe_vis, binned ? nullptr : head_words);
+  }
+  G5_HIP(hipGetLastError());
+  // after a bulk level, k_td_finish makes vis[cur^1] exactly this level's
+  // vertices and adds them to vis[cur]
+  if (!known_small)
+    hipLaunchKernelGGL(k_td_finish, dim3(grid_of((b.words + 15) / 16, kBlock / 64, 8192)), dim3(kBlock), 0,
+                       s, b.level.p, rows, b.words, (uint32_t)lvl, b.vis[cur].p, b.vis[cur ^ 1].p, cnt,
+                       b.prefix.p, nf);
+  G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
+  ++b.pub_seq;
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, 1, b.pub.d, b.pub_seq);
+  G5_HIP(hipGetLastError());
+  wait_published(b, s);
+  const int64_t nq = (int64_t)b.h_counters[C_FOUND];
+  const bool bulk = b.h_counters[C_AUX] > kTdSmall;
+  st.direction[lvl] = 1;
+  st.nq[lvl] = nq;
+  st.num_levels = lvl + 1;
+  float lms = 0;
+  G5_HIP(hipEventSynchronize(b.lev_end[lvl]));
+  G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[lvl], b.lev_end[lvl]));
+  st.level_ms[lvl] = lms;
+  ++state.lvl;
+  state.visited += nq;
+  state.nf = nq;
+  if (nq == 0) return;
+  // direction switch, mpi/bfs.hpp:2799-2829 (a top-down level hands over to bottom-up or goes on)
+  if (state.growing && nq > state.prev_nq && (double)nq > na / 2000.0) state.forward = 0;
+  state.prev_nq = nq;
+  // The next top-down level needs this level's vertices as a queue, unless
+  // the bottom-up body takes it.  A small level appended them to queue[qn];
+  // a bulk one left them in vis[cur^1].
+  if (!bulk) {
+    state.qi = qn;
+  } else if (state.forward &&
+             !tail_pulls(1, state.growing, b.tail_pull, nq, g.n_active - state.visited)) {
+    device_scan(FrontierBits{b.vis[cur ^ 1].p, nullptr}, FrontierEmit{b.vis[cur ^ 1].p, nullptr, b.queue[qi].p},
+                (size_t)b.words, b.scan_tmp.p, s);
+  }
+}
+
+// The frontier after a bottom-up level as a queue: vis[cur] & ~vis[cur ^ 1].
+static void queue_from_bitmaps(BfsState& b, hipStream_t s, StepState& state) {
+  const uint64_t *now = b.vis[state.cur].p, *before = b.vis[state.cur ^ 1].p;
+  device_scan(FrontierBits{now, before}, FrontierEmit{now, before, b.queue[state.qi].p}, (size_t)b.words, b.scan_tmp.p,
+              s);
+  state.queued = 1;
+}
+
+// Bottom-up levels launched one by one, the next once the count of the last
+// is known: on large graphs the round trip is small next to the level, and
+// k_bu runs more waves than a step.  Returns before a top-down level that
+// the top-down kernels take.
+static void host_bottom_up(g5_ctx* ctx, BfsState& b, hipStream_t s, const StepArgs& a, StepState& state) {
+  Graph& g = ctx->graph;
+  unsigned long long* cnt = (unsigned long long*)b.counters.p;
+  g5_bfs_stats& st = b.stats;
+  const int lvl0 = state.lvl + 1;
+  while (state.nf && (!state.forward || tail_pulls(state.forward, state.growing, b.tail_pull, state.nf,
+                                                   g.n_active - state.visited))) {
+    const int lvl = state.lvl + 1;
+    if (lvl > kStepMaxLevel) break;
+    G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
+    hipLaunchKernelGGL(k_bu, dim3(grid_of((b.words + a.span - 1) / a.span, kBlock / 64, 8192)), dim3(kBlock), 0, s, a,
+                       state.cur, lvl, cnt);
+    G5_HIP(hipGetLastError());
+    G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
+    ++b.pub_seq;
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, (int64_t)0, 0, b.pub.d, b.pub_seq);
+    G5_HIP(hipGetLastError());
+    wait_published(b, s);
+    const int64_t nq = (int64_t)b.h_counters[C_FOUND];
+    st.direction[lvl] = state.forward;
+    st.bu_kernel[lvl] = 1;
+    st.nq[lvl] = nq;
+    st.num_levels = lvl + 1;
+    state.cur ^= 1;
+    state.queued = 0;
+    step_fold(g.n_active, state, nq);
+  }
+  for (int l = lvl0; l <= state.lvl; ++l) {
+    float lms = 0;
+    G5_HIP(hipEventSynchronize(b.lev_end[l]));
+    G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[l], b.lev_end[l]));
+    st.level_ms[l] = lms;
+  }
+  state.stop = STEP_GO;
+  if (state.nf && state.forward) queue_from_bitmaps(b, s, state);
+}
+
+// Workgroups of a step: one for the smallest graphs; else enough waves for a
+// turn of every wave in a bottom-up level, and at least kStepMinGrid for the
+// top-down levels.
+static unsigned step_grid(const Graph& g, const BfsState& b, int span) {
+  if (b.words <= kStepAloneWords && g.nnz <= kStepAloneEdges) return 1;
+  return std::max(kStepMinGrid, grid_of((b.words + span - 1) / span, kStepThreads / 64, kStepTdGrid * 2));
+}
+
+// Steps until one stops; returns its state (see k_bfs_step).  k counts the
+// search's steps; kStepAhead of them wait behind the running one.
+static StepState run_steps(BfsState& b, hipStream_t s, unsigned grid, int lvl0, int& k) {
+  const uint64_t seq = ++b.step_seq;
+  const int k0 = k, ahead = grid == 1 ? 0 : kStepAhead;
+  const PublishBlock& pub = b.step_pub;
+  for (uint64_t spins = 1; !pub.ready(P_STOP, P_STOP + 1, seq); ++spins) {
+    const int started = pub.ready(P_STEP, P_STEP + 1, seq) ? (int)pub.value(P_STEP) : k0;
+    if (k - started < std::max(ahead, k == k0 ? 1 : 0) || k - k0 < ahead) {
+      hipLaunchKernelGGL(k_bfs_step, dim3(grid), dim3(kStepThreads), 0, s, (unsigned long long*)b.step_ctl.p, k, seq);
+      G5_HIP(hipGetLastError());
+      ++k;
+    } else if (spins % 4096 == 0) {
+      const hipError_t e = hipStreamQuery(s);
+      if (e == hipErrorNotReady) continue;
+      G5_HIP(e);
+      G5_CHECK(pub.ready(P_STEP, P_STEP + 1, seq), "g5_run_bfs: a step was not published");
+    }
+  }
+  pub.wait(P_STOP, P_NUM, seq, s, "g5_run_bfs: the last step's state was not published");
+  StepState r{};
+  r.stop = (int32_t)pub.value(P_STOP);
+  r.lvl = (int32_t)pub.value(P_LVL);
+  const uint64_t bits = pub.value(P_BITS);
+  r.forward = bits & 1;
+  r.growing = (bits >> 1) & 1;
+  r.cur = (bits >> 2) & 1;
+  r.queued = (bits >> 3) & 1;
+  r.qi = (int32_t)(bits >> 4);
+  r.nf = (int64_t)pub.value(P_NF);
+  r.prev_nq = (int64_t)pub.value(P_PREV);
+  r.visited = (int64_t)pub.value(P_VISITED);
+  r.edges = pub.value(P_EDGES);
+  const double tick_ms = 1.0 / (double)b.tick_khz;
+  g5_bfs_stats& st = b.stats;
+  pub.wait(2 * (lvl0 + 1), 2 * (r.lvl + 1), seq, s, "g5_run_bfs: levels were not published");
+  for (int l = lvl0 + 1; l <= r.lvl; ++l) {
+    const uint64_t v = pub.value(2 * l);
+    st.nq[l] = (int64_t)(v >> 2);
+    st.direction[l] = v & 1;
+    st.bu_kernel[l] = (v >> 1) & 1;
+    st.level_ms[l] = (double)pub.value(2 * l + 1) * tick_ms;
+    st.num_levels = l + 1;
+  }
+  st.device_ms = (double)pub.value(P_TICKS) * tick_ms;
+  return r;
+}
+
 void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   Graph& g = ctx->graph;
   G5_CHECK(b.prepared, "g5_run_bfs: call g5_prepare_bfs first");
@@ -1111,279 +1804,70 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
 
   if (b.hub_shift > 0 && b.hub_built_shift != b.hub_shift) bfs_tuning_buffers(ctx, b, s);
 
-  G5_HIP(hipEventRecord(b.ev0, s));
-  hipLaunchKernelGGL(k_bfs_init, dim3(grid_of(rows, kBlock, 4096)), dim3(kBlock), 0, s, b.level.p,
-                     b.vis[0].p, rows, b.words);
-  G5_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_bfs_root, dim3(1), dim3(kBlock), 0, s, g.old2new.p, root, rows, b.level.p,
-                     b.parent.p, b.vis[0].p, b.queue[0].p, cnt);
+  StepArgs a{};
+  a.offsets = g.offsets.p;
+  a.cols = g.cols.p;
+  a.first_nbr = g.first_nbr.p;
+  for (int i = 0; i < 2; ++i) a.vis[i] = b.vis[i].p;
+  for (int i = 0; i < 3; ++i) a.queue[i] = b.queue[i].p;
+  a.level = b.level.p;
+  a.parent = b.parent.p;
+  a.pub = b.step_pub.d;
+  a.words = b.words;
+  a.n_active = g.n_active;
+  a.small_edges = b.small_edges;
+  a.tail_pull = b.tail_pull;
+  // bitmap words per wave turn: as many as keep at least 32768 turns
+  a.span = 2;
+  while (a.span < 64 && b.words / (2 * a.span) >= 32768) a.span *= 2;
+  a.host_bu = b.words > kStepMaxWords;
+  const unsigned grid = step_grid(g, b, a.span);
+  hipLaunchKernelGGL(k_bfs_init, dim3(grid_of((rows + 15) / 16, kBlock, 2048)), dim3(kBlock), 0, s, g.old2new.p, root,
+                     rows, b.words, b.level.p, b.parent.p, b.vis[0].p, b.queue[0].p,
+                     (unsigned long long*)b.step_ctl.p, cnt, a);
   G5_HIP(hipGetLastError());
 
   // A root without edges (reachable only through a find_roots fallback) is
   // the whole tree: the reference's first top-down level finds nothing.
   const bool root_active = (g.has_edge_words[root >> 6] >> (root & 63)) & 1;
-  int cur = 0, qi = 0;
-  int64_t nf = 1;
-  bool next_forward = true, growing = true;
-  int64_t prev_nq = 0, visited = 1;
-  // frontier edges of the coming top-down level when a small level summed
-  // them (-1: unknown, both forms are launched and the device picks)
-  int64_t e_next = -1;
-  const double na = (double)g.n_active;
-  int lvl = 0;
   if (!root_active) {
     st.num_levels = 2;
     st.direction[1] = 1;
     st.nq[1] = 0;
+    G5_HIP(hipStreamSynchronize(s));
   }
-  // a fused launch that found the next frontier too large hands that level
-  // to the per-level path
-  bool fuse_next = true;
-  // A top-down level after the bottom-up phase whose frontier holds more
-  // than 1/tail_pull as many vertices as remain unvisited (and more than a
-  // fused launch takes) is found by the bottom-up kernel: an unvisited vertex
-  // with a visited neighbour is on this level (an older neighbour would have
-  // reached it before), so both kernels find the same vertices, and this one
-  // probes from the few unvisited ones instead of expanding the frontier.
-  // The level keeps its top-down place in the schedule.
-  const auto pulls = [&](bool fwd, int64_t frontier) {
-    return fwd && !growing && b.tail_pull > 0 && frontier > kFuseNf &&
-           b.tail_pull * frontier > g.n_active - visited;
+  StepState state{};
+  state.visited = 1;
+  int steps = 0;
+  bool resume = false;  // the state has gone on in host code since the last step
+  const auto bottom_up_next = [&] {
+    return !state.forward ||
+           tail_pulls(1, state.growing, b.tail_pull, state.nf, g.n_active - state.visited);
   };
   while (root_active) {
-    ++lvl;
-    G5_CHECK(lvl < 255, "g5_run_bfs: more than 254 levels (uint8 level array)");
-    const bool forward = next_forward;
-    G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
-    if (forward && fuse_next && b.small_edges > 0 && nf <= kFuseNf &&
-        (e_next < 0 || e_next <= b.small_edges)) {
-      // small top-down levels, as many as fit, in one single-workgroup launch
-      const int max_levels = std::min(kFuseMaxLevels, 254 - lvl);
-      ++b.fuse_seq;
-      hipLaunchKernelGGL(k_td_fused, dim3(1), dim3(kFuseThreads), 0, s, b.queue[0].p, b.queue[1].p, qi, nf,
-                         g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p, (uint32_t)lvl, max_levels,
-                         b.small_edges, na, prev_nq, growing ? 1 : 0, b.fuse.d, b.fuse_seq);
-      G5_HIP(hipGetLastError());
-      G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
-      const char* unpublished = "g5_run_bfs: fused levels were not published";
-      b.fuse.wait(F_LEVELS, F_NUM, b.fuse_seq, s, unpublished);
-      const int k = (int)b.fuse.value(F_LEVELS);
-      b.fuse.wait(0, k, b.fuse_seq, s, unpublished);
-      const uint64_t stop = b.fuse.value(F_STOP);
-      if (k == 0) {
-        // the first frontier was already too large: this level runs per level
-        fuse_next = false;
-        e_next = (int64_t)b.fuse.value(F_E);  // its edge count, when the launch summed it (0: not known)
-        if (e_next == 0) e_next = -1;
-        --lvl;
-        continue;
-      }
-      for (int j = 0; j < k; ++j) {
-        const int l = lvl + j;
-        const int64_t nq = (int64_t)b.fuse.value(j);
-        st.direction[l] = 1;
-        st.nq[l] = nq;
-        st.num_levels = l + 1;
-        visited += nq;
-        st.level_ms[l] = j ? 0 : -1;  // the launch's time is the first fused level's; the others show 0
-      }
-      prev_nq = (int64_t)b.fuse.value(k - 1);
-      qi = (int)b.fuse.value(F_QI);
-      nf = (int64_t)b.fuse.value(F_NF);
-      lvl += k - 1;
-      if (stop == FUSE_EMPTY) break;
-      next_forward = stop != FUSE_PULL;
-      fuse_next = stop != FUSE_LARGE;
-      e_next = stop == FUSE_LARGE && b.fuse.value(F_E) > 0 ? (int64_t)b.fuse.value(F_E) : -1;
+    if (resume && state.nf && a.host_bu && bottom_up_next() && state.lvl < kStepMaxLevel) {
+      host_bottom_up(ctx, b, s, a, state);
       continue;
     }
-    fuse_next = true;
-    const bool pull_td = pulls(forward, nf);
-    const bool td = forward && !pull_td;  // the top-down kernels run
-    if (td) {
-      device_scan(FrontierDegree{b.queue[qi].p, g.offsets.p, nf}, StoreU64{b.prefix.p},
-                  (size_t)nf + 1, b.scan_tmp.p, s);
-      if (b.bin_edges > 0) {
-        // the binned form sizes its pair buffer from E: wait for it
-        G5_HIP(hipMemcpyAsync(b.h_counters + 1, b.prefix.p + nf, 8, hipMemcpyDeviceToHost, s));
-        G5_HIP(hipStreamSynchronize(s));
-      }
-      const uint64_t E_known = b.bin_edges > 0 ? b.h_counters[1] : 0;
-      // past the bottom-up phase most targets are visited: a bulk level then
-      // tests the visited bitmap before the level array
-      const int probe_vis = (double)visited > na / 4 ? 1 : 0;
-      // the level's frontier edge count when the previous level summed it
-      const bool known_small = e_next >= 0 && (uint64_t)e_next <= kTdSmall;
-      const bool known_bulk = e_next >= 0 && (uint64_t)e_next > kTdSmall;
-      // while the search grows, a bulk level can take its rows block by
-      // block (exact target blocks) or piece by piece (positional pieces)
-      const int64_t seg_max = b.seg_max > 0 ? std::min<int64_t>(b.seg_max, kSegMax) : kSegMax;
-      const bool blocked = b.hub_shift > 0 && !probe_vis && nf * b.hub_pieces <= seg_max;
-      // a growing bulk level settles its highest-degree targets bottom-up
-      // first (degree order only)
-      bool head = b.td_head > 0 && !probe_vis && g.reorder_mode == 2;
-      if (head && e_next > (int64_t)kTdSmall) {
-        // E known on the host: no head when no row reaches the threshold
-        // (the same test k_td_head_size makes)
-        const double r = (double)g.nnz / (double)e_next;
-        if ((double)b.td_head / 16.0 * r * r > (double)g.max_degree) head = false;
-      }
-      unsigned long long* head_words = head ? cnt + C_HEAD : nullptr;
-      const bool pieces = blocked || (b.td_pieces > 0 && !probe_vis && nf * b.td_pieces <= seg_max);
-      // with a head and row order, the expansion walks row suffixes (one
-      // segment per frontier row: the segment count field bounds nf)
-      if (head && !pieces && nf > seg_max) head = false;
-      head_words = head ? cnt + C_HEAD : nullptr;
-      const bool suffix = head && !pieces;
-      const bool binned = b.bin_edges > 0 && E_known > kTdSmall && E_known >= (uint64_t)b.bin_edges;
-      // Without binning no launch waits for E on the host: chunk rows and the
-      // expansion take upper-bound grids and read E (prefix[nf]) on the
-      // device; the small and the bulk expansion are both launched and the
-      // one that does not fit E exits at once, as does k_td_finish after a
-      // small level.  The host learns E with the level's counters.
-      const uint64_t max_chunks = b.chunk_rows.n / 2;  // sized for every edge of the graph
-      const uint64_t nchunks = b.bin_edges > 0 ? (E_known + kEpb - 1) / kEpb : max_chunks;
-      const unsigned grid = b.bin_edges > 0 ? grid_of((int64_t)E_known, kEpb, 2048) : 2048u;
-      if (nchunks)
-        hipLaunchKernelGGL(k_chunk_rows<kEpb>,
-                           dim3(b.bin_edges > 0 ? grid_of((int64_t)(2 * nchunks), kBlock, 65536) : 4096u),
-                           dim3(kBlock), 0, s, b.prefix.p, nf, nchunks, b.chunk_rows.p);
-      if (!known_bulk)
-        hipLaunchKernelGGL(k_td_expand<false>, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
-                           b.chunk_rows.p, g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p,
-                           b.queue[qi ^ 1].p, cnt, (uint32_t)lvl, 0, nullptr);
-      if (head && !binned && !known_small) {
-        hipLaunchKernelGGL(k_td_head_size, dim3(1), dim3(1), 0, s, b.prefix.p, nf, g.offsets.p, rows, b.words,
-                           (double)g.nnz, (double)b.td_head / 16.0, head_words);
-        hipLaunchKernelGGL(k_td_head, dim3(grid_of(b.words, kBlock / 64, 8192)), dim3(kBlock), 0, s,
-                           b.vis[cur].p, g.first_nbr.p, g.offsets.p, g.cols.p, b.level.p, b.parent.p, head_words,
-                           (uint32_t)lvl);
-        G5_HIP(hipGetLastError());
-      }
-      if (known_small) {
-        // nothing else to launch: the small expansion keeps the queue exact
-      } else if (binned) {
-        // binned by target range (see k_td_bin_count)
-        const uint64_t E = E_known;
-        int shift = kBinShift;
-        while ((rows >> shift) >= kBinMaxBuckets) ++shift;
-        const int nb = (int)(((rows - 1) >> shift) + 1);
-        b.bin_pairs.alloc(E);
-        b.bin_cnt.alloc(2 * kBinMaxBuckets);
-        unsigned long long* bc = (unsigned long long*)b.bin_cnt.p;
-        G5_HIP(hipMemsetAsync(bc, 0, nb * 8, s));
-        hipLaunchKernelGGL(k_td_bin_count, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
-                           b.chunk_rows.p, g.offsets.p, g.cols.p, shift, nb, bc);
-        hipLaunchKernelGGL(k_td_bin_offsets, dim3(1), dim3(kBlock), 0, s, bc, nb, bc + kBinMaxBuckets);
-        hipLaunchKernelGGL(k_td_bin_scatter, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
-                           b.chunk_rows.p, g.offsets.p, g.cols.p, shift, nb, bc + kBinMaxBuckets, b.bin_pairs.p);
-        hipLaunchKernelGGL(k_td_bin_apply, dim3(grid_of((int64_t)E, kBlock, 2048)), dim3(kBlock), 0, s,
-                           b.bin_pairs.p, E, b.level.p, b.parent.p, (uint32_t)lvl);
-      } else if (pieces || suffix) {
-        // segment-list bulk level; a small level makes an empty segment list
-        // and the expansion exits (both read E on the device)
-        const size_t np = (size_t)(suffix ? nf : nf * (blocked ? b.hub_pieces : b.td_pieces)) + 1;
-        b.seg_pre.alloc(np);
-        b.seg_base.alloc(np);
-        b.seg_src.alloc(np);
-        b.seg_count.alloc(1);
-        b.seg_scan_tmp.alloc(scan_tmp_elems(np));
-        if (suffix) {
-          b.seg_start.alloc(np);
-          hipLaunchKernelGGL(k_suffix_start, dim3(grid_of(nf, kBlock, 4096)), dim3(kBlock), 0, s, b.queue[qi].p, nf,
-                             b.prefix.p, g.offsets.p, g.cols.p, head_words, b.seg_start.p);
-          const SuffixLen sl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, 1, b.seg_start.p};
-          device_scan(sl, PieceEmit<SuffixLen>{sl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
-                      b.seg_scan_tmp.p, s);
-        } else if (blocked) {
-          const BlockLen bl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, b.hub_pieces, b.hub_bnd.p, b.hub_rows};
-          device_scan(bl, PieceEmit<BlockLen>{bl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
-                      b.seg_scan_tmp.p, s);
-        } else {
-          const PieceLen pl{b.queue[qi].p, g.offsets.p, b.prefix.p, nf, b.td_pieces};
-          device_scan(pl, PieceEmit<PieceLen>{pl, b.seg_pre.p, b.seg_base.p, b.seg_src.p, b.seg_count.p}, np,
-                      b.seg_scan_tmp.p, s);
-        }
-        hipLaunchKernelGGL(k_chunk_segs, dim3(4096), dim3(kBlock), 0, s, b.seg_pre.p, b.seg_count.p, max_chunks,
-                           b.chunk_rows.p);
-        hipLaunchKernelGGL(k_td_expand_segs, dim3(grid), dim3(kBlock), 0, s, b.prefix.p, nf, b.seg_pre.p,
-                           b.seg_base.p, b.seg_src.p, b.seg_count.p, b.chunk_rows.p, g.cols.p, b.vis[cur].p,
-                           b.level.p, b.parent.p, (uint32_t)lvl, head_words);
-      } else {
-        hipLaunchKernelGGL(k_td_expand<true>, dim3(grid), dim3(kBlock), 0, s, b.queue[qi].p, nf, b.prefix.p,
-                           b.chunk_rows.p, g.offsets.p, g.cols.p, b.vis[cur].p, b.level.p, b.parent.p,
-                           (uint32_t*)nullptr, cnt, (uint32_t)lvl, probe_vis, binned ? nullptr : head_words);
-      }
+    if (resume && state.nf > kStepNf && !bottom_up_next() && state.lvl < kStepMaxLevel) {
+      large_top_down(ctx, b, s, state);
+      continue;
+    }
+    if (resume) {
+      hipLaunchKernelGGL(k_step_resume, dim3(1), dim3(1), 0, s, (unsigned long long*)b.step_ctl.p, state, steps);
       G5_HIP(hipGetLastError());
-      // after a bulk level, k_td_finish makes vis[cur^1] exactly this level's
-      // vertices and adds them to vis[cur]
-      if (!known_small)
-        hipLaunchKernelGGL(k_td_finish, dim3(grid_of((b.words + 15) / 16, kBlock / 64, 8192)), dim3(kBlock), 0,
-                           s, b.level.p, rows, b.words, (uint32_t)lvl, b.vis[cur].p, b.vis[cur ^ 1].p, cnt,
-                           b.prefix.p, nf);
-    } else {
-      // words per wave step: as many as keep at least 32768 wave steps
-      int span = 2;
-      while (span < 64 && b.words / (2 * span) >= 32768) span *= 2;
-      hipLaunchKernelGGL(k_bu, dim3(grid_of((b.words + span - 1) / span, kBlock / 64, 8192)), dim3(kBlock), 0, s,
-                         b.vis[cur].p, b.vis[cur ^ 1].p, g.first_nbr.p, g.offsets.p, g.cols.p,
-                         b.level.p, b.parent.p, b.words, span, (uint32_t)lvl, cnt);
     }
-    G5_HIP(hipGetLastError());
-    G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
-    ++b.pub_seq;
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, td ? 1 : 0, b.pub.d,
-                       b.pub_seq);
-    G5_HIP(hipGetLastError());
-    wait_published(b, s);
-    const int64_t nq = (int64_t)b.h_counters[0];
-    const bool bulk = td && b.h_counters[1] > kTdSmall;
-    // a small top-down level summed its winners' degrees
-    e_next = (td && !bulk) ? (int64_t)b.h_counters[C_NEXT_E] : -1;
-    st.direction[lvl] = forward ? 1 : 0;
-    st.bu_kernel[lvl] = td ? 0 : 1;
-    st.nq[lvl] = nq;
-    st.num_levels = lvl + 1;
-    st.level_ms[lvl] = -1;  // read from the events at the end
-    visited += nq;
-    if (nq == 0) break;
-    // direction switch, mpi/bfs.hpp:2799-2829
-    const int64_t unvisited = g.n_active - visited;
-    if (growing && nq > prev_nq) {
-      if (forward && (double)nq > na / 2000.0) next_forward = false;
-    } else {
-      if (!forward && unvisited < (int64_t)(na / 8.0)) {
-        next_forward = true;
-        growing = false;
-      }
-    }
-    prev_nq = nq;
-    // The next top-down level needs this level's vertices as a queue, unless
-    // the bottom-up kernel takes it.  A small top-down level appended them to
-    // queue[qi^1]; a bulk one left them in vis[cur^1]; the bottom-up kernel
-    // left them as vis[cur^1] & ~vis[cur].
-    if (td && !bulk) {
-      qi ^= 1;
-    } else if (next_forward && !pulls(true, nq)) {
-      const uint64_t* before = td ? nullptr : b.vis[cur].p;
-      device_scan(FrontierBits{b.vis[cur ^ 1].p, before},
-                  FrontierEmit{b.vis[cur ^ 1].p, before, b.queue[qi].p}, (size_t)b.words, b.scan_tmp.p, s);
-    }
-    if (!td) cur ^= 1;
-    nf = nq;
+    state = run_steps(b, s, grid, state.lvl, steps);
+    if (state.stop == STEP_DONE) break;
+    G5_CHECK(state.stop != STEP_LIMIT, "g5_run_bfs: more than 254 levels (uint8 level array)");
+    const int stop = state.stop;
+    state.stop = STEP_GO;
+    resume = true;
+    if (!state.queued && stop != STEP_BOTTOM_UP) queue_from_bitmaps(b, s, state);
+    if (stop == STEP_LARGE) large_top_down(ctx, b, s, state);
+    state.edges = 0;
   }
-  G5_HIP(hipEventRecord(b.ev1, s));
-  G5_HIP(hipEventSynchronize(b.ev1));
-  float ms = 0;
-  G5_HIP(hipEventElapsedTime(&ms, b.ev0, b.ev1));
-  st.device_ms = ms;
-  for (int l = 1; l <= lvl && root_active; ++l) {
-    if (st.level_ms[l] == 0) continue;
-    float lms = 0;
-    G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[l], b.lev_end[l]));
-    st.level_ms[l] = lms;
-  }
-  st.reached = visited;
+  st.reached = state.visited;
   b.have_result = true;
 }
 

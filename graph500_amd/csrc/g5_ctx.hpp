@@ -64,7 +64,7 @@ struct BfsState {
   DevBuf<uint64_t> vis[2];
   DevBuf<uint8_t> level;          // n_rows
   DevBuf<uint32_t> parent;        // n_rows
-  DevBuf<uint32_t> queue[2];      // n_rows
+  DevBuf<uint32_t> queue[3];      // n_rows
   DevBuf<uint64_t> prefix;        // n_rows + 1 (top-down edge prefix)
   DevBuf<uint32_t> chunk_rows;    // 2 per top-down edge chunk: first/last frontier index
   DevBuf<uint64_t> scan_tmp;
@@ -72,8 +72,10 @@ struct BfsState {
   uint64_t h_counters[8] = {};    // the last level's counters on the host
   PublishBlock pub;               // the level counters, published by k_publish
   uint64_t pub_seq = 0;
-  PublishBlock fuse;              // the fused small levels' state (g5_bfs.hip)
-  uint64_t fuse_seq = 0;
+  DevBuf<uint64_t> step_ctl;      // control words of the steps (g5_bfs.hip)
+  PublishBlock step_pub;          // what the steps publish
+  uint64_t step_seq = 0;
+  int tick_khz = 0;               // rate of the device clock the steps read
   int64_t small_edges = 8192;     // small top-down levels up to this many edges run fused (0: never)
   int64_t tail_pull = 4;          // post-bottom-up top-down levels with tail_pull * nf > unvisited run bottom-up
   DevBuf<int64_t> pred_out;       // n, built on demand by get_pred
@@ -96,8 +98,7 @@ struct BfsState {
   int64_t hub_rows = 0;           // rows [0, hub_rows) are indexed
   DevBuf<uint32_t> hub_bnd;       // hub_rows * hub_pieces
   g5_bfs_stats stats{};
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  std::vector<hipEvent_t> lev_begin, lev_end;  // per level
+  std::vector<hipEvent_t> lev_begin, lev_end;  // per level run from the host
   // the tuning (g5_bfs_set_tuning's fields) of another state
   void copy_tuning(const BfsState& o) {
     small_edges = o.small_edges;
@@ -117,6 +118,7 @@ struct BfsState {
     chunk_rows.release();
     scan_tmp.release();
     counters.release();
+    step_ctl.release();
     pred_out.release();
     level_out.release();
     bin_pairs.release();
@@ -136,8 +138,6 @@ struct BfsState {
   ~BfsState() {
     destroy_events(lev_begin);
     destroy_events(lev_end);
-    if (ev0) (void)hipEventDestroy(ev0);
-    if (ev1) (void)hipEventDestroy(ev1);
   }
 };
 
