@@ -39,6 +39,7 @@
 //              the whole wave 64 entries at a time with a ballot for the first
 //              hit.  The visited snapshot of the previous level is read-only;
 //              the next bitmap word is written once per wave from a ballot.
+#include "g5_answers.hpp"
 #include "g5_ctx.hpp"
 #include "g5_frontier.hpp"
 #include "g5_prims.hpp"
@@ -820,15 +821,81 @@ __global__ void k_make_pred(const uint32_t* __restrict__ old2new, const uint32_t
   }
 }
 
-__global__ void k_make_levels(const uint32_t* __restrict__ old2new, const uint8_t* __restrict__ level,
-                              int64_t n, int64_t rows, int64_t root_orig, uint8_t* __restrict__ out) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-       v += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t nv = old2new[v];
-    uint8_t l = 0xFF;
-    if (v == root_orig) l = 0;
-    else if ((int64_t)nv < rows) l = level[nv];
-    out[v] = l;
+__global__ void __launch_bounds__(kBlock) k_make_levels(const uint32_t* __restrict__ old2new,
+                                                        const uint8_t* __restrict__ level, int64_t n, int64_t rows,
+                                                        int64_t root_orig, uint8_t* __restrict__ out) {
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q * 16 < n; q += stride) {
+    const int m = n < 16 ? (int)n : 16;  // n is a power of two
+    uint32_t nv[16];
+    if (m == 16) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        reinterpret_cast<uint4*>(nv)[j] = reinterpret_cast<const uint4*>(old2new + q * 16)[j];
+    } else {
+      for (int j = 0; j < 16; ++j) nv[j] = j < m ? old2new[j] : 0xFFFFFFFFu;
+    }
+    uint32_t l[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) l[j] = j < m && (int64_t)nv[j] < rows ? level[nv[j]] : 0xFF;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = l[4 * j] | (l[4 * j + 1] << 8) | (l[4 * j + 2] << 16) | (l[4 * j + 3] << 24);
+    const int64_t r = root_orig - q * 16;  // also a root without edges, which is no row of the CSR
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (r >= 4 * j && r < 4 * j + 4) w[j] &= ~(0xFFu << (8 * (r & 3)));
+    if (m == 16) {
+      reinterpret_cast<uint4*>(out)[q] = uint4{w[0], w[1], w[2], w[3]};
+    } else {
+      for (int j = 0; j < m; ++j) out[j] = (uint8_t)(w[j >> 2] >> (8 * (j & 3)));
+    }
+  }
+}
+
+void launch_make_levels(const uint32_t* old2new, const uint8_t* row_level, int64_t n, int64_t rows, int64_t root,
+                        uint8_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_make_levels, dim3(grid_of((n + 15) / 16, kBlock, 4096)), dim3(kBlock), 0, s, old2new, row_level,
+                     n, rows, root, out);
+  G5_HIP(hipGetLastError());
+}
+
+// Tuple weights of the reached rows: 16 rows per thread and turn, one sum per
+// workgroup published to the host, which adds them up (at most kTepsGrid).
+// Bound by the 5 B read per row: 141 us at S28, 290 with adds to one word and
+// a copy of the sum.
+constexpr int kTepsGrid = 256;
+constexpr int kTepsThreads = 1024;
+__global__ void __launch_bounds__(kTepsThreads) k_teps(const uint8_t* __restrict__ level,
+                                                       const uint32_t* __restrict__ weight, int64_t rows,
+                                                       Published* pub, uint64_t seq) {
+  __shared__ uint64_t s_sum[kTepsThreads / 64];
+  uint64_t sum = 0;
+  const int64_t stride = (int64_t)gridDim.x * kTepsThreads;
+  for (int64_t q = (int64_t)blockIdx.x * kTepsThreads + threadIdx.x; q * 16 < rows; q += stride) {
+    if (q * 16 + 16 <= rows) {
+      uint32_t l[4];
+      *reinterpret_cast<uint4*>(l) = reinterpret_cast<const uint4*>(level)[q];
+      uint4 w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = reinterpret_cast<const uint4*>(weight)[q * 4 + j];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        sum += (l[j] & 0xFF) != 0xFF ? w[j].x : 0;
+        sum += ((l[j] >> 8) & 0xFF) != 0xFF ? w[j].y : 0;
+        sum += ((l[j] >> 16) & 0xFF) != 0xFF ? w[j].z : 0;
+        sum += (l[j] >> 24) != 0xFF ? w[j].w : 0;
+      }
+    } else {
+      for (int64_t v = q * 16; v < rows; ++v) sum += level[v] != 0xFF ? weight[v] : 0;
+    }
+  }
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const uint64_t t = wave_sum(threadIdx.x < kTepsThreads / 64 ? s_sum[threadIdx.x] : 0);
+    if (threadIdx.x == 0) publish(pub + blockIdx.x, t, seq);
   }
 }
 
@@ -1493,6 +1560,8 @@ void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   b.step_ctl.alloc(kStepWords);
   b.step_pub.alloc(P_NUM);
   b.step_seq = 0;
+  b.teps_pub.alloc(kTepsGrid);
+  b.teps_seq = 0;
   if (!b.tick_khz) {
     int khz = 0;
     G5_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
@@ -1875,37 +1944,35 @@ void bfs_get_pred(g5_ctx* ctx, int64_t* host_pred) {
   Graph& g = ctx->graph;
   BfsState& b = ctx->bfs;
   G5_CHECK(b.have_result, "g5_get_pred: no BFS result (call g5_run_bfs first)");
-  b.pred_out.alloc(g.n);
+  HostOut out(host_pred, (size_t)g.n, ctx->stage, b.pred_out, ctx->stream);
   hipLaunchKernelGGL(k_make_pred, dim3(grid_of(g.n, kBlock, 65536)), dim3(kBlock), 0, ctx->stream,
-                     g.old2new.p, g.new2old.p, b.level.p, b.parent.p, g.n, g.n_rows, b.root_orig,
-                     b.pred_out.p);
+                     g.old2new.p, g.new2old.p, b.level.p, b.parent.p, g.n, g.n_rows, b.root_orig, (int64_t*)out.p);
   G5_HIP(hipGetLastError());
-  G5_HIP(hipMemcpyAsync(host_pred, b.pred_out.p, g.n * 8, hipMemcpyDeviceToHost, ctx->stream));
-  G5_HIP(hipStreamSynchronize(ctx->stream));
+  out.finish();
 }
 
 void bfs_get_levels(g5_ctx* ctx, uint8_t* host_levels) {
   Graph& g = ctx->graph;
   BfsState& b = ctx->bfs;
   G5_CHECK(b.have_result, "g5_get_levels: no BFS result (call g5_run_bfs first)");
-  b.level_out.alloc(g.n);
-  hipLaunchKernelGGL(k_make_levels, dim3(grid_of(g.n, kBlock, 65536)), dim3(kBlock), 0, ctx->stream,
-                     g.old2new.p, b.level.p, g.n, g.n_rows, b.root_orig, b.level_out.p);
-  G5_HIP(hipGetLastError());
-  G5_HIP(hipMemcpyAsync(host_levels, b.level_out.p, g.n, hipMemcpyDeviceToHost, ctx->stream));
-  G5_HIP(hipStreamSynchronize(ctx->stream));
+  HostOut out(host_levels, (size_t)g.n, ctx->stage, b.level_out, ctx->stream);
+  launch_make_levels(g.old2new.p, b.level.p, g.n, g.n_rows, b.root_orig, (uint8_t*)out.p, ctx->stream);
+  out.finish();
 }
 
-int64_t bfs_teps_edges(g5_ctx* ctx) {
-  ctx->acc.alloc(4);
-  return bfs_teps_edges(ctx, ctx->bfs, ctx->acc, ctx->stream);
-}
+int64_t bfs_teps_edges(g5_ctx* ctx) { return bfs_teps_edges(ctx, ctx->bfs, ctx->stream); }
 
-int64_t bfs_teps_edges(g5_ctx* ctx, const BfsState& b, DevBuf<uint64_t>& acc, hipStream_t s) {
+int64_t bfs_teps_edges(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   Graph& g = ctx->graph;
   G5_CHECK(b.have_result, "g5_teps_edges: no BFS result (call g5_run_bfs first)");
-  G5_CHECK(acc.n >= 4, "g5_teps_edges: reduction buffer too small");
-  const uint64_t sum = device_reduce_sum(ReachedWeight{b.level.p, g.weight.p}, (size_t)g.n_rows, acc.p, s);
+  const unsigned grid = grid_of((g.n_rows + 15) / 16, kTepsThreads, kTepsGrid);
+  ++b.teps_seq;
+  hipLaunchKernelGGL(k_teps, dim3(grid), dim3(kTepsThreads), 0, s, b.level.p, g.weight.p, g.n_rows, b.teps_pub.d,
+                     b.teps_seq);
+  G5_HIP(hipGetLastError());
+  b.teps_pub.wait(0, (int)grid, b.teps_seq, s, "g5_teps_edges: a sum was not published");
+  uint64_t sum = 0;
+  for (unsigned i = 0; i < grid; ++i) sum += b.teps_pub.value(i);
   return (int64_t)(sum / 2);
 }
 

@@ -42,6 +42,21 @@ struct Graph {
   }
 };
 
+// Pinned host memory, allocated on first use and kept.
+struct HostStage {
+  void* h = nullptr;
+  HostStage() = default;
+  HostStage(const HostStage&) = delete;
+  HostStage& operator=(const HostStage&) = delete;
+  ~HostStage() {
+    if (h) (void)hipHostFree(h);
+  }
+  void* get(size_t bytes) {  // always the same size
+    if (!h) G5_HIP(hipHostMalloc(&h, bytes, hipHostMallocDefault));
+    return h;
+  }
+};
+
 // Events of a run's levels, created as levels are first reached.
 inline hipEvent_t level_event(std::vector<hipEvent_t>& v, int l) {
   if ((int)v.size() <= l) v.resize(l + 1, nullptr);
@@ -75,6 +90,8 @@ struct BfsState {
   DevBuf<uint64_t> step_ctl;      // control words of the steps (g5_bfs.hip)
   PublishBlock step_pub;          // what the steps publish
   uint64_t step_seq = 0;
+  PublishBlock teps_pub;          // per-workgroup sums of the traversed-edge count
+  uint64_t teps_seq = 0;
   int tick_khz = 0;               // rate of the device clock the steps read
   int64_t small_edges = 8192;     // small top-down levels up to this many edges run fused (0: never)
   int64_t tail_pull = 4;          // post-bottom-up top-down levels with tail_pull * nf > unvisited run bottom-up
@@ -197,6 +214,10 @@ struct MsState {
   std::vector<char> fr_exact;
   std::vector<int64_t> fr_count;  // per level: vertices the last run marked
   DevBuf<const uint64_t*> frp;  // device copy of the fr pointers
+  DevBuf<uint8_t> row_level;    // a lane's levels by row (g5_batch_get_levels on larger graphs)
+  DevBuf<uint64_t> teps_acc;    // striped traversed-edge sums, clear between calls
+  PublishBlock teps_pub;
+  uint64_t teps_seq = 0;
   DevBuf<uint32_t> queue;
   DevBuf<uint32_t> touch;    // vertices a sparse push level touched
   DevBuf<uint64_t> miss;     // one bit per vertex still missing a live root (tail pull levels)
@@ -221,6 +242,8 @@ struct MsState {
     fr_exact.clear();
     fr_count.clear();
     frp.release();
+    row_level.release();
+    teps_acc.release();
     queue.release();
     touch.release();
     miss.release();
@@ -275,6 +298,7 @@ struct g5_ctx {
   g5::BfsState bfs;
   g5::MsState ms;
   g5::DevBuf<uint64_t> acc;  // small reduction scratch
+  g5::HostStage stage;       // small answers on their way to the host
   int servers = 0;           // g5_server objects that serve this context's graph
 };
 
@@ -300,7 +324,7 @@ int64_t bfs_teps_edges(g5_ctx* ctx);
 void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s);
 void bfs_tuning_buffers(g5_ctx* ctx, BfsState& b, hipStream_t s);
 void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root_orig);
-int64_t bfs_teps_edges(g5_ctx* ctx, const BfsState& b, DevBuf<uint64_t>& acc, hipStream_t s);
+int64_t bfs_teps_edges(g5_ctx* ctx, BfsState& b, hipStream_t s);
 void bfs_model_bytes(g5_ctx* ctx, double* per_level, double* total);
 // g5_validate.hip
 void bfs_validate(g5_ctx* ctx, int64_t* errors_out);

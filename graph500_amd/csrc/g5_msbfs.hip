@@ -20,6 +20,7 @@
 //         zero" bitmap (n/8 bytes, cache resident) is tested first, so the
 //         8-byte frontier word is only read for frontier vertices
 // Per-lane levels equal the single-root BFS levels of the same root.
+#include "g5_answers.hpp"
 #include "g5_ctx.hpp"
 #include "g5_frontier.hpp"
 #include "g5_ms_device.hpp"
@@ -432,52 +433,135 @@ __global__ void __launch_bounds__(kBlock) k_ms_fill(uint64_t* __restrict__ a, in
   ms_zero_body(a, n, blockIdx.x, gridDim.x);
 }
 
-// Per-root level of every original vertex: the first level whose frontier
-// word holds the lane.
-__global__ void k_ms_levels(const uint32_t* __restrict__ old2new, int64_t n, int64_t rows,
-                            const uint64_t* const* __restrict__ fr, int nlevels, int lane, int64_t root,
-                            uint8_t* __restrict__ out) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t nv = old2new[v];
-    uint8_t l = 0xFF;
-    if (v == root)
-      l = 0;  // also a root without edges, which is no row of the CSR
-    else if ((int64_t)nv < rows)
-      for (int i = 0; i < nlevels; ++i)
-        if ((fr[i][nv] >> lane) & 1) {
-          l = (uint8_t)i;
-          break;
+// A lane's level is the first level whose frontier word holds it.  The levels'
+// frontier words and nonzero bitmaps travel in the argument block.
+constexpr int kMsArgLevels = 24;
+struct LevelWords {
+  const uint64_t* fr[kMsArgLevels];
+  const uint64_t* nz[kMsArgLevels];  // null where a level's bitmap does not describe its words
+  const uint64_t* const* more;       // the frontier words again, for deeper searches
+  int n;
+  __device__ const uint64_t* words(int i) const { return i < kMsArgLevels ? fr[i] : more[i]; }
+};
+
+// Levels by original id: 4 consecutive ids per thread, their words of one
+// level in flight together.  For graphs whose frontier words sit in the L2s.
+__global__ void __launch_bounds__(kBlock) k_ms_levels(const uint32_t* __restrict__ old2new, int64_t n, int64_t rows,
+                                                      LevelWords lw, int lane, int64_t root,
+                                                      uint8_t* __restrict__ out) {
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q * 4 < n; q += stride) {
+    const int m = n < 4 ? (int)n : 4;  // n is a power of two
+    uint32_t nv[4];
+    uint32_t l[4];
+    bool open[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      nv[j] = j < m ? old2new[q * 4 + j] : 0xFFFFFFFFu;
+      l[j] = 0xFF;
+      open[j] = (int64_t)nv[j] < rows;
+    }
+    for (int i = 0; i < lw.n && (open[0] || open[1] || open[2] || open[3]); ++i) {
+      const uint64_t* f = lw.words(i);
+      uint64_t x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = open[j] ? f[nv[j]] : 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if ((x[j] >> lane) & 1) {
+          l[j] = i;
+          open[j] = false;
         }
-    out[v] = l;
+    }
+    const int64_t r = root - q * 4;
+    if (r >= 0 && r < 4) {  // also a root without edges, which is no row of the CSR
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (r == j) l[j] = 0;
+    }
+    if (m == 4) {
+      reinterpret_cast<uint32_t*>(out)[q] = l[0] | (l[1] << 8) | (l[2] << 16) | (l[3] << 24);
+    } else {
+      for (int j = 0; j < m; ++j) out[j] = (uint8_t)l[j];
+    }
+  }
+}
+
+// Levels by row, for larger graphs: a wave takes 64 rows, and reads a level's
+// words (coalesced) only where the level's bitmap has one of its rows still
+// open; the lookup by original id is then one byte each (k_make_levels)
+// instead of a word per level.
+__global__ void __launch_bounds__(kBlock) k_ms_row_levels(LevelWords lw, int64_t rows, int lane_bit,
+                                                          uint8_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t words = (rows + 63) / 64, nwaves = (int64_t)gridDim.x * (kBlock / 64);
+  for (int64_t wd = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); wd < words; wd += nwaves) {
+    const int64_t v = wd * 64 + lane;
+    bool open = v < rows;
+    uint32_t l = 0xFF;
+    for (int i = 0; i < lw.n && __ballot(open); ++i) {
+      const uint64_t* nz = i < kMsArgLevels ? lw.nz[i] : nullptr;
+      const bool read = open && (!nz || ((nz[wd] >> lane) & 1));
+      if (read && ((lw.words(i)[v] >> lane_bit) & 1)) {
+        l = i;
+        open = false;
+      }
+    }
+    if (v < rows) out[v] = (uint8_t)l;
   }
 }
 
 // Traversed-edge numerators of all lanes: sum of weight over the vertices
-// each lane reached.  Vertices reached by every lane go to one accumulator.
+// each lane reached.  Vertices reached by every lane go to one sum; for the
+// others, thread i of a wave sums lane i's weights (readlane walk).  Workgroups
+// add to one of kTepsStripes copies; k_ms_teps_publish sums and clears them.
+// Bound by the words and weights read (12 B per row); one copy of the sums
+// held the workgroups up at its words (12 ns an add: S22 82 us, now 29).
+constexpr int kTepsStripes = 16;
+constexpr int kTepsStride = 72;
 __global__ void __launch_bounds__(kBlock) k_ms_teps(const uint64_t* __restrict__ seen,
                                                     const uint32_t* __restrict__ weight, int64_t rows,
                                                     uint64_t all, unsigned long long* __restrict__ acc) {
   __shared__ unsigned long long s_acc[65];
   if (threadIdx.x < 65) s_acc[threadIdx.x] = 0;
   __syncthreads();
-  uint64_t full = 0;
-  for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < rows; v += (int64_t)gridDim.x * kBlock) {
-    const uint64_t s = seen[v];
-    const uint64_t w = weight[v];
-    if (s == all) {
-      full += w;
-    } else {
-      uint64_t x = s;
-      while (x) {
-        atomicAdd(&s_acc[__builtin_ctzll(x)], (unsigned long long)w);
-        x &= x - 1;
-      }
+  const int me = threadIdx.x & 63;
+  const int64_t nwaves = (int64_t)gridDim.x * (kBlock / 64);
+  uint64_t full = 0, mine = 0;
+  for (int64_t wd = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); wd * 64 < rows; wd += nwaves) {
+    const int64_t v = wd * 64 + me;
+    const uint64_t x = v < rows ? seen[v] : 0;
+    const uint32_t w = v < rows ? weight[v] : 0;
+    if (x == all) full += w;
+    uint64_t m = __ballot(x != 0 && x != all);
+    while (m) {
+      const int t = __builtin_ctzll(m);
+      m &= m - 1;
+      const uint32_t xlo = __builtin_amdgcn_readlane((uint32_t)x, t);
+      const uint32_t xhi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), t);
+      const uint32_t wt = __builtin_amdgcn_readlane(w, t);
+      mine += ((me < 32 ? xlo >> me : xhi >> (me - 32)) & 1) ? wt : 0;
     }
   }
   full = wave_sum(full);
-  if ((threadIdx.x & 63) == 0 && full) atomicAdd(&s_acc[64], (unsigned long long)full);
+  if (me == 0 && full) atomicAdd(&s_acc[64], (unsigned long long)full);
+  if (mine) atomicAdd(&s_acc[me], (unsigned long long)mine);
   __syncthreads();
-  if (threadIdx.x < 65 && s_acc[threadIdx.x]) atomicAdd(acc + threadIdx.x, s_acc[threadIdx.x]);
+  if (threadIdx.x < 65 && s_acc[threadIdx.x])
+    atomicAdd(acc + (blockIdx.x % kTepsStripes) * kTepsStride + threadIdx.x, s_acc[threadIdx.x]);
+}
+
+__global__ void __launch_bounds__(128) k_ms_teps_publish(unsigned long long* __restrict__ acc, Published* pub,
+                                                         uint64_t seq) {
+  const int t = threadIdx.x;
+  if (t > 64) return;
+  uint64_t sum = 0;
+#pragma unroll
+  for (int i = 0; i < kTepsStripes; ++i) {
+    sum += acc[i * kTepsStride + t];
+    acc[i * kTepsStride + t] = 0;
+  }
+  publish(pub + t, sum, seq);
 }
 
 // --- batched byte model (evaluated after the run from the per-level words) ---
@@ -575,6 +659,10 @@ void ms_prepare(g5_ctx* ctx) {
   G5_HIP(hipStreamSynchronize(ctx->stream));  // the published block is reset below
   m.pub.alloc(kMsCounters);
   m.pub_seq = 0;
+  m.teps_pub.alloc(65);
+  m.teps_seq = 0;
+  m.teps_acc.alloc(kTepsStripes * kTepsStride);
+  G5_HIP(hipMemsetAsync(m.teps_acc.p, 0, m.teps_acc.bytes(), ctx->stream));
   if (!m.ev0) G5_HIP(hipEventCreate(&m.ev0));
   if (!m.ev1) G5_HIP(hipEventCreate(&m.ev1));
   m.prepared = true;
@@ -1161,37 +1249,57 @@ static void ms_upload_level_ptrs(MsState& m, int nlev, hipStream_t s) {
   G5_HIP(hipMemcpyAsync(m.frp.p, h.data(), nlev * sizeof(void*), hipMemcpyHostToDevice, s));
 }
 
+// From this many rows on a lane's levels are made by row first: below, the
+// levels' frontier words (8 B per row) fit the L2s and one launch is less
+// (one lane of S17: 21 us directly, 23 by row; S19, 335k rows: 32 both; S22,
+// by row: 124, and 162 with one id per thread and a copy behind it).
+constexpr int64_t kRowLevelsFrom = 1 << 19;
+
 void ms_get_levels(g5_ctx* ctx, int lane, uint8_t* host_levels) {
   Graph& g = ctx->graph;
   MsState& m = ctx->ms;
+  hipStream_t s = ctx->stream;
   G5_CHECK(m.have_result, "g5_batch_get_levels: no batch result");
   G5_CHECK(lane >= 0 && lane < m.nroots, "g5_batch_get_levels: lane out of range");
-  const int nlev = m.stats.num_levels;  // frontier words exist for levels 0..num_levels-1
-  ms_upload_level_ptrs(m, nlev, ctx->stream);
-  ctx->bfs.level_out.alloc(g.n);
-  hipLaunchKernelGGL(k_ms_levels, dim3(grid_of(g.n, kBlock, 65536)), dim3(kBlock), 0, ctx->stream, g.old2new.p,
-                     g.n, g.n_rows, (const uint64_t* const*)m.frp.p, nlev, lane, m.host_roots[lane],
-                     ctx->bfs.level_out.p);
-  G5_HIP(hipGetLastError());
-  G5_HIP(hipMemcpyAsync(host_levels, ctx->bfs.level_out.p, g.n, hipMemcpyDeviceToHost, ctx->stream));
-  G5_HIP(hipStreamSynchronize(ctx->stream));
+  LevelWords lw{};
+  lw.n = m.stats.num_levels;  // frontier words exist for levels 0..num_levels-1
+  for (int i = 0; i < lw.n && i < kMsArgLevels; ++i) {
+    lw.fr[i] = m.fr[i]->p;
+    lw.nz[i] = m.fr_exact[i] ? m.fr_dirty[i]->p : nullptr;
+  }
+  if (lw.n > kMsArgLevels) {
+    ms_upload_level_ptrs(m, lw.n, s);
+    lw.more = (const uint64_t* const*)m.frp.p;
+  }
+  HostOut out(host_levels, (size_t)g.n, ctx->stage, ctx->bfs.level_out, s);
+  if (g.n_rows < kRowLevelsFrom) {
+    hipLaunchKernelGGL(k_ms_levels, dim3(grid_of((g.n + 3) / 4, kBlock, 4096)), dim3(kBlock), 0, s, g.old2new.p, g.n,
+                       g.n_rows, lw, lane, m.host_roots[lane], (uint8_t*)out.p);
+    G5_HIP(hipGetLastError());
+  } else {
+    m.row_level.alloc(g.n_rows);
+    hipLaunchKernelGGL(k_ms_row_levels, dim3(grid_of((g.n_rows + 63) / 64, kBlock / 64, 8192)), dim3(kBlock), 0, s, lw,
+                       g.n_rows, lane, m.row_level.p);
+    G5_HIP(hipGetLastError());
+    launch_make_levels(g.old2new.p, m.row_level.p, g.n, g.n_rows, m.host_roots[lane], (uint8_t*)out.p, s);
+  }
+  out.finish();
 }
 
 void ms_teps_edges(g5_ctx* ctx, int64_t* out) {
   Graph& g = ctx->graph;
   MsState& m = ctx->ms;
   G5_CHECK(m.have_result, "g5_batch_teps_edges: no batch result");
-  ctx->acc.alloc(65);
   hipStream_t s = ctx->stream;
-  G5_HIP(hipMemsetAsync(ctx->acc.p, 0, 65 * 8, s));
   const uint64_t all = m.nroots == 64 ? ~UINT64_C(0) : ((UINT64_C(1) << m.nroots) - 1);
-  hipLaunchKernelGGL(k_ms_teps, dim3(grid_of(g.n_rows, kBlock, 4096)), dim3(kBlock), 0, s, m.seen.p,
-                     g.weight.p, g.n_rows, all, (unsigned long long*)ctx->acc.p);
+  ++m.teps_seq;
+  hipLaunchKernelGGL(k_ms_teps, dim3(grid_of((g.n_rows + 63) / 64, kBlock / 64, 2048)), dim3(kBlock), 0, s, m.seen.p,
+                     g.weight.p, g.n_rows, all, (unsigned long long*)m.teps_acc.p);
+  hipLaunchKernelGGL(k_ms_teps_publish, dim3(1), dim3(128), 0, s, (unsigned long long*)m.teps_acc.p, m.teps_pub.d,
+                     m.teps_seq);
   G5_HIP(hipGetLastError());
-  uint64_t h[65];
-  G5_HIP(hipMemcpyAsync(h, ctx->acc.p, 65 * 8, hipMemcpyDeviceToHost, s));
-  G5_HIP(hipStreamSynchronize(s));
-  for (int r = 0; r < m.nroots; ++r) out[r] = (int64_t)((h[r] + h[64]) / 2);
+  m.teps_pub.wait(0, 65, m.teps_seq, s, "g5_batch_teps_edges: the sums were not published");
+  for (int r = 0; r < m.nroots; ++r) out[r] = (int64_t)((m.teps_pub.value(r) + m.teps_pub.value(64)) / 2);
 }
 
 void ms_model_bytes(g5_ctx* ctx, double* per_level, double* total) {

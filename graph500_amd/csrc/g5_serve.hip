@@ -20,6 +20,7 @@
 //
 // Reference: there is no serving loop in the reference; each answer equals
 // BfsBase::run_bfs's levels for the same root (mpi/bfs.hpp:2651-2940).
+#include "g5_answers.hpp"
 #include "g5_ctx.hpp"
 #include "g5_ms_device.hpp"
 
@@ -299,15 +300,6 @@ __global__ void __launch_bounds__(kBlock) k_sv_teps(const uint64_t* __restrict__
   }
 }
 
-// Answer (new ids) -> levels by original id.
-__global__ void k_sv_levels(const uint32_t* __restrict__ old2new, int64_t n, int64_t rows,
-                            const uint8_t* __restrict__ ans, int64_t root, uint8_t* __restrict__ out) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t nv = old2new[v];
-    out[v] = (v == root) ? 0 : ((int64_t)nv < rows ? ans[nv] : 0xFF);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Host
 // ---------------------------------------------------------------------------
@@ -343,7 +335,6 @@ struct SoloSlot {
   BfsState* b = nullptr;     // the state the runs use
   hipStream_t s = nullptr;
   bool own_stream = false;
-  DevBuf<uint64_t> acc;      // the traversed-edge reduction's scratch
   std::thread th;
   std::atomic<int> state{0};  // 0 free, 1 running, 2 finished
   int64_t req = -1;
@@ -431,6 +422,7 @@ struct g5_server {
   int64_t run_done = 0;  // requests of the current run answered so far
   double t0 = 0;  // start of the current run (now_s clock)
   g5::DevBuf<uint8_t> lv_out;
+  g5::HostStage stage;  // small answers on their way to the host
 };
 
 namespace g5 {
@@ -453,7 +445,6 @@ static void sv_setup_solo(Engine& e, int slots) {
       bfs_prepare(ctx, sl->own, sl->s);
       sl->b = &sl->own;
     }
-    sl->acc.alloc(4);
     e.solo.push_back(std::move(sl));
   }
 }
@@ -802,7 +793,7 @@ static void sv_start_solo(g5_server* srv, Engine& e, SoloSlot& sl, double t) {
         G5_HIP(hipMemcpyAsync(ans, sp->b->level.p, (size_t)rows, hipMemcpyDeviceToDevice, sp->s));
         G5_HIP(hipStreamSynchronize(sp->s));
       }
-      sp->edges = bfs_teps_edges(ctx, *sp->b, sp->acc, sp->s);
+      sp->edges = bfs_teps_edges(ctx, *sp->b, sp->s);
       sp->levels = sp->b->stats.num_levels - 1;
       sp->done = now_s() - t0;
     } catch (const Error& x) {
@@ -1086,12 +1077,9 @@ int g5_server_get_levels(g5_server* srv, int64_t request, uint8_t* levels) {
     G5_CHECK(q.status == SV_DONE && q.buf >= 0,
              "g5_server_get_levels: request not complete, not kept (keep = 0) or released");
     Engine& e = *srv->eng[q.graph];
-    srv->lv_out.alloc(e.n);
-    hipLaunchKernelGGL(k_sv_levels, dim3(grid_of(e.n, kBlock, 65536)), dim3(kBlock), 0, e.s,
-                       e.ctx->graph.old2new.p, e.n, e.rows, e.bufs[q.buf]->p, q.root, srv->lv_out.p);
-    G5_HIP(hipGetLastError());
-    G5_HIP(hipMemcpyAsync(levels, srv->lv_out.p, e.n, hipMemcpyDeviceToHost, e.s));
-    G5_HIP(hipStreamSynchronize(e.s));
+    HostOut out(levels, (size_t)e.n, srv->stage, srv->lv_out, e.s);
+    launch_make_levels(e.ctx->graph.old2new.p, e.bufs[q.buf]->p, e.n, e.rows, q.root, (uint8_t*)out.p, e.s);
+    out.finish();
   });
 }
 
