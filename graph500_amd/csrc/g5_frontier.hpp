@@ -195,12 +195,4 @@ __device__ __forceinline__ void gather_strided(uint64_t e0, uint64_t e1, int cnt
   }
 }
 
-// Tuple weight of a reached vertex (0xFF = unreached); the traversed-edge
-// count of a run is the sum over all rows, halved.
-struct ReachedWeight {
-  const uint8_t* level;
-  const uint32_t* weight;
-  __device__ uint64_t operator()(size_t i) const { return level[i] != 0xFF ? weight[i] : 0; }
-};
-
 }  // namespace g5
