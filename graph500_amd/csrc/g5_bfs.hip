@@ -915,19 +915,17 @@ __global__ void __launch_bounds__(kTepsThreads) k_teps(const uint8_t* __restrict
 //     by binary search in LDS), test-and-set the visited bitmap and append
 //     the winners through an LDS list;
 //   * a bottom-up level: a wave reads `span` bitmap words at a time (one
-//     coalesced load, one word per lane, span a power of two from 2 to 64),
-//     copies the words whose vertices are all visited to the next bitmap (one
-//     coalesced store) and walks the others two at a time, one lane per vertex
-//     of each, so both words' first-neighbour probes are in flight together.
-//     The host sizes span so that the grid still has a step per wave or more;
-//     late levels, where almost every word is full, then cost little more than
-//     a pass over the bitmap.  The new vertices are listed as well, as far as
+//     coalesced load, one word per lane) and probes those with an unvisited
+//     vertex (step_bottom_up); late levels, where almost every word is full,
+//     cost little more than a pass over the bitmap.  The new vertices are listed as well, as far as
 //     each workgroup's LDS list holds them, for a top-down level that follows;
 // and hands any other level back to the host (larger top-down levels, a
 // frontier whose queue has to be rebuilt from the bitmaps).  Graphs of one
 // workgroup's size run all their levels in one step.
 constexpr int kStepThreads = 1024;
 constexpr int kStepNf = 4096;
+constexpr int kBuWords = 4;        // open words whose first probes are in flight together (bottom-up)
+constexpr int kBuSpan = 16;        // most words of a bottom-up turn
 constexpr int kStepList = 2048;    // LDS list of a workgroup's new vertices
 constexpr int kStepTdGrid = 256;   // workgroups of a top-down level: kTdSmall edges are 4,096 waves of 256
 constexpr int kStepMaxLevel = 254; // levels are bytes, 0xFF = unreached
@@ -971,7 +969,8 @@ struct StepArgs {
   uint32_t* parent;
   Published* pub;
   int64_t words, n_active, small_edges, tail_pull;
-  int span;
+  int span;   // words per wave turn of a bottom-up level
+  int share;  // its rows are shared out in the workgroup
   int host_bu;  // bottom-up levels go back to the host
 };
 
@@ -982,10 +981,13 @@ __device__ __forceinline__ void step_publish_level(const StepArgs& a, uint64_t s
 }
 
 // Least workgroups of a step, the bitmap words and edges up to which one
-// workgroup takes the whole search in one launch, the bitmap words beyond
+// workgroup takes the whole search in one launch (S10, 14 words: 47 us a
+// search, 48 in steps of many; S12, 53 words: its large level takes 38 us
+// alone and 13 in 64 workgroups), the bitmap words beyond
 // which bottom-up levels go back to the host, and the steps launched ahead.
 constexpr unsigned kStepMinGrid = 64;
-constexpr int64_t kStepAloneWords = 64;
+constexpr int64_t kStepAloneWords = 32;
+constexpr int64_t kStepShareWords = 8192;  // see step_bottom_up
 constexpr int64_t kStepAloneEdges = 1 << 18;
 constexpr int64_t kStepMaxWords = 100000;
 constexpr int kStepAhead = 3;
@@ -1024,8 +1026,19 @@ __host__ __device__ __forceinline__ bool tail_pulls(int forward, int growing, in
 
 static_assert(sizeof(StepArgs) <= 32 * 8, "argument block");
 
+// What a workgroup of kWaves waves keeps of a bottom-up turn.
+template <int kWaves>
+struct BuLds {
+  uint16_t miss[kWaves * kBuSpan * 64];
+  uint32_t got[kWaves * kBuSpan * 2];
+  uint32_t n[kWaves];
+};
+
 struct StepLds {
-  uint64_t base[kStepNf];     // cols index of frontier row i's first entry - pre[i]
+  union {
+    uint64_t base[kStepNf];  // cols index of frontier row i's first entry - pre[i]
+    BuLds<kStepThreads / 64> bu;
+  };
   uint32_t pre[kStepNf + 1];  // first virtual edge of the row
   uint32_t src[kStepNf];
   uint32_t list[kStepList];
@@ -1155,67 +1168,118 @@ __device__ __forceinline__ void step_expand(const StepArgs& a, const StepLds& L,
     }
 }
 
-// The bottom-up body over waves wave0, wave0 + nwaves, ...; with a list (LDS,
-// kStepList entries and their count) found vertices are appended to it.
-// Returns the wave's count (in every lane).
-template <int kU, int kR>
-__device__ __forceinline__ uint64_t step_bottom_up(const StepArgs& a, uint32_t* list, uint32_t* list_n,
-                                                   const uint64_t* __restrict__ vis, uint64_t* __restrict__ vis_next,
-                                                   int lvl, int64_t wave0, int64_t nwaves) {
-  const int lane = threadIdx.x & 63, span = a.span;
+// The bottom-up body.  A wave of the workgroup takes `span` words a turn,
+// probes the first neighbours of kBuWords open words at a time and lists who
+// missed; the rows of those are then searched with every lane busy, whatever
+// words they come from (got gathers who was found).  Searched word by word, a
+// turn of 128 vertices waited for six dependent loads (searches, us: S14 85,
+// now 67; S21 131, 119; S24 318, 302; S28 2,525-2,590, 2,450-2,500; k_bu's
+// largest level there moves 1 GB in 500 us).  `share`: the
+// workgroup's waves share the rows out, so that a word of hubs, whose long
+// rows one wave searches one after another, does not hold the level up;
+// where waves have words enough that costs more than it gives (S14 18 -> 13
+// us a level, S23 36 -> 40).  With a list (LDS, kStepList entries and their
+// count) found vertices are appended to it.  Every thread of the workgroup
+// calls it.  kSpread: neighbouring turns go to different workgroups (hubs are
+// neighbours).  Returns the lane's share of the count.
+template <int kWaves, int kU, int kR, bool kSpread>
+__device__ __forceinline__ uint64_t step_bottom_up(const StepArgs& a, BuLds<kWaves>& B, uint32_t* list,
+                                                   uint32_t* list_n, const uint64_t* __restrict__ vis,
+                                                   uint64_t* __restrict__ vis_next, int lvl, bool share) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, span = a.span;
   const uint64_t below = lane ? ~UINT64_C(0) >> (64 - lane) : 0;
+  // list position of the first of n new vertices (a full list stays full: further counts are not needed)
+  const auto list_at = [&](uint32_t n) {
+    uint32_t pos = kStepList;
+    if (lane == 0 && n && *list_n <= (uint32_t)kStepList) pos = atomicAdd(list_n, n);
+    return (uint32_t)__builtin_amdgcn_readfirstlane(pos);
+  };
+  const auto found = [&](int64_t v, uint32_t p, uint32_t pos) {
+    a.level[v] = (uint8_t)lvl;
+    a.parent[v] = p;
+    if (list && pos < (uint32_t)kStepList) list[pos] = (uint32_t)v;
+  };
   uint64_t total = 0;
-  for (int64_t base = wave0 * span; base < a.words; base += nwaves * span) {
-    const int64_t wl = base + lane;
+  // word j of wave w's turn has slot w * kBuSpan + j
+  const auto word_of = [&](int64_t turn, int slot) {
+    const int w = slot / kBuSpan;
+    const int64_t at = kSpread ? (turn * kWaves + w) * gridDim.x + blockIdx.x
+                               : (turn * gridDim.x + blockIdx.x) * kWaves + w;
+    return at * span + slot % kBuSpan;
+  };
+  uint32_t* got = B.got + wave * kBuSpan * 2;
+  uint32_t* count = share ? B.n : B.n + wave;
+  uint16_t* miss = share ? B.miss : B.miss + wave * kBuSpan * 64;
+  const int first = share ? wave : 0, step = share ? kWaves : 1;
+  const auto sync = [&] {
+    if (share) __syncthreads();
+    else __builtin_amdgcn_wave_barrier();
+  };
+  for (int64_t turn = 0; turn * kWaves * gridDim.x * span < a.words; ++turn) {
+    const int64_t base = word_of(turn, wave * kBuSpan), wl = base + lane;
     const bool mine = lane < span && wl < a.words;
     const uint64_t cl = mine ? vis[wl] : ~UINT64_C(0);  // lanes beyond the span or the end read as visited
-    uint64_t open = __ballot(cl != ~UINT64_C(0));        // words with an unvisited vertex
-    if (mine && cl == ~UINT64_C(0)) vis_next[wl] = cl;
-    while (open) {
-      // the next two open words (identical in every lane)
-      const int j0 = __builtin_ctzll(open);
-      open &= open - 1;
-      const bool has1 = open != 0;
-      const int j1 = has1 ? __builtin_ctzll(open) : j0;
-      if (has1) open &= open - 1;
-      const uint64_t c0 = __shfl(cl, j0, 64);
-      const uint64_t c1 = has1 ? __shfl(cl, j1, 64) : ~UINT64_C(0);
-      const int64_t w0 = base + j0, w1 = base + j1;
-      const uint32_t v0 = (uint32_t)(w0 * 64 + lane), v1 = (uint32_t)(w1 * 64 + lane);
-      const bool a0 = !((c0 >> lane) & 1), a1 = !((c1 >> lane) & 1);
-      const uint32_t f0 = a0 ? a.first_nbr[v0] : kNoNbr;
-      const uint32_t f1 = a1 ? a.first_nbr[v1] : kNoNbr;
-      const bool h0 = f0 != kNoNbr && bit_set(vis, f0);
-      const bool h1 = f1 != kNoNbr && bit_set(vis, f1);
-      uint32_t p0 = f0, p1 = f1;
-      // every lane makes both calls (the long-row scan needs the whole wave)
-      const bool r0 = row_marked_nbr<kU, kR>(f0 != kNoNbr && !h0, v0, vis, a.offsets, a.cols, p0);
-      const bool r1 = row_marked_nbr<kU, kR>(f1 != kNoNbr && !h1, v1, vis, a.offsets, a.cols, p1);
-      const bool g0 = h0 || r0, g1 = h1 || r1;
-      const uint64_t m0 = __ballot(g0), m1 = __ballot(g1);
-      const uint32_t n0 = (uint32_t)__popcll(m0), n1 = (uint32_t)__popcll(m1);
-      uint32_t pos = 0;
-      if (lane == 0) {
-        vis_next[w0] = c0 | m0;
-        if (has1) vis_next[w1] = c1 | m1;
-        // a full list stays full: further counts are not needed
-        pos = kStepList;
-        if (list && n0 + n1 && *list_n <= (uint32_t)kStepList) pos = atomicAdd(list_n, n0 + n1);
+    if (lane < 2 * span) got[lane] = 0;
+    if (share ? threadIdx.x == 0 : lane == 0) *count = 0;
+    sync();
+    for (uint64_t open = __ballot(cl != ~UINT64_C(0)); open;) {
+      int j[kBuWords];
+      uint32_t f[kBuWords];
+      bool h[kBuWords];
+      uint64_t m[kBuWords], r[kBuWords];
+#pragma unroll
+      for (int i = 0; i < kBuWords; ++i) {
+        j[i] = open ? __builtin_ctzll(open) : -1;
+        open &= open - 1;
+        const uint64_t c = j[i] >= 0 ? __shfl(cl, j[i], 64) : ~UINT64_C(0);
+        f[i] = (c >> lane) & 1 ? kNoNbr : a.first_nbr[(base + j[i]) * 64 + lane];
       }
-      if (list) pos = __builtin_amdgcn_readfirstlane(pos);
-      if (g0) {
-        a.level[v0] = (uint8_t)lvl;
-        a.parent[v0] = p0;
-        const uint32_t i = pos + (uint32_t)__popcll(m0 & below);
-        if (list && i < (uint32_t)kStepList) list[i] = v0;
+#pragma unroll
+      for (int i = 0; i < kBuWords; ++i) h[i] = f[i] != kNoNbr && bit_set(vis, f[i]);
+      uint32_t pos = 0, out = 0;
+#pragma unroll
+      for (int i = 0; i < kBuWords; ++i) {
+        m[i] = __ballot(h[i]);
+        r[i] = __ballot(f[i] != kNoNbr && !h[i]);
+        pos += (uint32_t)__popcll(m[i]);
+        out += (uint32_t)__popcll(r[i]);
       }
-      if (g1) {
-        a.level[v1] = (uint8_t)lvl;
-        a.parent[v1] = p1;
-        const uint32_t i = pos + n0 + (uint32_t)__popcll(m1 & below);
-        if (list && i < (uint32_t)kStepList) list[i] = v1;
+      if (list) pos = list_at(pos);
+      if (out) {
+        if (lane == 0) out = atomicAdd(count, out);
+        out = __builtin_amdgcn_readfirstlane(out);
       }
-      total += n0 + n1;
+#pragma unroll
+      for (int i = 0; i < kBuWords; ++i) {
+        if (j[i] < 0) continue;
+        if (lane < 2) got[2 * j[i] + lane] = (uint32_t)(m[i] >> (32 * lane));
+        if (h[i]) found((base + j[i]) * 64 + lane, f[i], pos + (uint32_t)__popcll(m[i] & below));
+        pos += (uint32_t)__popcll(m[i]);
+        if ((r[i] >> lane) & 1)
+          miss[out + (uint32_t)__popcll(r[i] & below)] = (uint16_t)((wave * kBuSpan + j[i]) * 64 + lane);
+        out += (uint32_t)__popcll(r[i]);
+      }
+    }
+    sync();
+    const int nmiss = (int)*count;
+    for (int i = first; i < nmiss; i += step * 64) {
+      const bool in = i + lane * step < nmiss;
+      const int x = in ? miss[i + lane * step] : 0;
+      const int64_t v = word_of(turn, x >> 6) * 64 + (x & 63);
+      uint32_t p = 0;
+      const bool hit = row_marked_nbr<kU, kR>(in, (uint32_t)v, vis, a.offsets, a.cols, p);
+      const uint64_t r = __ballot(hit);
+      const uint32_t pos = list ? list_at((uint32_t)__popcll(r)) : 0;
+      if (hit) {
+        found(v, p, pos + (uint32_t)__popcll(r & below));
+        atomicOr(B.got + (x >> 5), 1u << (x & 31));
+      }
+    }
+    sync();
+    if (mine) {
+      const uint64_t n = got[2 * lane] | (uint64_t)got[2 * lane + 1] << 32;
+      vis_next[wl] = cl | n;
+      total += __popcll(n);
     }
   }
   return total;
@@ -1345,9 +1409,9 @@ __global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* _
       __syncthreads();
       const StepArgs& a = step_args(ctl);
       const int cur = __builtin_amdgcn_readfirstlane(L.st.cur);
-      const uint64_t f = step_bottom_up<8, 4>(a, L.list, &L.n, a.vis[cur], a.vis[cur ^ 1], lvl,
-                                              (int64_t)blockIdx.x * (kStepThreads / 64) + wave,
-                                              (int64_t)gridDim.x * (kStepThreads / 64));
+      const uint64_t f = wave_sum(step_bottom_up<kStepThreads / 64, 8, 4, true>(a, L.bu, L.list, &L.n, a.vis[cur],
+                                                                          a.vis[cur ^ 1], lvl,
+                                                                          a.share));
       if (lane == 0) L.wave[wave] = f;
     }
     __syncthreads();
@@ -1422,10 +1486,9 @@ __global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* _
 // 256-thread workgroups without a list, at twice the waves per CU a step
 // leaves room for (its registers and LDS hold 16).
 __global__ void __launch_bounds__(kBlock) k_bu(StepArgs a, int cur, int lvl, unsigned long long* __restrict__ counters) {
-  const uint64_t f = step_bottom_up<4, 1>(a, nullptr, nullptr, a.vis[cur], a.vis[cur ^ 1], lvl,
-                                          (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6),
-                                          (int64_t)gridDim.x * (kBlock / 64));
-  block_add((threadIdx.x & 63) == 0 ? f : 0, stripe_of(counters + kStripeBase, S_FOUND));
+  __shared__ BuLds<kBlock / 64> bu;
+  const uint64_t f = step_bottom_up<kBlock / 64, 4, 1, false>(a, bu, nullptr, nullptr, a.vis[cur], a.vis[cur ^ 1], lvl, false);
+  block_add(f, stripe_of(counters + kStripeBase, S_FOUND));
 }
 
 // The state a row of steps goes on from after a level run by the host (slot:
@@ -1807,9 +1870,21 @@ static void host_bottom_up(g5_ctx* ctx, BfsState& b, hipStream_t s, const StepAr
 // Workgroups of a step: one for the smallest graphs; else enough waves for a
 // turn of every wave in a bottom-up level, and at least kStepMinGrid for the
 // top-down levels.
+static bool step_alone(const Graph& g, const BfsState& b) {
+  return b.words <= kStepAloneWords && g.nnz <= kStepAloneEdges;
+}
+// Bitmap words per wave turn of a bottom-up level.  In a step, what gives
+// every wave the same number of turns; for k_bu, 8, or 16 where a wave still
+// has ten turns or more (S26 8/16: 674/685 us a search, S28: 2,521/2,469).
+static int bottom_up_span(const Graph& g, const BfsState& b) {
+  if (b.words > kStepMaxWords) return b.words >= (INT64_C(1) << 20) ? 16 : 8;
+  const int64_t waves = (step_alone(g, b) ? 1 : kStepTdGrid) * (kStepThreads / 64);
+  const int64_t turns = (b.words + waves * kBuSpan - 1) / (waves * kBuSpan);
+  return (int)((b.words + waves * turns - 1) / (waves * turns));
+}
 static unsigned step_grid(const Graph& g, const BfsState& b, int span) {
-  if (b.words <= kStepAloneWords && g.nnz <= kStepAloneEdges) return 1;
-  return std::max(kStepMinGrid, grid_of((b.words + span - 1) / span, kStepThreads / 64, kStepTdGrid * 2));
+  if (step_alone(g, b)) return 1;
+  return std::max(kStepMinGrid, grid_of((b.words + span - 1) / span, kStepThreads / 64, kStepTdGrid));
 }
 
 // Steps until one stops; returns its state (see k_bfs_step).  k counts the
@@ -1886,10 +1961,9 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   a.n_active = g.n_active;
   a.small_edges = b.small_edges;
   a.tail_pull = b.tail_pull;
-  // bitmap words per wave turn: as many as keep at least 32768 turns
-  a.span = 2;
-  while (a.span < 64 && b.words / (2 * a.span) >= 32768) a.span *= 2;
   a.host_bu = b.words > kStepMaxWords;
+  a.span = bottom_up_span(g, b);
+  a.share = b.words <= kStepShareWords;
   const unsigned grid = step_grid(g, b, a.span);
   hipLaunchKernelGGL(k_bfs_init, dim3(grid_of((rows + 15) / 16, kBlock, 2048)), dim3(kBlock), 0, s, g.old2new.p, root,
                      rows, b.words, b.level.p, b.parent.p, b.vis[0].p, b.queue[0].p,

@@ -78,3 +78,17 @@ def test_many_claims_of_few_words(oracle_mod):
     dst = np.tile(np.arange(4000, 4200), 3000)
     root = np.stack([np.zeros(3000, np.int64), np.arange(1, 3001)], 1)
     check(oracle_mod, tuples(np.concatenate([root, np.stack([src, dst], 1)])), [0, 4100, 17])
+
+
+@pytest.mark.parametrize("rows", [2047, 2048, 2049, 262143, 262145, 524288, 524289, 1048577])
+def test_bottom_up_turns(oracle_mod, rows):
+    """Bottom-up levels where one workgroup ends (32 words), where a turn grows
+    from one word to two and three (4,096 and 8,192 words) and rows are no
+    longer shared out: some hubs, short rows whose first neighbour misses, and
+    a path that goes on after them."""
+    rng = np.random.default_rng(rows)
+    hubs = rng.integers(0, rows // 100, (rows * 2, 1))
+    p = np.concatenate([np.concatenate([hubs, rng.integers(0, rows, (rows * 2, 1))], 1),
+                        rng.integers(0, rows, (rows, 2)),
+                        np.stack([np.arange(rows - 20, rows - 1), np.arange(rows - 19, rows)], 1)])
+    check(oracle_mod, tuples(p), [0, rows - 1, int(p[7, 1])])
