@@ -9,7 +9,18 @@
 namespace g5 {
 
 constexpr uint32_t kMsNoNbr = 0xFFFFFFFFu;
-constexpr int kMsShortRow = 32;
+// Pulls: rows up to kMsShortRow entries are searched by their lane, longer ones
+// by groups of kMsGroup lanes for up to kMsGroupTurns turns, and what is left
+// of very long ones by whole waves.  A pull is bound by its lookups of frontier
+// words past the L2 (about 55 a nanosecond): a whole wave per row looked up 64
+// at least where the first 16 mostly settle the row, and a lane per row read
+// its columns alone.  Batches of 64, us: S22 1,165 with rows up to 32 by their
+// lane and the others by waves, 971 so (groups of 8: 996); S24 3,490, 2,735
+// (2,770); S26 13,420, 11,110 (11,560); the limit 4, 16 or 32 in place of 8:
+// 10,950, 11,190, 11,520 at S26 and 990, 997, 990 at S22.
+constexpr int kMsShortRow = 8;
+constexpr int kMsGroup = 16;
+constexpr int kMsGroupTurns = 16;
 
 enum { M_LIVE = 0, M_PAIRS = 1, M_NZ = 2, M_FDEG = 3, M_NUM = 8 };
 
@@ -41,6 +52,18 @@ __device__ __forceinline__ uint64_t wave_or(uint64_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
   return v;
+}
+
+// OR over each group of 16 lanes, in all of them
+__device__ __forceinline__ uint32_t group_or(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);   // quad_perm 1,0,3,2
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2,3,0,1
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
+  return v;
+}
+__device__ __forceinline__ uint64_t group_or(uint64_t v) {
+  return group_or((uint32_t)v) | (uint64_t)group_or((uint32_t)(v >> 32)) << 32;
 }
 
 // Block-wide OR / sums of the level counters, one atomic each per workgroup.
@@ -317,7 +340,7 @@ struct CompactEmit {
 
 // The probes of one pull step for each lane's vertex v (need: the lanes v
 // still has to find; 0 for a lane with nothing to do): its first neighbour,
-// then its short row lane-sequentially or its long row by the whole wave.
+// then the rest of its row (see kMsShortRow).
 // Every lane of the wave calls it.  Returns the OR of the frontier words
 // probed (at least the needed lanes when they are all present).
 template <int kU, int kW>
@@ -355,7 +378,59 @@ __device__ __forceinline__ uint64_t ms_pull_probe(const FrontView& fv, int64_t v
     }
     more = false;
   }
-  uint64_t lm = __ballot(more);
+  // rows of more entries by groups of kMsGroup lanes, 64 / kMsGroup rows at a
+  // time, a group taking the next row as soon as its own is done
+  const int gid = lane / kMsGroup, gl = lane % kMsGroup;
+  uint64_t lm = __ballot(more), rest = 0;
+  int src = -1, turn = 0;
+  uint64_t b = 0, e = 0, nd = 0, a = 0;
+  for (;;) {
+    const uint64_t idle = __ballot(src < 0);
+    if (idle) {
+      if (!lm && idle == ~UINT64_C(0)) break;
+      const int rank = __popcll(idle & ((UINT64_C(1) << (gid * kMsGroup)) - 1)) / kMsGroup;
+      int take = -1;
+      for (int i = 0; i < __popcll(idle) / kMsGroup && lm; ++i) {
+        if (i == rank) take = __builtin_ctzll(lm);
+        lm &= lm - 1;
+      }
+      const int from = take < 0 ? lane : take;
+      const uint64_t b1 = __shfl(rb, from, 64), e1 = __shfl(re, from, 64);
+      const uint64_t n1 = __shfl(need, from, 64), a1 = __shfl(acc, from, 64);
+      if (src < 0 && take >= 0) {
+        src = take;
+        b = b1;
+        e = e1;
+        nd = n1;
+        a = a1;
+        turn = 0;
+      }
+    }
+    const bool in = src >= 0 && b + gl < e;
+    const uint32_t w = in ? cols[b + gl] : 0;
+    a |= group_or(in ? front_of(fv, w) : UINT64_C(0));
+    b += kMsGroup;
+    ++turn;
+    const bool full = (a & nd) == nd, done = src >= 0 && (full || b >= e);
+    const bool pass = src >= 0 && !done && turn >= kMsGroupTurns && e - b > 64 * kW;  // left to the whole wave
+    const uint64_t out = __ballot(done || pass);
+    if (out) {
+#pragma unroll
+      for (int g = 0; g < 64 / kMsGroup; ++g) {
+        if (!((out >> (g * kMsGroup)) & 1)) continue;
+        const int s = __builtin_amdgcn_readlane(src, g * kMsGroup);
+        const uint64_t ga = __shfl(a, g * kMsGroup, 64), gb = __shfl(b, g * kMsGroup, 64);
+        if (lane == s) {
+          acc = ga;
+          rb = gb;
+        }
+        rest |= (uint64_t)(__builtin_amdgcn_readlane((int)pass, g * kMsGroup) & 1) << s;
+      }
+      if (done || pass) src = -1;
+    }
+  }
+  // what the groups left of long rows, by the whole wave
+  lm = rest;
   while (lm) {
     const int src = __ffsll((unsigned long long)lm) - 1;
     lm &= lm - 1;
@@ -381,7 +456,14 @@ __device__ __forceinline__ uint64_t ms_pull_probe(const FrontView& fv, int64_t v
 
 // kU: independent probes per step of a lane's short row; kW: entries per lane
 // and step of the wave's scan of a long row (kW x 64 per step).
-template <class Epi = NoEpilogue, int kU = 4, int kW = 2>
+template <int kRows>
+__device__ __forceinline__ void store_bits(uint64_t* words, int64_t turn, uint64_t bits) {
+  if (kRows == 64) words[turn] = bits;
+  else reinterpret_cast<uint16_t*>(words)[turn] = (uint16_t)bits;
+}
+
+// A wave takes kRows rows a turn.
+template <class Epi = NoEpilogue, int kU = 4, int kW = 2, int kRows = 64>
 __device__ __forceinline__ void ms_pull_body(uint64_t* __restrict__ seen, const FrontView fv,
                                              uint64_t* __restrict__ next, uint64_t* __restrict__ nz_next,
                                              const uint32_t* __restrict__ first_nbr,
@@ -393,11 +475,12 @@ __device__ __forceinline__ void ms_pull_body(uint64_t* __restrict__ seen, const 
   const int lane = threadIdx.x & 63;
   const int64_t nwaves = (int64_t)nblk * (kBlock / 64);
   uint64_t live = 0, pairs = 0, nz = 0, fdeg = 0;
-  const int64_t words = (rows + 63) / 64;
+  static_assert(kRows == 64 || kRows == 16, "bits of a turn are stored as one word or quarter word");
+  const int64_t turns = (rows + 63) / 64 * (64 / kRows);
   epi.begin();
-  for (int64_t wd = (int64_t)bid * (kBlock / 64) + (threadIdx.x >> 6); wd < words; wd += nwaves) {
-    const int64_t v = wd * 64 + lane;
-    const bool inb = v < rows;
+  for (int64_t wd = (int64_t)bid * (kBlock / 64) + (threadIdx.x >> 6); wd < turns; wd += nwaves) {
+    const int64_t v = wd * kRows + lane;
+    const bool inb = lane < kRows && v < rows;
     const uint64_t s0 = inb ? seen[v] : ~UINT64_C(0);
     const uint64_t s = inb ? (s0 & keep) : s0;
     const uint64_t need = ~s & live_in;
@@ -410,10 +493,10 @@ __device__ __forceinline__ void ms_pull_body(uint64_t* __restrict__ seen, const 
     // one bit per vertex still missing a live lane, for the list-driven tail levels
     if (miss) {
       const uint64_t mb = __ballot(inb && (live_in & ~(s | nw)) != 0);
-      if (lane == 0) miss[wd] = mb;
+      if (lane == 0) store_bits<kRows>(miss, wd, mb);
     }
     const uint64_t b = __ballot(nw != 0);
-    if (lane == 0) nz_next[wd] = b;
+    if (lane == 0) store_bits<kRows>(nz_next, wd, b);
     if (inb) {
       // with merge the array was cleared before the push and holds zeros or
       // pushed lanes: only words that change are written

@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_finish(uint64_t* __restrict__ see
   ms_finish_body(seen, next, nz_next, offsets, rows, ms_stripe(c), blockIdx.x, gridDim.x);
 }
 
-template <int kU, int kW>
+template <int kU, int kW, int kRows = 64>
 __global__ void __launch_bounds__(kBlock) k_ms_pull(uint64_t* __restrict__ seen, const uint64_t* __restrict__ front,
                                                     const uint64_t* __restrict__ nz_front, uint64_t* __restrict__ next,
                                                     uint64_t* __restrict__ nz_next,
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull(uint64_t* __restrict__ seen,
                                                     const uint64_t* __restrict__ compact, uint32_t filter_from,
                                                     unsigned long long* __restrict__ c, uint64_t* __restrict__ miss) {
   const FrontView fv{front, nz_front, pack, compact, mode, filter_from};
-  ms_pull_body<NoEpilogue, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+  ms_pull_body<NoEpilogue, kU, kW, kRows>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
                                    blockIdx.x, gridDim.x, ~UINT64_C(0), NoEpilogue(), false, miss);
 }
 
@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_finish_lanes(uint64_t* __restrict
 
 // Pull for the lanes in live_in; with merge, next already holds this level's
 // pushed lanes, which are folded in.
-template <int kU, int kW>
+template <int kU, int kW, int kRows = 64>
 __global__ void __launch_bounds__(kBlock) k_ms_pull_lanes(uint64_t* __restrict__ seen, const uint64_t* __restrict__ front,
                                                           const uint64_t* __restrict__ nz_front, uint64_t* __restrict__ next,
                                                           uint64_t* __restrict__ nz_next,
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull_lanes(uint64_t* __restrict__
   LaneEpi epi = epi_in;  // a copy in registers: the epilogue accumulates per thread
   epi.lane_nq = ms_stripe(epi.lane_nq);
   const FrontView fv{front, nz_front, nullptr, nullptr, filter ? kFrontFilter : kFrontPlain, 0};
-  ms_pull_body<LaneEpi, kU, kW>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+  ms_pull_body<LaneEpi, kU, kW, kRows>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
                                 blockIdx.x, gridDim.x, ~UINT64_C(0), epi, merge != 0);
 }
 
@@ -286,6 +286,15 @@ constexpr double kListBelow = 16.0;
 // shorter than its bound, and workgroups that find nothing to do still cost
 // (SCALE 28, per listed level: 0.070 ms on up to 4,096, 0.093 on 16,384).
 constexpr int64_t kListGrid = 2048;
+
+// Pulls of graphs up to this many words take 16 rows a turn instead of 64: a
+// wave with the 64 rows of the largest hubs outlasts the rest of a small
+// graph (the first pull of S12 87 us, now 49; S16 120, 68; S18 152, 95).  A
+// pull that follows finds most rows done, and turns cost more than they give
+// from S19 on (5,200 words: 9 us a level, now 20); a first one loses from S21
+// (167 us, 178; S20 133, 113).
+constexpr int64_t kPartWords = 4096;
+constexpr int64_t kPartWordsFirst = 12288;
 
 // A push level lists the vertices it touches when its frontier edges times
 // this are fewer than the rows (the touched vertices are at most the edges).
@@ -767,6 +776,8 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
   uint64_t pulled = 0;  // roots that have pulled: they pull from then on
   const uint64_t* h_lane = m.h_counters.data() + kMsLanes;
   unsigned* d_list_count = (unsigned*)(cnt + M_NUM);
+  // turns of a pull that takes 16 rows each up to `limit` words
+  const auto pull_turns = [&](int64_t limit) { return m.pull_unroll == 0 && words <= limit ? words * 4 : words; };
   bool have_miss = false;  // m.miss holds the vertices still missing a live root
   int l = l0 - 1;
   while (live) {
@@ -792,12 +803,18 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       // reached (the roots' own level pushes; all pull in the beta tail); a
       // root that has pulled keeps pulling, so once every live root pulls
       // the level is a plain pull with no per-root statistics
+      // A level pulls only when the union of the frontiers has edges enough:
+      // a pull reads the rows of everything unreached however few roots it is
+      // for, a push the union's rows (S26, 2 of 64 roots over the line at 3 %
+      // of the edges: pull 4.7 ms, push of all 1.6; the least a pull pays at
+      // is 1/8 of the edges, at larger alpha 16/alpha).
       const bool tail = total_pairs - reached < unseen_frac * total_pairs;
+      const bool enough = (double)fdeg * std::max(8.0, m.alpha / 16.0) > (double)g.nnz;
       for (int r = 0; r < 64; ++r) {
         const uint64_t bit = UINT64_C(1) << r;
         if (!(live & bit)) continue;
         const double unreached = (double)g.nnz - lane_vd[r];
-        const bool pull_r = tail || (pulled & bit) || (l > 1 && lane_fd[r] * m.alpha > unreached);
+        const bool pull_r = tail || (pulled & bit) || (l > 1 && enough && lane_fd[r] * m.alpha > unreached);
         (pull_r ? bu : td) |= bit;
       }
       pulled |= bu;
@@ -862,9 +879,9 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         case 5: kpl = k_ms_pull_lanes<1, 1>; break;
         case 6: kpl = k_ms_pull_lanes<2, 2>; break;
         case 7: kpl = k_ms_pull_lanes<1, 2>; break;
-        default: break;
+        default: if (words <= kPartWordsFirst) kpl = k_ms_pull_lanes<4, 2, 16>;
       }
-      hipLaunchKernelGGL(kpl, dim3(grid_of(words, kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
+      hipLaunchKernelGGL(kpl, dim3(grid_of(pull_turns(kPartWordsFirst), kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
                          nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, rows, bu,
                          m.pull_filter == 1 ? 1 : 0, 1, cnt, lepi);
     } else if (push) {
@@ -934,7 +951,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         case 5: kp = k_ms_pull<1, 1>; break;
         case 6: kp = k_ms_pull<2, 2>; break;
         case 7: kp = k_ms_pull<1, 2>; break;
-        default: break;
+        default: if (words <= kPartWords) kp = k_ms_pull<4, 2, 16>;
       }
       // Tail levels: once fewer than rows / kListBelow (root, vertex) pairs
       // are unreached, a pull also marks the vertices still missing a live
@@ -961,7 +978,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         // the pull writes every word of the level's frontier array (clearing
         // its old words first, one store per marked vertex, so that the pull
         // could skip its zero words, measured no faster)
-        hipLaunchKernelGGL(kp, dim3(grid_of(words, kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
+        hipLaunchKernelGGL(kp, dim3(grid_of(pull_turns(kPartWords), kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
                            nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, rows, live, mode,
                            m.pack.p, m.compact.p, filter_from, cnt, mark ? m.miss.p : nullptr);
         list_level = mark;
