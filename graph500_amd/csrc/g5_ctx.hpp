@@ -232,8 +232,8 @@ struct MsState {
   PublishBlock pub;             // the counters as each level publishes them (g5_msbfs.hip)
   uint64_t pub_seq = 0;
   g5_batch_stats stats{};
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  std::vector<hipEvent_t> lev_begin, lev_end;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;  // around a persistent run
+  DevBuf<uint64_t> stamps;                  // device clock at a batch's and a level's start
   void release() {
     seen.release();
     for (auto& b : nz) b.release();
@@ -244,6 +244,7 @@ struct MsState {
     frp.release();
     row_level.release();
     teps_acc.release();
+    stamps.release();
     queue.release();
     touch.release();
     miss.release();
@@ -276,8 +277,6 @@ struct MsState {
   }
   // events and published blocks stay with the state from one graph to the next
   ~MsState() {
-    destroy_events(lev_begin);
-    destroy_events(lev_end);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
   }

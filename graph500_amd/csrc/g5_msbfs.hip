@@ -15,10 +15,12 @@
 //   pull  one lane per vertex: the lanes it still lacks (and whose frontier
 //         is not empty) are collected by OR-ing the neighbours' frontier
 //         words in ascending (highest degree first) order until every needed
-//         lane is found or the row ends; long rows are scanned by the whole
-//         wave with a wave-wide OR.  A 1-bit-per-vertex "frontier word is not
-//         zero" bitmap (n/8 bytes, cache resident) is tested first, so the
-//         8-byte frontier word is only read for frontier vertices
+//         lane is found or the row ends, rows over 8 entries by groups of 16
+//         lanes.  On request a 1-bit-per-vertex "frontier word is not zero"
+//         bitmap (n/8 bytes) is tested before an 8-byte frontier word
+// Small graphs are bound by launches: a level is at most five (select, ready,
+// push, pull, publish), a pull two, a start two (S12, 64 roots: 41 launches
+// and 242 us, now 24 and 162).
 // Per-lane levels equal the single-root BFS levels of the same root.
 #include "g5_answers.hpp"
 #include "g5_ctx.hpp"
@@ -33,6 +35,15 @@ namespace g5 {
 constexpr int kMsCounters = kMsLanes + 128;  // level counters, a list count, per-lane counts and degree sums
 constexpr size_t kMsCounterWords = (size_t)kMsStripes * kMsStride;
 static_assert(kMsCounters <= kMsStride, "a counter copy holds every counter");
+
+// Device clock at the start of a batch and of a level (m.stamps); a level's
+// first kernel stamps it, and every publish sends the times since both.
+// (Events around each level took 7 us a level of the stream's time.)
+enum { T_BATCH = 0, T_LEVEL = 1, T_NUM = 2 };
+__device__ __forceinline__ void ms_stamp(uint64_t* stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+__global__ void k_ms_stamp(uint64_t* stamp) { ms_stamp(stamp); }
 
 __global__ void __launch_bounds__(kBlock) k_ms_clear(uint64_t* __restrict__ a, uint64_t* __restrict__ b,
                                                      int64_t n) {
@@ -74,6 +85,63 @@ __global__ void k_ms_roots(const uint32_t* __restrict__ old2new, const int64_t* 
 }
 
 // Level-0 nonzero bitmap: the root vertices (lane r, root r).
+// The roots of a level-by-level batch, in the argument block.
+struct MsRoots {
+  int64_t root[64];
+  int n;
+};
+
+// A batch's start in two launches.  k_ms_begin clears the reached lanes, level
+// 0's frontier words (the ones its last run marked, or all), their marks and
+// the level counters (which every publish clears again); k_ms_place puts the
+// roots in and publishes the first level's counters.
+__global__ void __launch_bounds__(kBlock) k_ms_begin(uint64_t* __restrict__ seen, uint64_t* __restrict__ fr0,
+                                                     uint64_t* __restrict__ nz0, int64_t rows, int64_t words,
+                                                     int marked, unsigned long long* __restrict__ counters,
+                                                     uint64_t* __restrict__ stamps) {
+  ms_stamp(stamps + T_BATCH);
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x, stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t v = t; v < rows; v += stride) {
+    seen[v] = 0;
+    if (!marked) fr0[v] = 0;
+  }
+  for (int64_t wd = t; wd < words; wd += stride) {
+    if (marked)
+      for (uint64_t b = nz0[wd]; b; b &= b - 1) {
+        const int64_t v = wd * 64 + __builtin_ctzll(b);
+        if (v < rows) fr0[v] = 0;
+      }
+    nz0[wd] = 0;
+  }
+  for (int64_t i = t; i < (int64_t)kMsCounterWords; i += stride) counters[i] = 0;
+}
+
+__global__ void __launch_bounds__(64) k_ms_place(const uint32_t* __restrict__ old2new, MsRoots roots, int64_t rows,
+                                                 const uint64_t* __restrict__ offsets, uint64_t* __restrict__ seen,
+                                                 uint64_t* __restrict__ fr0, uint64_t* __restrict__ nz0,
+                                                 Published* __restrict__ pub, uint64_t seq,
+                                                 const uint64_t* __restrict__ stamps) {
+  const int r = threadIdx.x;
+  bool act = false, first = false;
+  uint64_t deg = 0;
+  if (r < roots.n) {
+    const uint32_t v = old2new[roots.root[r]];
+    act = (int64_t)v < rows;  // a root without edges discovers nothing
+    if (act) {
+      const unsigned long long bit = 1ull << r;
+      atomicOr((unsigned long long*)(seen + v), bit);
+      atomicOr((unsigned long long*)(nz0 + (v >> 6)), 1ull << (v & 63));
+      first = atomicOr((unsigned long long*)(fr0 + v), bit) == 0;
+      if (first) deg = offsets[v + 1] - offsets[v];
+    }
+  }
+  const uint64_t live = __ballot(act);
+  const uint64_t nz = (uint64_t)__popcll(__ballot(first));
+  const uint64_t fdeg = wave_sum(deg);
+  if (r < T_NUM) publish(pub + kMsCounters + r, wall_clock64() - stamps[T_BATCH], seq);
+  if (r < M_NUM) publish(pub + r, r == M_LIVE ? live : r == M_NZ ? nz : r == M_FDEG ? fdeg : 0, seq);
+}
+
 __global__ void k_ms_roots_nz(const uint32_t* __restrict__ old2new, const int64_t* __restrict__ roots, int nroots,
                               int64_t rows, uint64_t* __restrict__ nz0) {
   const int r = threadIdx.x;
@@ -177,7 +245,9 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull(uint64_t* __restrict__ seen,
                                                     const uint32_t* __restrict__ cols, int64_t rows,
                                                     uint64_t live_in, int mode, const uint64_t* __restrict__ pack,
                                                     const uint64_t* __restrict__ compact, uint32_t filter_from,
-                                                    unsigned long long* __restrict__ c, uint64_t* __restrict__ miss) {
+                                                    unsigned long long* __restrict__ c, uint64_t* __restrict__ miss,
+                                                    uint64_t* __restrict__ stamp) {
+  ms_stamp(stamp);
   const FrontView fv{front, nz_front, pack, compact, mode, filter_from};
   ms_pull_body<NoEpilogue, kU, kW, kRows>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
                                    blockIdx.x, gridDim.x, ~UINT64_C(0), NoEpilogue(), false, miss);
@@ -228,7 +298,8 @@ __global__ void __launch_bounds__(kBlock) k_ms_pull_lanes(uint64_t* __restrict__
 
 // One bit per vertex whose frontier word has one of `lanes`.
 __global__ void __launch_bounds__(kBlock) k_ms_select(const uint64_t* __restrict__ front, int64_t rows, uint64_t lanes,
-                                                      uint64_t* __restrict__ nz_sel) {
+                                                      uint64_t* __restrict__ nz_sel, uint64_t* __restrict__ stamp) {
+  ms_stamp(stamp);
   ms_select_body(front, rows, lanes, nz_sel, blockIdx.x, gridDim.x);
 }
 
@@ -664,9 +735,13 @@ void ms_prepare(g5_ctx* ctx) {
   m.fr_exact.assign(m.fr.size(), 0);
   m.fr_count.assign(m.fr.size(), 0);
   if (m.compact_below > 0) ms_alloc_compact(ctx);
-  m.h_counters.assign(kMsCounters, 0);
+  m.h_counters.assign(kMsCounters + T_NUM, 0);
   G5_HIP(hipStreamSynchronize(ctx->stream));  // the published block is reset below
-  m.pub.alloc(kMsCounters);
+  m.pub.alloc(kMsCounters + T_NUM);
+  m.stamps.alloc(T_NUM);
+  int khz = 0;
+  G5_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+  m.clock_khz = khz > 0 ? khz : 100000;
   m.pub_seq = 0;
   m.teps_pub.alloc(65);
   m.teps_seq = 0;
@@ -681,8 +756,9 @@ void ms_prepare(g5_ctx* ctx) {
 // are published to coherent host memory, each tagged with the level's
 // sequence number, and every counter is cleared for the next level (so no
 // fill starts a level).
-__global__ void k_ms_publish(unsigned long long* __restrict__ c, int n_pub, Published* __restrict__ p,
-                             uint64_t seq) {
+__global__ void k_ms_publish(unsigned long long* __restrict__ c, int n_pub, Published* __restrict__ p, uint64_t seq,
+                             const uint64_t* __restrict__ stamps) {
+  if (threadIdx.x < T_NUM) publish(p + kMsCounters + threadIdx.x, wall_clock64() - stamps[threadIdx.x], seq);
   // one thread per counter; counters past the published ones (the per-lane
   // sums of a level that kept none) were not written, but for the list count
   const int n = n_pub > M_NUM ? n_pub : M_NUM + 1;
@@ -694,13 +770,19 @@ __global__ void k_ms_publish(unsigned long long* __restrict__ c, int n_pub, Publ
   }
 }
 
+static void ms_wait(MsState& m, int n_pub, hipStream_t s) {
+  m.pub.wait(0, n_pub, m.pub_seq, s, "g5_run_bfs_batch: level counters were not published");
+  m.pub.wait(kMsCounters, kMsCounters + T_NUM, m.pub_seq, s, "g5_run_bfs_batch: level times were not published");
+  for (int i = 0; i < n_pub; ++i) m.h_counters[i] = m.pub.value(i);
+  for (int i = kMsCounters; i < kMsCounters + T_NUM; ++i) m.h_counters[i] = m.pub.value(i);
+}
+
 static void ms_publish_wait(MsState& m, int n_pub, hipStream_t s) {
   ++m.pub_seq;
   hipLaunchKernelGGL(k_ms_publish, dim3(1), dim3(kBlock), 0, s, (unsigned long long*)m.counters.p, n_pub, m.pub.d,
-                     m.pub_seq);
+                     m.pub_seq, m.stamps.p);
   G5_HIP(hipGetLastError());
-  m.pub.wait(0, n_pub, m.pub_seq, s, "g5_run_bfs_batch: level counters were not published");
-  for (int i = 0; i < n_pub; ++i) m.h_counters[i] = m.pub.value(i);
+  ms_wait(m, n_pub, s);
 }
 
 // Frontier words of level l, allocated on first use and kept for reuse.
@@ -716,31 +798,158 @@ static uint64_t* ms_level(MsState& m, int l, int64_t rows) {
   return m.fr[l]->p;
 }
 
-// Zeroes level l's frontier words before a level that writes them sparsely
-// (a push's atomic ORs, a listed fold or pull): only the words its last run
-// left non-zero when those are known, else the whole array.
+// What a level that writes its frontier words sparsely (a push's atomic ORs, a
+// listed fold or pull) needs cleared: the words its last run left non-zero
+// when those are known and few, else all of them, and where the level only
+// sets bits of them the level's own marks.
+struct MsClear {
+  uint64_t* fr;
+  uint64_t* nz;       // the level's marks
+  int64_t rows, words;
+  int marked;         // fr is non-zero exactly where marked
+  int zero_nz;
+  uint64_t* stamp;    // of the level, or null
+};
 // One bitmap word per lane (the marks are read coalesced); a lane zeroes the
-// frontier words of its word's set bits (used for sparse marks only).
-__global__ void __launch_bounds__(kBlock) k_ms_clear_marked(const uint64_t* __restrict__ marked, int64_t words,
-                                                            int64_t rows, uint64_t* __restrict__ fr) {
-  for (int64_t wd = (int64_t)blockIdx.x * kBlock + threadIdx.x; wd < words; wd += (int64_t)gridDim.x * kBlock) {
-    for (uint64_t b = marked[wd]; b; b &= b - 1) {
-      const int64_t v = wd * 64 + __builtin_ctzll(b);
-      if (v < rows) fr[v] = 0;
-    }
+// frontier words of its word's set bits.
+__device__ __forceinline__ void ms_clear_body(const MsClear& c, int64_t t, int64_t stride) {
+  if (c.stamp && t == 0) *c.stamp = wall_clock64();
+  if (!c.marked)
+    for (int64_t v = t; v < c.rows; v += stride) c.fr[v] = 0;
+  for (int64_t wd = t; wd < c.words; wd += stride) {
+    if (c.marked)
+      for (uint64_t b = c.nz[wd]; b; b &= b - 1) {
+        const int64_t v = wd * 64 + __builtin_ctzll(b);
+        if (v < c.rows) c.fr[v] = 0;
+      }
+    if (c.zero_nz) c.nz[wd] = 0;
   }
 }
 
-static void ms_clear_frontier(MsState& m, int l, int64_t rows, hipStream_t s, bool marked) {
-  const int64_t words = (rows + 63) / 64;
-  // a dense mark set is cleared faster by a plain fill
-  if (marked && m.fr_count[l] * 16 < rows) {
-    hipLaunchKernelGGL(k_ms_clear_marked, dim3(grid_of(words, kBlock, 8192)), dim3(kBlock), 0, s,
-                       m.fr_dirty[l]->p, words, rows, m.fr[l]->p);
-    G5_HIP(hipGetLastError());
-  } else {
-    G5_HIP(hipMemsetAsync(m.fr[l]->p, 0, rows * 8, s));
+// A level's frontier as a queue: the vertices of `bits` in ascending order,
+// and for a push the prefix sums of their degrees and the queue rows of every
+// kEpb-edge chunk.  Small ones are made by one workgroup beside the clears of
+// the others (k_ms_ready: up to kReadyWords bitmap words and kReadyRows
+// vertices); a scan each takes a launch or three, and beyond those sizes one
+// workgroup takes longer than they do.
+struct MsQueue {
+  const uint64_t* bits;
+  uint32_t* queue;
+  uint64_t* count;     // null: not stored
+  uint64_t* prefix;    // null: the queue alone
+  int64_t nf;          // vertices, at most (entries past the count add nothing)
+  const uint64_t* offsets;
+  uint32_t* chunk_rows;
+  uint64_t nchunks;    // at most
+  uint64_t* bits_out;  // null, or bits again: cleared
+};
+constexpr int kReadyThreads = 1024;
+constexpr int64_t kReadyWords = 16384;
+constexpr int kReadyPer = 8;
+constexpr int64_t kReadyRows = (int64_t)kReadyThreads * kReadyPer;
+
+__device__ __forceinline__ uint64_t ready_scan(uint64_t v, uint64_t* s_wave, uint64_t& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t inc = wave_incl_scan(v);
+  __syncthreads();
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  uint64_t run = inc - v;
+  total = 0;
+  for (int w = 0; w < kReadyThreads / 64; ++w) {
+    if (w < wave) run += s_wave[w];
+    total += s_wave[w];
   }
+  return run;
+}
+
+__global__ void __launch_bounds__(kReadyThreads) k_ms_ready(MsQueue q, MsClear c) {
+  if (blockIdx.x != 0) {
+    ms_clear_body(c, (int64_t)(blockIdx.x - 1) * kReadyThreads + threadIdx.x,
+                  (int64_t)(gridDim.x - 1) * kReadyThreads);
+    return;
+  }
+  __shared__ uint64_t s_wave[kReadyThreads / 64];
+  __shared__ uint64_t s_pre[kReadyRows + 1];
+  const int t = threadIdx.x;
+  const int64_t per = (c.words + kReadyThreads - 1) / kReadyThreads, w0 = t * per;
+  uint64_t n = 0, total, E;
+  for (int64_t w = w0; w < w0 + per && w < c.words; ++w) n += (uint64_t)__popcll(q.bits[w]);
+  uint64_t at = ready_scan(n, s_wave, total);
+  for (int64_t w = w0; w < w0 + per && w < c.words; ++w) {
+    for (uint64_t x = q.bits[w]; x; x &= x - 1) q.queue[at++] = (uint32_t)(w * 64 + __builtin_ctzll(x));
+    if (q.bits_out) q.bits_out[w] = 0;
+  }
+  if (t == 0 && q.count) *q.count = total;
+  if (!q.prefix) return;
+  __syncthreads();  // the queue is read back
+  uint64_t d[kReadyPer], sum = 0;
+#pragma unroll
+  for (int j = 0; j < kReadyPer; ++j) {
+    const int64_t i = (int64_t)t * kReadyPer + j;
+    d[j] = 0;
+    if (i < q.nf && i < (int64_t)total) {
+      const uint32_t u = q.queue[i];
+      d[j] = q.offsets[u + 1] - q.offsets[u];
+    }
+    sum += d[j];
+  }
+  uint64_t run = ready_scan(sum, s_wave, E);
+#pragma unroll
+  for (int j = 0; j < kReadyPer; ++j) {
+    s_pre[t * kReadyPer + j] = run;
+    run += d[j];
+  }
+  if (t == 0) s_pre[kReadyRows] = E;
+  __syncthreads();
+  for (int64_t i = t; i <= q.nf; i += kReadyThreads) q.prefix[i] = s_pre[i];
+  const uint64_t nc = (E + kEpb - 1) / kEpb < q.nchunks ? (E + kEpb - 1) / kEpb : q.nchunks;
+  for (uint64_t k = t; k < 2 * nc; k += kReadyThreads) {
+    uint64_t key = (k >> 1) * kEpb;
+    if (k & 1) key = ((key + kEpb < E) ? key + kEpb : E) - 1;
+    int64_t lo = 0, hi = q.nf - 1;  // last row with prefix <= key
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) >> 1;
+      if (s_pre[mid] <= key) lo = mid; else hi = mid - 1;
+    }
+    q.chunk_rows[k] = (uint32_t)lo;
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_ms_clear_level(MsClear c) {
+  ms_clear_body(c, (int64_t)blockIdx.x * kBlock + threadIdx.x, (int64_t)gridDim.x * kBlock);
+}
+
+// BitsEmitN that clears the bits it has listed (out: the same words, or null).
+struct BitsTakeN {
+  BitsEmitN emit;
+  uint64_t* out;
+  __device__ void operator()(size_t w, uint64_t pre) const {
+    emit(w, pre);
+    if (out && (int64_t)w < emit.words) out[w] = 0;
+  }
+};
+
+// The level's queue (see MsQueue) and clears.
+static void ms_ready(g5_ctx* ctx, const MsQueue& q, const MsClear& c, hipStream_t s) {
+  MsState& m = ctx->ms;
+  const int64_t items = c.marked ? c.words : c.rows;
+  if (c.words <= kReadyWords && q.nf <= kReadyRows) {
+    hipLaunchKernelGGL(k_ms_ready, dim3(1 + grid_of(items, kReadyThreads, 255)), dim3(kReadyThreads), 0, s, q, c);
+    G5_HIP(hipGetLastError());
+    return;
+  }
+  hipLaunchKernelGGL(k_ms_clear_level, dim3(grid_of(items, kBlock, 8192)), dim3(kBlock), 0, s, c);
+  device_scan(BitsCountN{q.bits, c.words}, BitsTakeN{{q.bits, c.words, q.queue, m.ulist_count.p}, q.bits_out},
+              (size_t)c.words + 1, m.scan_tmp.p, s);
+  if (q.prefix) {
+    device_scan(FrontierDegreeN{q.queue, q.offsets, m.ulist_count.p}, StoreU64{q.prefix}, (size_t)q.nf + 1,
+                m.scan_tmp.p, s);
+    if (q.nchunks)
+      hipLaunchKernelGGL(k_chunk_rows<kEpb>, dim3(grid_of((int64_t)(2 * q.nchunks), kBlock, 65536)), dim3(kBlock), 0,
+                         s, q.prefix, q.nf, q.nchunks, q.chunk_rows);
+  }
+  G5_HIP(hipGetLastError());
 }
 
 // Level l's nonzero bitmap (one bit per vertex whose frontier word is not
@@ -777,6 +986,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
   const uint64_t* h_lane = m.h_counters.data() + kMsLanes;
   unsigned* d_list_count = (unsigned*)(cnt + M_NUM);
   // turns of a pull that takes 16 rows each up to `limit` words
+  m.ulist_count.alloc(1);
   const auto pull_turns = [&](int64_t limit) { return m.pull_unroll == 0 && words <= limit ? words * 4 : words; };
   bool have_miss = false;  // m.miss holds the vertices still missing a live root
   int l = l0 - 1;
@@ -794,6 +1004,12 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     // for the next batch's clear of them
     uint64_t* nz_next = ms_marks(m, l, words);
     const uint64_t* nz_front = m.fr_dirty[l - 1]->p;
+    // (a dense mark set is cleared faster by a plain fill)
+    uint64_t* const stamp = m.stamps.p + T_LEVEL;
+    const auto clear = [&](bool zero_nz, bool first) {
+      return MsClear{next, nz_next, rows, words, marked && m.fr_count[l] * 16 < rows ? 1 : 0, zero_nz ? 1 : 0,
+                     first ? stamp : nullptr};
+    };
     bool push = (double)fdeg < push_limit && total_pairs - reached >= unseen_frac * total_pairs;
     bool sweep = !push && m.sweep_chunks && reached < sweep_limit;
     uint64_t td = 0, bu = 0;
@@ -824,7 +1040,6 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     }
     m.level_push[l] = push ? live : td;
     m.level_pull[l] = push ? 0 : (lanes_mode ? bu : live);
-    G5_HIP(hipEventRecord(level_event(m.lev_begin, l), s));
     // statistics for the roots still choosing (a root that pulled keeps pulling)
     const LaneEpi lepi{cnt + kMsLanes, g.offsets.p, lanes_mode ? td : live};
     if (lanes_mode && td && bu) {
@@ -832,8 +1047,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       // pushed lanes
       m.nz_sel.alloc(words);
       hipLaunchKernelGGL(k_ms_select, dim3(grid_of(words, kBlock / 64, 8192)), dim3(kBlock), 0, s, front, rows, td,
-                         m.nz_sel.p);
-      ms_clear_frontier(m, l, rows, s, marked);
+                         m.nz_sel.p, stamp);
       if (m.mixed_push == 1) {
         // the pushing roots' frontier vertices as a queue (the count stays on
         // the device), their rows as one edge-balanced virtual edge list; the
@@ -846,21 +1060,17 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         }
         const int64_t nf = (int64_t)std::min<double>(nf_ub, (double)rows);
         const uint64_t E_ub = (uint64_t)std::min<double>(fd_ub, (double)g.nnz);
-        m.ulist_count.alloc(1);
-        device_scan(BitsCountN{m.nz_sel.p, words}, BitsEmitN{m.nz_sel.p, words, m.queue.p, m.ulist_count.p},
-                    (size_t)words + 1, m.scan_tmp.p, s);
-        device_scan(FrontierDegreeN{m.queue.p, g.offsets.p, m.ulist_count.p}, StoreU64{m.prefix.p}, (size_t)nf + 1,
-                    m.scan_tmp.p, s);
         const uint64_t nchunks = (E_ub + kEpb - 1) / kEpb;
         G5_CHECK(2 * nchunks <= m.chunk_rows.n, "g5_run_bfs_batch: chunk table too small");
-        if (nchunks) {
-          hipLaunchKernelGGL(k_chunk_rows<kEpb>, dim3(grid_of((int64_t)(2 * nchunks), kBlock, 65536)), dim3(kBlock),
-                             0, s, m.prefix.p, nf, nchunks, m.chunk_rows.p);
+        ms_ready(ctx, MsQueue{m.nz_sel.p, m.queue.p, m.ulist_count.p, m.prefix.p, nf, g.offsets.p, m.chunk_rows.p,
+                              nchunks, nullptr}, clear(false, false), s);
+        if (nchunks)
           hipLaunchKernelGGL(k_ms_push, dim3(grid_of((int64_t)E_ub, kEpb, 8192)), dim3(kBlock), 0, s, m.queue.p, nf,
                              m.prefix.p, m.chunk_rows.p, g.offsets.p, g.cols.p, front, next, td);
-        }
       } else {
         // over the CSR chunks holding one of the pushing roots' frontier vertices
+        hipLaunchKernelGGL(k_ms_clear_level, dim3(grid_of(clear(false, false).marked ? words : rows, kBlock, 8192)), dim3(kBlock),
+                           0, s, clear(false, false));
         m.chunk_list.alloc(m.sweep_chunks);
         hipLaunchKernelGGL(k_ms_collect, dim3(grid_of((int64_t)m.sweep_chunks, kBlock, 4096)), dim3(kBlock), 0, s,
                            m.sweep_rows.p, m.sweep_chunks, m.nz_sel.p, m.chunk_list.p, d_list_count);
@@ -885,24 +1095,18 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
                          nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, rows, bu,
                          m.pull_filter == 1 ? 1 : 0, 1, cnt, lepi);
     } else if (push) {
-      device_scan(UnionCount{nz_front}, UnionEmit{nz_front, m.queue.p}, (size_t)words, m.scan_tmp.p, s);
       const int64_t nf = (int64_t)nz;
-      device_scan(FrontierDegree{m.queue.p, g.offsets.p, nf}, StoreU64{m.prefix.p}, (size_t)nf + 1,
-                  m.scan_tmp.p, s);
       const uint64_t nchunks = (fdeg + kEpb - 1) / kEpb;
       G5_CHECK(2 * nchunks <= m.chunk_rows.n, "g5_run_bfs_batch: chunk table too small");
-      if (nchunks)
-        hipLaunchKernelGGL(k_chunk_rows<kEpb>, dim3(grid_of((int64_t)(2 * nchunks), kBlock, 65536)),
-                           dim3(kBlock), 0, s, m.prefix.p, nf, nchunks, m.chunk_rows.p);
-      ms_clear_frontier(m, l, rows, s, marked);
       // a push whose frontier edges are few next to the rows lists what it
       // touches, and only those vertices are folded
       const uint64_t touch_cap = std::min<uint64_t>(fdeg, (uint64_t)rows);
       const bool touch = (double)fdeg * kTouchBelow < (double)rows;
+      ms_ready(ctx, MsQueue{nz_front, m.queue.p, m.ulist_count.p, m.prefix.p, nf, g.offsets.p, m.chunk_rows.p,
+                            nchunks, nullptr}, clear(touch, true), s);
       if (touch) {
         m.touch.alloc(std::max<uint64_t>(touch_cap, 1));
         unsigned long long* touch_count = cnt + M_NUM;  // cleared with the counters
-        G5_HIP(hipMemsetAsync(nz_next, 0, words * 8, s));
         hipLaunchKernelGGL(k_ms_push_touch, dim3(grid_of((int64_t)fdeg, kEpb, 2048)), dim3(kBlock), 0, s,
                            m.queue.p, nf, m.prefix.p, m.chunk_rows.p, g.offsets.p, g.cols.p, front, next, m.touch.p,
                            touch_count);
@@ -923,6 +1127,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         hipLaunchKernelGGL(k_ms_finish, dim3(grid_of(words, kBlock / 64, 8192)), dim3(kBlock), 0, s, m.seen.p,
                            next, nz_next, g.offsets.p, rows, cnt);
     } else if (sweep) {
+      hipLaunchKernelGGL(k_ms_stamp, dim3(1), dim3(64), 0, s, stamp);
       hipLaunchKernelGGL(k_ms_sweep_clear, dim3(grid_of((int64_t)m.sweep_chunks, kBlock, 4096)), dim3(kBlock), 0,
                          s, m.sweep_rows.p, m.sweep_chunks, g.offsets.p, next);
       hipLaunchKernelGGL(k_ms_sweep, dim3(grid_of((int64_t)m.sweep_chunks, 1, m.sweep_grid)), dim3(kBlock), 0, s,
@@ -937,6 +1142,7 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         // frontier words of few vertices: pack them densely
         m.pack.alloc(2 * words);
         m.compact.alloc(rows);
+        hipLaunchKernelGGL(k_ms_stamp, dim3(1), dim3(64), 0, s, stamp);
         device_scan(CompactCount{nz_front}, CompactEmit{nz_front, front, m.pack.p, m.compact.p}, (size_t)words,
                     m.scan_tmp.p, s);
         mode = kFrontCompact;
@@ -962,12 +1168,8 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       if (have_miss && mode == kFrontPlain) {
         const uint64_t ub = (uint64_t)std::min<double>((double)rows, unreached);  // list length bound
         m.ulist.alloc(std::max<uint64_t>(ub, 1));
-        m.ulist_count.alloc(1);
-        device_scan(BitsCountN{m.miss.p, words}, BitsEmitN{m.miss.p, words, m.ulist.p, m.ulist_count.p},
-                    (size_t)words + 1, m.scan_tmp.p, s);
-        ms_clear_frontier(m, l, rows, s, marked);
-        G5_HIP(hipMemsetAsync(nz_next, 0, words * 8, s));
-        G5_HIP(hipMemsetAsync(m.miss.p, 0, words * 8, s));
+        ms_ready(ctx, MsQueue{m.miss.p, m.ulist.p, m.ulist_count.p, nullptr, 0, nullptr, nullptr, 0, m.miss.p},
+                 clear(true, true), s);
         hipLaunchKernelGGL(k_ms_pull_list, dim3(grid_of((int64_t)ub, kBlock, std::min(m.pull_grid, kListGrid))), dim3(kBlock), 0, s,
                            m.seen.p, front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, m.ulist.p,
                            m.ulist_count.p, live, m.miss.p, cnt);
@@ -980,13 +1182,13 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
         // could skip its zero words, measured no faster)
         hipLaunchKernelGGL(kp, dim3(grid_of(pull_turns(kPartWords), kBlock / 64, m.pull_grid)), dim3(kBlock), 0, s, m.seen.p, front,
                            nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, rows, live, mode,
-                           m.pack.p, m.compact.p, filter_from, cnt, mark ? m.miss.p : nullptr);
+                           m.pack.p, m.compact.p, filter_from, cnt, mark ? m.miss.p : nullptr,
+                           mode == kFrontCompact ? nullptr : stamp);
         list_level = mark;
       }
     }
     G5_HIP(hipGetLastError());
     m.fr_exact[l] = 1;  // every level form leaves next non-zero exactly at the bits of nz_next
-    G5_HIP(hipEventRecord(level_event(m.lev_end, l), s));
     ms_publish_wait(m, lane_stats ? kMsCounters : M_NUM, s);
     st.direction[l] = (lanes_mode && td && bu) ? 3 : (push ? 1 : (sweep ? 2 : 0));
     if (lane_stats)
@@ -998,20 +1200,11 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
     st.pairs[l] = (int64_t)m.h_counters[M_PAIRS];
     reached += (double)m.h_counters[M_PAIRS];
     st.num_levels = l + 1;
+    st.level_ms[l] = (double)m.h_counters[kMsCounters + T_LEVEL] / (double)m.clock_khz;
     live = m.h_counters[M_LIVE];
     nz = m.h_counters[M_NZ];
     m.fr_count[l] = (int64_t)nz;
     fdeg = m.h_counters[M_FDEG];
-  }
-  // level times, once the last level's events are complete (a level's
-  // published counters can reach the host before its end event is)
-  if (st.num_levels - 1 >= l0) {
-    G5_HIP(hipEventSynchronize(m.lev_end[st.num_levels - 1]));
-    for (int k = l0; k < st.num_levels; ++k) {
-      float lms = 0;
-      G5_HIP(hipEventElapsedTime(&lms, m.lev_begin[k], m.lev_end[k]));
-      st.level_ms[k] = lms;
-    }
   }
 }
 
@@ -1063,9 +1256,6 @@ static void ms_persistent_setup(g5_ctx* ctx) {
   G5_CHECK(grid <= (int64_t)kBarGroup * kBarMaxGroups, "g5_run_bfs_batch: persistent grid beyond the barrier's groups");
   if (m.persist_grid > 0 && m.persist_grid < grid) grid = m.persist_grid;
   m.p_grid = (unsigned)grid;
-  int rate_khz = 0;
-  G5_HIP(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, ctx->device));
-  m.clock_khz = rate_khz > 0 ? rate_khz : 100000;
 
   MsPersistArgs a{};
   a.offsets = g.offsets.p;
@@ -1228,34 +1418,34 @@ void ms_run(g5_ctx* ctx, const int64_t* roots, int nroots) {
 
   if (m.persistent && m.sweep_chunks) {
     ms_run_persistent(ctx, roots, nroots);
+    G5_HIP(hipEventRecord(m.ev1, s));
+    G5_HIP(hipEventSynchronize(m.ev1));
+    float ms = 0;
+    G5_HIP(hipEventElapsedTime(&ms, m.ev0, m.ev1));
+    st.device_ms = ms;
   } else {
     uint64_t* fr0 = ms_level(m, 0, rows);
     const int64_t words = (rows + 63) / 64;
     uint64_t* nz0 = ms_marks(m, 0, words);
-    G5_HIP(hipMemcpyAsync(m.roots.p, roots, nroots * sizeof(int64_t), hipMemcpyHostToDevice, s));
-    G5_HIP(hipEventRecord(m.ev0, s));
-    G5_HIP(hipMemsetAsync(m.counters.p, 0, kMsCounterWords * 8, s));  // then cleared by every publish
-    G5_HIP(hipMemsetAsync(m.seen.p, 0, rows * 8, s));
-    const bool marked = m.fr_exact[0] != 0;
+    MsRoots mr{};
+    mr.n = nroots;
+    std::copy(roots, roots + nroots, mr.root);
+    const bool marked = m.fr_exact[0] != 0;  // by the previous batch's roots
     m.fr_exact[0] = 0;
-    ms_clear_frontier(m, 0, rows, s, marked);  // the previous batch's roots, or everything
-    G5_HIP(hipMemsetAsync(nz0, 0, words * 8, s));
-    hipLaunchKernelGGL(k_ms_roots, dim3(1), dim3(64), 0, s, g.old2new.p, m.roots.p, nroots, rows, g.offsets.p,
-                       m.seen.p, fr0, cnt);
-    hipLaunchKernelGGL(k_ms_roots_nz, dim3(1), dim3(64), 0, s, g.old2new.p, m.roots.p, nroots, rows, nz0);
+    hipLaunchKernelGGL(k_ms_begin, dim3(grid_of(rows, kBlock, 4096)), dim3(kBlock), 0, s, m.seen.p, fr0, nz0, rows,
+                       words, marked ? 1 : 0, cnt, m.stamps.p);
+    ++m.pub_seq;
+    hipLaunchKernelGGL(k_ms_place, dim3(1), dim3(64), 0, s, g.old2new.p, mr, rows, g.offsets.p, m.seen.p, fr0, nz0,
+                       m.pub.d, m.pub_seq, m.stamps.p);
     G5_HIP(hipGetLastError());
     m.fr_exact[0] = 1;
     m.fr_count[0] = nroots;
-    ms_publish_wait(m, M_NUM, s);
+    ms_wait(m, M_NUM, s);
     const uint64_t live = m.h_counters[M_LIVE];
     const double roots_live = (double)__builtin_popcountll(live);
     ms_host_levels(ctx, 1, live, m.h_counters[M_NZ], m.h_counters[M_FDEG], roots_live, roots_live);
+    st.device_ms = (double)m.h_counters[kMsCounters + T_BATCH] / (double)m.clock_khz;
   }
-  G5_HIP(hipEventRecord(m.ev1, s));
-  G5_HIP(hipEventSynchronize(m.ev1));
-  float ms = 0;
-  G5_HIP(hipEventElapsedTime(&ms, m.ev0, m.ev1));
-  st.device_ms = ms;
   m.nlevels = st.num_levels - 1 > 0 ? st.num_levels - 1 : 1;  // levels with frontier words 0..L-1
   m.have_result = true;
 }

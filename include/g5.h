@@ -72,7 +72,7 @@ typedef struct g5_bfs_stats {
   int32_t num_levels;               /* levels executed + 1 (last level finds nothing) */
   int32_t direction[G5_MAX_LEVELS]; /* 1 = top-down, 0 = bottom-up */
   int64_t nq[G5_MAX_LEVELS];        /* vertices discovered at that level */
-  double level_ms[G5_MAX_LEVELS];   /* device time of each level's kernels (HIP events) */
+  double level_ms[G5_MAX_LEVELS];   /* device time of each level's kernels (device clock or HIP events) */
   double device_ms;                 /* device time of the whole run (HIP events) */
   int64_t reached;                  /* vertices with a level, root included */
   int32_t bu_kernel[G5_MAX_LEVELS]; /* 1 = the level's vertices were found by the bottom-up kernel
@@ -88,7 +88,7 @@ typedef struct g5_batch_stats {
                                        2 = edge-parallel pull sweep, 3 = some roots push and
                                        the others pull (lane_rule 1) */
   int64_t pairs[G5_MAX_LEVELS];     /* (root, vertex) pairs discovered at that level */
-  double level_ms[G5_MAX_LEVELS];   /* device time per level (HIP events) */
+  double level_ms[G5_MAX_LEVELS];   /* device time per level, from its first kernel to its counters (device clock) */
   double device_ms;                 /* device time of the whole batch */
   int32_t persistent_grid;          /* workgroups of the persistent launch (0: per-level launches) */
   int32_t persistent_levels;        /* levels run inside the persistent launch */

@@ -52,3 +52,35 @@ def test_pull_rows(oracle_mod, words, mode):
             c.run_bfs_batch(roots)
             for lane, r in enumerate(roots):
                 assert np.array_equal(c.batch_levels(lane), want[r]), (tuning, lane, r)
+
+
+@pytest.mark.parametrize("leaves,words", [(8191, 700), (8192, 700), (8193, 700), (30000, 700), (3000, 16384), (3000, 16385)])
+def test_level_queue(oracle_mod, leaves, words):
+    """Frontiers and bitmaps on both sides of what one workgroup lists beside
+    the clears (8,192 vertices, 16,384 words), in pushes, in levels with both
+    directions and in the listed pulls at the end of long paths."""
+    import graph500_amd
+    rng = np.random.default_rng(leaves + words)
+    n = 64 * words
+    hubs = np.array([0, 1, 2])
+    star = np.concatenate([np.stack([np.full(leaves, h), 8 + h * 64 + np.arange(leaves)], 1) for h in hubs])
+    field = rng.integers(3, n - 40, (2 * n, 2))
+    every = np.stack([np.arange(n - 41), rng.integers(3, n - 41, n - 41)], 1)
+    tail = np.stack([np.arange(n - 41, n - 1), np.arange(n - 40, n)], 1)
+    p = np.concatenate([star, field, every, tail])
+    t = np.zeros(len(p), graph500_amd.EDGE_DTYPE)
+    t["v0_low"], t["v1_low"] = p[:, 0], p[:, 1]
+    oc = oracle_mod.Csr(t)
+    roots = [0, 1, n - 1, int(p[7, 1]), 0, 2, n - 20, 5]
+    want = {r: oc.bfs(r)[0] for r in set(roots)}
+    with graph500_amd.G5Context(0) as c:
+        c.edges_append(t)
+        c.construct(2)
+        c.batch_prepare()
+        for tuning in ({}, {"alpha": 1e-9}, {"alpha": 1.5}, {"mixed_push": 0, "alpha": 64.0}):
+            c.batch_set_tuning(**tuning)
+            for again in range(2):  # the second batch clears what the first marked
+                print(leaves, words, tuning, flush=True)
+                c.run_bfs_batch(roots)
+                for lane, r in enumerate(roots):
+                    assert np.array_equal(c.batch_levels(lane), want[r]), (tuning, lane, r)
