@@ -55,6 +55,7 @@ struct ServeEpi {
 // (read by readlane where a wave writes lane r's bytes) and lane i's counts
 // (a readlane walk over the wave's vertices, as LaneEpi), so no shared
 // counter is touched until the block's LDS reduction at the end.
+template <int kRows = 64>  // vertices a wave has at a time
 struct ServeLocal {
   const ServeEpi& p;
   mutable uint64_t n_acc = 0, d_acc = 0, my_ans = 0;
@@ -103,7 +104,7 @@ struct ServeLocal {
         atomicOr((unsigned long long*)(p.nz_sel + (v >> 6)), 1ull << (v & 63));
     } else {
       const uint64_t bs = __ballot(inb && (nw & p.sel) != 0);
-      if (me == 0) p.nz_sel[v >> 6] = bs;
+      if (me == 0) store_bits<kRows>(p.nz_sel, v / kRows, bs);
     }
   }
   __device__ void end() const {
@@ -124,23 +125,53 @@ struct ServeLocal {
 // level finished, and its counters, by polling host memory, with no copy
 // commands on the stream.
 constexpr int kSvTeps = M_NUM + 128;
-constexpr int kSvPub = kSvTeps + 64;
+constexpr int kSvTicks = kSvTeps + 64;  // device time since the level's first kernel
+constexpr int kSvPub = kSvTicks + 1;
 constexpr int kSvTouch = kMsLanes + 128;  // device counter slot of a listed push's touched vertices
 constexpr size_t kSvCounterWords = (size_t)kMsStripes * kMsStride;
-static_assert(kSvTouch < kMsStride, "a counter copy holds every counter");
-__global__ void k_sv_publish(const unsigned long long* __restrict__ c, const unsigned long long* __restrict__ tacc,
-                             Published* __restrict__ p, uint64_t seq) {
+static_assert(kSvTouch < kMsStride && kMsStride <= kBlock, "a counter copy holds every counter");
+constexpr int64_t kSvPartWords = 4096;  // pulls of graphs up to this many words take 16 rows a turn
+// The weight sums have copies too, chosen by workgroup (see ms_stripe).
+constexpr int kTaccStripes = 16;
+constexpr int kTaccStride = 72;
+// Counters and weight sums are clear again for the next level behind it.
+__global__ void __launch_bounds__(kBlock) k_sv_publish(unsigned long long* __restrict__ c,
+                                                       unsigned long long* __restrict__ tacc,
+                                                       Published* __restrict__ p, uint64_t seq,
+                                                       const uint64_t* __restrict__ stamp) {
   const int t = threadIdx.x;
   // [0, M_NUM) level counters, [M_NUM, kSvTeps) per-lane sums, then the weight sums
   if (t < kSvTeps) publish(p + t, ms_stripe_total(c, t < M_NUM ? t : kMsLanes + t - M_NUM), seq);
-  else if (t < kSvPub) publish(p + t, tacc[t - kSvTeps], seq);
+  else if (t < kSvTicks) {
+    uint64_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < kTaccStripes; ++i) {
+      sum += tacc[i * kTaccStride + t - kSvTeps];
+      tacc[i * kTaccStride + t - kSvTeps] = 0;
+    }
+    publish(p + t, sum, seq);
+  } else if (t == kSvTicks) {
+    publish(p + t, wall_clock64() - *stamp, seq);
+  }
+  __syncthreads();
+  if (t < kMsStride)
+#pragma unroll 8
+    for (int i = 0; i < kMsStripes; ++i) c[i * kMsStride + t] = 0;
 }
 
+// The start of a level: its first kernel stamps the device clock.
+__device__ __forceinline__ void sv_stamp(uint64_t* stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+
+// Queries admitted together.
 struct ServeRoots {
-  int64_t root[64];  // original id of the query admitted into each lane, -1 = none
+  int64_t root[64];  // original id
   uint8_t* ans[64];
+  uint8_t lane[64];
 };
 
+template <int kRows>
 __global__ void __launch_bounds__(kBlock) k_sv_pull(uint64_t* __restrict__ seen, const uint64_t* __restrict__ front,
                                                     const uint64_t* __restrict__ nz_front, uint64_t* __restrict__ next,
                                                     uint64_t* __restrict__ nz_next,
@@ -148,13 +179,14 @@ __global__ void __launch_bounds__(kBlock) k_sv_pull(uint64_t* __restrict__ seen,
                                                     const uint64_t* __restrict__ offsets,
                                                     const uint32_t* __restrict__ cols, int64_t rows, uint64_t live_in,
                                                     int filter, unsigned long long* __restrict__ c, uint64_t keep,
-                                                    int merge, ServeEpi epi) {
+                                                    int merge, ServeEpi epi, uint64_t* __restrict__ stamp) {
+  sv_stamp(stamp);
   const FrontView fv{front, nz_front, nullptr, nullptr, filter ? kFrontFilter : kFrontPlain, 0};
-  const ServeLocal el{epi};
+  const ServeLocal<kRows> el{epi};
   // two probes per step on a short row, one per lane and step on a long row:
   // the batch's fastest pull unrolling at SCALE 28 (fewer probes past the
   // point where a vertex's searches are all found)
-  ms_pull_body<ServeLocal, 2, 1>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
+  ms_pull_body<ServeLocal<kRows>, 2, 1, kRows>(seen, fv, next, nz_next, first_nbr, offsets, cols, rows, live_in, ms_stripe(c),
                                  blockIdx.x, gridDim.x, keep, el, merge != 0);
 }
 
@@ -163,7 +195,7 @@ __global__ void __launch_bounds__(kBlock) k_sv_finish(uint64_t* __restrict__ see
                                                       const uint64_t* __restrict__ offsets, int64_t rows,
                                                       unsigned long long* __restrict__ c, uint64_t keep,
                                                       ServeEpi epi) {
-  const ServeLocal el{epi};
+  const ServeLocal<> el{epi};
   ms_finish_body(seen, next, nz_next, offsets, rows, ms_stripe(c), blockIdx.x, gridDim.x, keep, el);
 }
 
@@ -207,33 +239,39 @@ __global__ void __launch_bounds__(kBlock) k_sv_finish_list(uint64_t* __restrict_
                                                            const uint32_t* __restrict__ touch,
                                                            const unsigned long long* __restrict__ touch_count,
                                                            unsigned long long* __restrict__ c, ServeEpi epi) {
-  const ServeLocal el{epi};
+  const ServeLocal<> el{epi};
   ms_finish_list_body(seen, next, nz_next, offsets, touch, (uint64_t)*touch_count, ms_stripe(c), blockIdx.x,
                       gridDim.x, el);
 }
 
-// Zeroes the frontier words marked in a nonzero bitmap (one bitmap word per
-// lane; for sparse marks).
-__global__ void __launch_bounds__(kBlock) k_sv_clear_marked(const uint64_t* __restrict__ marked, int64_t words,
-                                                            int64_t rows, uint64_t* __restrict__ fr) {
-  for (int64_t wd = (int64_t)blockIdx.x * kBlock + threadIdx.x; wd < words; wd += (int64_t)gridDim.x * kBlock)
-    for (uint64_t b = marked[wd]; b; b &= b - 1) {
-      const int64_t v = wd * 64 + __builtin_ctzll(b);
-      if (v < rows) fr[v] = 0;
-    }
+// Clears what a pushing level writes sparsely: the frontier words (where
+// marked, for sparse marks, or all), and for a listed push the marks and the
+// top-down lanes' marks, whose bits it sets one by one.
+__global__ void __launch_bounds__(kBlock) k_sv_clear_level(uint64_t* __restrict__ nz, int64_t words, int64_t rows,
+                                                           uint64_t* __restrict__ fr, int marked,
+                                                           uint64_t* __restrict__ nz_sel, uint64_t* __restrict__ stamp) {
+  sv_stamp(stamp);
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x, stride = (int64_t)gridDim.x * kBlock;
+  if (!marked)
+    for (int64_t v = t; v < rows; v += stride) fr[v] = 0;
+  for (int64_t wd = t; wd < words; wd += stride) {
+    if (marked)
+      for (uint64_t b = nz[wd]; b; b &= b - 1) {
+        const int64_t v = wd * 64 + __builtin_ctzll(b);
+        if (v < rows) fr[v] = 0;
+      }
+    if (nz_sel) nz[wd] = nz_sel[wd] = 0;
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) k_sv_select(const uint64_t* __restrict__ front, int64_t rows, uint64_t lanes,
-                                                      uint64_t* __restrict__ nz_sel) {
+                                                      uint64_t* __restrict__ nz_sel, uint64_t* __restrict__ stamp) {
+  sv_stamp(stamp);
   ms_select_body(front, rows, lanes, nz_sel, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(kBlock) k_sv_zero(uint64_t* __restrict__ a, int64_t n) {
   ms_zero_body(a, n, blockIdx.x, gridDim.x);
-}
-
-__global__ void __launch_bounds__(kBlock) k_sv_fill_bytes(uint8_t* __restrict__ p, int64_t n, uint8_t val) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) p[i] = val;
 }
 
 // seen &= keep over all rows (lanes cooling while the engine is idle).
@@ -244,21 +282,30 @@ __global__ void __launch_bounds__(kBlock) k_sv_clear(uint64_t* __restrict__ seen
   }
 }
 
-// Places the admitted roots into seen / frontier / nonzero bitmap and their
-// answers; one thread per lane (lanes may share a root vertex).
-__global__ void k_sv_admit(const uint32_t* __restrict__ old2new, int64_t rows, ServeRoots rs,
-                           uint64_t* __restrict__ seen, uint64_t* __restrict__ front, uint64_t* __restrict__ nz_front,
-                           uint64_t* __restrict__ nz_sel_front) {
-  const int r = threadIdx.x;
-  if (r >= 64 || rs.root[r] < 0) return;
-  const uint32_t v = old2new[rs.root[r]];
-  if ((int64_t)v >= rows) return;  // a root without edges reaches nothing
-  const unsigned long long bit = 1ull << r;
-  atomicOr((unsigned long long*)(seen + v), bit);
-  atomicOr((unsigned long long*)(front + v), bit);
-  atomicOr((unsigned long long*)(nz_front + (v >> 6)), 1ull << (v & 63));
-  atomicOr((unsigned long long*)(nz_sel_front + (v >> 6)), 1ull << (v & 63));
-  rs.ans[r][v] = 0;
+// Admits queries, one per blockIdx.y: its answer array unreached but for the
+// root, its root in seen, the frontier and the nonzero bitmaps (queries may
+// share a root vertex).  (A fill launch per query took 3 us of the stream each.)
+__global__ void __launch_bounds__(kBlock) k_sv_admit(const uint32_t* __restrict__ old2new, int64_t rows, ServeRoots rs,
+                                                     uint64_t* __restrict__ seen, uint64_t* __restrict__ front,
+                                                     uint64_t* __restrict__ nz_front,
+                                                     uint64_t* __restrict__ nz_sel_front) {
+  const int q = blockIdx.y;
+  const int64_t v = old2new[rs.root[q]];  // >= rows: a root without edges reaches nothing
+  uint8_t* ans = rs.ans[q];
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i * 16 < rows; i += (int64_t)gridDim.x * kBlock) {
+    if (i * 16 + 16 <= rows && (v < i * 16 || v >= i * 16 + 16)) {
+      reinterpret_cast<uint4*>(ans)[i] = uint4{~0u, ~0u, ~0u, ~0u};
+    } else {
+      for (int64_t w = i * 16; w < i * 16 + 16 && w < rows; ++w) ans[w] = w == v ? 0 : 0xFF;
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && v < rows) {
+    const unsigned long long bit = 1ull << rs.lane[q];
+    atomicOr((unsigned long long*)(seen + v), bit);
+    atomicOr((unsigned long long*)(front + v), bit);
+    atomicOr((unsigned long long*)(nz_front + (v >> 6)), 1ull << (v & 63));
+    atomicOr((unsigned long long*)(nz_sel_front + (v >> 6)), 1ull << (v & 63));
+  }
 }
 
 // Per-lane sums of the tuple weights of the reached vertices, lanes in mask.
@@ -296,7 +343,7 @@ __global__ void __launch_bounds__(kBlock) k_sv_teps(const uint64_t* __restrict__
   __syncthreads();
   if (threadIdx.x < 64) {
     const unsigned long long t = s_acc[threadIdx.x] + (((mask >> threadIdx.x) & 1) ? s_acc[64] : 0);
-    if (t) atomicAdd(acc + threadIdx.x, t);
+    if (t) atomicAdd(acc + (blockIdx.x % kTaccStripes) * kTaccStride + threadIdx.x, t);
   }
 }
 
@@ -367,7 +414,8 @@ struct Engine {
   unsigned long long* h = nullptr;   // pinned: the per-lane weight sums of a retirement, copied at the end
   PublishBlock pub;                  // the level counters and per-lane counts (k_sv_publish)
   uint64_t pub_seq = 0;              // sequence number of the level in flight
-  hipEvent_t ev_start = nullptr, ev_end = nullptr;  // timing of the level in flight
+  DevBuf<uint64_t> stamp;  // device clock at the start of the level in flight
+  int clock_khz = 100000;
   g5_server_graph_stats st{};
   std::vector<std::unique_ptr<DevBuf<uint8_t>>> bufs;
   std::vector<int> free_bufs;
@@ -402,8 +450,6 @@ struct Engine {
   ~Engine() {
     solo.clear();  // joins the runs still going
     if (h) (void)hipHostFree(h);
-    if (ev_start) (void)hipEventDestroy(ev_start);
-    if (ev_end) (void)hipEventDestroy(ev_end);
   }
 };
 
@@ -468,12 +514,15 @@ static void sv_setup_engine(g5_server* srv, Engine& e, g5_ctx* ctx) {
   e.chunk_list.alloc(e.nchunks + 1);
   e.cnt.alloc(kSvCounterWords);
   e.touch.alloc(e.rows ? e.rows : 1);
-  e.tacc.alloc(64);
-  G5_HIP(hipMemsetAsync(e.tacc.p, 0, 64 * 8, e.s));
-  G5_HIP(hipHostMalloc((void**)&e.h, 64 * sizeof(unsigned long long), hipHostMallocDefault));
+  e.tacc.alloc(kTaccStripes * kTaccStride);
+  G5_HIP(hipMemsetAsync(e.tacc.p, 0, e.tacc.bytes(), e.s));
+  G5_HIP(hipMemsetAsync(e.cnt.p, 0, e.cnt.bytes(), e.s));
+  G5_HIP(hipHostMalloc((void**)&e.h, e.tacc.bytes(), hipHostMallocDefault));
+  e.stamp.alloc(1);
+  int khz = 0;
+  G5_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+  e.clock_khz = khz > 0 ? khz : 100000;
   e.pub.alloc(kSvPub);
-  G5_HIP(hipEventCreate(&e.ev_start));
-  G5_HIP(hipEventCreate(&e.ev_end));
   hipStream_t s = e.s;
   if (e.nchunks)
     hipLaunchKernelGGL(k_chunk_rows<kSweepEpb>, dim3(grid_of((int64_t)(2 * e.nchunks), kBlock, 65536)), dim3(kBlock),
@@ -504,8 +553,11 @@ static void sv_setup_engine(g5_server* srv, Engine& e, g5_ctx* ctx) {
 static void sv_take_teps(g5_server* srv, Engine& e, bool from_level) {
   if (!e.teps_pending) return;
   if (!from_level) {
-    G5_HIP(hipMemcpyAsync(e.h, e.tacc.p, 64 * 8, hipMemcpyDeviceToHost, e.s));
+    G5_HIP(hipMemcpyAsync(e.h, e.tacc.p, e.tacc.bytes(), hipMemcpyDeviceToHost, e.s));
+    G5_HIP(hipMemsetAsync(e.tacc.p, 0, e.tacc.bytes(), e.s));
     G5_HIP(hipStreamSynchronize(e.s));
+    for (int r = 0; r < 64; ++r)
+      for (int i = 1; i < kTaccStripes; ++i) e.h[r] += e.h[i * kTaccStride + r];
   }
   uint64_t m = e.teps_mask;
   while (m) {
@@ -559,7 +611,6 @@ static void sv_complete_level(g5_server* srv, Engine& e, double t) {
   }
   if (finished) {
     // traversed edges of the finished lanes, before their bits are cleared
-    G5_HIP(hipMemsetAsync(e.tacc.p, 0, 64 * 8, e.s));
     hipLaunchKernelGGL(k_sv_teps, dim3(grid_of(e.rows, kBlock, 2048)), dim3(kBlock), 0, e.s, e.seen.p,
                        e.ctx->graph.weight.p, e.rows, finished, e.tacc.p);
     G5_HIP(hipGetLastError());
@@ -614,11 +665,8 @@ static uint64_t sv_admit(g5_server* srv, Engine& e, double t) {
     const double waited = t - srv->req[e.waiting.front()].arrival;
     if (!young && can < want && waited < srv->cfg.max_wait_s) return 0;
   }
-  ServeRoots rs;
-  for (int r = 0; r < 64; ++r) {
-    rs.root[r] = -1;
-    rs.ans[r] = nullptr;
-  }
+  ServeRoots rs{};
+  int n = 0;
   uint64_t admitted = 0;
   for (int r = 0; r < 64 && !e.waiting.empty() && !e.free_bufs.empty(); ++r) {
     if ((busy_lanes >> r) & 1) continue;
@@ -638,21 +686,20 @@ static uint64_t sv_admit(g5_server* srv, Engine& e, double t) {
     e.lane_prev_nq[r] = 0;
     e.lane_visited[r] = 1;
     e.lane_vdeg[r] = 0;
-    uint8_t* ans = e.bufs[q.buf]->p;
-    hipLaunchKernelGGL(k_sv_fill_bytes, dim3(grid_of(e.rows, kBlock, 2048)), dim3(kBlock), 0, e.s, ans, e.rows,
-                       (uint8_t)0xFF);
-    rs.root[r] = q.root;
-    rs.ans[r] = ans;
+    rs.root[n] = q.root;
+    rs.ans[n] = e.bufs[q.buf]->p;
+    rs.lane[n] = (uint8_t)r;
+    ++n;
     admitted |= UINT64_C(1) << r;
   }
   if (admitted) {
-    hipLaunchKernelGGL(k_sv_admit, dim3(1), dim3(64), 0, e.s, e.ctx->graph.old2new.p, e.rows, rs, e.seen.p,
-                       e.fr[e.level & 1].p, e.nz[e.level & 1].p, e.nzs[e.level & 1].p);
+    hipLaunchKernelGGL(k_sv_admit, dim3(grid_of((e.rows + 15) / 16, kBlock, 256), n), dim3(kBlock), 0, e.s,
+                       e.ctx->graph.old2new.p, e.rows, rs, e.seen.p, e.fr[e.level & 1].p, e.nz[e.level & 1].p, e.nzs[e.level & 1].p);
     G5_HIP(hipGetLastError());
     e.nzs_lanes[e.level & 1] |= admitted;
     e.nzc[e.level & 1] += __builtin_popcountll(admitted);  // their roots' words join the marks
     e.active |= admitted;
-    const int64_t k = __builtin_popcountll(admitted);
+    const int64_t k = n;
     (in_flight ? e.st.admitted_busy : e.st.admitted_idle) += k;
     ++e.admit_events;
   }
@@ -702,11 +749,12 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
   const uint64_t* nz_push = e.nzs[cur].p;
   const bool reselect = td && e.nzs_lanes[cur] != td;
   e.nzs_lanes[cur ^ 1] = td;
-  G5_HIP(hipEventRecord(e.ev_start, s));
-  if (reselect)
+  uint64_t* stamp = e.stamp.p;
+  if (reselect) {
     hipLaunchKernelGGL(k_sv_select, dim3(grid_of(e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, front, e.rows, td,
-                       e.nzs[cur].p);
-  G5_HIP(hipMemsetAsync(c, 0, kSvCounterWords * 8, s));
+                       e.nzs[cur].p, stamp);
+    stamp = nullptr;
+  }
   ++e.st.levels;
   if (td && bu) ++e.st.mixed_levels; else if (td) ++e.st.push_levels; else ++e.st.pull_levels;
   e.st.lane_levels += __builtin_popcountll(e.active);
@@ -718,16 +766,13 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
   if (td) {
     // next held the frontier of two levels back, non-zero exactly at the
     // bits of nz_next's last contents: few of them are cleared one by one
-    if (e.nzc[cur ^ 1] * 16 < e.rows)
-      hipLaunchKernelGGL(k_sv_clear_marked, dim3(grid_of(e.words, kBlock, 4096)), dim3(kBlock), 0, s, nz_next,
-                         e.words, e.rows, next);
-    else
-      hipLaunchKernelGGL(k_sv_zero, dim3(grid_of(e.rows, kBlock, 4096)), dim3(kBlock), 0, s, next, e.rows);
+    const bool marked = e.nzc[cur ^ 1] * 16 < e.rows;
+    hipLaunchKernelGGL(k_sv_clear_level, dim3(grid_of(marked ? e.words : e.rows, kBlock, 4096)), dim3(kBlock), 0, s,
+                       nz_next, e.words, e.rows, next, marked ? 1 : 0, listed ? epi.nz_sel : nullptr, stamp);
+    stamp = nullptr;
     hipLaunchKernelGGL(k_sv_collect, dim3(grid_of((int64_t)e.nchunks, kBlock, 4096)), dim3(kBlock), 0, s,
                        e.chunk_rows.p, e.nchunks, nz_push, e.chunk_list.p, (unsigned*)(c + M_NUM));
     if (listed) {
-      G5_HIP(hipMemsetAsync(nz_next, 0, e.words * 8, s));  // after the clear above read it
-      G5_HIP(hipMemsetAsync(epi.nz_sel, 0, e.words * 8, s));
       hipLaunchKernelGGL(k_sv_push_touch, dim3(grid_of((int64_t)e.nchunks, 1, 4096)), dim3(kBlock), 0, s,
                          e.chunk_list.p, (const unsigned*)(c + M_NUM), e.chunk_rows.p, (uint64_t)e.nnz, g.offsets.p,
                          g.cols.p, front, nz_front, next, td, e.touch.p, c + kSvTouch);
@@ -741,16 +786,19 @@ static void sv_launch_level(g5_server* srv, Engine& e) {
     hipLaunchKernelGGL(k_sv_finish_list, dim3(grid_of(e.rows / 8 + 1, kBlock, 2048)), dim3(kBlock), 0, s, e.seen.p,
                        next, nz_next, g.offsets.p, e.touch.p, (const unsigned long long*)(c + kSvTouch), c, epi);
   } else if (bu) {
-    hipLaunchKernelGGL(k_sv_pull, dim3(grid_of(e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, e.seen.p, front,
+    // 16 rows a turn on small graphs, as in a batch
+    const bool part = e.words <= kSvPartWords;
+    hipLaunchKernelGGL(part ? k_sv_pull<16> : k_sv_pull<64>,
+                       dim3(grid_of(part ? 4 * e.words : e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, e.seen.p, front,
                        nz_front, next, nz_next, g.first_nbr.p, g.offsets.p, g.cols.p, e.rows, bu,
-                       srv->cfg.pull_filter, c, keep, td ? 1 : 0, epi);
+                       srv->cfg.pull_filter, c, keep, td ? 1 : 0, epi, stamp);
   } else {
     hipLaunchKernelGGL(k_sv_finish, dim3(grid_of(e.words, kBlock / 64, 8192)), dim3(kBlock), 0, s, e.seen.p, next,
                        nz_next, g.offsets.p, e.rows, c, keep, epi);
   }
   G5_HIP(hipGetLastError());
-  G5_HIP(hipEventRecord(e.ev_end, s));
-  hipLaunchKernelGGL(k_sv_publish, dim3(1), dim3(kBlock), 0, s, c, e.tacc.p, e.pub.d, ++e.pub_seq);
+  hipLaunchKernelGGL(k_sv_publish, dim3(1), dim3(kBlock), 0, s, c, e.tacc.p, e.pub.d, ++e.pub_seq,
+                     e.stamp.p);
   G5_HIP(hipGetLastError());
   e.level = l;
   e.busy = true;
@@ -862,9 +910,7 @@ static bool sv_step(g5_server* srv, Engine& e, double t) {
       G5_CHECK(e.pub.ready(0, kSvPub, e.pub_seq), "serving: a level's counters were not published");
     }
     e.busy = false;
-    float lms = 0;
-    G5_HIP(hipEventSynchronize(e.ev_end));  // recorded before the publish: already complete
-    if (hipEventElapsedTime(&lms, e.ev_start, e.ev_end) == hipSuccess) e.st.busy_ms += lms;
+    e.st.busy_ms += (double)e.pub.value(kSvTicks) / (double)e.clock_khz;
     sv_complete_level(srv, e, t);
   }
   if (!e.active && e.cooling && !e.waiting.empty()) {

@@ -415,7 +415,7 @@ typedef struct g5_server_graph_stats {
   int64_t pull_levels;    /* levels with bottom-up lanes only */
   int64_t mixed_levels;   /* levels with both */
   int64_t lane_levels;    /* sum over levels of the active lanes */
-  double busy_ms;         /* device time of the levels (HIP events) */
+  double busy_ms;         /* device time of the levels (device clock) */
   int64_t completed;      /* queries answered */
   int64_t admitted_busy;  /* queries admitted while other searches of this graph were in flight */
   int64_t admitted_idle;  /* queries admitted into an idle graph */
