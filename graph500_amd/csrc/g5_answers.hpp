@@ -17,6 +17,9 @@ namespace g5 {
 
 // Where a kernel writes an answer of `bytes` for host memory `host`.
 struct HostOut {
+  // Up to here the host's copy out of the pinned buffer (about 10 GB/s) costs
+  // less than the copy command it replaces (15-20 us with its kernel).
+  static constexpr size_t kStageBytes = size_t(256) << 10;
   void* p = nullptr;  // the kernel's output, 16-byte aligned
   // dev is used only for answers the GPU cannot store to the host itself
   template <class T>
@@ -41,9 +44,6 @@ struct HostOut {
   }
 
  private:
-  // Up to here the host's copy out of the pinned buffer (about 10 GB/s) costs
-  // less than the copy command it replaces (15-20 us with its kernel).
-  static constexpr size_t kStageBytes = size_t(256) << 10;
   // one allocation of host memory that the GPU addresses by the same pointer
   static bool pinned(const void* q, size_t bytes) {
     hipPointerAttribute_t at{};

@@ -16,6 +16,7 @@
 // entries relabelled range by range, grouped by row ranges, then by estimated
 // position, sorted and deduplicated in LDS (g5_entries.hpp).  The tuples
 // themselves are never re-sorted.
+#include "g5_answers.hpp"
 #include "g5_ctx.hpp"
 #include "g5_entries.hpp"
 #include "g5_prims.hpp"
@@ -34,7 +35,7 @@ __device__ __forceinline__ uint64_t tuple_v1(const g5_packed_edge& e) {
 // One atomic per workgroup, and none once the bits are there: a wave's OR per
 // wave of a 65,536-workgroup grid spent 3 ms on that one word (12 ns each).
 __global__ void __launch_bounds__(kBlock) k_or_ids(const g5_packed_edge* __restrict__ e, int64_t m,
-                                                   unsigned long long* out) {
+                                                   Published* __restrict__ pub, uint64_t seq) {
   __shared__ uint64_t s_or[kBlock / 64];
   uint64_t acc = 0;
   const int64_t stride = (int64_t)gridDim.x * kBlock;
@@ -49,9 +50,24 @@ __global__ void __launch_bounds__(kBlock) k_or_ids(const g5_packed_edge* __restr
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < kBlock / 64; ++w) acc |= s_or[w];
-    if (acc & ~__hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      atomicOr(out, (unsigned long long)acc);
+    publish(pub + blockIdx.x, acc, seq);
   }
+}
+
+// Zeroes two arrays (a fill call each is one launch or two).
+__global__ void __launch_bounds__(kBlock) k_zero2(uint32_t* __restrict__ a, int64_t na, uint32_t* __restrict__ b,
+                                                  int64_t nb) {
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x, stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t i = t; i < na; i += stride) a[i] = 0;
+  for (int64_t i = t; i < nb; i += stride) b[i] = 0;
+}
+
+// The info words, and the columns in all rows, to the host.
+__global__ void __launch_bounds__(64) k_publish_info(const unsigned long long* __restrict__ info,
+                                                     const uint64_t* __restrict__ nnz, Published* __restrict__ pub,
+                                                     uint64_t seq) {
+  if (threadIdx.x < I_NUM) publish(pub + threadIdx.x, info[threadIdx.x], seq);
+  if (threadIdx.x == I_NUM) publish(pub + I_NUM, *nnz, seq);
 }
 
 // Sort keys for the vertex order: smaller key first, stable by id.
@@ -136,12 +152,23 @@ __global__ void k_first_nbr(const uint64_t* __restrict__ offsets, const uint32_t
 
 // has_edge bitmap by original id (one wave writes one 64-bit word).
 __global__ void __launch_bounds__(kBlock) k_has_edge_bits(const uint32_t* __restrict__ deg, int64_t n,
-                                                          uint64_t* __restrict__ words) {
-  for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v - (threadIdx.x & 63) < n;
-       v += (int64_t)gridDim.x * kBlock) {
-    const bool has = v < n && deg[v] > 0;
-    const uint64_t w = __ballot(has);
-    if ((threadIdx.x & 63) == 0) words[v >> 6] = w;
+                                                          uint64_t* __restrict__ words,
+                                                          const unsigned long long* __restrict__ info,
+                                                          Published* __restrict__ pub, uint64_t seq) {
+  // the host goes on with the info words while the bits are made
+  if (blockIdx.x == 0 && threadIdx.x < I_NUM) publish(pub + threadIdx.x, info[threadIdx.x], seq);
+  // a wave makes 16 words, stored together (they may go to the host's memory)
+  const int lane = threadIdx.x & 63;
+  const int64_t nw = (n + 63) / 64, waves = (int64_t)gridDim.x * (kBlock / 64);
+  for (int64_t w0 = ((int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * 16; w0 < nw; w0 += waves * 16) {
+    uint64_t mine = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int64_t v = (w0 + j) * 64 + lane;
+      const uint64_t w = __ballot(v < n && deg[v] > 0);
+      if (lane == j) mine = w;
+    }
+    if (lane < 16 && w0 + lane < nw) words[w0 + lane] = mine;
   }
 }
 
@@ -192,6 +219,13 @@ static void partition(const Src& src, unsigned long long* cursor, uint64_t* out,
   G5_HIP(hipGetLastError());
 }
 
+// What a construction publishes: the OR of the ids by workgroup, then the info
+// words after the degrees and, with the columns' count, after the sort.
+constexpr int kPubOr = (int)kTupleGrid;
+// Up to this many ids the bitmap of used ones fits the pinned stage, and
+// scratch is kept to the end instead of given back on the way (12 B an id).
+constexpr int64_t kSmallIds = (int64_t)HostOut::kStageBytes * 8;
+
 void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   G5_CHECK(mode >= 0 && mode <= 2, "g5_construct: reorder_mode must be 0, 1 or 2");
   G5_CHECK(ctx->num_edges > 0, "g5_construct: the edge list is empty");
@@ -202,19 +236,23 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   const int64_t m = ctx->num_edges;
   const g5_packed_edge* e = ctx->edges.p;
 
+  // What the host needs on the way is published to it (the OR of the ids by
+  // workgroup, the info words twice); a copy and a wait each took 25 us more.
+  ctx->build_pub.alloc_once(kPubOr + 2 * (I_NUM + 1));
+  PublishBlock& pub = ctx->build_pub;
+  const uint64_t seq = ++ctx->build_seq;
   hipEvent_t t0, t1;
   G5_HIP(hipEventCreate(&t0));
   G5_HIP(hipEventCreate(&t1));
   G5_HIP(hipEventRecord(t0, s));
 
   // 1. estimated SCALE
-  G5_HIP(hipMemsetAsync(ctx->acc.p, 0, 8, s));
-  hipLaunchKernelGGL(k_or_ids, dim3(std::min(grid_for(m, kBlock * 8), kTupleGrid)), dim3(kBlock), 0, s, e, m,
-                     (unsigned long long*)ctx->acc.p);
+  const unsigned or_grid = std::min(grid_for(m, kBlock * 8), kTupleGrid);
+  hipLaunchKernelGGL(k_or_ids, dim3(or_grid), dim3(kBlock), 0, s, e, m, pub.d, seq);
   G5_HIP(hipGetLastError());
+  pub.wait(0, (int)or_grid, seq, s, "g5_construct: the ids' bits were not published");
   uint64_t orv = 0;
-  G5_HIP(hipMemcpyAsync(&orv, ctx->acc.p, 8, hipMemcpyDeviceToHost, s));
-  G5_HIP(hipStreamSynchronize(s));
+  for (unsigned i = 0; i < or_grid; ++i) orv |= pub.value((int)i);
   int scale = 0;
   while (scale < 64 && (orv >> scale)) ++scale;
   G5_CHECK(scale >= 1, "g5_construct: all vertex ids are zero");
@@ -242,8 +280,8 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   uint64_t* range_off = (uint64_t*)(cur2 + pad);
   uint64_t* l1_base = range_off + kPartMax + 1;
   unsigned long long* info = cur2 + pad + 2 * (kPartMax + 1);
-  G5_HIP(hipMemsetAsync(ctl.p, 0, ctl.bytes(), s));
-  G5_HIP(hipMemsetAsync(loops.p, 0, n * 4, s));
+  hipLaunchKernelGGL(k_zero2, dim3(grid_for(std::max<int64_t>(n, (int64_t)ctl.n * 2), kBlock * 4)), dim3(kBlock), 0, s,
+                     (uint32_t*)ctl.p, (int64_t)ctl.n * 2, loops.p, n);
   hipLaunchKernelGGL(k_part_count, dim3(std::min(grid_for(m, kBlock * 8), kTupleGrid)), dim3(kBlock), 0, s, e, m, shift, nb,
                      counts, info);
   hipLaunchKernelGGL(k_part_offsets, dim3(1), dim3(kPartMax), 0, s, counts, nb, range_off, cur0, cur1);
@@ -253,47 +291,51 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   partition(SrcTuples{e, m, loops.p, shift}, cur0, xa.p, s);
   hipLaunchKernelGGL(k_bucket_degrees, dim3((unsigned)nb << (shift - sub_shift)), dim3(1024), 0, s, xa.p, range_off,
                      shift, sub_shift, n, deg.p, info);
+  // has_edge bitmap by original id, kept on the host for root selection; small
+  // ones are written to pinned host memory by the kernel
+  DevBuf<uint64_t> words;
+  const int64_t nw = (n + 63) / 64;
+  const bool small = n <= kSmallIds;
+  uint64_t* h_words = nullptr;
+  if (small) {
+    h_words = (uint64_t*)ctx->stage.get(HostOut::kStageBytes);
+  } else {
+    words.alloc(nw);
+  }
+  hipLaunchKernelGGL(k_has_edge_bits, dim3(grid_for(n, kBlock * 16)), dim3(kBlock), 0, s, deg.p, n, small ? h_words : words.p, info,
+                     pub.d + kPubOr, seq);
   G5_HIP(hipGetLastError());
   uint64_t h_info[I_NUM];
-  G5_HIP(hipMemcpyAsync(h_info, info, sizeof(h_info), hipMemcpyDeviceToHost, s));
-  G5_HIP(hipStreamSynchronize(s));
+  const auto read_info = [&](int at, int count) {
+    pub.wait(at, at + count, seq, s, "g5_construct: counts were not published");
+    for (int i = 0; i < I_NUM; ++i) h_info[i] = pub.value(at + i);
+  };
+  read_info(kPubOr, I_NUM);
   g.max_degree = (int64_t)h_info[I_MAXDEG];
   g.self_loops = (int64_t)h_info[I_LOOPS];
   g.n_active = (int64_t)h_info[I_ACTIVE];
   g.directed_before = 2 * (m - g.self_loops);
   g.n_rows = (mode == 0) ? n : g.n_active;
-  if (release_edges) {
+  if (release_edges && !small) {
     ctx->edges.release();
     ctx->num_edges = 0;
   }
-
-  // has_edge bitmap by original id, kept on the host for root selection
-  {
-    DevBuf<uint64_t> words;
-    const int64_t nw = (n + 63) / 64;
-    words.alloc(nw);
-    hipLaunchKernelGGL(k_has_edge_bits, dim3(grid_for(n)), dim3(kBlock), 0, s, deg.p, n, words.p);
-    G5_HIP(hipGetLastError());
-    g.has_edge_words.resize(nw);
+  g.has_edge_words.resize(nw);
+  if (!small) {
     G5_HIP(hipMemcpyAsync(g.has_edge_words.data(), words.p, nw * 8, hipMemcpyDeviceToHost, s));
     G5_HIP(hipStreamSynchronize(s));
-    g.max_used_vertex = 0;
-    for (int64_t w = nw - 1; w >= 0; --w)
-      if (g.has_edge_words[w]) {
-        g.max_used_vertex = w * 64 + 63 - __builtin_clzll(g.has_edge_words[w]);
-        break;
-      }
+    words.drop();
   }
 
   // 3. vertex order
   g.new2old.alloc(n);
   g.old2new.alloc(n);
   RadixScratch rs;
+  DevBuf<uint32_t> k0, k1, v1;
   if (mode == 0) {
     hipLaunchKernelGGL(k_iota, dim3(grid_for(n)), dim3(kBlock), 0, s, n, g.new2old.p);
     G5_HIP(hipGetLastError());
   } else {
-    DevBuf<uint32_t> k0, k1, v1;
     k0.alloc(n);
     k1.alloc(n);
     v1.alloc(n);
@@ -305,9 +347,13 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     while (bits < 32 && (kmax >> bits)) ++bits;
     uint32_t *kp = k0.p, *ka = k1.p, *vp = g.new2old.p, *va = v1.p;
     radix_sort_pairs_u32(&kp, &ka, &vp, &va, (size_t)n, 0, bits, rs, s);
-    if (vp != g.new2old.p)
-      G5_HIP(hipMemcpyAsync(g.new2old.p, vp, n * 4, hipMemcpyDeviceToDevice, s));
-    G5_HIP(hipStreamSynchronize(s));
+    if (vp != g.new2old.p) g.new2old.swap(v1);
+    if (!small) {  // the memory is needed below
+      G5_HIP(hipStreamSynchronize(s));
+      k0.drop();
+      k1.drop();
+      v1.drop();
+    }
   }
   const int64_t rows = g.n_rows;
   g.weight.alloc(rows);
@@ -331,6 +377,9 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   const uint64_t E = (uint64_t)g.directed_before;
   xb.alloc(nkeys);
   uint64_t nnz = 0;
+  DevBuf<uint64_t> sub64;  // first position | first entry | first unique column
+  DevBuf<uint32_t> sub32;  // entries | first row | unique columns | L1 first sub-buckets | column shares
+  DevBuf<uint64_t> stmp;
   if (E == 0) {
     g.cols.alloc(0);
     G5_HIP(hipMemsetAsync(g.offsets.p, 0, (rows + 1) * 8, s));
@@ -338,8 +387,6 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     const int sub = sub_shift_for(E), wshift = l1_shift(E, sub);
     const int nb1 = (int)(((E - 1) >> wshift) + 1);
     const size_t max_subs = (size_t)(E >> sub) + nb1 + 1;
-    DevBuf<uint64_t> sub64;  // first position | first entry | first unique column
-    DevBuf<uint32_t> sub32;  // entries | first row | unique columns | L1 first sub-buckets | column shares
     sub64.alloc(3 * (max_subs + 1));
     sub32.alloc(3 * max_subs + kPartMax + 1 + kFracMax);
     uint64_t *sub_pos = sub64.p, *sub_off = sub_pos + max_subs + 1, *out_off = sub_off + max_subs + 1;
@@ -374,7 +421,8 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     }
     hipLaunchKernelGGL(k_refine, dim3((unsigned)nb1), dim3(1024), 0, s, grouped, refined, sub, l1_base, l1_sub0,
                        sub_pos, sub_off, sub_cnt, info);
-    G5_HIP(hipMemsetAsync(row_cnt.p, 0, (rows + 1) * 4, s));
+    hipLaunchKernelGGL(k_zero2, dim3(grid_for(rows + 1, kBlock * 4)), dim3(kBlock), 0, s, row_cnt.p, rows + 1,
+                       (uint32_t*)nullptr, (int64_t)0);
     if (sub == 11)
       hipLaunchKernelGGL(k_sort_sub<11>, dim3((unsigned)max_subs), dim3(SubSort<11>::kThreads), 0, s, refined, sub_off,
                          sub_cnt, sub_pos, sub_row, P.p, rows, row_cnt.p, sub_unique, info);
@@ -382,13 +430,14 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
       hipLaunchKernelGGL(k_sort_sub<12>, dim3((unsigned)max_subs), dim3(SubSort<12>::kThreads), 0, s, refined, sub_off,
                          sub_cnt, sub_pos, sub_row, P.p, rows, row_cnt.p, sub_unique, info);
     G5_HIP(hipGetLastError());
-    DevBuf<uint64_t> stmp;
     stmp.alloc(scan_tmp_elems(max_subs));
     device_scan(LoadU32{row_cnt.p}, StoreU64{g.offsets.p}, (size_t)rows + 1, tmp.p, s);
     device_scan(LoadU32{sub_unique}, StoreU64{out_off}, max_subs, stmp.p, s);
-    G5_HIP(hipMemcpyAsync(h_info, info, sizeof(h_info), hipMemcpyDeviceToHost, s));
-    G5_HIP(hipMemcpyAsync(&nnz, g.offsets.p + rows, 8, hipMemcpyDeviceToHost, s));
-    G5_HIP(hipStreamSynchronize(s));
+    hipLaunchKernelGGL(k_publish_info, dim3(1), dim3(64), 0, s, info, g.offsets.p + rows, pub.d + kPubOr + I_NUM + 1,
+                       seq);
+    G5_HIP(hipGetLastError());
+    read_info(kPubOr + I_NUM + 1, I_NUM + 1);
+    nnz = pub.value(kPubOr + 2 * I_NUM + 1);
     if (!h_info[I_WIDE] && !h_info[I_OVERFLOW]) {
       g.cols.alloc(nnz);
       hipLaunchKernelGGL(k_compact, dim3((unsigned)max_subs), dim3(kBlock), 0, s, refined, sub_off, sub_unique, out_off,
@@ -412,7 +461,6 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
                          g.offsets.p);
       G5_HIP(hipGetLastError());
     }
-    G5_HIP(hipStreamSynchronize(s));
   }
   g.nnz = (int64_t)nnz;
 
@@ -427,6 +475,21 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   g.construct_ms = ms;
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
+  // all work is done: the scratch goes back without a wait each
+  if (small) std::copy(h_words, h_words + nw, g.has_edge_words.begin());
+  g.max_used_vertex = 0;
+  for (int64_t w = nw - 1; w >= 0; --w)
+    if (g.has_edge_words[w]) {
+      g.max_used_vertex = w * 64 + 63 - __builtin_clzll(g.has_edge_words[w]);
+      break;
+    }
+  if (release_edges && small) {
+    ctx->edges.drop();
+    ctx->num_edges = 0;
+  }
+  for (DevBuf<uint32_t>* b : {&deg, &loops, &k0, &k1, &v1, &row_cnt, &sub32}) b->drop();
+  for (DevBuf<uint64_t>* b : {&xa, &xb, &P, &tmp, &row_word, &sub64, &stmp}) b->drop();
+  ctl.drop();
   g.built = true;
 }
 

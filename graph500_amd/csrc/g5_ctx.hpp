@@ -298,6 +298,8 @@ struct g5_ctx {
   g5::MsState ms;
   g5::DevBuf<uint64_t> acc;  // small reduction scratch
   g5::HostStage stage;       // small answers on their way to the host
+  g5::PublishBlock build_pub;  // what a construction publishes on its way
+  uint64_t build_seq = 0;
   int servers = 0;           // g5_server objects that serve this context's graph
 };
 

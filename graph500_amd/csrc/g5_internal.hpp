@@ -13,6 +13,7 @@
 //                 parent uint32[n_active], frontier queues uint32[2][n_active]
 #pragma once
 
+#include <utility>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -57,7 +58,7 @@ constexpr int kWave = 64;
 // a pass in hipMalloc and hipFree for 55 ms of kernels.
 // ---------------------------------------------------------------------------
 hipError_t pool_alloc(void** p, size_t bytes);
-void pool_free(void* p);
+void pool_free(void* p, bool idle = false);  // idle: the caller has waited for all work on the block
 void pool_context(int device, int delta);  // a context comes (+1) or goes (-1)
 
 // ---------------------------------------------------------------------------
@@ -88,6 +89,16 @@ struct DevBuf {
     if (p) pool_free(p);
     p = nullptr;
     n = 0;
+  }
+  // release() without its wait for the device: all work on the buffer is known to be done
+  void drop() {
+    if (p) pool_free(p, true);
+    p = nullptr;
+    n = 0;
+  }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
   }
   size_t bytes() const { return n * sizeof(T); }
 };

@@ -1,7 +1,7 @@
 // g5_pool.hip -- device memory with freed blocks kept for reuse.
 //
 // A freed block joins its device's list (after the wait for the device that
-// hipFree makes, so whoever takes it next, on whatever stream or thread,
+// hipFree makes, or the owner's own wait for all work on it, so whoever takes it next, on whatever stream or thread,
 // finds no work of the previous owner on it) and serves a later request of
 // at least 4/5 of its size.  The list holds at most 1/8 of the device's
 // memory; older blocks go back to the driver first, larger ones at once.  A
@@ -84,7 +84,7 @@ hipError_t pool_alloc(void** p, size_t bytes) {
   return e;
 }
 
-void pool_free(void* p) {
+void pool_free(void* p, bool idle) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
     const auto it = g_live.find(p);
@@ -92,7 +92,7 @@ void pool_free(void* p) {
     if (it != g_live.end()) g_live.erase(it);
     if (b.device >= 0 && b.device == current()) {
       Pool& pl = g_pool[b.device];
-      if (pl.contexts > 0 && b.bytes <= pl.limit && hipDeviceSynchronize() == hipSuccess) {
+      if (pl.contexts > 0 && b.bytes <= pl.limit && (idle || hipDeviceSynchronize() == hipSuccess)) {
         trim(pl, pl.limit - b.bytes);
         pl.kept.push_back({p, b.bytes});
         pl.total += b.bytes;

@@ -51,6 +51,10 @@ struct PublishBlock {
     G5_HIP(hipHostGetDevicePointer((void**)&d, h, 0));
     n = count;
   }
+  // an equal block as it is (tags of earlier sequence numbers may be set)
+  void alloc_once(int count) {
+    if (!h || n != count) alloc(count);
+  }
   void release() {
     if (h) (void)hipHostFree(h);
     h = d = nullptr;
