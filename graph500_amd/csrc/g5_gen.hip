@@ -16,6 +16,7 @@
 #include "g5_internal.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace g5 {
 
@@ -230,31 +231,66 @@ struct GenParams {
   uint64_t val0, val1;
   int64_t start, count;
   int scale;
-  uint32_t a_num, bc_num;
+  uint32_t t1, t2, t3;  // floor(k * 2^32 / 10000) for the thresholds bc, 2 bc, 2 bc + a
   int groups;  // 256-tuple groups per workgroup
 };
 
-// One draw's quadrant number below 10000 (draws under the rejection bound
-// 2^32 mod 10000 are taken again, as the generator defines it).
-__device__ __forceinline__ uint32_t ddraw(DState& st) {
-  constexpr uint32_t kLimit = UINT32_C(0xFFFFFFFF) % 10000u;  // 7295
-  uint32_t v = dstep(st);
-  while (v < kLimit) v = dstep(st);
-  return v - __umul24(v / 10000u, 10000u);  // the quotient has 18 bits: one full-rate multiply
+// Draws under 2^32 mod 10000 are taken again, as the generator defines it.
+constexpr uint32_t kLimit = UINT32_C(0xFFFFFFFF) % 10000u;  // 7295
+
+// The next draw from the latest one and the one five back.  Twice the
+// products, so that the fold's parts are the two halves.
+__device__ __forceinline__ uint32_t dnext(uint32_t z1, uint32_t z5) {
+  const uint64_t x = (uint64_t)(2 * kX) * z1 + (uint64_t)(2 * kY) * z5;  // < 2^60
+  const uint32_t r = (uint32_t)(x >> 32) + ((uint32_t)x >> 1);
+  return min(r, r - kM);
 }
+
+// 2^32 times the fraction of v / 10000 (v < 2^31), rounded down or to the
+// integer above: exact enough that v mod 10000 >= k where it is at least
+// floor(k * 2^32 / 10000) (neighbouring residues are 429,496 apart).
+__device__ __forceinline__ uint32_t dfrac(uint32_t v) {
+  constexpr uint64_t kInv = UINT64_MAX / 10000 + 1;
+  return v * (uint32_t)(kInv >> 32) + __umulhi(v, (uint32_t)kInv);
+}
+
+// acc = 2 acc + (f >= limit)
+__device__ __forceinline__ void dpush(uint32_t& acc, uint32_t f, uint32_t limit) {
+  asm("v_cmp_le_u32 vcc, %2, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(acc) : "v"(f), "s"(limit) : "vcc");
+}
+__device__ __forceinline__ void dpush(uint64_t& acc, uint32_t f, uint32_t limit) { acc = 2 * acc + (f >= limit); }
+
+// A tuple's quadrant draws so far, one bit per level: at least bc, 2 bc, 2 bc + a.
+template <class Bits>
+struct DBits {
+  Bits c1 = 0, c2 = 0, c3 = 0;
+  __device__ __forceinline__ void add(const GenParams& p, uint32_t v) {
+    const uint32_t f = dfrac(v);
+    dpush(c1, f, p.t1);
+    dpush(c2, f, p.t2);
+    dpush(c3, f, p.t3);
+  }
+};
 
 // tab: the 8 byte-tables of the middle exponent word (entries [8*256, 16*256)).
 // A workgroup takes p.groups runs of 256 tuple indices, aligned to 256, so
 // that a run shares every byte of its indices but the lowest: thread k makes
 // run k's state once (LDS), and lane t applies the low byte's transition,
-// which it keeps in registers over all runs.  The kernel is bound by the
-// integer multiplies of the draws (two 64-bit multiply-adds and a high
-// multiply per level, quarter rate); with four transitions per tuple, read
-// from the table, SCALE 25 (2^29 tuples) took 17.3 ms.
+// which it keeps in registers over all runs.
+//
+// The kernel is bound by its instructions (no memory but the 12 bytes
+// written), so a level is little more than the draw: five levels unrolled
+// rotate the state without moves, the thresholds meet the scaled fraction of
+// the draw instead of its residue and shift their outcomes into bit strings,
+// and what depends on all levels (which quadrant, clip-and-flip, a draw to be
+// taken again, 1 tuple in 11,000) is looked at once per tuple.  730 vector
+// instructions per tuple of SCALE 25 took 9.0 ms for 2^29 tuples, 500 take 7.0
+// (17.3 with four transitions per tuple read from the table).
 template <bool k32>
 __global__ void __launch_bounds__(256) k_kronecker(g5_packed_edge* __restrict__ out,
                                                    const DevEntry* __restrict__ tab,
                                                    GenParams p) {
+  using Bits = typename std::conditional<k32, uint32_t, uint64_t>::type;
   __shared__ DState s_run[256];
   const int t = threadIdx.x;
   const int64_t g0 = (p.start >> 8) + (int64_t)blockIdx.x * p.groups;
@@ -269,37 +305,62 @@ __global__ void __launch_bounds__(256) k_kronecker(g5_packed_edge* __restrict__ 
   }
   const DevEntry low = tab[t];
   __syncthreads();
-  const uint32_t bc = p.bc_num, bc2 = 2 * p.bc_num, abc = bc2 + p.a_num;
+  const int fives = p.scale / 5, ones = p.scale % 5;
+  const Bits all = (Bits)(~UINT64_C(0) >> (64 - p.scale));
   for (int k = 0; k < p.groups; ++k) {
     const int64_t i = ((g0 + k) << 8) + t - p.start;
     if (i < 0 || i >= p.count) continue;
     DState st = s_run[k];
     dapply(low, st);
-    uint64_t bs = 0, bt = 0;
-    uint32_t bs32 = 0, bt32 = 0;
-    bool same = true;  // bs == bt so far
-    for (int lvl = p.scale - 1; lvl >= 0; --lvl) {
-      const uint32_t val = ddraw(st);
-      // below bc: quadrant 1, below 2 bc: 2, below 2 bc + a: 0, else 3
-      const bool both = val >= abc;
-      bool so = both || (val >= bc && val < bc2), to = both || val < bc;
-      if (same && so && !to) {  // clip-and-flip
-        so = false;
-        to = true;
+    const DState start = st;
+    DBits<Bits> q;
+    uint32_t least = UINT32_MAX;
+    for (int l = 0; l < ones; ++l) {
+      const uint32_t v = dstep(st);
+      least = min(least, v);
+      q.add(p, v);
+    }
+    for (int l = 0; l < fives; ++l) {
+      st.z5 = dnext(st.z1, st.z5);
+      q.add(p, st.z5);
+      st.z4 = dnext(st.z5, st.z4);
+      q.add(p, st.z4);
+      least = min(least, min(st.z5, st.z4));
+      st.z3 = dnext(st.z4, st.z3);
+      q.add(p, st.z3);
+      st.z2 = dnext(st.z3, st.z2);
+      q.add(p, st.z2);
+      least = min(least, min(st.z3, st.z2));
+      st.z1 = dnext(st.z2, st.z1);
+      q.add(p, st.z1);
+      least = min(least, st.z1);
+      // the latest draw is z1 again and the one five back z5
+    }
+    if (least < kLimit) {  // some draw has to be taken again: this tuple from its start
+      st = start;
+      q = DBits<Bits>();
+      for (int l = 0; l < p.scale; ++l) {
+        uint32_t v = dstep(st);
+        while (v < kLimit) v = dstep(st);
+        q.add(p, v);
       }
-      same = same && so == to;
-      if (k32) {
-        bs32 = 2 * bs32 + so;
-        bt32 = 2 * bt32 + to;
-      } else {
-        bs = 2 * bs + so;
-        bt = 2 * bt + to;
+    }
+    // below bc: (0, 1), below 2 bc: (1, 0), below 2 bc + a: (0, 0), else (1, 1)
+    Bits bs = q.c3 | (q.c1 & ~q.c2), bt = q.c3 | (~q.c1 & all);
+    // clip-and-flip: (1, 0) at the first level where the two differ becomes (0, 1)
+    const Bits diff = bs ^ bt;
+    if (diff) {
+      const Bits first = k32 ? (Bits)(UINT32_C(0x80000000) >> __builtin_clz((uint32_t)diff))
+                             : (Bits)(UINT64_C(0x8000000000000000) >> __builtin_clzll((uint64_t)diff));
+      if (bs & first) {
+        bs ^= first;
+        bt ^= first;
       }
     }
     g5_packed_edge r;
     if (k32) {
-      r.v0_low = dscramble32(bs32, p.scale, p.val0, p.val1);
-      r.v1_low = dscramble32(bt32, p.scale, p.val0, p.val1);
+      r.v0_low = dscramble32((uint32_t)bs, p.scale, p.val0, p.val1);
+      r.v1_low = dscramble32((uint32_t)bt, p.scale, p.val0, p.val1);
       r.high = 0;
     } else {
       const uint64_t v0 = dscramble(bs, p.scale, p.val0, p.val1);
@@ -423,8 +484,11 @@ void launch_kronecker(int device, g5_packed_edge* out, int64_t start, int64_t co
   p.start = start;
   p.count = count;
   p.scale = scale;
-  p.a_num = (uint32_t)a_num;
-  p.bc_num = (uint32_t)bc_num;
+  // a draw's fraction is below 2^32 - 1, which a threshold of 10000 becomes
+  const auto limit = [](int k) { return k >= 10000 ? UINT32_MAX : (uint32_t)(((uint64_t)k << 32) / 10000); };
+  p.t1 = limit(bc_num);
+  p.t2 = limit(2 * bc_num);
+  p.t3 = limit(2 * bc_num + a_num);
   if (count <= 0) return;
   // Edge indices up to 2^64 use at most the 8 middle-word tables.
   const int64_t runs = ((start + count + 255) >> 8) - (start >> 8);

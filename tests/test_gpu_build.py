@@ -117,3 +117,14 @@ def test_generator_slices(oracle_mod, scale, edgefactor):
             got = c.edges_download(start, 1001 if start + 1001 <= m else m - start)
             exp = oracle_mod.generate_edges(scale, edgefactor, 5, 9, start=start, end=start + len(got))
             assert np.array_equal(got, exp), start
+
+
+@pytest.mark.parametrize("scale", [1, 2, 3, 4, 5, 6, 9, 10, 11])
+@pytest.mark.parametrize("a,bc", [(5700, 1900), (5500, 100), (10000, 0), (0, 5000), (0, 0), (1, 4999), (9998, 1)])
+def test_generator_parameters(oracle_mod, scale, a, bc):
+    """Levels in fives and the rest, and thresholds at the ends of their range."""
+    import graph500_amd
+    with graph500_amd.G5Context(0) as c:
+        c.generate_kronecker(scale, 23, 7, 11, a, bc)
+        got = c.edges_download()
+        assert np.array_equal(got, oracle_mod.generate_edges(scale, 23, 7, 11, a, bc)), (scale, a, bc)
