@@ -51,6 +51,13 @@ namespace g5 {
 constexpr uint64_t kTdSmall = 1 << 20;  // top-down levels up to this many edges use the atomic path
 constexpr int kBinShift = 19;           // binned top-down: at least 2^19 targets per bucket
 constexpr int kShortRow = 32;    // bottom-up: lane-sequential scan up to this length
+// Searches of many rows at a time (kR = 1: k_bu, k_td_head): rows over
+// kShortRow1 entries go to groups of 16 lanes, and what kGroupTurns turns
+// leave of a very long one to the whole wave.  A wave per row read 64 entries
+// where a few decide, one row after another (S26 700 us a search, S28 2,396;
+// so 646 and 2,224; with the limit 8 and 32: 644 and 662, 2,244 and 2,190).
+constexpr int kShortRow1 = 16;
+constexpr int kGroupTurns = 8;
 constexpr uint32_t kNoNbr = 0xFFFFFFFFu;
 
 // counters: vertices found; the root (new id); head words (k_td_head_size);
@@ -390,7 +397,7 @@ __global__ void __launch_bounds__(kBlock) k_td_expand_segs(
 // active=false only help.  Rows up to kShortRow are scanned by their lane, kU
 // entries a turn; longer rows by the whole wave, kR rows a turn, 64 entries of
 // each (the last one left takes all kR x 64), a ballot giving a row's first
-// hit.  A turn is a chain of two dependent loads, so on small graphs, whose
+// hit; with kR = 1 by groups of 16 lanes first (see kShortRow1).  A turn is a chain of two dependent loads, so on small graphs, whose
 // bottom-up levels are a few such chains, the turns are what counts (kU 8, kR
 // 4); on large ones the probes past a hit are (kU 4, kR 1 with two per lane).
 template <int kU, int kR>
@@ -405,7 +412,7 @@ __device__ __forceinline__ bool row_marked_nbr(bool active, uint32_t v, const ui
     re = offsets[v + 1];
     need = rb < re;
   }
-  if (need && re - rb <= (uint64_t)kShortRow) {
+  if (need && re - rb <= (uint64_t)(kR == 1 ? kShortRow1 : kShortRow)) {
     // independent probes (entries past the row repeat the first); any marked
     // neighbour is a valid parent, the first is taken
     for (uint64_t k = rb; k < re && !found; k += kU) {
@@ -426,6 +433,62 @@ __device__ __forceinline__ bool row_marked_nbr(bool active, uint32_t v, const ui
     need = false;
   }
   uint64_t lm = __ballot(need);
+  if (kR == 1) {
+    // by groups of 16 lanes, four rows at a time, a group taking the next row
+    // as soon as its own is done
+    const int gid = lane / 16, gl = lane % 16;
+    uint64_t rest = 0;
+    int src = -1, turn = 0;
+    uint64_t b = 0, e = 0;
+    for (;;) {
+      const uint64_t idle = __ballot(src < 0);
+      if (idle) {
+        if (!lm && idle == ~UINT64_C(0)) break;
+        const int rank = __popcll(idle & ((UINT64_C(1) << (gid * 16)) - 1)) / 16;
+        int take = -1;
+        for (int i = 0; i < __popcll(idle) / 16 && lm; ++i) {
+          if (i == rank) take = __builtin_ctzll(lm);
+          lm &= lm - 1;
+        }
+        const int from = take < 0 ? lane : take;
+        const uint64_t b1 = __shfl(rb, from, 64), e1 = __shfl(re, from, 64);
+        if (src < 0 && take >= 0) {
+          src = take;
+          b = b1;
+          e = e1;
+          turn = 0;
+        }
+      }
+      const bool in = src >= 0 && b + gl < e;
+      const uint32_t c = in ? cols[b + gl] : 0;
+      const uint64_t m = __ballot(in && bit_set(bm, c));
+      b += 16;
+      ++turn;
+      const bool done = src >= 0 && (((m >> (gid * 16)) & 0xFFFF) || b >= e);
+      const bool pass = src >= 0 && !done && turn >= kGroupTurns && e - b > 128;  // left to the whole wave
+      const uint64_t out = __ballot(done || pass);
+      if (out) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if (!((out >> (g * 16)) & 1)) continue;
+          const int s = __builtin_amdgcn_readlane(src, g * 16);
+          const uint32_t gm = (uint32_t)(m >> (g * 16)) & 0xFFFF;
+          const uint32_t hp = __shfl(c, g * 16 + (gm ? __builtin_ctz(gm) : 0), 64);
+          const uint64_t gb = __shfl(b, g * 16, 64);
+          if (lane == s) {
+            if (gm) {
+              found = true;
+              p = hp;
+            }
+            rb = gb;
+          }
+          rest |= (uint64_t)(__builtin_amdgcn_readlane((int)pass, g * 16) & 1) << s;
+        }
+        if (done || pass) src = -1;
+      }
+    }
+    lm = rest;
+  }
   while (lm) {
     constexpr int kSlots = kR > 1 ? kR : 2;
     int src[kSlots];
@@ -1173,8 +1236,8 @@ __device__ __forceinline__ void step_expand(const StepArgs& a, const StepLds& L,
 // missed; the rows of those are then searched with every lane busy, whatever
 // words they come from (got gathers who was found).  Searched word by word, a
 // turn of 128 vertices waited for six dependent loads (searches, us: S14 85,
-// now 67; S21 131, 119; S24 318, 302; S28 2,525-2,590, 2,450-2,500; k_bu's
-// largest level there moves 1 GB in 500 us).  `share`: the
+// now 67; S21 131, 119; S24 318, 302; S28 2,560, 2,475; with the rows by groups
+// 294 and 2,224, where k_bu's largest level moves 1 GB in 500 us).  `share`: the
 // workgroup's waves share the rows out, so that a word of hubs, whose long
 // rows one wave searches one after another, does not hold the level up;
 // where waves have words enough that costs more than it gives (S14 18 -> 13
@@ -1875,7 +1938,7 @@ static bool step_alone(const Graph& g, const BfsState& b) {
 }
 // Bitmap words per wave turn of a bottom-up level.  In a step, what gives
 // every wave the same number of turns; for k_bu, 8, or 16 where a wave still
-// has ten turns or more (S26 8/16: 674/685 us a search, S28: 2,521/2,469).
+// has ten turns or more (S26 8/16: 674/685 us a search, S28: 2,521/2,469, before rows went to groups).
 static int bottom_up_span(const Graph& g, const BfsState& b) {
   if (b.words > kStepMaxWords) return b.words >= (INT64_C(1) << 20) ? 16 : 8;
   const int64_t waves = (step_alone(g, b) ? 1 : kStepTdGrid) * (kStepThreads / 64);

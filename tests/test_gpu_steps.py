@@ -92,3 +92,17 @@ def test_bottom_up_turns(oracle_mod, rows):
                         rng.integers(0, rows, (rows, 2)),
                         np.stack([np.arange(rows - 20, rows - 1), np.arange(rows - 19, rows)], 1)])
     check(oracle_mod, tuples(p), [0, rows - 1, int(p[7, 1])])
+
+
+def test_large_bottom_up_rows(oracle_mod):
+    """Bottom-up levels of a graph beyond the steps (over 100,000 bitmap
+    words): rows of every length that is searched another way, many of them
+    with few reached neighbours."""
+    rng = np.random.default_rng(12)
+    n = 6_600_000
+    ring = np.stack([np.arange(n), rng.integers(0, n, n)], 1)
+    lengths = np.concatenate([rng.integers(14, 40, 30000), rng.integers(40, 400, 3000), rng.integers(400, 3000, 60)])
+    src = np.repeat(rng.permutation(n)[: len(lengths)], lengths)
+    extra = np.stack([src, rng.integers(0, n, len(src))], 1)
+    hub = np.stack([np.zeros(9000, np.int64), rng.integers(0, n, 9000)], 1)
+    check(oracle_mod, tuples(np.concatenate([ring, extra, hub])), [0, int(src[0]), n - 5])
