@@ -567,27 +567,52 @@ __global__ void __launch_bounds__(kBlock) k_ms_levels(const uint32_t* __restrict
   }
 }
 
-// Levels by row, for larger graphs: a wave takes 64 rows, and reads a level's
-// words (coalesced) only where the level's bitmap has one of its rows still
-// open; the lookup by original id is then one byte each (k_make_levels)
-// instead of a word per level.
+// Levels by row, for larger graphs: a lane takes 4 consecutive rows and reads
+// a level's words of them only where the level's bitmap has one that is still
+// open, the bitmap words of 4 levels in flight together; the lookup by
+// original id is then one byte each (k_make_levels) instead of a word per
+// level.  A lane's levels of S26 (34 M rows, 0.4 GB read), one row per thread
+// and a bitmap word at a time: 390 us, bound by the chain of loads.
 __global__ void __launch_bounds__(kBlock) k_ms_row_levels(LevelWords lw, int64_t rows, int lane_bit,
                                                           uint8_t* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t words = (rows + 63) / 64, nwaves = (int64_t)gridDim.x * (kBlock / 64);
-  for (int64_t wd = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); wd < words; wd += nwaves) {
-    const int64_t v = wd * 64 + lane;
-    bool open = v < rows;
-    uint32_t l = 0xFF;
-    for (int i = 0; i < lw.n && __ballot(open); ++i) {
-      const uint64_t* nz = i < kMsArgLevels ? lw.nz[i] : nullptr;
-      const bool read = open && (!nz || ((nz[wd] >> lane) & 1));
-      if (read && ((lw.words(i)[v] >> lane_bit) & 1)) {
-        l = i;
-        open = false;
+  const int64_t quads = (rows + 3) / 4, stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q < quads; q += stride) {
+    const int64_t v = q * 4;
+    const int m = rows - v < 4 ? (int)(rows - v) : 4;
+    const int sh = (int)(v & 63);
+    uint32_t open = (1u << m) - 1, l = 0xFFFFFFFFu;
+    for (int i0 = 0; i0 < lw.n && open; i0 += 4) {
+      uint32_t nz[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + j;
+        const uint64_t* w = i < lw.n && i < kMsArgLevels ? lw.nz[i] : nullptr;
+        nz[j] = i >= lw.n ? 0u : w ? (uint32_t)(w[v >> 6] >> sh) & 15u : 15u;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (!(nz[j] & open)) continue;
+        const uint64_t* f = lw.words(i0 + j) + v;
+        uint64_t x[4];
+        if (m == 4) {
+          *reinterpret_cast<ulonglong2*>(x) = *reinterpret_cast<const ulonglong2*>(f);
+          *reinterpret_cast<ulonglong2*>(x + 2) = *reinterpret_cast<const ulonglong2*>(f + 2);
+        } else {
+          for (int k = 0; k < 4; ++k) x[k] = k < m ? f[k] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (((open >> k) & 1) && ((x[k] >> lane_bit) & 1)) {
+            l = (l & ~(0xFFu << (8 * k))) | (uint32_t)(i0 + j) << (8 * k);
+            open &= ~(1u << k);
+          }
       }
     }
-    if (v < rows) out[v] = (uint8_t)l;
+    if (m == 4) {
+      reinterpret_cast<uint32_t*>(out)[q] = l;
+    } else {
+      for (int k = 0; k < m; ++k) out[v + k] = (uint8_t)(l >> (8 * k));
+    }
   }
 }
 
@@ -1459,7 +1484,7 @@ static void ms_upload_level_ptrs(MsState& m, int nlev, hipStream_t s) {
 // From this many rows on a lane's levels are made by row first: below, the
 // levels' frontier words (8 B per row) fit the L2s and one launch is less
 // (one lane of S17: 21 us directly, 23 by row; S19, 335k rows: 32 both; S22,
-// by row: 124, and 162 with one id per thread and a copy behind it).
+// by row: 112, and 162 with one id per thread and a copy behind it).
 constexpr int64_t kRowLevelsFrom = 1 << 19;
 
 void ms_get_levels(g5_ctx* ctx, int lane, uint8_t* host_levels) {
@@ -1485,7 +1510,7 @@ void ms_get_levels(g5_ctx* ctx, int lane, uint8_t* host_levels) {
     G5_HIP(hipGetLastError());
   } else {
     m.row_level.alloc(g.n_rows);
-    hipLaunchKernelGGL(k_ms_row_levels, dim3(grid_of((g.n_rows + 63) / 64, kBlock / 64, 8192)), dim3(kBlock), 0, s, lw,
+    hipLaunchKernelGGL(k_ms_row_levels, dim3(grid_of((g.n_rows + 3) / 4, kBlock, 8192)), dim3(kBlock), 0, s, lw,
                        g.n_rows, lane, m.row_level.p);
     G5_HIP(hipGetLastError());
     launch_make_levels(g.old2new.p, m.row_level.p, g.n, g.n_rows, m.host_roots[lane], (uint8_t*)out.p, s);
