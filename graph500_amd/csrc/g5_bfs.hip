@@ -1548,7 +1548,9 @@ __global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* _
 // A bottom-up level of a large graph, launched by the host: the body above in
 // 256-thread workgroups without a list, at twice the waves per CU a step
 // leaves room for (its registers and LDS hold 16).
-__global__ void __launch_bounds__(kBlock) k_bu(StepArgs a, int cur, int lvl, unsigned long long* __restrict__ counters) {
+__global__ void __launch_bounds__(kBlock) k_bu(StepArgs a, int cur, int lvl, unsigned long long* __restrict__ counters,
+                                               uint64_t* __restrict__ stamp) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();  // the level starts
   __shared__ BuLds<kBlock / 64> bu;
   const uint64_t f = step_bottom_up<kBlock / 64, 4, 1, false>(a, bu, nullptr, nullptr, a.vis[cur], a.vis[cur ^ 1], lvl, false);
   block_add(f, stripe_of(counters + kStripeBase, S_FOUND));
@@ -1608,10 +1610,15 @@ __global__ void __launch_bounds__(kBlock) k_bfs_init(const uint32_t* __restrict_
 // the host need not wait for a copy and a stream synchronisation.
 // One wave: lane i takes stripe i.
 static_assert(kStripes == 64, "k_publish sums one stripe per lane of a wave");
+// The time since the level's stamp is published behind the counters (an event
+// on either side of a level took 7 us of the stream).
+__global__ void k_stamp(uint64_t* stamp) { *stamp = wall_clock64(); }
 __global__ void __launch_bounds__(64) k_publish(unsigned long long* __restrict__ counters,
                                                 const uint64_t* __restrict__ prefix, int64_t nf, int forward,
-                                                Published* pub, uint64_t seq) {
+                                                Published* pub, uint64_t seq,
+                                                const uint64_t* __restrict__ stamp) {
   const int t = threadIdx.x;
+  if (t == C_NUM) publish(pub + t, wall_clock64() - *stamp, seq);
   unsigned long long* mine = counters + kStripeBase + t * kStripeWords;
   const uint64_t found = wave_sum(mine[S_FOUND]);
   const uint64_t next_e = wave_sum(mine[S_NEXT_E]);
@@ -1629,8 +1636,8 @@ __global__ void __launch_bounds__(64) k_publish(unsigned long long* __restrict__
 
 // Waits for the level's counters (see PublishBlock::wait).
 static void wait_published(BfsState& b, hipStream_t s) {
-  b.pub.wait(0, C_NUM, b.pub_seq, s, "g5_run_bfs: level counters were not published");
-  for (int i = 0; i < C_NUM; ++i) b.h_counters[i] = b.pub.value(i);
+  b.pub.wait(0, C_NUM + 1, b.pub_seq, s, "g5_run_bfs: level counters were not published");
+  for (int i = 0; i <= C_NUM; ++i) b.h_counters[i] = b.pub.value(i);
 }
 
 static void build_hub_index(g5_ctx* ctx, BfsState& b, hipStream_t s);
@@ -1679,9 +1686,10 @@ void bfs_prepare(g5_ctx* ctx, BfsState& b, hipStream_t s) {
   b.scan_tmp.alloc(scan_tmp_elems(scan_n));
   b.counters.alloc(kBfsCounters);
   bfs_tuning_buffers(ctx, b, s);
-  static_assert(C_NUM <= sizeof(b.h_counters) / 8, "host counters");
+  static_assert(C_NUM < sizeof(b.h_counters) / 8, "host counters");
   G5_HIP(hipStreamSynchronize(s));  // the published blocks are reset below
-  b.pub.alloc(C_NUM);
+  b.pub.alloc(C_NUM + 1);
+  b.stamp.alloc(1);
   b.pub_seq = 0;
   b.step_ctl.alloc(kStepWords);
   b.step_pub.alloc(P_NUM);
@@ -1727,7 +1735,7 @@ static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& s
   // the frontier's edges when the step summed them (-1: not known, both forms
   // are launched and the device picks)
   const int64_t e_next = state.edges ? (int64_t)state.edges : -1;
-  G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
+  hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, s, b.stamp.p);
   device_scan(FrontierDegree{b.queue[qi].p, g.offsets.p, nf}, StoreU64{b.prefix.p},
               (size_t)nf + 1, b.scan_tmp.p, s);
   if (b.bin_edges > 0) {
@@ -1848,9 +1856,9 @@ static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& s
     hipLaunchKernelGGL(k_td_finish, dim3(grid_of((b.words + 15) / 16, kBlock / 64, 8192)), dim3(kBlock), 0,
                        s, b.level.p, rows, b.words, (uint32_t)lvl, b.vis[cur].p, b.vis[cur ^ 1].p, cnt,
                        b.prefix.p, nf);
-  G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
   ++b.pub_seq;
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, 1, b.pub.d, b.pub_seq);
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, nf, 1, b.pub.d, b.pub_seq,
+                     b.stamp.p);
   G5_HIP(hipGetLastError());
   wait_published(b, s);
   const int64_t nq = (int64_t)b.h_counters[C_FOUND];
@@ -1858,10 +1866,7 @@ static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& s
   st.direction[lvl] = 1;
   st.nq[lvl] = nq;
   st.num_levels = lvl + 1;
-  float lms = 0;
-  G5_HIP(hipEventSynchronize(b.lev_end[lvl]));
-  G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[lvl], b.lev_end[lvl]));
-  st.level_ms[lvl] = lms;
+  st.level_ms[lvl] = (double)b.h_counters[C_NUM] / (double)b.tick_khz;
   ++state.lvl;
   state.visited += nq;
   state.nf = nq;
@@ -1897,34 +1902,27 @@ static void host_bottom_up(g5_ctx* ctx, BfsState& b, hipStream_t s, const StepAr
   Graph& g = ctx->graph;
   unsigned long long* cnt = (unsigned long long*)b.counters.p;
   g5_bfs_stats& st = b.stats;
-  const int lvl0 = state.lvl + 1;
   while (state.nf && (!state.forward || tail_pulls(state.forward, state.growing, b.tail_pull, state.nf,
                                                    g.n_active - state.visited))) {
     const int lvl = state.lvl + 1;
     if (lvl > kStepMaxLevel) break;
-    G5_HIP(hipEventRecord(level_event(b.lev_begin, lvl), s));
     hipLaunchKernelGGL(k_bu, dim3(grid_of((b.words + a.span - 1) / a.span, kBlock / 64, 8192)), dim3(kBlock), 0, s, a,
-                       state.cur, lvl, cnt);
+                       state.cur, lvl, cnt, b.stamp.p);
     G5_HIP(hipGetLastError());
-    G5_HIP(hipEventRecord(level_event(b.lev_end, lvl), s));
     ++b.pub_seq;
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, (int64_t)0, 0, b.pub.d, b.pub_seq);
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, cnt, b.prefix.p, (int64_t)0, 0, b.pub.d, b.pub_seq,
+                       b.stamp.p);
     G5_HIP(hipGetLastError());
     wait_published(b, s);
     const int64_t nq = (int64_t)b.h_counters[C_FOUND];
     st.direction[lvl] = state.forward;
     st.bu_kernel[lvl] = 1;
     st.nq[lvl] = nq;
+    st.level_ms[lvl] = (double)b.h_counters[C_NUM] / (double)b.tick_khz;
     st.num_levels = lvl + 1;
     state.cur ^= 1;
     state.queued = 0;
     step_fold(g.n_active, state, nq);
-  }
-  for (int l = lvl0; l <= state.lvl; ++l) {
-    float lms = 0;
-    G5_HIP(hipEventSynchronize(b.lev_end[l]));
-    G5_HIP(hipEventElapsedTime(&lms, b.lev_begin[l], b.lev_end[l]));
-    st.level_ms[l] = lms;
   }
   state.stop = STEP_GO;
   if (state.nf && state.forward) queue_from_bitmaps(b, s, state);

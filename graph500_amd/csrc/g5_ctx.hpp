@@ -57,18 +57,6 @@ struct HostStage {
   }
 };
 
-// Events of a run's levels, created as levels are first reached.
-inline hipEvent_t level_event(std::vector<hipEvent_t>& v, int l) {
-  if ((int)v.size() <= l) v.resize(l + 1, nullptr);
-  if (!v[l]) G5_HIP(hipEventCreate(&v[l]));
-  return v[l];
-}
-inline void destroy_events(std::vector<hipEvent_t>& v) {
-  for (auto e : v)
-    if (e) (void)hipEventDestroy(e);
-  v.clear();
-}
-
 // Single-root BFS state.
 struct BfsState {
   bool prepared = false;
@@ -115,7 +103,7 @@ struct BfsState {
   int64_t hub_rows = 0;           // rows [0, hub_rows) are indexed
   DevBuf<uint32_t> hub_bnd;       // hub_rows * hub_pieces
   g5_bfs_stats stats{};
-  std::vector<hipEvent_t> lev_begin, lev_end;  // per level run from the host
+  DevBuf<uint64_t> stamp;         // device clock at the start of a level run from the host
   // the tuning (g5_bfs_set_tuning's fields) of another state
   void copy_tuning(const BfsState& o) {
     small_edges = o.small_edges;
@@ -146,17 +134,13 @@ struct BfsState {
     seg_count.release();
     seg_scan_tmp.release();
     seg_start.release();
+    stamp.release();
     hub_bnd.release();
     hub_built_shift = 0;
     prepared = false;
     have_result = false;
   }
-  // events and published blocks stay with the state from one graph to the next
-  ~BfsState() {
-    destroy_events(lev_begin);
-    destroy_events(lev_end);
-  }
-};
+};  // the published blocks stay with the state from one graph to the next
 
 // Batched (up to 64 roots) BFS state.
 struct MsState {

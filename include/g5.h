@@ -72,8 +72,8 @@ typedef struct g5_bfs_stats {
   int32_t num_levels;               /* levels executed + 1 (last level finds nothing) */
   int32_t direction[G5_MAX_LEVELS]; /* 1 = top-down, 0 = bottom-up */
   int64_t nq[G5_MAX_LEVELS];        /* vertices discovered at that level */
-  double level_ms[G5_MAX_LEVELS];   /* device time of each level's kernels (device clock or HIP events) */
-  double device_ms;                 /* device time of the whole run (HIP events) */
+  double level_ms[G5_MAX_LEVELS];   /* device time of each level's kernels (device clock) */
+  double device_ms;                 /* device time of the whole run (device clock) */
   int64_t reached;                  /* vertices with a level, root included */
   int32_t bu_kernel[G5_MAX_LEVELS]; /* 1 = the level's vertices were found by the bottom-up kernel
                                        (every bottom-up level, and the top-down levels tail_pull
