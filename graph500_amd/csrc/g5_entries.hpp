@@ -42,6 +42,8 @@ constexpr int kCursorPad = 8;   // a bucket cursor has a 64-byte line of its own
 constexpr int kSubMax = 8192;     // sub-buckets of one L1 bucket
 constexpr int kFracMax = 6401;    // entries of the column share table
 constexpr int kDegVerts = 32768;  // vertices counted by one workgroup (128 KB of LDS)
+constexpr int kDegLoads = 4;      // 16-byte loads in flight per thread there
+constexpr int kDegBatch = 1024 * 2 * kDegLoads;
 constexpr int kDegBits = 28;      // low bits of a row word (k_row_words): its degree
 constexpr uint64_t kDegMask = (UINT64_C(1) << kDegBits) - 1;
 
@@ -395,7 +397,15 @@ __global__ void __launch_bounds__(kPartMax) k_part_offsets(const unsigned long l
 
 // Degrees (duplicates counted) of the vertices [base, base + 2^sub_shift):
 // their bucket's entries counted in LDS.  A bucket of more than kDegVerts
-// vertices takes several workgroups, each reading the whole bucket.
+// vertices takes several workgroups, each reading the whole bucket; 8 apart
+// in the grid, they run on one XCD at the same time and all but the first
+// find the entries in its L2 (there are 1024 buckets then, a multiple of 8).
+// Bound by the loads in flight: with 128 KB of LDS there are 16 waves on a CU,
+// so a thread has four 16-byte loads under way.  Against one 8-byte load after
+// another and the parts of a bucket next to each other in the grid: SCALE 18
+// 67 -> 56 us, 22 0.56 -> 0.36 ms, 25 2.94 -> 1.71 ms (5.0 TB/s), 26 (2 parts)
+// 9.6 -> 3.6 ms, 28 (8 parts) 131.6 -> 31.7 ms (17 TB/s out of the L2; 83 ms
+// with the parts next to each other, 36 ms with 8 loads, 33 ms with 16).
 __global__ void __launch_bounds__(1024) k_bucket_degrees(const uint64_t* __restrict__ in,
                                                          const uint64_t* __restrict__ off, int shift, int sub_shift,
                                                          int64_t n, uint32_t* __restrict__ deg,
@@ -403,18 +413,40 @@ __global__ void __launch_bounds__(1024) k_bucket_degrees(const uint64_t* __restr
   __shared__ uint32_t s[kDegVerts];
   __shared__ uint32_t s_red[2];
   const int t = threadIdx.x;
-  const int64_t bucket = (int64_t)blockIdx.x >> (shift - sub_shift);
+  const int parts = shift - sub_shift;  // log2 of the workgroups per bucket
+  uint32_t bucket = blockIdx.x, part = 0;
+  if (parts) {
+    bucket = (blockIdx.x >> (3 + parts) << 3) + (blockIdx.x & 7);
+    part = blockIdx.x >> 3 & ((1u << parts) - 1);
+  }
   const uint32_t width = 1u << sub_shift;
-  const uint32_t base = (uint32_t)((uint64_t)blockIdx.x << sub_shift);
+  const uint32_t base = (bucket << shift) + (part << sub_shift);
   for (uint32_t i = t; i < width; i += 1024) s[i] = 0;
   if (t < 2) s_red[t] = 0;
   __syncthreads();
   const uint64_t end = off[bucket + 1];
-#pragma unroll 4
-  for (uint64_t i = off[bucket] + t; i < end; i += 1024) {
-    const uint32_t d = (uint32_t)(in[i] >> 32) - base;
+  const auto count = [&](uint64_t e) {
+    const uint32_t d = (uint32_t)(e >> 32) - base;
     if (d < width) atomicAdd(&s[d], 1u);
+  };
+  uint64_t at = off[bucket];
+  if ((at & 1) && at < end) {  // to a 16-byte boundary
+    if (t == 0) count(in[at]);
+    ++at;
   }
+  for (; at + kDegBatch <= end; at += kDegBatch) {
+    const ulonglong2* p = (const ulonglong2*)(in + at) + t;
+    ulonglong2 e[kDegLoads];
+#pragma unroll
+    for (int j = 0; j < kDegLoads; ++j) e[j] = p[j * 1024];
+#pragma unroll
+    for (int j = 0; j < kDegLoads; ++j) {
+      count(e[j].x);
+      count(e[j].y);
+    }
+  }
+#pragma unroll 4
+  for (at += t; at < end; at += 1024) count(in[at]);
   __syncthreads();
   uint32_t mx = 0, act = 0;
   for (uint32_t i = t; i < width; i += 1024) {

@@ -82,6 +82,19 @@ def test_many_copies_of_one_tuple(ctx, copies, mode):
     check(ctx, a, b, mode, "copies %d" % copies)
 
 
+@pytest.mark.parametrize("scale", [25, 26, 27])
+def test_degrees_of_wide_ranges(ctx, scale):
+    """One, two and four workgroups count a range of ids; ranges of entries
+    below, at and beyond a workgroup's batch (8,192), from odd places on."""
+    rng = np.random.default_rng(scale)
+    n, width = 1 << scale, 1 << (scale - 10)
+    sizes = [1, 8190, 8191, 8192, 8193, 16385, 3, 24575, 40001]
+    a = np.concatenate([rng.integers(k * 7 * width, (k * 7 + 1) * width, size) for k, size in enumerate(sizes)])
+    a = np.append(a, [n - 1, 70 * width, 71 * width - 1])
+    b = rng.integers(100 * width, n, len(a))
+    check(ctx, a, b, 1, "wide %d" % scale)
+
+
 @pytest.mark.parametrize("mode", [0, 2])
 def test_only_loops_and_loops_between(ctx, mode):
     a = np.array([3, 3, 5], np.int64)
