@@ -624,6 +624,8 @@ __global__ void __launch_bounds__(1024) k_refine(const uint64_t* __restrict__ in
   }
 }
 
+typedef uint16_t half_word __attribute__((may_alias));  // bins are counted by pairs, read one by one
+
 // One workgroup per sub-bucket: its entries sorted by (position, column) in
 // LDS and deduplicated; the unique columns replace the entries in place (as
 // uint32 from the sub-bucket's first byte on).  A bin is one position, so the
@@ -631,8 +633,14 @@ __global__ void __launch_bounds__(1024) k_refine(const uint64_t* __restrict__ in
 // about one entry each, so the ranking takes a couple of LDS reads per entry.
 // Unique counts per row: a stored value for a row that lies inside the
 // sub-bucket, an atomic add for the rows that cross its ends.  A sub-bucket
-// may hold twice its positions; the register bound keeps four workgroups of
-// 2^11 positions per CU (the compiler's own choice left one).
+// may hold twice its positions; the register bound keeps at least four
+// workgroups of 2^11 positions per CU (the compiler's own choice left one).
+// Bound by LDS operations, so neighbouring lanes take neighbouring words: the
+// bins are 16-bit counts, eight in one uint4 a thread, and places are numbered
+// by groups of 64 (a ballot and a scan of the groups).  With 32-bit bins and
+// sixteen consecutive places a thread, 8 and 16 lanes met in a bank: SCALE 20
+// 221 -> 183 us, 22 0.82 -> 0.66 ms, 25 6.42 -> 5.03 ms (2.6 TB/s), 27 30.9 ->
+// 25.6 ms.  Ranking two or four entries of a thread at once: 2 % slower.
 template <int kSub>
 struct SubSort {
   static constexpr int kWidth = 1 << kSub, kCap = 2 * kWidth, kPer = 16, kThreads = kCap / kPer;
@@ -646,8 +654,12 @@ __global__ void __launch_bounds__(SubSort<kSub>::kThreads, 4)
   constexpr int kWidth = SubSort<kSub>::kWidth, kCap = SubSort<kSub>::kCap, kPer = SubSort<kSub>::kPer;
   constexpr int kThreads = SubSort<kSub>::kThreads;
   constexpr int kBins = kWidth / kThreads;  // bins per thread in the scan
+  constexpr int kGroups = kCap / 64;
+  __shared__ uint32_t s_g[kGroups];
   __shared__ uint32_t s_col[kCap];
-  __shared__ uint32_t s_start[kWidth + 1];
+  __shared__ uint4 s_bins[kWidth / 8 + 1];  // entries per bin, then first places: 16 bits each
+  half_word* const s_start = reinterpret_cast<half_word*>(s_bins);
+  uint32_t* const s_pair = reinterpret_cast<uint32_t*>(s_bins);
   __shared__ uint16_t s_up[kCap + 1];  // unique flags, then unique entries before a place
   __shared__ uint32_t s_w[kThreads / 64];
   const uint32_t sub = blockIdx.x;
@@ -663,8 +675,8 @@ __global__ void __launch_bounds__(SubSort<kSub>::kThreads, 4)
   }
   const uint64_t off = sub_off[sub], pos = sub_pos[sub], pos_end = sub_pos[sub + 1];
   const int64_t row0 = sub_row[sub];
-#pragma unroll
-  for (int j = 0; j < kBins; ++j) s_start[j * kThreads + t] = 0;
+  static_assert(kBins == 8, "a thread's bins are one uint4");
+  s_bins[t] = uint4{0, 0, 0, 0};
   __syncthreads();
   uint32_t col[kPer], br[kPer];  // bin << 16 | arrival in the bin
 #pragma unroll
@@ -676,22 +688,25 @@ __global__ void __launch_bounds__(SubSort<kSub>::kThreads, 4)
   }
 #pragma unroll
   for (int j = 0; j < kPer; ++j)
-    if ((uint32_t)(j * kThreads + t) < cnt) br[j] = (br[j] << 16) | atomicAdd(&s_start[br[j]], 1u);
+    if ((uint32_t)(j * kThreads + t) < cnt) {
+      const uint32_t at = br[j] & 1 ? 16 : 0, old = atomicAdd(&s_pair[br[j] >> 1], 1u << at);
+      br[j] = (br[j] << 16) | (old >> at & 0xFFFF);
+    }
   __syncthreads();
   {
-    uint32_t c[kBins], sum = 0, total;
+    const uint4 c = s_bins[t];
+    uint32_t w[4] = {c.x, c.y, c.z, c.w}, sum = 0, total;
 #pragma unroll
-    for (int j = 0; j < kBins; ++j) {
-      c[j] = s_start[t * kBins + j];
-      sum += c[j];
-    }
+    for (int j = 0; j < 4; ++j) sum += (w[j] & 0xFFFF) + (w[j] >> 16);
     uint32_t run = block_excl_scan32<kThreads>(sum, s_w, total);
 #pragma unroll
-    for (int j = 0; j < kBins; ++j) {
-      s_start[t * kBins + j] = run;
-      run += c[j];
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t odd = run + (w[j] & 0xFFFF), next = odd + (w[j] >> 16);
+      w[j] = run | odd << 16;
+      run = next;
     }
-    if (t == 0) s_start[kWidth] = cnt;
+    s_bins[t] = uint4{w[0], w[1], w[2], w[3]};
+    if (t == 0) s_start[kWidth] = (half_word)cnt;
   }
   __syncthreads();
 #pragma unroll
@@ -720,24 +735,33 @@ __global__ void __launch_bounds__(SubSort<kSub>::kThreads, 4)
       s_up[br[j] >> 1] = (uint16_t)(br[j] & 1);
     }
   __syncthreads();
-  // unique entries before every place; kPer consecutive places per thread
-  uint32_t flags = 0, total;
+  // unique entries before every place, counted by groups of 64 places
+  uint32_t flags = 0, total = 0;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const uint32_t p = t * kPer + j;
-    if (p < cnt) {
+    const uint32_t p = j * kThreads + t;
+    const bool u = p < cnt && s_up[p];
+    if (u) {
       col[j] = s_col[p];
-      flags |= (uint32_t)s_up[p] << j;
+      flags |= 1u << j;
     }
+    const uint64_t m = __ballot(u);
+    br[j] = __popcll(m & ((UINT64_C(1) << (t & 63)) - 1));
+    if ((t & 63) == 0) s_g[p >> 6] = (uint32_t)__popcll(m);
   }
-  // its barriers: every flag and column has been read
-  uint32_t run = block_excl_scan32<kThreads>(__popc(flags), s_w, total);
+  __syncthreads();
+  {
+    const uint32_t v = t < kGroups ? s_g[t] : 0, before = block_excl_scan32<kThreads>(v, s_w, total);
+    if (t < kGroups) s_g[t] = before;
+  }
+  __syncthreads();
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const uint32_t p = t * kPer + j;
+    const uint32_t p = j * kThreads + t;
     if (p < cnt) {
+      const uint32_t run = s_g[p >> 6] + br[j];
       s_up[p] = (uint16_t)run;
-      if ((flags >> j) & 1) s_col[run++] = col[j];
+      if ((flags >> j) & 1) s_col[run] = col[j];
     }
   }
   if (t == 0) {
