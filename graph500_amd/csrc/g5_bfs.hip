@@ -22,23 +22,24 @@
 //              the row suffixes beyond them (k_td_expand_segs).
 //              After the bottom-up phase, a top-down level whose frontier is
 //              large against the unvisited vertices is found by the bottom-up
-//              kernel (same vertices, far fewer probes); consecutive small
-//              top-down levels run fused in one single-workgroup launch
-//              (k_td_fused) that applies the switch rule itself.
-//   host loop  one round trip per level: a one-lane kernel publishes the
-//              level's counters to coherent host memory, each value tagged
-//              with the level's sequence number, where the host reads them
-//              for the alpha/beta rule.
+//              kernel (same vertices, far fewer probes).
+//   steps      k_bfs_step: one launch per level, whose workgroups all apply
+//              the switch rule to the last level's counts, so that no level
+//              waits for the host; it runs small and mid top-down levels and,
+//              on graphs up to kStepMaxWords bitmap words, bottom-up levels.
+//   host loop  the other levels: a one-wave kernel publishes the level's
+//              counters to coherent host memory, each value tagged with the
+//              level's sequence number, where the host reads them for the
+//              alpha/beta rule.
 //   queues     a top-down frontier that comes from a bitmap is rebuilt by an
 //              exclusive scan of per-word popcounts (ascending vertex order).
-//   bottom-up  k_bu: one wave per two 64-vertex bitmap words, one lane per
-//              vertex of each (both words' first probes in flight together).
-//              Unvisited lanes first probe their first (highest-degree)
-//              neighbour from the coalesced first_nbr array; misses with a
-//              short row scan it lane-sequentially, long rows are scanned by
-//              the whole wave 64 entries at a time with a ballot for the first
-//              hit.  The visited snapshot of the previous level is read-only;
-//              the next bitmap word is written once per wave from a ballot.
+//   bottom-up  step_bottom_up (in steps and in k_bu): a wave takes up to 16
+//              64-vertex bitmap words a turn.  Unvisited vertices first probe
+//              their first (highest-degree) neighbour from the coalesced
+//              first_nbr array, four words in flight; the rows of those who
+//              missed are searched with every lane busy.  The visited snapshot
+//              of the previous level is read-only; the next bitmap's words are
+//              written once per turn.
 #include "g5_answers.hpp"
 #include "g5_ctx.hpp"
 #include "g5_frontier.hpp"

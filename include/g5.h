@@ -120,7 +120,8 @@ typedef struct g5_batch_tuning {
   double filter_from;      /* pull_filter 2 threshold, a fraction of the rows */
   int32_t pull_unroll;     /* probes in flight per lane in the per-level pulls: 0 = 4 per short-row step
                               and 2 per long-row step, 1 = 8/2, 2 = 8/4, 3 = 4/4, 4 = 2/1, 5 = 1/1,
-                              6 = 2/2, 7 = 1/2 */
+                              6 = 2/2, 7 = 1/2 (rows over 8 entries are searched by groups of
+                              16 lanes first, very long ones by whole waves after that) */
   int32_t lane_rule;       /* 0: one direction per level for all roots (the rule on alpha above);
                               1: a direction per root and level (per-level launches, reorder modes
                               1 and 2): a root pulls when its frontier's edges exceed 1/alpha of the
