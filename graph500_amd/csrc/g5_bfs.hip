@@ -1939,6 +1939,7 @@ static bool step_alone(const Graph& g, const BfsState& b) {
 // every wave the same number of turns; for k_bu, 8, or 16 where a wave still
 // has ten turns or more (S26 8/16: 674/685 us a search, S28: 2,521/2,469, before rows went to groups).
 static int bottom_up_span(const Graph& g, const BfsState& b) {
+  if (b.words == 0) return 1;  // a graph without rows has no turns to share out
   if (b.words > kStepMaxWords) return b.words >= (INT64_C(1) << 20) ? 16 : 8;
   const int64_t waves = (step_alone(g, b) ? 1 : kStepTdGrid) * (kStepThreads / 64);
   const int64_t turns = (b.words + waves * kBuSpan - 1) / (waves * kBuSpan);
