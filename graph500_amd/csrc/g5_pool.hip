@@ -73,14 +73,15 @@ hipError_t pool_alloc(void** p, size_t bytes) {
     }
   }
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && pl && !pl->kept.empty()) {
-    trim(*pl, 0);
-    e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // or a launch's check finds it, though the next try succeeds
+    if (pl && !pl->kept.empty()) {
+      trim(*pl, 0);
+      e = hipMalloc(p, bytes);
+      if (e != hipSuccess) (void)hipGetLastError();
+    }
   }
-  if (e == hipSuccess)
-    g_live[*p] = {bytes, dev};
-  else
-    (void)hipGetLastError();
+  if (e == hipSuccess) g_live[*p] = {bytes, dev};
   return e;
 }
 

@@ -1,0 +1,183 @@
+// Checks of the block pool (g5_pool.hip) on the CPU; argv[1] names one.
+#include "g5_internal.hpp"
+
+#include <stdlib.h>
+#include <string.h>
+
+#include <map>
+#include <mutex>
+
+namespace {
+
+constexpr size_t kTotal = 8000;  // the pool keeps up to an eighth
+std::mutex mu;
+std::map<void*, size_t> blocks;
+size_t used;
+int mallocs, frees, waits;
+thread_local int device;
+thread_local hipError_t last;
+uintptr_t next_p = 0x1000;
+
+}  // namespace
+
+const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "out of memory"; }
+hipError_t hipMalloc(void** p, size_t bytes) {
+  std::lock_guard<std::mutex> lk(mu);
+  ++mallocs;
+  if (used + bytes > kTotal) return last = hipErrorOutOfMemory;
+  *p = (void*)next_p;
+  next_p += 0x1000;
+  blocks[*p] = bytes;
+  used += bytes;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lk(mu);
+  ++frees;
+  const auto it = blocks.find(p);
+  if (it == blocks.end()) {
+    fprintf(stderr, "freed twice\n");
+    abort();
+  }
+  used -= it->second;
+  blocks.erase(it);
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* dev) {
+  *dev = device;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() {
+  ++waits;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = last;
+  last = hipSuccess;
+  return e;
+}
+hipError_t hipMemGetInfo(size_t* free_b, size_t* total_b) {
+  *free_b = kTotal - used;
+  *total_b = kTotal;
+  return hipSuccess;
+}
+
+using namespace g5;
+
+#define CHECK(x)                                              \
+  do {                                                        \
+    if (!(x)) {                                               \
+      fprintf(stderr, "line %d: %s\n", __LINE__, #x);         \
+      exit(1);                                                \
+    }                                                         \
+  } while (0)
+
+static void* get(size_t bytes) {
+  void* p = nullptr;
+  CHECK(pool_alloc(&p, bytes) == hipSuccess && p);
+  return p;
+}
+
+// A request takes the smallest kept block it fills to 4/5.
+static void sizes() {
+  pool_context(0, 1);
+  void *a = get(500), *b = get(450);
+  pool_free(a);
+  pool_free(b);
+  CHECK(frees == 0 && waits == 2 && used == 950);
+  CHECK(get(400) == b);
+  CHECK(get(400) == a);
+  void* c = get(399);
+  CHECK(c != a && c != b && mallocs == 3);
+  pool_free(a);
+  CHECK(get(501) != a);
+  CHECK(get(399) != a);
+  CHECK(get(500) == a);
+}
+
+// At most an eighth is kept: older blocks go back first, a larger one at once.
+static void bound() {
+  pool_context(0, 1);
+  void *a = get(400), *b = get(410), *c = get(420), *d = get(1001);
+  pool_free(a);
+  pool_free(b, true);
+  CHECK(waits == 1);
+  pool_free(c);
+  CHECK(frees == 1 && blocks.count(a) == 0 && blocks.count(b) == 1);
+  pool_free(d);
+  CHECK(blocks.count(d) == 0 && used == 830);
+}
+
+// A request the device cannot fill takes back what is kept, and leaves no
+// error for the next call's check to find; one beyond that fails, likewise.
+static void refill() {
+  pool_context(0, 1);
+  void *a = get(900), *b = get(6900);
+  pool_free(a);
+  CHECK(used == 7800);
+  void* c = get(1000);
+  CHECK(hipGetLastError() == hipSuccess);
+  CHECK(blocks.count(a) == 0 && used == 7900);
+  void* d = nullptr;
+  CHECK(pool_alloc(&d, 200) == hipErrorOutOfMemory);
+  CHECK(hipGetLastError() == hipSuccess);
+  pool_free(b);
+  pool_free(c);
+}
+
+// Nothing is kept without a context, beside other devices, or past the last one.
+static void contexts() {
+  void* a = get(100);
+  pool_free(a);
+  CHECK(blocks.empty());
+  pool_context(0, 1);
+  pool_context(0, 1);
+  pool_context(1, 1);
+  a = get(100);
+  device = 1;
+  pool_free(a);
+  CHECK(blocks.empty());
+  a = get(100);
+  pool_free(a);
+  device = 0;
+  void* b = get(100);
+  CHECK(b != a);
+  pool_free(b);
+  pool_context(0, -1);
+  CHECK(used == 200);
+  pool_context(0, -1);
+  CHECK(used == 100);
+  pool_context(1, -1);
+  CHECK(blocks.empty());
+}
+
+// The wrapper: a buffer that cannot be had is an error of the library, and
+// what it held before has gone back.
+static void buffer() {
+  pool_context(0, 1);
+  DevBuf<uint64_t> x;
+  x.alloc(100);
+  const void* p = x.p;
+  x.alloc(90);
+  CHECK(x.p == p && x.bytes() == 800);
+  try {
+    x.alloc(2000);
+    CHECK(false);
+  } catch (const Error& e) {
+    CHECK(e.code == G5_ERR_MEM);
+  }
+  CHECK(!x.p && x.n == 0 && hipGetLastError() == hipSuccess && blocks.empty());
+}
+
+int main(int argc, char** argv) {
+  const struct {
+    const char* name;
+    void (*f)();
+  } checks[] = {{"sizes", sizes}, {"bound", bound}, {"refill", refill}, {"contexts", contexts}, {"buffer", buffer}};
+  for (const auto& c : checks)
+    if (argc > 1 && !strcmp(argv[1], c.name)) {
+      c.f();
+      return 0;
+    }
+  return 2;
+}
