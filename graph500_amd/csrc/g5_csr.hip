@@ -348,24 +348,22 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     uint32_t *kp = k0.p, *ka = k1.p, *vp = g.new2old.p, *va = v1.p;
     radix_sort_pairs_u32(&kp, &ka, &vp, &va, (size_t)n, 0, bits, rs, s);
     if (vp != g.new2old.p) g.new2old.swap(v1);
-    if (!small) {  // the memory is needed below
-      G5_HIP(hipStreamSynchronize(s));
-      k0.drop();
-      k1.drop();
-      v1.drop();
-    }
   }
   const int64_t rows = g.n_rows;
   g.weight.alloc(rows);
-  g.offsets.alloc(rows + 1);
   DevBuf<uint32_t> row_cnt;  // degrees with duplicates, then unique entries per row
-  DevBuf<uint64_t> P, tmp;   // degree prefix: P[r] = entries of the rows before r
   row_cnt.alloc(rows + 1);
-  P.alloc(rows + 1);
-  tmp.alloc(scan_tmp_elems(rows + 1));
   hipLaunchKernelGGL(k_row_info, dim3(grid_for(rows + 1)), dim3(kBlock), 0, s, g.new2old.p, deg.p,
                      g.self_loops ? loops.p : nullptr, rows, row_cnt.p, g.weight.p);
   G5_HIP(hipGetLastError());
+  if (!small) {  // the memory is needed below
+    G5_HIP(hipStreamSynchronize(s));
+    for (DevBuf<uint32_t>* b : {&k0, &k1, &v1, &deg, &loops}) b->drop();
+  }
+  g.offsets.alloc(rows + 1);
+  DevBuf<uint64_t> P, tmp;  // degree prefix: P[r] = entries of the rows before r
+  P.alloc(rows + 1);
+  tmp.alloc(scan_tmp_elems(rows + 1));
   device_scan(LoadU32{row_cnt.p}, StoreU64{P.p}, (size_t)rows + 1, tmp.p, s);
   DevBuf<uint64_t> row_word;
   row_word.alloc(n);
@@ -380,6 +378,15 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   DevBuf<uint64_t> sub64;  // first position | first entry | first unique column
   DevBuf<uint32_t> sub32;  // entries | first row | unique columns | L1 first sub-buckets | column shares
   DevBuf<uint64_t> stmp;
+  // Before the columns are allocated: all scratch but the sorted entries in
+  // `kept`, once nothing in flight reads it (at SCALE 28, edgefactor 16, the
+  // peak is 145 GB instead of 181).
+  const auto drop_idle = [&](const uint64_t* kept) {
+    if (small) return;
+    (kept == xa.p ? xb : xa).drop();
+    row_word.drop();
+    P.drop();
+  };
   if (E == 0) {
     g.cols.alloc(0);
     G5_HIP(hipMemsetAsync(g.offsets.p, 0, (rows + 1) * 8, s));
@@ -439,6 +446,7 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     read_info(kPubOr + I_NUM + 1, I_NUM + 1);
     nnz = pub.value(kPubOr + 2 * I_NUM + 1);
     if (!h_info[I_WIDE] && !h_info[I_OVERFLOW]) {
+      drop_idle(refined);
       g.cols.alloc(nnz);
       hipLaunchKernelGGL(k_compact, dim3((unsigned)max_subs), dim3(kBlock), 0, s, refined, sub_off, sub_unique, out_off,
                          info, g.cols.p);
@@ -454,6 +462,7 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
       radix_sort_u64(&kp, &ka, E, 32, 32 + scale, rs, s);
       const UniqueFlag flag{kp, (size_t)E};
       nnz = device_reduce_sum(flag, E, ctx->acc.p, s);
+      drop_idle(kp);
       g.cols.alloc(nnz);
       stmp.alloc(scan_tmp_elems(E));
       device_scan(flag, UniqueStore{kp, (size_t)E, 32, g.cols.p, g.offsets.p}, E, stmp.p, s);
