@@ -1570,7 +1570,8 @@ __global__ void __launch_bounds__(kBlock) k_bfs_init(const uint32_t* __restrict_
                                                      int64_t rows, int64_t words, uint8_t* __restrict__ level,
                                                      uint32_t* __restrict__ parent, uint64_t* __restrict__ vis,
                                                      uint32_t* __restrict__ queue, unsigned long long* __restrict__ ctl,
-                                                     unsigned long long* __restrict__ counters, StepArgs args) {
+                                                     unsigned long long* __restrict__ counters, StepArgs args,
+                                                     int active) {
   const int64_t stride = (int64_t)gridDim.x * kBlock, me = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t r = old2new[root_orig];  // >= rows for a root without edges (modes 1 and 2)
   for (int64_t q = me; q * 16 < rows; q += stride) {
@@ -1595,7 +1596,8 @@ __global__ void __launch_bounds__(kBlock) k_bfs_init(const uint32_t* __restrict_
       *reinterpret_cast<StepArgs*>(ctl + kStepArgs) = args;
       StepState st{};
       st.forward = st.growing = st.queued = 1;
-      st.nf = st.visited = 1;
+      st.nf = active;  // a root without edges is the whole tree: the first step finds the end
+      st.visited = 1;
       *reinterpret_cast<StepState*>(ctl + kStepState + kStateWords) = st;  // the slot step 0 reads
       if (r < rows) {
         parent[r] = (uint32_t)r;
@@ -2028,20 +2030,14 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   a.span = bottom_up_span(g, b);
   a.share = b.words <= kStepShareWords;
   const unsigned grid = step_grid(g, b, a.span);
-  hipLaunchKernelGGL(k_bfs_init, dim3(grid_of((rows + 15) / 16, kBlock, 2048)), dim3(kBlock), 0, s, g.old2new.p, root,
-                     rows, b.words, b.level.p, b.parent.p, b.vis[0].p, b.queue[0].p,
-                     (unsigned long long*)b.step_ctl.p, cnt, a);
-  G5_HIP(hipGetLastError());
-
   // A root without edges (reachable only through a find_roots fallback) is
   // the whole tree: the reference's first top-down level finds nothing.
   const bool root_active = (g.has_edge_words[root >> 6] >> (root & 63)) & 1;
-  if (!root_active) {
-    st.num_levels = 2;
-    st.direction[1] = 1;
-    st.nq[1] = 0;
-    G5_HIP(hipStreamSynchronize(s));
-  }
+  hipLaunchKernelGGL(k_bfs_init, dim3(grid_of((rows + 15) / 16, kBlock, 2048)), dim3(kBlock), 0, s, g.old2new.p, root,
+                     rows, b.words, b.level.p, b.parent.p, b.vis[0].p, b.queue[0].p,
+                     (unsigned long long*)b.step_ctl.p, cnt, a, root_active ? 1 : 0);
+  G5_HIP(hipGetLastError());
+
   StepState state{};
   state.visited = 1;
   int steps = 0;
@@ -2050,7 +2046,7 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     return !state.forward ||
            tail_pulls(1, state.growing, b.tail_pull, state.nf, g.n_active - state.visited);
   };
-  while (root_active) {
+  for (;;) {
     if (resume && state.nf && a.host_bu && bottom_up_next() && state.lvl < kStepMaxLevel) {
       host_bottom_up(ctx, b, s, a, state);
       continue;
@@ -2072,6 +2068,10 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     if (!state.queued && stop != STEP_BOTTOM_UP) queue_from_bitmaps(b, s, state);
     if (stop == STEP_LARGE) large_top_down(ctx, b, s, state);
     state.edges = 0;
+  }
+  if (!root_active) {  // the level that finds nothing was not run
+    st.num_levels = 2;
+    st.direction[1] = 1;
   }
   st.reached = state.visited;
   b.have_result = true;
