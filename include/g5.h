@@ -141,7 +141,12 @@ typedef struct g5_batch_tuning {
 /* ---- context ---- */
 const char* g5_version(void);
 int g5_device_count(int* count);
-/* Creates a context on HIP device 'device' with its own stream. */
+/* Creates a context on HIP device 'device' with its own stream.
+ * While a context exists on a device, up to an eighth of the device's memory
+ * stays with the library after it was freed (scratch of a construction, the
+ * arrays of a graph that was replaced), for its own later requests: other
+ * users of the device find that much less free.  It goes back when a request
+ * of the library is refused, and whole with the device's last context. */
 int g5_create(int device, g5_ctx** out);
 /* Frees the context and everything it holds.  Returns G5_ERR_STATE, and
  * frees nothing, while a g5_server created over the context still exists

@@ -4,6 +4,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <functional>
+#include <future>
 #include <map>
 #include <mutex>
 
@@ -17,6 +19,13 @@ int mallocs, frees, waits;
 thread_local int device;
 thread_local hipError_t last;
 uintptr_t next_p = 0x1000;
+std::function<void()> on_wait;  // runs while a call waits for the device (a free waits for it too)
+
+void wait_for_device() {
+  std::function<void()> f;
+  std::swap(f, on_wait);
+  if (f) f();
+}
 
 }  // namespace
 
@@ -32,6 +41,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+  wait_for_device();
   std::lock_guard<std::mutex> lk(mu);
   ++frees;
   const auto it = blocks.find(p);
@@ -49,6 +59,7 @@ hipError_t hipGetDevice(int* dev) {
 }
 hipError_t hipDeviceSynchronize() {
   ++waits;
+  wait_for_device();
   return hipSuccess;
 }
 hipError_t hipGetLastError() {
@@ -151,6 +162,40 @@ static void contexts() {
   CHECK(blocks.empty());
 }
 
+// While one thread waits for the device (a free, a block that goes back to the
+// driver, the last context), others get and return blocks; none of it is lost.
+static void threads() {
+  bool ran = false;
+  const auto other_goes_on = [&ran] {
+    ran = true;
+    auto f = std::async(std::launch::async, [] { pool_free(get(50), true); });
+    if (f.wait_for(std::chrono::seconds(5)) == std::future_status::timeout) {
+      fprintf(stderr, "a request waited for another thread's wait for the device\n");
+      _Exit(1);
+    }
+  };
+  const auto check = [&](const std::function<void()>& call) {
+    ran = false;
+    on_wait = other_goes_on;
+    call();
+    CHECK(ran && !on_wait);
+  };
+  pool_context(0, 1);
+  pool_free(get(50));
+  void *a = get(500), *b = get(600), *c = get(5000);
+  check([&] { pool_free(a); });        // kept
+  check([&] { pool_free(b, true); });  // kept, a goes back
+  CHECK(blocks.count(a) == 0 && blocks.count(b) == 1);
+  check([&] { pool_free(c); });        // too large to be kept
+  CHECK(blocks.count(c) == 0);
+  c = get(7250);
+  check([&] { pool_free(get(640)); });  // the kept blocks go back and the request succeeds
+  CHECK(blocks.count(b) == 0 && hipGetLastError() == hipSuccess);
+  pool_free(c);
+  check([&] { pool_context(0, -1); });
+  CHECK(used <= 50);  // what the other thread may have kept before the context was gone
+}
+
 // The wrapper: a buffer that cannot be had is an error of the library, and
 // what it held before has gone back.
 static void buffer() {
@@ -173,7 +218,8 @@ int main(int argc, char** argv) {
   const struct {
     const char* name;
     void (*f)();
-  } checks[] = {{"sizes", sizes}, {"bound", bound}, {"refill", refill}, {"contexts", contexts}, {"buffer", buffer}};
+  } checks[] = {{"sizes", sizes}, {"bound", bound}, {"refill", refill}, {"contexts", contexts}, {"buffer", buffer},
+                {"threads", threads}};
   for (const auto& c : checks)
     if (argc > 1 && !strcmp(argv[1], c.name)) {
       c.f();
