@@ -367,6 +367,15 @@ constexpr int64_t kListGrid = 2048;
 constexpr int64_t kPartWords = 4096;
 constexpr int64_t kPartWordsFirst = 12288;
 
+// Below this many entries a level costs its launches, two for a pull and four
+// for a push, and a root pulls by its own frontier alone (lane_rule 1): long
+// graphs never have a union large enough (2 and 8 roots, us, with the union
+// rule and without: a path of 200 6,214 / 6,047 and 3,382 / 4,142, 128 x 1,024
+// vertices in a grid with chords 3,998 / 7,038 and 2,811 / 3,838), Kronecker
+// graphs up to S18 are equal; S19 with 8 roots 218 with, 251 without, S23 811
+// and 894.
+constexpr int64_t kUnionFrom = INT64_C(1) << 22;
+
 // A push level lists the vertices it touches when its frontier edges times
 // this are fewer than the rows (the touched vertices are at most the edges).
 constexpr double kTouchBelow = 8.0;
@@ -1044,13 +1053,14 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       // reached (the roots' own level pushes; all pull in the beta tail); a
       // root that has pulled keeps pulling, so once every live root pulls
       // the level is a plain pull with no per-root statistics
-      // A level pulls only when the union of the frontiers has edges enough:
-      // a pull reads the rows of everything unreached however few roots it is
-      // for, a push the union's rows (S26, 2 of 64 roots over the line at 3 %
-      // of the edges: pull 4.7 ms, push of all 1.6; the least a pull pays at
-      // is 1/8 of the edges, at larger alpha 16/alpha).
+      // On graphs of kUnionFrom entries and more a level pulls only when the
+      // union of the frontiers has edges enough: a pull reads the rows of
+      // everything unreached however few roots it is for, a push the union's
+      // rows (S26, 2 of 64 roots over the line at 3 % of the edges: pull 4.7
+      // ms, push of all 1.6; the least a pull pays at is 1/8 of the edges, at
+      // larger alpha 16/alpha).
       const bool tail = total_pairs - reached < unseen_frac * total_pairs;
-      const bool enough = (double)fdeg * std::max(8.0, m.alpha / 16.0) > (double)g.nnz;
+      const bool enough = g.nnz < kUnionFrom || (double)fdeg * std::max(8.0, m.alpha / 16.0) > (double)g.nnz;
       for (int r = 0; r < 64; ++r) {
         const uint64_t bit = UINT64_C(1) << r;
         if (!(live & bit)) continue;
