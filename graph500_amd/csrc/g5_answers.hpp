@@ -21,11 +21,12 @@ struct HostOut {
   // less than the copy command it replaces (15-20 us with its kernel).
   static constexpr size_t kStageBytes = size_t(256) << 10;
   void* p = nullptr;  // the kernel's output, 16-byte aligned
-  // dev is used only for answers the GPU cannot store to the host itself
+  // dev is used only for answers the GPU does not store to the host itself:
+  // those for memory it cannot address, and those of more than `direct` bytes
   template <class T>
-  HostOut(T* host, size_t count, HostStage& stage, DevBuf<T>& dev, hipStream_t s)
+  HostOut(T* host, size_t count, HostStage& stage, DevBuf<T>& dev, hipStream_t s, size_t direct = SIZE_MAX)
       : host_(host), bytes_(count * sizeof(T)), s_(s) {
-    if (pinned(host, bytes_)) {
+    if (bytes_ <= direct && pinned(host, bytes_)) {
       p = host;
     } else if (bytes_ <= kStageBytes) {
       p = stage.get(kStageBytes);

@@ -2077,11 +2077,17 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
   b.have_result = true;
 }
 
+// Predecessors are 8 B an id, made faster than the link takes them, so large
+// ones are bound by the link alone: 53 GB/s of a kernel's stores, 57 of the
+// copy engine (S22/S24/S26: 664, 2,613 and 10,414 us stored, 646, 2,495 and
+// 10,040 copied; S18, S20 and S21 51, 174 and 337 against 60, 180 and 337).
+constexpr size_t kPredDirect = size_t(16) << 20;
+
 void bfs_get_pred(g5_ctx* ctx, int64_t* host_pred) {
   Graph& g = ctx->graph;
   BfsState& b = ctx->bfs;
   G5_CHECK(b.have_result, "g5_get_pred: no BFS result (call g5_run_bfs first)");
-  HostOut out(host_pred, (size_t)g.n, ctx->stage, b.pred_out, ctx->stream);
+  HostOut out(host_pred, (size_t)g.n, ctx->stage, b.pred_out, ctx->stream, kPredDirect);
   hipLaunchKernelGGL(k_make_pred, dim3(grid_of(g.n, kBlock, 65536)), dim3(kBlock), 0, ctx->stream,
                      g.old2new.p, g.new2old.p, b.level.p, b.parent.p, g.n, g.n_rows, b.root_orig, (int64_t*)out.p);
   G5_HIP(hipGetLastError());
