@@ -1277,7 +1277,7 @@ __device__ __forceinline__ uint64_t step_bottom_up(const StepArgs& a, BuLds<kWav
   const int first = share ? wave : 0, step = share ? kWaves : 1;
   const auto sync = [&] {
     if (share) __syncthreads();
-    else __builtin_amdgcn_wave_barrier();
+    else wave_sync();
   };
   for (int64_t turn = 0; turn * kWaves * gridDim.x * span < a.words; ++turn) {
     const int64_t base = word_of(turn, wave * kBuSpan), wl = base + lane;

@@ -15,6 +15,15 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return lane ? (~UINT64_C(0) >> (64 - lane)) : 0;
 }
 
+// What a lane has stored to LDS is there for the other lanes of its wave.  The
+// barrier alone orders the schedule, not memory: the fences keep the compiler
+// from moving an access of one lane past it (no instruction of their own).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Inclusive scan across the 64 lanes of a wave.
 __device__ __forceinline__ uint64_t wave_incl_scan(uint64_t v) {
   const int lane = threadIdx.x & 63;

@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(kValThreads) k_val_edges(const uint8_t* __rest
         off[i] = o <= k0 ? 0 : o - k0 < len ? (uint32_t)(o - k0) : len;
       }
       rl[lane] = v0 + lane < rows ? level[v0 + lane] : 0xFF;
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       const uint32_t end = off[64];
       int row = 0;  // the row of entry cur
       while (cur < end) {
@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(kValThreads) k_val_edges(const uint8_t* __rest
         }
         cur = cur + 64 * kValU < end ? cur + 64 * kValU : end;
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
     }
   }
   bad = wave_sum(bad);
