@@ -891,7 +891,7 @@ __global__ void __launch_bounds__(kBlock) k_make_levels(const uint32_t* __restri
   const int64_t stride = (int64_t)gridDim.x * kBlock;
   for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q * 16 < n; q += stride) {
     const int m = n < 16 ? (int)n : 16;  // n is a power of two
-    uint32_t nv[16];
+    alignas(16) uint32_t nv[16];
     if (m == 16) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -938,7 +938,7 @@ __global__ void __launch_bounds__(kTepsThreads) k_teps(const uint8_t* __restrict
   const int64_t stride = (int64_t)gridDim.x * kTepsThreads;
   for (int64_t q = (int64_t)blockIdx.x * kTepsThreads + threadIdx.x; q * 16 < rows; q += stride) {
     if (q * 16 + 16 <= rows) {
-      uint32_t l[4];
+      alignas(16) uint32_t l[4];
       *reinterpret_cast<uint4*>(l) = reinterpret_cast<const uint4*>(level)[q];
       uint4 w[4];
 #pragma unroll

@@ -602,7 +602,7 @@ __global__ void __launch_bounds__(kBlock) k_ms_row_levels(LevelWords lw, int64_t
       for (int j = 0; j < 4; ++j) {
         if (!(nz[j] & open)) continue;
         const uint64_t* f = lw.words(i0 + j) + v;
-        uint64_t x[4];
+        alignas(16) uint64_t x[4];
         if (m == 4) {
           *reinterpret_cast<ulonglong2*>(x) = *reinterpret_cast<const ulonglong2*>(f);
           *reinterpret_cast<ulonglong2*>(x + 2) = *reinterpret_cast<const ulonglong2*>(f + 2);

@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(kValThreads) k_val_edges(const uint8_t* __rest
                                                            const uint64_t* __restrict__ offsets,
                                                            const uint32_t* __restrict__ cols, int64_t rows, uint64_t nnz,
                                                            uint32_t run, unsigned long long* __restrict__ err) {
-  __shared__ uint8_t s_hot[kValHot];
+  __shared__ alignas(16) uint8_t s_hot[kValHot];  // filled 16 bytes at a time
   __shared__ uint32_t s_off[kValThreads / 64][65];  // row bounds, relative to the run
   __shared__ uint8_t s_lv[kValThreads / 64][64];
   __shared__ uint64_t s_bad;
