@@ -1735,8 +1735,8 @@ static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& s
   const double na = (double)g.n_active;
   unsigned long long* cnt = (unsigned long long*)b.counters.p;
   g5_bfs_stats& st = b.stats;
-  // the frontier's edges when the step summed them (-1: not known, both forms
-  // are launched and the device picks)
+  // the frontier's edges when the step or the level before summed them (-1:
+  // not known, both forms are launched and the device picks)
   const int64_t e_next = state.edges ? (int64_t)state.edges : -1;
   hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, s, b.stamp.p);
   device_scan(FrontierDegree{b.queue[qi].p, g.offsets.p, nf}, StoreU64{b.prefix.p},
@@ -1873,6 +1873,7 @@ static void large_top_down(g5_ctx* ctx, BfsState& b, hipStream_t s, StepState& s
   ++state.lvl;
   state.visited += nq;
   state.nf = nq;
+  state.edges = bulk ? 0 : b.h_counters[C_NEXT_E];  // a bulk level does not sum them
   if (nq == 0) return;
   // direction switch, mpi/bfs.hpp:2799-2829 (a top-down level hands over to bottom-up or goes on)
   if (state.growing && nq > state.prev_nq && (double)nq > na / 2000.0) state.forward = 0;
@@ -1895,6 +1896,7 @@ static void queue_from_bitmaps(BfsState& b, hipStream_t s, StepState& state) {
   device_scan(FrontierBits{now, before}, FrontierEmit{now, before, b.queue[state.qi].p}, (size_t)b.words, b.scan_tmp.p,
               s);
   state.queued = 1;
+  state.edges = 0;
 }
 
 // Bottom-up levels launched one by one, the next once the count of the last
@@ -2067,7 +2069,6 @@ void bfs_run(g5_ctx* ctx, BfsState& b, hipStream_t s, int64_t root) {
     resume = true;
     if (!state.queued && stop != STEP_BOTTOM_UP) queue_from_bitmaps(b, s, state);
     if (stop == STEP_LARGE) large_top_down(ctx, b, s, state);
-    state.edges = 0;
   }
   if (!root_active) {  // the level that finds nothing was not run
     st.num_levels = 2;
