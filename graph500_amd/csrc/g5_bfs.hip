@@ -991,7 +991,7 @@ constexpr int kStepNf = 4096;
 constexpr int kBuWords = 4;        // open words whose first probes are in flight together (bottom-up)
 constexpr int kBuSpan = 16;        // most words of a bottom-up turn
 constexpr int kStepList = 2048;    // LDS list of a workgroup's new vertices
-constexpr int kStepTdGrid = 256;   // workgroups of a top-down level: kTdSmall edges are 4,096 waves of 256
+constexpr int kStepMaxGrid = 256;  // most workgroups of a step: kTdSmall edges are 4,096 waves of 256
 constexpr int kStepMaxLevel = 254; // levels are bytes, 0xFF = unreached
 enum { STEP_GO = 0, STEP_DONE = 1, STEP_LARGE = 2, STEP_QUEUE = 3, STEP_LIMIT = 4, STEP_BOTTOM_UP = 5 };
 
@@ -1050,6 +1050,7 @@ __device__ __forceinline__ void step_publish_level(const StepArgs& a, uint64_t s
 // alone and 13 in 64 workgroups), the bitmap words beyond
 // which bottom-up levels go back to the host, and the steps launched ahead.
 constexpr unsigned kStepMinGrid = 64;
+static_assert(kStepMinGrid <= (unsigned)kStepMaxGrid, "workgroups of a step");
 constexpr int64_t kStepAloneWords = 32;
 constexpr int64_t kStepShareWords = 8192;  // see step_bottom_up
 constexpr int64_t kStepAloneEdges = 1 << 18;
@@ -1409,7 +1410,6 @@ __global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* _
       else if (td && L.st.nf > kStepNf) stop = STEP_LARGE;
       else if (!td && a.host_bu) stop = STEP_BOTTOM_UP;
       if (!stop && td) {
-        if (blockIdx.x >= kStepTdGrid) return;
         E = step_prefix(L, a.queue[L.st.qi], (int)L.st.nf, a.offsets);
         if (E > kTdSmall) stop = STEP_LARGE;
       }
@@ -1459,7 +1459,7 @@ __global__ void __launch_bounds__(kStepThreads) k_bfs_step(unsigned long long* _
       }
       // consecutive stretches go to different workgroups, so that the winners
       // spread over their lists (past a full list each costs a global atomic)
-      const uint32_t nblk = gridDim.x < kStepTdGrid ? gridDim.x : kStepTdGrid;
+      const uint32_t nblk = gridDim.x;
       for (uint32_t c = wave * nblk + blockIdx.x; (uint64_t)c * 256 < E; c += nblk * (kStepThreads / 64)) {
         const uint64_t end = (uint64_t)(c + 1) * 256 < E ? (uint64_t)(c + 1) * 256 : E;
         step_expand(a, L, nf, vis, c * 256 + lane, (uint32_t)end, 64, lvl, [&](uint32_t w) {
@@ -1607,15 +1607,15 @@ __global__ void __launch_bounds__(kBlock) k_bfs_init(const uint32_t* __restrict_
   }
 }
 
+__global__ void k_stamp(uint64_t* stamp) { *stamp = wall_clock64(); }  // a level starts
+
 // Level end: the counters the host decides the next level with (and the
 // level's frontier edge count after a top-down level) are published straight
 // into coherent host memory, each tagged with the level's sequence number, so
-// the host need not wait for a copy and a stream synchronisation.
-// One wave: lane i takes stripe i.
+// the host need not wait for a copy and a stream synchronisation; behind them
+// the time since the level's stamp (an event on either side of a level took 7
+// us of the stream).  One wave: lane i takes stripe i.
 static_assert(kStripes == 64, "k_publish sums one stripe per lane of a wave");
-// The time since the level's stamp is published behind the counters (an event
-// on either side of a level took 7 us of the stream).
-__global__ void k_stamp(uint64_t* stamp) { *stamp = wall_clock64(); }
 __global__ void __launch_bounds__(64) k_publish(unsigned long long* __restrict__ counters,
                                                 const uint64_t* __restrict__ prefix, int64_t nf, int forward,
                                                 Published* pub, uint64_t seq,
@@ -1933,9 +1933,7 @@ static void host_bottom_up(g5_ctx* ctx, BfsState& b, hipStream_t s, const StepAr
   if (state.nf && state.forward) queue_from_bitmaps(b, s, state);
 }
 
-// Workgroups of a step: one for the smallest graphs; else enough waves for a
-// turn of every wave in a bottom-up level, and at least kStepMinGrid for the
-// top-down levels.
+// One workgroup takes the whole search of the smallest graphs.
 static bool step_alone(const Graph& g, const BfsState& b) {
   return b.words <= kStepAloneWords && g.nnz <= kStepAloneEdges;
 }
@@ -1945,13 +1943,16 @@ static bool step_alone(const Graph& g, const BfsState& b) {
 static int bottom_up_span(const Graph& g, const BfsState& b) {
   if (b.words == 0) return 1;  // a graph without rows has no turns to share out
   if (b.words > kStepMaxWords) return b.words >= (INT64_C(1) << 20) ? 16 : 8;
-  const int64_t waves = (step_alone(g, b) ? 1 : kStepTdGrid) * (kStepThreads / 64);
+  const int64_t waves = (step_alone(g, b) ? 1 : kStepMaxGrid) * (kStepThreads / 64);
   const int64_t turns = (b.words + waves * kBuSpan - 1) / (waves * kBuSpan);
   return (int)((b.words + waves * turns - 1) / (waves * turns));
 }
+// Workgroups of a step: one for the smallest graphs; else enough waves for a
+// turn of every wave in a bottom-up level, and at least kStepMinGrid for the
+// top-down levels.
 static unsigned step_grid(const Graph& g, const BfsState& b, int span) {
   if (step_alone(g, b)) return 1;
-  return std::max(kStepMinGrid, grid_of((b.words + span - 1) / span, kStepThreads / 64, kStepTdGrid));
+  return std::max(kStepMinGrid, grid_of((b.words + span - 1) / span, kStepThreads / 64, kStepMaxGrid));
 }
 
 // Steps until one stops; returns its state (see k_bfs_step).  k counts the

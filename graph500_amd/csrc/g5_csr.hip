@@ -32,8 +32,9 @@ __device__ __forceinline__ uint64_t tuple_v1(const g5_packed_edge& e) {
   return (uint64_t)e.v1_low | ((uint64_t)(e.high >> 16) << 32);
 }
 
-// One atomic per workgroup, and none once the bits are there: a wave's OR per
-// wave of a 65,536-workgroup grid spent 3 ms on that one word (12 ns each).
+// The OR of all ids, by workgroup: each publishes its own to the host, which
+// combines them (atomics by every wave of a 65,536-workgroup grid spent 3 ms on
+// one word, 12 ns each).
 __global__ void __launch_bounds__(kBlock) k_or_ids(const g5_packed_edge* __restrict__ e, int64_t m,
                                                    Published* __restrict__ pub, uint64_t seq) {
   __shared__ uint64_t s_or[kBlock / 64];
@@ -150,7 +151,7 @@ __global__ void k_first_nbr(const uint64_t* __restrict__ offsets, const uint32_t
   }
 }
 
-// has_edge bitmap by original id (one wave writes one 64-bit word).
+// has_edge bitmap by original id.
 __global__ void __launch_bounds__(kBlock) k_has_edge_bits(const uint32_t* __restrict__ deg, int64_t n,
                                                           uint64_t* __restrict__ words,
                                                           const unsigned long long* __restrict__ info,

@@ -126,25 +126,6 @@ __device__ __forceinline__ int stage_chunk(uint64_t c, const uint32_t* __restric
   return cnt;
 }
 
-// Calls f(target, source) for this lane's kEpt consecutive edges of [e0, e1):
-// one LDS binary search, then a forward walk across row boundaries.
-template <class F>
-__device__ __forceinline__ void walk_lane(uint64_t e0, uint64_t e1, int cnt, const ChunkRows& cr,
-                                          const uint32_t* __restrict__ cols, F&& f) {
-  const uint64_t my0 = e0 + (uint64_t)threadIdx.x * kEpt;
-  if (my0 >= e1) return;
-  int lo = 0, hi = cnt - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cr.pre[mid] <= my0) lo = mid; else hi = mid - 1;
-  }
-  const uint64_t my1 = (my0 + kEpt < e1) ? my0 + kEpt : e1;
-  for (uint64_t e = my0; e < my1; ++e) {
-    while (lo + 1 < cnt && cr.pre[lo + 1] <= e) ++lo;
-    f(cols[cr.base[lo] + e], cr.src[lo]);
-  }
-}
-
 // Calls f(target, source) for the edges e0 + threadIdx.x + j * kBlock of
 // [e0, e1): consecutive lanes take consecutive edges, so a wave reads 256
 // contiguous bytes of cols per step and, within a sorted hub row, probes

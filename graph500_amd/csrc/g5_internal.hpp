@@ -10,7 +10,7 @@
 //                 (non-loop degree + 2 * self loops) for the TEPS count
 //   old2new, new2old : uint32[n]
 //   BFS state   : visited bitmaps uint64[2][W], level uint8[n_active],
-//                 parent uint32[n_active], frontier queues uint32[2][n_active]
+//                 parent uint32[n_active], frontier queues uint32[3][n_active]
 #pragma once
 
 #include <utility>
@@ -47,8 +47,6 @@ struct Error {
   do {                                                        \
     if (!(cond)) throw ::g5::Error{std::string(text), (code)}; \
   } while (0)
-
-constexpr int kWave = 64;
 
 // ---------------------------------------------------------------------------
 // Device memory (g5_pool.hip): hipMalloc with freed blocks kept for reuse, at

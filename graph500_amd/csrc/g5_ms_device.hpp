@@ -99,14 +99,9 @@ __device__ __forceinline__ void ms_block_counters(uint64_t live, uint64_t pairs,
 }
 
 
-// Vertices of the frontier union (set bits of the nonzero bitmap) -> queue,
-// ascending, through a scan of per-word popcounts.
-struct UnionCount {
-  const uint64_t* nz;
-  __device__ uint64_t operator()(size_t w) const { return (uint64_t)__popcll(nz[w]); }
-};
-// The same over words [0, words) with one more element whose prefix, the
-// total, goes to *count.
+// Set bits of a bitmap -> list, ascending, through a scan of the popcounts of
+// words [0, words) with one more element whose prefix, the total, goes to
+// *count.
 struct BitsCountN {
   const uint64_t* bits;
   int64_t words;
@@ -129,19 +124,6 @@ struct BitsEmitN {
     }
   }
 };
-struct UnionEmit {
-  const uint64_t* nz;
-  uint32_t* queue;
-  __device__ void operator()(size_t w, uint64_t pre) const {
-    uint64_t x = nz[w];
-    while (x) {
-      queue[pre++] = (uint32_t)(w * 64 + __builtin_ctzll(x));
-      x &= x - 1;
-    }
-  }
-};
-
-
 // Per-level hooks of the finish and pull steps.  keep: lanes of seen that
 // stay (the others belong to finished searches and are cleared on the way);
 // epi(v, inb, nw): called by every lane of a wave with its vertex's new lanes;
@@ -454,15 +436,16 @@ __device__ __forceinline__ uint64_t ms_pull_probe(const FrontView& fv, int64_t v
   return acc;
 }
 
-// kU: independent probes per step of a lane's short row; kW: entries per lane
-// and step of the wave's scan of a long row (kW x 64 per step).
+// A turn's bits (one per row) to their place in a bitmap of 64-bit words.
 template <int kRows>
 __device__ __forceinline__ void store_bits(uint64_t* words, int64_t turn, uint64_t bits) {
   if (kRows == 64) words[turn] = bits;
   else reinterpret_cast<uint16_t*>(words)[turn] = (uint16_t)bits;
 }
 
-// A wave takes kRows rows a turn.
+// kU: independent probes per step of a lane's short row; kW: entries per lane
+// and step of the wave's scan of a long row (kW x 64 per step).  A wave takes
+// kRows rows a turn.
 template <class Epi = NoEpilogue, int kU = 4, int kW = 2, int kRows = 64>
 __device__ __forceinline__ void ms_pull_body(uint64_t* __restrict__ seen, const FrontView fv,
                                              uint64_t* __restrict__ next, uint64_t* __restrict__ nz_next,

@@ -84,7 +84,6 @@ __global__ void k_ms_roots(const uint32_t* __restrict__ old2new, const int64_t* 
   }
 }
 
-// Level-0 nonzero bitmap: the root vertices (lane r, root r).
 // The roots of a level-by-level batch, in the argument block.
 struct MsRoots {
   int64_t root[64];
@@ -142,6 +141,7 @@ __global__ void __launch_bounds__(64) k_ms_place(const uint32_t* __restrict__ ol
   if (r < M_NUM) publish(pub + r, r == M_LIVE ? live : r == M_NZ ? nz : r == M_FDEG ? fdeg : 0, seq);
 }
 
+// Level-0 nonzero bitmap: the root vertices (lane r, root r).
 __global__ void k_ms_roots_nz(const uint32_t* __restrict__ old2new, const int64_t* __restrict__ roots, int nroots,
                               int64_t rows, uint64_t* __restrict__ nz0) {
   const int r = threadIdx.x;

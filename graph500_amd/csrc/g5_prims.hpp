@@ -172,28 +172,6 @@ __global__ void __launch_bounds__(kBlock) k_reduce_sum(In in, size_t n, unsigned
   }
 }
 
-template <class In>
-__global__ void __launch_bounds__(kBlock) k_reduce_max(In in, size_t n, unsigned long long* d_out) {
-  __shared__ uint64_t s_wave[kBlock / 64];
-  uint64_t m = 0;
-  for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
-    const uint64_t v = in(i);
-    m = v > m ? v : m;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint64_t t = __shfl_xor(m, o, 64);
-    m = t > m ? t : m;
-  }
-  if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t t = 0;
-    for (int w = 0; w < kBlock / 64; ++w) t = s_wave[w] > t ? s_wave[w] : t;
-    atomicMax(d_out, (unsigned long long)t);
-  }
-}
-
 inline unsigned reduce_grid(size_t n) {
   size_t b = (n + kBlock - 1) / kBlock;
   if (b > 2048) b = 2048;
@@ -206,20 +184,6 @@ uint64_t device_reduce_sum(In in, size_t n, uint64_t* d_acc, hipStream_t s) {
   G5_HIP(hipMemsetAsync(d_acc, 0, sizeof(uint64_t), s));
   if (n) {
     hipLaunchKernelGGL(k_reduce_sum<In>, dim3(reduce_grid(n)), dim3(kBlock), 0, s, in, n,
-                       (unsigned long long*)d_acc);
-    G5_HIP(hipGetLastError());
-  }
-  uint64_t h = 0;
-  G5_HIP(hipMemcpyAsync(&h, d_acc, sizeof(h), hipMemcpyDeviceToHost, s));
-  G5_HIP(hipStreamSynchronize(s));
-  return h;
-}
-
-template <class In>
-uint64_t device_reduce_max(In in, size_t n, uint64_t* d_acc, hipStream_t s) {
-  G5_HIP(hipMemsetAsync(d_acc, 0, sizeof(uint64_t), s));
-  if (n) {
-    hipLaunchKernelGGL(k_reduce_max<In>, dim3(reduce_grid(n)), dim3(kBlock), 0, s, in, n,
                        (unsigned long long*)d_acc);
     G5_HIP(hipGetLastError());
   }
