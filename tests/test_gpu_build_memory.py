@@ -34,12 +34,14 @@ def test_peak_is_two_key_arrays(hip):
         # the columns (about 8 m bytes) do not fit beside the keys
         leave = 32 * m + 48 * n - 12 * m
         try:
-            each = (free_bytes(hip) - leave) // 8
-            for _ in range(8):
+            # in pieces, to within 1.5 GB (the unfreed key array would need 2.1 more than there is)
+            while (left := free_bytes(hip) - leave) > 3 << 29:
                 p = ctypes.c_void_p()
-                assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(each)) == 0
+                if hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(max(1 << 30, left // 4))) != 0:
+                    pytest.skip("the device's free memory cannot be had in pieces")
                 held.append(p)
-            print("held", 8 * each, "free", free_bytes(hip), flush=True)
+            print("held in", len(held), "free", free_bytes(hip), flush=True)
+            assert left >= 0
             ctx.construct(2, release_edges=True)
             info = ctx.graph_info()
         finally:
