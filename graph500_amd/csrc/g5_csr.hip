@@ -349,22 +349,24 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     uint32_t *kp = k0.p, *ka = k1.p, *vp = g.new2old.p, *va = v1.p;
     radix_sort_pairs_u32(&kp, &ka, &vp, &va, (size_t)n, 0, bits, rs, s);
     if (vp != g.new2old.p) g.new2old.swap(v1);
+    if (!small) {  // the memory is needed below
+      G5_HIP(hipStreamSynchronize(s));
+      k0.drop();
+      k1.drop();
+      v1.drop();
+    }
   }
   const int64_t rows = g.n_rows;
   g.weight.alloc(rows);
+  g.offsets.alloc(rows + 1);
   DevBuf<uint32_t> row_cnt;  // degrees with duplicates, then unique entries per row
+  DevBuf<uint64_t> P, tmp;   // degree prefix: P[r] = entries of the rows before r
   row_cnt.alloc(rows + 1);
+  P.alloc(rows + 1);
+  tmp.alloc(scan_tmp_elems(rows + 1));
   hipLaunchKernelGGL(k_row_info, dim3(grid_for(rows + 1)), dim3(kBlock), 0, s, g.new2old.p, deg.p,
                      g.self_loops ? loops.p : nullptr, rows, row_cnt.p, g.weight.p);
   G5_HIP(hipGetLastError());
-  if (!small) {  // the memory is needed below
-    G5_HIP(hipStreamSynchronize(s));
-    for (DevBuf<uint32_t>* b : {&k0, &k1, &v1, &deg, &loops}) b->drop();
-  }
-  g.offsets.alloc(rows + 1);
-  DevBuf<uint64_t> P, tmp;  // degree prefix: P[r] = entries of the rows before r
-  P.alloc(rows + 1);
-  tmp.alloc(scan_tmp_elems(rows + 1));
   device_scan(LoadU32{row_cnt.p}, StoreU64{P.p}, (size_t)rows + 1, tmp.p, s);
   DevBuf<uint64_t> row_word;
   row_word.alloc(n);
@@ -374,20 +376,29 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
 
   // 4. entries to sorted, deduplicated rows
   const uint64_t E = (uint64_t)g.directed_before;
-  xb.alloc(nkeys);
+  // Where the device is short, a request is tried again once the scratch that
+  // no later pass reads has gone back; else that stays to the end, from where
+  // the next construction takes it (given back earlier, it left the pool in an
+  // order in which a repeated SCALE 26 build waits for the driver to clear
+  // memory: 100 ms, then 0.4-1.5 s).
+  std::vector<DevBuf<uint32_t>*> idle32{&deg, &loops};
+  std::vector<DevBuf<uint64_t>*> idle64;
+  const auto alloc = [&](auto& buf, size_t count) {
+    try {
+      buf.alloc(count);
+    } catch (const Error& err) {
+      if (err.code != G5_ERR_MEM) throw;
+      G5_HIP(hipStreamSynchronize(s));
+      for (DevBuf<uint32_t>* b : idle32) b->drop();
+      for (DevBuf<uint64_t>* b : idle64) b->drop();
+      buf.alloc(count);
+    }
+  };
+  alloc(xb, nkeys);
   uint64_t nnz = 0;
   DevBuf<uint64_t> sub64;  // first position | first entry | first unique column
   DevBuf<uint32_t> sub32;  // entries | first row | unique columns | L1 first sub-buckets | column shares
   DevBuf<uint64_t> stmp;
-  // Before the columns are allocated: all scratch but the sorted entries in
-  // `kept`, once nothing in flight reads it (at SCALE 28, edgefactor 16, the
-  // peak is 145 GB instead of 181).
-  const auto drop_idle = [&](const uint64_t* kept) {
-    if (small) return;
-    (kept == xa.p ? xb : xa).drop();
-    row_word.drop();
-    P.drop();
-  };
   if (E == 0) {
     g.cols.alloc(0);
     G5_HIP(hipMemsetAsync(g.offsets.p, 0, (rows + 1) * 8, s));
@@ -395,8 +406,8 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     const int sub = sub_shift_for(E), wshift = l1_shift(E, sub);
     const int nb1 = (int)(((E - 1) >> wshift) + 1);
     const size_t max_subs = (size_t)(E >> sub) + nb1 + 1;
-    sub64.alloc(3 * (max_subs + 1));
-    sub32.alloc(3 * max_subs + kPartMax + 1 + kFracMax);
+    alloc(sub64, 3 * (max_subs + 1));
+    alloc(sub32, 3 * max_subs + kPartMax + 1 + kFracMax);
     uint64_t *sub_pos = sub64.p, *sub_off = sub_pos + max_subs + 1, *out_off = sub_off + max_subs + 1;
     uint32_t *sub_cnt = sub32.p, *sub_row = sub_cnt + max_subs, *sub_unique = sub_row + max_subs;
     uint32_t *l1_sub0 = sub_unique + max_subs, *frac = l1_sub0 + kPartMax + 1;
@@ -438,7 +449,7 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
       hipLaunchKernelGGL(k_sort_sub<12>, dim3((unsigned)max_subs), dim3(SubSort<12>::kThreads), 0, s, refined, sub_off,
                          sub_cnt, sub_pos, sub_row, P.p, rows, row_cnt.p, sub_unique, info);
     G5_HIP(hipGetLastError());
-    stmp.alloc(scan_tmp_elems(max_subs));
+    alloc(stmp, scan_tmp_elems(max_subs));
     device_scan(LoadU32{row_cnt.p}, StoreU64{g.offsets.p}, (size_t)rows + 1, tmp.p, s);
     device_scan(LoadU32{sub_unique}, StoreU64{out_off}, max_subs, stmp.p, s);
     hipLaunchKernelGGL(k_publish_info, dim3(1), dim3(64), 0, s, info, g.offsets.p + rows, pub.d + kPubOr + I_NUM + 1,
@@ -447,8 +458,8 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
     read_info(kPubOr + I_NUM + 1, I_NUM + 1);
     nnz = pub.value(kPubOr + 2 * I_NUM + 1);
     if (!h_info[I_WIDE] && !h_info[I_OVERFLOW]) {
-      drop_idle(refined);
-      g.cols.alloc(nnz);
+      idle64 = {refined == xa.p ? &xb : &xa, &row_word, &P, &tmp};
+      alloc(g.cols, nnz);
       hipLaunchKernelGGL(k_compact, dim3((unsigned)max_subs), dim3(kBlock), 0, s, refined, sub_off, sub_unique, out_off,
                          info, g.cols.p);
       G5_HIP(hipGetLastError());
@@ -463,9 +474,9 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
       radix_sort_u64(&kp, &ka, E, 32, 32 + scale, rs, s);
       const UniqueFlag flag{kp, (size_t)E};
       nnz = device_reduce_sum(flag, E, ctx->acc.p, s);
-      drop_idle(kp);
-      g.cols.alloc(nnz);
-      stmp.alloc(scan_tmp_elems(E));
+      idle64 = {kp == xa.p ? &xb : &xa, &row_word, &P, &tmp};
+      alloc(g.cols, nnz);
+      alloc(stmp, scan_tmp_elems(E));
       device_scan(flag, UniqueStore{kp, (size_t)E, 32, g.cols.p, g.offsets.p}, E, stmp.p, s);
       hipLaunchKernelGGL(k_offsets_tail, dim3(grid_for(rows)), dim3(kBlock), 0, s, kp, (size_t)E, 32, rows, nnz,
                          g.offsets.p);
@@ -474,7 +485,9 @@ void build_graph(g5_ctx* ctx, int mode, bool release_edges) {
   }
   g.nnz = (int64_t)nnz;
 
-  g.first_nbr.alloc(rows);
+  idle32 = {&deg, &loops, &row_cnt, &sub32};
+  idle64 = {&xa, &xb, &row_word, &P, &tmp, &sub64, &stmp};
+  alloc(g.first_nbr, rows);
   hipLaunchKernelGGL(k_first_nbr, dim3(grid_for(rows)), dim3(kBlock), 0, s, g.offsets.p, g.cols.p,
                      rows, g.first_nbr.p);
   G5_HIP(hipGetLastError());
