@@ -367,13 +367,13 @@ constexpr int64_t kListGrid = 2048;
 constexpr int64_t kPartWords = 4096;
 constexpr int64_t kPartWordsFirst = 12288;
 
-// Below this many entries a level costs its launches, two for a pull and four
-// for a push, and a root pulls by its own frontier alone (lane_rule 1): long
-// graphs never have a union large enough (2 and 8 roots, us, with the union
-// rule and without: a path of 200 6,214 / 6,047 and 3,382 / 4,142, 128 x 1,024
-// vertices in a grid with chords 3,998 / 7,038 and 2,811 / 3,838), Kronecker
-// graphs up to S18 are equal; S19 with 8 roots 218 with, 251 without, S23 811
-// and 894.
+// Below this many entries a root waits for the union one level only (lane_rule
+// 1): a level costs its launches there, two for a pull and four for a push,
+// and long graphs never have a union large enough (2 and 8 roots, us, waiting
+// and not: a path of 200 6,214 / 6,047 and 3,467 / 4,254, 128 x 1,024 vertices
+// in a grid with chords 3,998 / 7,038 and 2,834 / 3,771).  The one level stays
+// for graphs that grow: from the next on their union is large enough, and a
+// mixed level in between costs S14 to S18 5 to 8 %.
 constexpr int64_t kUnionFrom = INT64_C(1) << 22;
 
 // A push level lists the vertices it touches when its frontier edges times
@@ -1016,7 +1016,8 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
   const bool lanes_mode = m.lane_rule == 1 && m.sweep_chunks && l0 == 1;
   m.level_masks = lanes_mode;
   double lane_fd[64] = {}, lane_vd[64] = {};
-  uint64_t pulled = 0;  // roots that have pulled: they pull from then on
+  uint64_t pulled = 0;   // roots that have pulled: they pull from then on
+  uint64_t waiting = 0;  // roots over their own threshold that pushed the last level
   const uint64_t* h_lane = m.h_counters.data() + kMsLanes;
   unsigned* d_list_count = (unsigned*)(cnt + M_NUM);
   // turns of a pull that takes 16 rows each up to `limit` words
@@ -1053,20 +1054,24 @@ static void ms_host_levels(g5_ctx* ctx, int l0, uint64_t live, uint64_t nz, uint
       // reached (the roots' own level pushes; all pull in the beta tail); a
       // root that has pulled keeps pulling, so once every live root pulls
       // the level is a plain pull with no per-root statistics
-      // On graphs of kUnionFrom entries and more a level pulls only when the
-      // union of the frontiers has edges enough: a pull reads the rows of
-      // everything unreached however few roots it is for, a push the union's
-      // rows (S26, 2 of 64 roots over the line at 3 % of the edges: pull 4.7
-      // ms, push of all 1.6; the least a pull pays at is 1/8 of the edges, at
-      // larger alpha 16/alpha).
+      // A level pulls only when the union of the frontiers has edges enough:
+      // a pull reads the rows of everything unreached however few roots it is
+      // for, a push the union's rows (S26, 2 of 64 roots over the line at 3 %
+      // of the edges: pull 4.7 ms, push of all 1.6; the least a pull pays at
+      // is 1/8 of the edges, at larger alpha 16/alpha).  Below kUnionFrom
+      // entries a root that has waited a level for that pulls.
       const bool tail = total_pairs - reached < unseen_frac * total_pairs;
-      const bool enough = g.nnz < kUnionFrom || (double)fdeg * std::max(8.0, m.alpha / 16.0) > (double)g.nnz;
+      const bool enough = (double)fdeg * std::max(8.0, m.alpha / 16.0) > (double)g.nnz;
+      const uint64_t waited = g.nnz < kUnionFrom ? waiting : 0;
+      waiting = 0;
       for (int r = 0; r < 64; ++r) {
         const uint64_t bit = UINT64_C(1) << r;
         if (!(live & bit)) continue;
         const double unreached = (double)g.nnz - lane_vd[r];
-        const bool pull_r = tail || (pulled & bit) || (l > 1 && enough && lane_fd[r] * m.alpha > unreached);
+        const bool over = l > 1 && lane_fd[r] * m.alpha > unreached;
+        const bool pull_r = tail || ((pulled | waited) & bit) || (over && enough);
         (pull_r ? bu : td) |= bit;
+        if (over && !pull_r) waiting |= bit;
       }
       pulled |= bu;
       push = bu == 0;

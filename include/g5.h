@@ -125,10 +125,10 @@ typedef struct g5_batch_tuning {
   int32_t lane_rule;       /* 0: one direction per level for all roots (the rule on alpha above);
                               1: a direction per root and level (per-level launches, reorder modes
                               1 and 2): a root pulls when its frontier's edges exceed 1/alpha of the
-                              edges of the vertices it has not reached, and, on graphs of 2^22
-                              directed entries and more, those of all frontiers together
-                              1/max(8, alpha/16) of the graph's, else pushes; a level with
-                              both kinds pushes first, then pulls and merges */
+                              edges of the vertices it has not reached, and those of all frontiers
+                              together 1/max(8, alpha/16) of the graph's (on graphs of fewer than
+                              2^22 directed entries it waits one level for that), else pushes; a
+                              level with both kinds pushes first, then pulls and merges */
   double compact_below;    /* per-level pulls (persistent = 0) read frontier words from a compact
                               copy holding only the frontier's words when the frontier spans fewer
                               than compact_below x rows vertices; 0 disables */

@@ -1,6 +1,6 @@
-"""Which levels of a batch pull, on both sides of the size from which the
-union of the frontiers decides with each root's own frontier; levels against
-the oracle either way."""
+"""Which levels of a batch pull, on both sides of the size from which a root
+that is over its own threshold waits for the union of the frontiers for good;
+levels against the oracle either way."""
 import numpy as np
 import pytest
 
@@ -27,8 +27,8 @@ def run(ctx, oc, roots):
 @pytest.mark.parametrize("n,w", [(200, 1), (120, 4), (200, 4)])
 @pytest.mark.parametrize("nroots", [2, 8])
 def test_long_small_graphs_pull(oracle_mod, n, w, nroots):
-    """A frontier of a few vertices of a small graph: once a root pulls it
-    keeps pulling, as its own frontier says."""
+    """A frontier of a few vertices of a small graph: a root waits one level
+    for the union, pulls, and keeps pulling."""
     import graph500_amd
     print("grid", n, w, nroots, flush=True)
     a, b = grid(n, w)
@@ -42,17 +42,39 @@ def test_long_small_graphs_pull(oracle_mod, n, w, nroots):
         assert d.count(PULL) >= len(d) - 8
 
 
-@pytest.mark.parametrize("scale,mixed", [(16, True), (19, False)])
-def test_union_decides_on_large_graphs(oracle_mod, scale, mixed):
-    """8 roots, of which some are over their own threshold at level 2 where
-    the union of all is below its own: the small graph pulls for them, the
-    large one pushes for all."""
+@pytest.mark.parametrize("w,large", [(1024, False), (8192, True)])
+def test_large_graphs_wait(oracle_mod, w, large):
+    """Two roots in a grid with chords, 110 to 145 levels: the small graph
+    pulls for them most of the time, the large one pushes."""
+    import graph500_amd
+    print("chords", w, flush=True)
+    a, b = grid(128, w)
+    i = np.arange(128 * w)
+    at = i[i // 128 % 16 == 0]
+    rng = np.random.default_rng(3)
+    a = np.concatenate([a, at])
+    b = np.concatenate([b, (at + 128 * 16 * rng.integers(0, w // 16, len(at))) % (128 * w)])
+    t = np.zeros(len(a), graph500_amd.EDGE_DTYPE)
+    t["v0_low"], t["v1_low"] = a, b
+    with graph500_amd.G5Context(0) as ctx:
+        ctx.edges_append(t)
+        ctx.construct(2)
+        assert (ctx.graph_info()["nnz"] >= 1 << 22) == large
+        d = run(ctx, oracle_mod.Csr(t), ctx.find_roots(2, 7, 3))
+        assert len(d) > 90
+        assert d.count(PUSH) > 0.8 * len(d) if large else d.count(PUSH) < 0.4 * len(d)
+
+
+@pytest.mark.parametrize("scale", [14, 16, 19])
+def test_growing_graphs_wait_one_level(oracle_mod, scale):
+    """8 roots of a Kronecker graph, of which some are over their own threshold
+    at level 2 where the union of all is below its own, and no longer at level
+    3: all push at level 2, no mixed level."""
     import graph500_amd
     print("scale", scale, flush=True)
     with graph500_amd.G5Context(0) as ctx:
-        ctx.generate_kronecker(scale, 16, 5, 9)
+        ctx.generate_kronecker(scale, 16, 2, 3)
         t = ctx.edges_download()
         ctx.construct(2)
-        assert (ctx.graph_info()["nnz"] < 1 << 22) == mixed
-        d = run(ctx, oracle_mod.Csr(t), ctx.find_roots(8, 7, 3))
-        assert d[0] == PUSH and (d[1] == PUSH) != mixed
+        d = run(ctx, oracle_mod.Csr(t), ctx.find_roots(4 if scale == 16 else 8, 7, 3))
+        assert d[:3] == [PUSH, PUSH, PULL]
