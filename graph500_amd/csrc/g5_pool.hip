@@ -18,6 +18,7 @@
 
 #include <list>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 
 namespace g5 {
@@ -102,8 +103,13 @@ hipError_t pool_alloc(void** p, size_t bytes) {
     }
   }
   if (e == hipSuccess) {
-    std::lock_guard<std::mutex> lk(g_mu);
-    g_live[*p] = {bytes, dev};
+    try {
+      std::lock_guard<std::mutex> lk(g_mu);
+      g_live[*p] = {bytes, dev};
+    } catch (const std::bad_alloc&) {
+      (void)hipFree(*p);
+      e = hipErrorOutOfMemory;
+    }
   }
   return e;
 }
@@ -123,10 +129,20 @@ void pool_free(void* p, bool idle) {
       keep = pl.contexts > 0 && b.bytes <= pl.limit;
     }
   }
+  // the list's entry: without host memory the block goes back at once (this
+  // runs in destructors)
+  std::list<Block> entry;
+  if (keep) {
+    try {
+      entry.push_back({p, b.bytes});
+    } catch (const std::bad_alloc&) {
+      keep = false;
+    }
+  }
   if (keep && (idle || hipDeviceSynchronize() == hipSuccess)) {
     Pool& pl = g_pool[b.device];
     const auto add = [&] {
-      pl.kept.push_back({p, b.bytes});
+      pl.kept.splice(pl.kept.end(), entry);
       pl.total += b.bytes;
     };
     {

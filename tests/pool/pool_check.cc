@@ -8,6 +8,17 @@
 #include <future>
 #include <map>
 #include <mutex>
+#include <new>
+
+// Host allocations fail while this is set.
+static bool no_memory;
+void* operator new(size_t n) {
+  void* p = no_memory ? nullptr : malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 namespace {
 
@@ -19,6 +30,7 @@ int mallocs, frees, waits;
 thread_local int device;
 thread_local hipError_t last;
 uintptr_t next_p = 0x1000;
+bool fail_after_malloc;  // host memory ends with the next device allocation
 std::function<void()> on_wait;  // runs while a call waits for the device (a free waits for it too)
 
 void wait_for_device() {
@@ -38,6 +50,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   next_p += 0x1000;
   blocks[*p] = bytes;
   used += bytes;
+  no_memory = fail_after_malloc;
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
@@ -196,6 +209,32 @@ static void threads() {
   CHECK(used <= 50);  // what the other thread may have kept before the context was gone
 }
 
+// Without host memory a returned block goes to the driver (it comes from
+// destructors: an exception there ends the process), and so does a new one that
+// cannot be entered: the request fails as one for device memory.
+static void host_memory() {
+  pool_context(0, 1);
+  void *a = get(500), *b = get(600);
+  no_memory = true;
+  pool_free(a);
+  no_memory = false;
+  CHECK(blocks.count(a) == 0 && used == 600);
+  void *c = get(500), *d = get(500);
+  pool_free(c);
+  no_memory = true;
+  pool_free(d, true);  // where an older block would have to go back for it
+  no_memory = false;
+  CHECK(blocks.count(d) == 0 && blocks.count(c) == 1);
+  fail_after_malloc = true;
+  void* e = nullptr;
+  const hipError_t rc = pool_alloc(&e, 450 + 300);
+  no_memory = fail_after_malloc = false;
+  CHECK(rc == hipErrorOutOfMemory && used == 1100);
+  CHECK(get(500) == c);
+  pool_free(b);
+  pool_free(c);
+}
+
 // The wrapper: a buffer that cannot be had is an error of the library, and
 // what it held before has gone back.
 static void buffer() {
@@ -219,7 +258,7 @@ int main(int argc, char** argv) {
     const char* name;
     void (*f)();
   } checks[] = {{"sizes", sizes}, {"bound", bound}, {"refill", refill}, {"contexts", contexts}, {"buffer", buffer},
-                {"threads", threads}};
+                {"threads", threads}, {"host_memory", host_memory}};
   for (const auto& c : checks)
     if (argc > 1 && !strcmp(argv[1], c.name)) {
       c.f();

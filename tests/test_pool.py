@@ -1,7 +1,8 @@
 """The pool of freed device blocks, built for the CPU over a device that is
 only bookkeeping (tests/pool): which requests reuse a block, the bound on what
-is kept, what a request the device cannot fill does, when all goes back, and
-that no thread waits for another's wait for the device."""
+is kept, what a request the device cannot fill does, when all goes back, that
+no thread waits for another's wait for the device, and what happens without
+host memory."""
 import os
 import subprocess
 
@@ -20,7 +21,7 @@ def binary(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["sizes", "bound", "refill", "contexts", "buffer", "threads"])
+@pytest.mark.parametrize("check", ["sizes", "bound", "refill", "contexts", "buffer", "threads", "host_memory"])
 def test_pool(binary, check):
     r = subprocess.run([binary, check], capture_output=True, text=True, timeout=20)
     assert r.returncode == 0, r.stderr
